@@ -19,7 +19,9 @@ struct eo_index {
   int learned = 0;
   uint64_t n = 0;
   int log2nb = 0;
-  uint32_t *keys = nullptr, *pays = nullptr, *off = nullptr;
+  char *mem = nullptr;  // one allocation: entries, offsets or directory, model
+  eo_tuple *ent = nullptr;
+  uint32_t *off = nullptr;  // hash: bucket offsets; sorted: the directory
   void *model = nullptr;
   uint64_t bytes = 0;
   double build_ms = 0.0;
@@ -31,18 +33,23 @@ namespace {
 
 using namespace eo;
 
-eo_status alloc_dev(void **p, size_t bytes, uint64_t *acc) {
-  EO_TRY_HIP(hipMalloc(p, std::max<size_t>(bytes, 256)), "index allocation");
-  *acc += bytes;
+// Allocates the index's memory: its entries, `words` u32 and `model` bytes.
+eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
+  Layout L;
+  const size_t o_ent = L.add(index_entries(ix->n) * sizeof(eo_tuple));
+  const size_t o_off = L.add(words * sizeof(uint32_t));
+  const size_t o_model = L.add(model);
+  EO_TRY_HIP(hipMalloc((void **)&ix->mem, L.total), "index allocation");
+  ix->bytes = L.total;
+  ix->ent = (eo_tuple *)(ix->mem + o_ent);
+  ix->off = (uint32_t *)(ix->mem + o_off);
+  if (model) ix->model = ix->mem + o_model;
   return EO_OK;
 }
 
 void free_index(eo_index *ix) {
   if (!ix) return;
-  if (ix->keys) (void)hipFree(ix->keys);
-  if (ix->pays) (void)hipFree(ix->pays);
-  if (ix->off) (void)hipFree(ix->off);
-  if (ix->model) (void)hipFree(ix->model);
+  if (ix->mem) (void)hipFree(ix->mem);
   delete ix;
 }
 
@@ -82,16 +89,14 @@ eo_status eo_hidx_build(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_join
   ix->kind = EO_INDEX_HASH;
   ix->n = nR;
   ix->log2nb = log2nb;
-  eo_status st = alloc_dev((void **)&ix->keys, nR * 4, &ix->bytes);
-  if (st == EO_OK) st = alloc_dev((void **)&ix->pays, nR * 4, &ix->bytes);
-  if (st == EO_OK) st = alloc_dev((void **)&ix->off, (nb + 1) * 4, &ix->bytes);
+  eo_status st = alloc_index(ix, nb + 1, 0);
   if (st != EO_OK) {
     free_index(ix);
     return st;
   }
   Layout L;
   const size_t o_in = L.add(host ? nR * sizeof(eo_tuple) : 0);
-  const size_t o_cur = L.add(nb * 4);
+  const size_t o_rank = L.add(nR * 4);
   const size_t o_scr = L.add(scan_scratch_bytes_u32(nb + 1));
   hipError_t e = hipStreamSynchronize(s);
   if (e == hipSuccess) e = c->arena.reserve(L.total);
@@ -107,7 +112,7 @@ eo_status eo_hidx_build(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_join
   }
   PhaseClock clk(c, s, true);
   clk.mark();
-  e = hidx_build(dR, nR, log2nb, ix->keys, ix->pays, ix->off, (uint32_t *)(A + o_cur), A + o_scr, c->d_err, s);
+  e = hidx_build(dR, nR, log2nb, ix->ent, ix->off, (uint32_t *)(A + o_rank), A + o_scr, c->d_err, s);
   clk.mark();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
@@ -143,9 +148,7 @@ static eo_status sidx_build_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, int 
   ix->kind = EO_INDEX_SORTED;
   ix->learned = learned ? 1 : 0;
   ix->n = nR;
-  eo_status st = alloc_dev((void **)&ix->keys, nR * 4, &ix->bytes);
-  if (st == EO_OK) st = alloc_dev((void **)&ix->pays, nR * 4, &ix->bytes);
-  if (st == EO_OK && learned) st = alloc_dev(&ix->model, learned_model_bytes(), &ix->bytes);
+  eo_status st = alloc_index(ix, index_dir_words(nR), learned ? learned_model_bytes() : 0);
   if (st != EO_OK) {
     free_index(ix);
     return st;
@@ -200,12 +203,14 @@ static eo_status sidx_build_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, int 
   }
   if (nR) {
     for (int k = 0; k < 4 && e == hipSuccess && !presorted; ++k) {
-      eo_tuple *dst = (k % 2 == 0) ? bufa : bufb;
+      eo_tuple *dst = k == 3 ? ix->ent : (k % 2 == 0) ? bufa : bufb;
       e = partition_pass(pp[k], src, dst, nullptr, A + o_scr, c->d_err, s);
       src = dst;
     }
-    if (e == hipSuccess) e = sidx_split(src, nR, ix->keys, ix->pays, s);
-    if (e == hipSuccess && learned) e = learned_fit(ix->keys, nR, ix->model, (uint16_t *)(A + o_leaf), s);
+    if (e == hipSuccess && presorted)
+      e = hipMemcpyAsync(ix->ent, dR, nR * sizeof(eo_tuple), hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = index_dir_build(ix->ent, nR, ix->off, s);
+    if (e == hipSuccess && learned) e = learned_fit(ix->ent, nR, ix->model, (uint16_t *)(A + o_leaf), s);
   }
   clk.mark();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -340,8 +345,8 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
       e = fill_u32(none, 0u, matched_words(nS), s);
       if (e == hipSuccess) e = emit_unmatched(dS, nS, none, small, out ? dout : nullptr, out ? out_cap : 0, wide, s);
     } else {
-      e = index_probe(kind, out != nullptr, ix->n, ix->log2nb, ix->keys, ix->pays, ix->off, ix->model, dS, nS,
-                      nullptr, small, out ? dout : nullptr, out ? out_cap : 0, nullptr, wide, outer, s);
+      e = index_probe(kind, out != nullptr, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS,
+                      nullptr, small, out ? dout : nullptr, out ? out_cap : 0, nullptr, wide, outer, c->props.cus, s);
     }
     clk.mark();
     uint64_t total = 0;
@@ -366,8 +371,8 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
     if (st != EO_OK) return st;
     return (out && total > out_cap) ? EO_ECAPACITY : EO_OK;
   }
-  EO_TRY_HIP(index_probe(kind, false, ix->n, ix->log2nb, ix->keys, ix->pays, ix->off, ix->model, dS, nS, cnt, nullptr,
-                         nullptr, 0, nullptr, false, outer, s),
+  EO_TRY_HIP(index_probe(kind, false, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS, cnt, nullptr,
+                         nullptr, 0, nullptr, false, outer, c->props.cus, s),
              "index count");
   EO_TRY_HIP(scan_u64(cnt, cnt, tiles, small, A + o_scr, c->d_err, s), "index scan");
   clk.mark();
@@ -382,8 +387,8 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
   if (total) {
     eo_pair *dout = out;
     if (host) EO_TRY_HIP(hipMallocAsync((void **)&dout, total * row, s), "output staging");
-    hipError_t e = index_probe(kind, true, ix->n, ix->log2nb, ix->keys, ix->pays, ix->off, ix->model, dS, nS, cnt,
-                               nullptr, dout, total, nullptr, wide, outer, s);
+    hipError_t e = index_probe(kind, true, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS, cnt,
+                               nullptr, dout, total, nullptr, wide, outer, c->props.cus, s);
     clk.mark();
     if (e == hipSuccess && host) e = hipMemcpyAsync(out, dout, total * row, hipMemcpyDeviceToHost, s);
     if (host) (void)hipFreeAsync(dout, s);
@@ -426,8 +431,8 @@ eo_status eo_index_lookup(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint
   PhaseClock clk(c, s, o && o->stats);
   ScopedTimer tmr(c, o ? o->stats : nullptr);
   clk.mark();
-  EO_TRY_HIP(index_probe(kind, false, ix->n, ix->log2nb, ix->keys, ix->pays, ix->off, ix->model, dS, nS, nullptr, nullptr,
-                         nullptr, 0, dpos, false, false, s),
+  EO_TRY_HIP(index_probe(kind, false, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS, nullptr, nullptr,
+                         nullptr, 0, dpos, false, false, c->props.cus, s),
              "index lookup");
   clk.mark();
   if (host) EO_TRY_HIP(hipMemcpyAsync(pos, dpos, nS * sizeof(uint64_t), hipMemcpyDeviceToHost, s), "d2h");
@@ -444,10 +449,18 @@ eo_status eo_index_lookup(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint
 eo_status eo_index_export(eo_ctx *c, const eo_index *ix, uint32_t *keys, uint32_t *pays) {
   if (!c || !ix || (ix->n && (!keys || !pays))) return EO_EINVAL;
   DeviceGuard g(c->device);
-  if (ix->n) {
-    EO_TRY_HIP(hipMemcpy(keys, ix->keys, ix->n * 4, hipMemcpyDeviceToHost), "export keys");
-    EO_TRY_HIP(hipMemcpy(pays, ix->pays, ix->n * 4, hipMemcpyDeviceToHost), "export payloads");
-  }
+  if (!ix->n) return EO_OK;
+  // the entries are pairs: split on the device, then two copies
+  hipStream_t s = c->stream;
+  Layout L;
+  const size_t o_k = L.add(ix->n * 4), o_p = L.add(ix->n * 4);
+  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
+  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  char *A = c->arena.base;
+  EO_TRY_HIP(index_split(ix->ent, ix->n, (uint32_t *)(A + o_k), (uint32_t *)(A + o_p), s), "export split");
+  EO_TRY_HIP(hipMemcpyAsync(keys, A + o_k, ix->n * 4, hipMemcpyDeviceToHost, s), "export keys");
+  EO_TRY_HIP(hipMemcpyAsync(pays, A + o_p, ix->n * 4, hipMemcpyDeviceToHost, s), "export payloads");
+  EO_TRY_HIP(hipStreamSynchronize(s), "export sync");
   return EO_OK;
 }
 

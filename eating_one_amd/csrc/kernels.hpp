@@ -160,30 +160,38 @@ hipError_t emit_unmatched(const eo_tuple *S, uint64_t n, const uint32_t *matched
                           uint64_t out_cap, bool wide, hipStream_t stream);
 
 // ---- index.hip --------------------------------------------------------------
-// Resident indexes.  kind 0: hash (keys/pays grouped by bucket, off[NB+1]);
-// kind 1: sorted (binary search); kind 2: sorted with the learned model.
+// Resident indexes, entries as (key, payload) pairs.  kind 0: hash (grouped by
+// bucket, off[NB+1]); kind 1: sorted (off: the directory); kind 2: sorted with
+// the learned model.
 uint64_t index_probe_tiles(uint64_t nS);
 int learned_leaves();
 int learned_knots();
 size_t learned_model_bytes();
-hipError_t hidx_build(const eo_tuple *R, uint64_t n, int log2nb, uint32_t *keys, uint32_t *pays, uint32_t *off,
-                      uint32_t *cursor, void *scan_scratch, uint32_t *err, hipStream_t stream);
-hipError_t sidx_split(const eo_tuple *sorted, uint64_t n, uint32_t *keys, uint32_t *pays, hipStream_t stream);
+// Entries to allocate for n (whole 128-byte lines), u32 words of the directory
+// of a sorted index.
+uint64_t index_entries(uint64_t n);
+uint64_t index_dir_words(uint64_t n);
+// rank: n u32 of scratch.
+hipError_t hidx_build(const eo_tuple *R, uint64_t n, int log2nb, eo_tuple *ent, uint32_t *off, uint32_t *rank,
+                      void *scan_scratch, uint32_t *err, hipStream_t stream);
+// The directory of n sorted entries (and the padding of their last line).
+hipError_t index_dir_build(eo_tuple *ent, uint64_t n, uint32_t *dir, hipStream_t stream);
+hipError_t index_split(const eo_tuple *ent, uint64_t n, uint32_t *keys, uint32_t *pays, hipStream_t stream);
 // *flag (device) = 1 if in[] is not sorted by signed key, else 0.
 hipError_t check_sorted(const eo_tuple *in, uint64_t n, uint32_t *flag, hipStream_t stream);
-// Fits the learned model over sorted keys; leaf_scratch: n u16.
-hipError_t learned_fit(const uint32_t *keys, uint64_t n, void *model, uint16_t *leaf_scratch, hipStream_t stream);
+// Fits the learned model over sorted entries; leaf_scratch: n u16.
+hipError_t learned_fit(const eo_tuple *entries, uint64_t n, void *model, uint16_t *leaf_scratch, hipStream_t stream);
 // Count (write = false: per-tile counts into tile_cnt, or, with tile_cnt ==
 // NULL, the total added into *cursor) or write (write = true: tile_cnt holds
 // exclusive-scanned tile offsets, or, with tile_cnt == NULL, every tile
 // reserves its range from *cursor and positions >= out_cap are counted only).
-// lb_out (optional, nS u64): the index position each probe starts from
-// (lower bound for sorted kinds).  outer: a probe without a match counts
-// (and writes) one null-padded row (left outer join).
-hipError_t index_probe(int kind, bool write, uint64_t n, int log2nb, const uint32_t *keys, const uint32_t *pays,
-                       const uint32_t *off, const void *model, const eo_tuple *S, uint64_t nS,
-                       uint64_t *tile_cnt, uint64_t *cursor, eo_pair *out, uint64_t out_cap, uint64_t *lb_out,
-                       bool wide, bool outer, hipStream_t stream);
+// lb_out (optional, nS u64, write = false): the index position each probe
+// starts from (lower bound for sorted kinds).  outer: a probe without a match
+// counts (and writes) one null-padded row (left outer join).
+hipError_t index_probe(int kind, bool write, uint64_t n, int log2nb, const eo_tuple *ent, const uint32_t *off,
+                       const void *model, const eo_tuple *S, uint64_t nS, uint64_t *tile_cnt, uint64_t *cursor,
+                       eo_pair *out, uint64_t out_cap, uint64_t *lb_out, bool wide, bool outer, int cus,
+                       hipStream_t stream);
 
 // Two-pass MSD partition (high digit bits_hi over the whole array, then the
 // low digit bits_lo inside each first-pass partition) from a single

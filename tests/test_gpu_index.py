@@ -149,3 +149,47 @@ def test_sidx_import_from_reference_index_file(ctx, tmp_path):
         built.free()
     with pytest.raises(eo.EOError):
         ctx.sidx_import(R)  # not sorted
+
+
+@pytest.mark.parametrize("nR", [1, 15, 16, 17, 512, 65536, 65537, 131073, 2097152, 2097153])
+@pytest.mark.parametrize("dup", [1, 5, 40])
+def test_sorted_index_directory_edges(ctx, nR, dup):
+    """Sizes at the edges of the directory's lines and levels (16 entries and 32 keys a line, a
+    top level of 4096 keys), runs of equal keys within, at the end of and across lines, probes
+    below, between, equal to and above every key, and the key that pads the last line."""
+    rng = np.random.default_rng(nR * 64 + dup)
+    top = (1 << 31) - 1
+    keys = np.repeat(np.arange((nR + dup - 1) // dup, dtype=np.int64) * 3 - nR, dup)[:nR]
+    if nR > 15:
+        keys[-(nR % 7 + 1):] = top  # the padding's key, also as a real one
+    order = rng.permutation(nR)
+    R = np.stack([keys[order], order], 1).astype(np.int32)
+    probes = np.concatenate([keys[rng.integers(0, nR, 3000)], keys[rng.integers(0, nR, 500)] - 1,
+                             [keys[0] - 5, keys[-1], min(keys[-1] + 1, top), top, -top - 1]])
+    S = np.stack([probes, np.arange(len(probes))], 1).astype(np.int32)
+    want = brute_join(R, S)
+    for learned in (False, True):
+        ix = ctx.sidx_build(R, learned=learned)
+        try:
+            pos = ix.lookup(S, _abi.EO_LOOKUP_BINARY)
+            assert np.array_equal(pos, np.searchsorted(keys, S[:, 0], side="left").astype(np.uint64))
+            assert same_multiset(ix.join(S), want)
+            assert same_multiset(ix.join(S, deterministic=True), want)
+        finally:
+            ix.free()
+
+
+@pytest.mark.parametrize("nS", [255, 257, (1 << 20) - 1, (1 << 20) + 1, (1 << 20) + 2049])
+def test_index_join_probe_tiles(ctx, nS):
+    """Probe counts at the edges of the tiles and of the choice between them."""
+    R, S = gen.c3(seed=nS, nR=50000, nS=nS, key_range=200000)
+    want = brute_join(R, S)
+    for ix in (ctx.hidx_build(R), ctx.sidx_build(R)):
+        try:
+            assert same_multiset(ix.join(S), want)
+            outer = ix.join(S, left_outer=True)
+            null = outer[:, 0] == _abi.EO_NULL_PAYLOAD
+            assert same_multiset(outer[~null], want)
+            assert np.array_equal(np.sort(outer[null, 1]), np.flatnonzero(~np.isin(S[:, 0], R[:, 0])))
+        finally:
+            ix.free()
