@@ -1041,7 +1041,8 @@ eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_
   }
   EO_TRY_HIP(fill_u64(small, 0, 1, s), "cursor reset");
   clk.mark();
-  hipError_t e = nlj_dist(dR, nR, dS, nS, distance * distance, small, out ? dout : nullptr, out ? out_cap : 0, s);
+  hipError_t e = nlj_dist(dR, nR, dS, nS, distance * distance, small, out ? dout : nullptr, out ? out_cap : 0,
+                          c->props.cus, s);
   clk.mark();
   uint64_t total = 0;
   eo_status st = EO_OK;

@@ -251,15 +251,36 @@ __global__ __launch_bounds__(kNljNT) void k_nlj_fused(const uint2 *__restrict__ 
 // that order with every subtraction, product and sum rounded on its own
 // (__dsub_rn / __dmul_rn / __dadd_rn: no fused multiply-add), which makes each
 // decision bit-identical to the reference's unfused x86-64 arithmetic.  Same
-// fused single-pass structure as k_nlj_fused: R tile (1024 points, SoA
-// doubles) in LDS, 4 S points per lane, OR-accumulated ballots per group of 8
-// R points, per-wave hit-group list, one output reservation per wave.
+// fused single-pass structure as k_nlj_fused: an R tile (up to 1024 points) in
+// LDS, 8 S points per lane, OR-accumulated ballots per group of 8 R points,
+// per-wave hit-group list, one output reservation per wave.
+//
+// The exact predicate takes 9 FP64 instructions per pair.  Every pair first
+// passes a filter of 4 (three FMAs and a compare) that never rejects a match:
+//   |r|^2 - 2 r.s < d2 - |s|^2,   both sides widened by kDistSlack of the terms
+// and only the S registers of a group in which it holds for some pair evaluate
+// the predicate (on coordinates read again, so that the loop keeps only the
+// filter's registers).  8 S points per lane, because the R point that they
+// share is a 32-byte LDS broadcast: with 4 the CU's LDS port is as busy as its
+// four FP64 pipes.
+// Rounding: with u = 2^-53 the filter's left side is off by at most 3u |r|^2
+// (the squares' sum) + 3u (|r|^2 + 2 |r||s|) (the FMAs) <= 9u (|r|^2 + |s|^2),
+// the right side by 4u (|s|^2 + d2), and the reference's own sum is within 8u
+// of the real squared distance, at most 8u d2 at the threshold: together
+// under 16u (|r|^2 + |s|^2 + d2); kDistSlack is 128u.  A point whose squared
+// length is not below 2^1000 (infinities and NaN included) makes every pair
+// of it pass.  FP64 issue bound (0.89 of the VALU's cycles): 2^17 x 2^17 points
+// in 3.69 ms with the exact predicate on every pair, 2.27 ms with the filter
+// (4 S points per lane 2.35, a running minimum instead of the compares 2.33).
 constexpr int kDistNT = 256;
 constexpr int kDistNW = kDistNT / kWave;
-constexpr int kDistK = 4;
-constexpr int kDistSTile = kDistNT * kDistK;  // 1024
+constexpr int kDistK = 8;
+constexpr int kDistSTile = kDistNT * kDistK;  // 2048
 constexpr int kDistRTile = 1024;
 constexpr int kDistGroup = 8;
+constexpr double kDistSlack = 0x1p-46;
+constexpr double kDistHuge = 0x1p1000;
+constexpr double kDistTiny = 0x1p-1060;  // covers squares that round to a multiple of 2^-1074
 
 struct Point3 {
   int32_t id, pad;
@@ -274,36 +295,46 @@ __device__ __forceinline__ bool dist_lt(double sx, double sy, double sz, double 
   return acc < d2;
 }
 
+// An R point as the filter reads it: c = |r|^2 lowered by the slack, or -inf.
+struct alignas(16) DistPoint {
+  double x, y, z, c;
+};
+
 template <bool WRITE>
-__global__ __launch_bounds__(kDistNT) void k_nlj_dist(const Point3 *__restrict__ R, uint64_t nR,
+__global__ __launch_bounds__(kDistNT) __attribute__((amdgpu_waves_per_eu(4))) void k_nlj_dist(const Point3 *__restrict__ R, uint64_t nR,
                                                       const Point3 *__restrict__ S, uint64_t nS, uint32_t s_tiles,
-                                                      double d2, uint64_t *cursor, uint2 *__restrict__ out,
-                                                      uint64_t out_cap) {
-  __shared__ double rx[kDistRTile], ry[kDistRTile], rz[kDistRTile];
+                                                      uint32_t r_tile, double d2, uint64_t *cursor,
+                                                      uint2 *__restrict__ out, uint64_t out_cap) {
+  __shared__ DistPoint rp[kDistRTile];
   __shared__ uint16_t hits[WRITE ? kDistNW : 1][WRITE ? kDistRTile / kDistGroup : 1];
   const uint32_t b = blockIdx.x;
   const uint32_t st = b % s_tiles, rt = b / s_tiles;
-  const uint64_t r0 = (uint64_t)rt * kDistRTile;
-  const uint32_t rn = (uint32_t)std::min<uint64_t>(kDistRTile, nR - r0);
+  const uint64_t r0 = (uint64_t)rt * r_tile;
+  const uint32_t rn = (uint32_t)std::min<uint64_t>(r_tile, nR - r0);
   for (uint32_t i = threadIdx.x; i < rn; i += kDistNT) {
     const Point3 &p = R[r0 + i];
-    rx[i] = p.v[0];
-    ry[i] = p.v[1];
-    rz[i] = p.v[2];
+    const double x = p.v[0], y = p.v[1], z = p.v[2], q = x * x + y * y + z * z;
+    rp[i] = DistPoint{x, y, z, q < kDistHuge ? q - kDistSlack * q : -__builtin_inf()};
   }
+  // the last group is filled with points that pass no pair
+  for (uint32_t i = rn + threadIdx.x; i < (rn + kDistGroup - 1) / kDistGroup * kDistGroup; i += kDistNT)
+    rp[i] = DistPoint{0.0, 0.0, 0.0, __builtin_inf()};
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   const uint64_t s0 = (uint64_t)st * kDistSTile + (uint64_t)w * kWave * kDistK;
-  double sx[kDistK], sy[kDistK], sz[kDistK];
-  uint64_t valid[kDistK];
+  double mx[kDistK], my[kDistK], mz[kDistK], thr[kDistK];
 #pragma unroll
   for (int k = 0; k < kDistK; ++k) {
     const uint64_t i = s0 + (uint64_t)k * kWave + lane;
     const bool ok = i < nS;
-    sx[k] = ok ? S[i].v[0] : 0.0;
-    sy[k] = ok ? S[i].v[1] : 0.0;
-    sz[k] = ok ? S[i].v[2] : 0.0;
-    valid[k] = __ballot(ok);
+    const double x = ok ? S[i].v[0] : 0.0, y = ok ? S[i].v[1] : 0.0, z = ok ? S[i].v[2] : 0.0;
+    const double q = x * x + y * y + z * z;
+    const bool h = !(q < kDistHuge);
+    mx[k] = h ? 0.0 : -2.0 * x;
+    my[k] = h ? 0.0 : -2.0 * y;
+    mz[k] = h ? 0.0 : -2.0 * z;
+    // (a lane past the end of S passes nothing but huge R points)
+    thr[k] = h ? __builtin_inf() : ok ? d2 - q + (kDistSlack * (q + d2) + kDistTiny) : -__builtin_inf();
   }
   __syncthreads();
   const uint64_t lt = lanemask_lt();
@@ -313,25 +344,43 @@ __global__ __launch_bounds__(kDistNT) void k_nlj_dist(const Point3 *__restrict__
   for (uint32_t gi = 0; gi < ngroups; ++gi) {
     const uint32_t g = gi * kDistGroup;
     const uint32_t gn = rn - g < (uint32_t)kDistGroup ? rn - g : (uint32_t)kDistGroup;  // wave-uniform
-    uint64_t acc = 0;
+    uint64_t acc[kDistK] = {};
 #pragma unroll
     for (int q = 0; q < kDistGroup; ++q) {
-      const uint32_t j = g + (q < (int)gn ? q : 0);
-      const double x = rx[j], y = ry[j], z = rz[j];
+      const DistPoint p = rp[g + q];
+      double v[kDistK];  // coordinate by coordinate: kDistK independent FMAs in a row
 #pragma unroll
-      for (int k = 0; k < kDistK; ++k) acc |= __ballot(dist_lt(sx[k], sy[k], sz[k], x, y, z, d2));
+      for (int k = 0; k < kDistK; ++k) v[k] = __builtin_fma(mz[k], p.z, p.c);
+#pragma unroll
+      for (int k = 0; k < kDistK; ++k) v[k] = __builtin_fma(my[k], p.y, v[k]);
+#pragma unroll
+      for (int k = 0; k < kDistK; ++k) v[k] = __builtin_fma(mx[k], p.x, v[k]);
+#pragma unroll
+      for (int k = 0; k < kDistK; ++k) acc[k] |= __ballot(!(v[k] >= thr[k]));  // (not "less": a NaN passes)
     }
-    if (!acc) continue;
-    uint64_t cnt = 0;
-    for (uint32_t q = 0; q < gn; ++q) {
-      const double x = rx[g + q], y = ry[g + q], z = rz[g + q];
+    uint32_t pass = 0;  // S registers with a pair that passes
 #pragma unroll
-      for (int k = 0; k < kDistK; ++k) cnt += __popcll(__ballot(dist_lt(sx[k], sy[k], sz[k], x, y, z, d2)) & valid[k]);
+    for (int k = 0; k < kDistK; ++k) pass |= acc[k] ? 1u << k : 0u;
+    if (!pass) continue;
+    uint64_t cnt = 0;
+    uint32_t hit = 0;
+    for (uint32_t left = pass; left; left &= left - 1) {  // wave-uniform
+      const uint32_t k = (uint32_t)__ffs(left) - 1u;
+      const uint64_t i = s0 + (uint64_t)k * kWave + lane;
+      const Point3 &sp = S[min(i, nS - 1)];
+      const double x = sp.v[0], y = sp.v[1], z = sp.v[2];
+      uint64_t c = 0;
+      for (uint32_t q = 0; q < gn; ++q) {
+        const DistPoint p = rp[g + q];
+        c += __popcll(__ballot(i < nS && dist_lt(x, y, z, p.x, p.y, p.z, d2)));
+      }
+      cnt += c;
+      hit |= c ? 1u << k : 0u;
     }
     if (cnt) {
       total += cnt;
       if (WRITE) {
-        if (lane == 0) hits[w][nh] = (uint16_t)gi;
+        if (lane == 0) hits[w][nh] = (uint16_t)(gi << 8 | hit);
         ++nh;
       }
     }
@@ -344,19 +393,22 @@ __global__ __launch_bounds__(kDistNT) void k_nlj_dist(const Point3 *__restrict__
   if (!WRITE || total == 0) return;
   uint64_t running = 0;
   for (uint32_t h = 0; h < nh; ++h) {
-    const uint32_t g = (uint32_t)hits[w][h] * kDistGroup;
+    const uint32_t rec = (uint32_t)__builtin_amdgcn_readfirstlane((int)hits[w][h]);
+    const uint32_t g = (rec >> 8) * kDistGroup;
     const uint32_t gn = rn - g < (uint32_t)kDistGroup ? rn - g : (uint32_t)kDistGroup;
-    for (uint32_t q = 0; q < gn; ++q) {
-      const double x = rx[g + q], y = ry[g + q], z = rz[g + q];
-#pragma unroll
-      for (int k = 0; k < kDistK; ++k) {
-        const bool eq = dist_lt(sx[k], sy[k], sz[k], x, y, z, d2) && ((valid[k] >> lane) & 1);
+    for (uint32_t left = rec & 0xffu; left; left &= left - 1) {
+      const uint32_t k = (uint32_t)__ffs(left) - 1u;
+      const uint64_t i = s0 + (uint64_t)k * kWave + lane;
+      const Point3 &sp = S[min(i, nS - 1)];
+      const double x = sp.v[0], y = sp.v[1], z = sp.v[2];
+      for (uint32_t q = 0; q < gn; ++q) {
+        const DistPoint p = rp[g + q];
+        const bool eq = i < nS && dist_lt(x, y, z, p.x, p.y, p.z, d2);
         const uint64_t m = __ballot(eq);
         if (m) {
           if (eq) {
             const uint64_t pos = base + running + __popcll(m & lt);
-            const uint64_t si = s0 + (uint64_t)k * kWave + lane;
-            if (pos < out_cap) out[pos] = make_uint2((uint32_t)R[r0 + g + q].id, (uint32_t)S[si].id);
+            if (pos < out_cap) out[pos] = make_uint2((uint32_t)R[r0 + g + q].id, (uint32_t)sp.id);
           }
           running += __popcll(m);
         }
@@ -364,6 +416,8 @@ __global__ __launch_bounds__(kDistNT) void k_nlj_dist(const Point3 *__restrict__
     }
   }
 }
+
+static_assert(kDistK <= 8 && kDistRTile / kDistGroup <= 256, "a hit record: group << 8 | S registers");
 
 }  // namespace
 
@@ -420,21 +474,33 @@ hipError_t nlj_write(const NljPlan &p, const eo_tuple *R, const eo_tuple *S, con
   return hipGetLastError();
 }
 
+// R tuples per tile: `full`, or fewer (whole groups, at least 64) while the
+// grid has less than four workgroups of 256 threads per CU: a small join is
+// bound by the length of one workgroup's loop (2^12 x 2^12 points in 16 tile
+// pairs of 1024 x 1024: 279 us; in 128 of 64 x 2048, with the filter: 58 us).
+static uint32_t nlj_r_tile(uint64_t nR, uint64_t s_tiles, uint32_t full, uint32_t group, int cus) {
+  const uint64_t want = 4ull * (uint64_t)std::max(cus, 8) / std::max<uint64_t>(s_tiles, 1);  // R tiles
+  uint64_t t = want > 1 ? (nR + want - 1) / want : full;
+  t = (t + group - 1) / group * group;
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(t, 64), full);
+}
+
 hipError_t nlj_dist(const eo_point3 *R, uint64_t nR, const eo_point3 *S, uint64_t nS, double d2, uint64_t *cursor,
-                    eo_pair *out, uint64_t out_cap, hipStream_t stream) {
-  const uint64_t r_tiles = (nR + kDistRTile - 1) / kDistRTile, s_tiles = (nS + kDistSTile - 1) / kDistSTile;
-  const uint64_t grid = r_tiles * s_tiles;
+                    eo_pair *out, uint64_t out_cap, int cus, hipStream_t stream) {
+  const uint64_t s_tiles = (nS + kDistSTile - 1) / kDistSTile;
+  const uint32_t r_tile = nlj_r_tile(nR, s_tiles, kDistRTile, kDistGroup, cus);
+  const uint64_t grid = (nR + r_tile - 1) / r_tile * s_tiles;
   if (grid == 0) return hipSuccess;
   if (grid >= (1ull << 31)) return hipErrorInvalidValue;
   const Point3 *vR = reinterpret_cast<const Point3 *>(R), *vS = reinterpret_cast<const Point3 *>(S);
   if (out)
     EO_TIMED("nlj_dist", stream,
              hipLaunchKernelGGL(k_nlj_dist<true>, dim3((uint32_t)grid), dim3(kDistNT), 0, stream, vR, nR, vS, nS,
-                                (uint32_t)s_tiles, d2, cursor, reinterpret_cast<uint2 *>(out), out_cap));
+                                (uint32_t)s_tiles, r_tile, d2, cursor, reinterpret_cast<uint2 *>(out), out_cap));
   else
     EO_TIMED("nlj_dist_count", stream,
              hipLaunchKernelGGL(k_nlj_dist<false>, dim3((uint32_t)grid), dim3(kDistNT), 0, stream, vR, nR, vS, nS,
-                                (uint32_t)s_tiles, d2, cursor, nullptr, 0));
+                                (uint32_t)s_tiles, r_tile, d2, cursor, nullptr, 0));
   return hipGetLastError();
 }
 

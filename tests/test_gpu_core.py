@@ -371,6 +371,34 @@ def test_nlj_dist_join_equals_oracle(ctx, nR, nS, dist):
     assert ctx.nlj_dist_join(R, S, dist, count_only=True) == len(want)
 
 
+@pytest.mark.parametrize("scale,offset,dist", [
+    (1.0, 0.0, 0.3), (1.0, 1e9, 0.3), (1e-3, -1e6, 2e-4), (1e-160, 0.0, 3e-161), (1e-150, 0.0, 3e-151),
+    (1e153, 0.0, 3e152), (1e140, 5e150, 3e139), (1.0, 0.0, 0.0), (1.0, 0.0, float("inf")),
+])
+@pytest.mark.parametrize("nR,nS", [(63, 70), (1030, 515)])
+def test_nlj_dist_filter_keeps_every_match(ctx, nR, nS, scale, offset, dist):
+    """Coordinates far from the origin, near underflow and near overflow, with infinities and
+    NaN among them: the decisions are the oracle's for every pair."""
+    rng = np.random.default_rng(int(nR + nS))
+    R = np.zeros(nR, dtype=oracle.POINT3)
+    S = np.zeros(nS, dtype=oracle.POINT3)
+    R["id"], S["id"] = np.arange(nR), np.arange(nS) + 10 ** 6
+    R["v"] = rng.uniform(-1, 1, size=(nR, 3)) * scale + offset
+    S["v"] = rng.uniform(-1, 1, size=(nS, 3)) * scale + offset
+    S["v"][:20] = R["v"][:20]                                     # equal points
+    if 0.0 < dist < np.inf:
+        S["v"][20:40] = R["v"][20:40] + np.array([0.0, dist, 0.0])  # at the distance, up to rounding
+    special = [np.inf, -np.inf, np.nan, 1.7e308, -1.7e308, 1.4e154, 5e-324, -0.0]
+    for i, x in enumerate(special):
+        R["v"][40 + i, i % 3] = x
+        S["v"][50 + i, i % 3] = x
+    S["v"][58] = R["v"][45]
+    with np.errstate(all="ignore"):
+        want = oracle.nlj_dist_join(R, S, dist)
+    got = ctx.nlj_dist_join(R, S, dist)
+    assert len(got) == len(want) and same_multiset(got, want)
+
+
 @pytest.mark.parametrize("hot", [0.3, 0.7, 1.0])
 def test_two_pass_hot_key(ctx, hot):
     """One key holding up to all of S: one first-pass segment far larger than the
