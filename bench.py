@@ -420,9 +420,10 @@ def run_c3_nlj(a):
             det.append(stats.ms_total)
     compares = len(R) * len(S)
     peak = info["cus"] * 64 * info["clock_khz"] * 1e3  # one 32-bit compare per lane per clock
-    dom = max(ms.items(), key=lambda x: x[1])
     total_ms = sum(ms.values())
-    rate = compares / (dom[1] * 1e-3)
+    # the default order looks inner blocks up in LDS hash tables: its pairs are
+    # covered, not compared; the deterministic order's two passes compare each
+    rate = 2 * compares / (sum(det) / len(det) * 1e-3)
     # measured issue rates: the NLJ's own compare loop without hits, and plain
     # integer adds (eo_valu_probe), best over workgroups per CU
     measured = {}
@@ -435,11 +436,11 @@ def run_c3_nlj(a):
             best = max(best, r.value)
         measured[name] = best
         log(f"measured {name}: {best / 1e12:.2f} T/s ({best / peak:.2f} of 1 per lane per clock)")
-    res = {"metric": "NLJ compares/s, 2^18 x 2^18 (C3)", "value": compares / (total_ms * 1e-3),
-           "unit": "compares/s", "ms_per_step": total_ms, "n_out": n.value, "kernels_ms": ms,
+    res = {"metric": "NLJ tuple pairs/s, 2^18 x 2^18 (C3)", "value": compares / (total_ms * 1e-3),
+           "unit": "pairs/s", "ms_per_step": total_ms, "n_out": n.value, "kernels_ms": ms,
            "deterministic_ms": sum(det) / len(det),
            "roofline": {"bound": "valu", "achieved": rate / 1e9, "peak": peak / 1e9, "unit": "Gcompares/s",
-                        "frac": rate / peak, "kernel": dom[0],
+                        "frac": rate / peak, "kernel": "nlj_count + nlj_write (deterministic order)",
                         "measured_compare_loop": measured["compare_loop"] / 1e9,
                         "measured_int_add": measured["int_add"] / 1e9,
                         "frac_of_compare_loop": rate / measured["compare_loop"]}}
@@ -865,8 +866,8 @@ def other_configs(a):
     out["c1"] = {"workload": "C1 hash join 2^16 x 2^20", "ms_per_join": c1["ms_per_step"], "tuples_per_s": c1["value"]}
     nlj = run_c3_nlj(b)
     out["c3_nlj"] = {"workload": "C3 block NLJ 2^18 x 2^18", "ms_per_join": nlj["ms_per_step"],
-                     "compares_per_s": nlj["value"], "frac_of_nominal": nlj["roofline"]["frac"],
-                     "frac_of_compare_loop": nlj["roofline"].get("frac_of_compare_loop")}
+                     "pairs_per_s": nlj["value"], "deterministic_ms": nlj["deterministic_ms"],
+                     "deterministic_frac_of_compare_loop": nlj["roofline"].get("frac_of_compare_loop")}
     hidx = run_c3_hidx(b)
     out["c3_hidx"] = {"workload": "C3 hash-index join 2^18 x 2^18", "ms_per_probe_pass": hidx["ms_per_step"],
                       "probes_per_s": hidx["value"], "build_ms": hidx.get("build_ms")}

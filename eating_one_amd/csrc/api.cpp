@@ -81,6 +81,37 @@ eo_status read_u64(eo_ctx *ctx, const uint64_t *dev, uint64_t *host, int n, hipS
   return EO_OK;
 }
 
+eo_status begin_results(eo_ctx *ctx, hipStream_t stream) {
+  if (ctx->words_dirty) EO_TRY_HIP(fill_u64(ctx->d_words, 0, 8, stream), "result reset");
+  ctx->words_dirty = true;
+  return EO_OK;
+}
+
+eo_status end_results(eo_ctx *ctx, hipStream_t stream, uint64_t *words, int n, uint32_t *flags) {
+  uint64_t *h = ctx->h_pinned + 48;
+  EO_TRY_HIP(publish_results(ctx->d_words, n, ctx->d_err, h, stream), "result readback");
+  EO_TRY_HIP(hipStreamSynchronize(stream), "result sync");
+  ctx->words_dirty = false;
+  if (n) std::memcpy(words, h, sizeof(uint64_t) * n);
+  *flags = (uint32_t)h[n];
+  return EO_OK;
+}
+
+eo_status end_results_checked(eo_ctx *ctx, hipStream_t stream, uint64_t *words, int n) {
+  uint32_t flags = 0;
+  const eo_status st = end_results(ctx, stream, words, n, &flags);
+  if (st != EO_OK || !flags) return st;
+  set_last_error("device error flags 0x" + std::to_string(flags));
+  return EO_EINTERNAL;
+}
+
+eo_status ensure_arena(eo_ctx *ctx, hipStream_t stream, size_t bytes) {
+  if (bytes <= ctx->arena.cap) return EO_OK;
+  EO_TRY_HIP(hipStreamSynchronize(stream), "sync");
+  EO_TRY_HIP(ctx->arena.reserve(bytes), "arena");
+  return EO_OK;
+}
+
 eo_status check_device_errors(eo_ctx *ctx, hipStream_t stream) {
   EO_TRY_HIP(hipMemcpyAsync(ctx->h_pinned + 63, ctx->d_err, sizeof(uint32_t), hipMemcpyDeviceToHost, stream),
              "error flag readback");
@@ -213,6 +244,7 @@ eo_status eo_ctx_create(eo_ctx **out, int device, const eo_ctx_opts *opts) {
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void **)&c->d_err, 256);
   if (e == hipSuccess) e = hipMemset(c->d_err, 0, 256);
+  if (e == hipSuccess) c->d_words = (uint64_t *)c->d_err + 8;
   if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_pinned, 64 * sizeof(uint64_t), hipHostMallocDefault);
   for (int i = 0; i < 8 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
   for (int i = 0; i < 2 * kMaxTimedLaunches && e == hipSuccess; ++i) e = hipEventCreate(&c->timer.ev[i]);
@@ -587,6 +619,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const bool gap_try = !fx && !outer && !deterministic && hp.passes == 2 && !(o && (o->flags & EO_F_EXACT_PARTITIONS));
   const bool gapR = gap_try && gap_supported(nR, hp.bits_pass2, hp.bits_pass1);
   const bool gapS = gap_try && gap_supported(nS, hp.bits_pass2, hp.bits_pass1);
+  const bool direct = !deterministic && hp.passes == 0;  // unpartitioned: the tiles are planned here
   const uint64_t rp_rows = gapR ? gap_out_rows(nR, hp.bits_pass2, hp.bits_pass1) : nR;
   const uint64_t sp_rows = gapS ? gap_out_rows(nS, hp.bits_pass2, hp.bits_pass1) : nS;
   const uint64_t tmp_rows = std::max(gapR ? gap_tmp_rows(nR, hp.bits_pass2, hp.bits_pass1) : nR,
@@ -603,7 +636,6 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_re = L.add(gapR ? P * sizeof(uint32_t) : 0);
   const size_t o_se = L.add(gapS ? P * sizeof(uint32_t) : 0);
   const size_t o_ts = L.add((P + 1) * sizeof(uint32_t));
-  const size_t o_small = L.add(8 * sizeof(uint64_t));
   const size_t o_bits = L.add(outer ? matched_words(nS) * sizeof(uint32_t) : 0);
   const uint64_t ublocks = outer ? unmatched_blocks(nS) : 0;  // deterministic outer rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
@@ -627,10 +659,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   } else {
     // growing the arena frees the old one: nothing may still use it; when it
     // is large enough, this call's work follows earlier work on the stream
-    if (L.total > c->arena.cap) {
-      EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-      EO_TRY_HIP(c->arena.reserve(L.total), "arena");
-    }
+    if ((st = ensure_arena(c, s, L.total)) != EO_OK) return st;
     A = c->arena.base;
   }
   const eo_tuple *dR = host ? (eo_tuple *)(A + o_rin) : R;
@@ -639,12 +668,13 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   uint32_t *s_start = (uint32_t *)(A + o_ss);
   const uint32_t *r_end = r_start + 1, *s_end = s_start + 1;  // contiguous partitions
   uint32_t *tile_start = (uint32_t *)(A + o_ts);
-  uint64_t *small = (uint64_t *)(A + o_small);
   if (host) {
     EO_TRY_HIP(hipMemcpyAsync((void *)dR, R, nR * sizeof(eo_tuple), hipMemcpyHostToDevice, s), "h2d R");
     EO_TRY_HIP(hipMemcpyAsync((void *)dS, S, nS * sizeof(eo_tuple), hipMemcpyHostToDevice, s), "h2d S");
   }
 
+  st = begin_results(c, s);
+  if (st != EO_OK) return st;
   PhaseClock clk(c, s, stats != nullptr);
   ScopedTimer tmr(c, stats);
   clk.mark();  // 0
@@ -686,7 +716,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     used_gap = gr || gs;
     Rp = rp;
     Sp = sp;
-  } else {
+  } else if (!direct) {
     EO_TRY_HIP(fill_u32(r_start, 0u, 1, s), "fill");
     EO_TRY_HIP(fill_u32(r_start + 1, (uint32_t)nR, 1, s), "fill");
     EO_TRY_HIP(fill_u32(s_start, 0u, 1, s), "fill");
@@ -696,9 +726,13 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
 
   // both orders use the fused probe's tiles: (partition, R chunk, S span)
   const uint32_t cap = join_fused_cap(hp.lds_cap);
-  EO_TRY_HIP(join_fused_plan(P, hp.s_span, cap, r_start, r_end, s_start, s_end, tile_start, small, A + o_jscr,
-                             c->d_err, s),
-             "tile plan");
+  // result words: the tile count, the match count, (deterministic) the null rows
+  uint64_t *const n_tiles_dev = c->d_words, *const cursor = c->d_words + 1;
+  const DirectPlan dp = direct ? plan_direct(nR, nS, &eff, c->props.cus) : DirectPlan{};
+  if (!direct)
+    EO_TRY_HIP(join_fused_plan(P, hp.s_span, cap, r_start, r_end, s_start, s_end, tile_start, n_tiles_dev, A + o_jscr,
+                               c->d_err, s),
+               "tile plan");
   if (stats) {
     stats->radix_bits = (uint32_t)hp.bits;
     stats->passes = (uint32_t)hp.passes;
@@ -719,21 +753,24 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
       EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
-    EO_TRY_HIP(fill_u64(small + 1, 0, 1, s), "cursor reset");
     uint32_t *matched = outer ? (uint32_t *)(A + o_bits) : nullptr;
     if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(nS), s), "match bitmap reset");
     clk.mark();  // 2
-    hipError_t e = join_fused(P, hp.s_span, cap, join_fused_grid(P, nR, nS, tiles_est, c->props.cus), small, Rp,
-                              r_start, r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, small + 1, wide, matched,
-                              c->d_err, s, swapped);
-    if (e == hipSuccess && outer) e = emit_unmatched(Sp, nS, matched, small + 1, dout, cap_dev, wide, s);
+    hipError_t e;
+    if (direct)
+      e = join_direct(dp, Rp, nR, Sp, nS, cap_dev ? dout : nullptr, cap_dev, cursor, wide, matched, swapped, "probe", s);
+    else
+      e = join_fused(P, hp.s_span, cap, join_fused_grid(P, nR, nS, tiles_est, c->props.cus), n_tiles_dev, Rp, r_start,
+                     r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, cursor, wide, matched, c->d_err, s, swapped);
+    if (e == hipSuccess && outer) e = emit_unmatched(Sp, nS, matched, cursor, dout, cap_dev, wide, s);
     clk.mark();  // 3
-    uint64_t words[3] = {0, 0, 0};  // tiles, matches, error flags
-    if (e == hipSuccess) e = take_error_flags(c->d_err, small + 2, s);
+    uint64_t words[2] = {0, 0};  // tiles, matches
+    uint32_t flags = 0;
     if (e == hipSuccess) {
-      st = read_u64(c, small, words, 3, s);
+      st = end_results(c, s, words, 2, &flags);
+      if (direct) words[0] = (uint64_t)dp.chunks * dp.spans;
       total = words[1];
-      if (st == EO_OK && used_gap && words[2] == kErrCapacity) {
+      if (st == EO_OK && used_gap && flags == kErrCapacity) {
         // a sampled region was too small: the rows are incomplete, so the
         // join runs again from the caller's inputs with exact partitions
         if (staged) (void)hipFreeAsync(dout, s);
@@ -745,7 +782,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
         if (stats) stats->sampled = 2u;
         return st;
       }
-      if (st == EO_OK && !words[2] && staged && total) {  // on overflow: the out_cap rows that were written
+      if (st == EO_OK && !flags && staged && total) {  // on overflow: the out_cap rows that were written
         e = hipMemcpyAsync(out, dout, std::min(total, out_cap) * row, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
       }
@@ -753,8 +790,8 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     if (staged) (void)hipFreeAsync(dout, s);
     if (e != hipSuccess) return hip_fail(e, "fused probe");
     if (st != EO_OK) return st;
-    if (words[2]) {
-      set_last_error("device error flags 0x" + std::to_string(words[2]) +
+    if (flags) {
+      set_last_error("device error flags 0x" + std::to_string(flags) +
                      (words[0] >= (1ull << 31) ? " (2^31 or more join tiles)" : ""));
       return EO_EINTERNAL;
     }
@@ -771,54 +808,55 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     return (out && total > out_cap) ? EO_ECAPACITY : EO_OK;
   }
 
-  // Deterministic order: the count and write grids are exact, so the tile
-  // count is read first.
-  uint64_t n_tiles = 0;
-  st = read_u64(c, small, &n_tiles, 1, s);
-  if (st != EO_OK) return st;
-  if (n_tiles >= (1ull << 31)) {
-    set_last_error("too many join tiles");
-    return EO_EINTERNAL;
-  }
-  if (stats) stats->tiles = (uint32_t)n_tiles;
-
   // Deterministic order: count -> scan -> write, nothing written on EO_ECAPACITY.
-  char *B = A + o_tc;
-  bool side = false;
-  size_t o_cnt = 0, o_cscr = tiles_est * sizeof(uint64_t);
-  if (n_tiles > tiles_est) {
-    Layout L2;
-    o_cnt = L2.add(n_tiles * sizeof(uint64_t));
-    o_cscr = L2.add(scan_scratch_bytes_u64(n_tiles));
-    EO_TRY_HIP(hipMallocAsync((void **)&B, L2.total, s), "tile count buffer");
-    side = true;
-  }
-  uint64_t *tile_cnt = (uint64_t *)(B + o_cnt);
-  auto free_side = [&]() {
-    if (side) (void)hipFreeAsync(B, s);
-  };
+  // The counts are taken for the host's estimate of the tile count (0 past the
+  // real one), so that nothing is read back before them; a join with more
+  // tiles (heavily skewed keys) counts again with the exact number.
   // Left outer: the count pass marks matched S tuples; the null rows follow
   // the inner rows, in S order, at scanned per-block offsets.
   uint32_t *bits = outer ? (uint32_t *)(A + o_bits) : nullptr;
   uint64_t *ub = (uint64_t *)(A + o_ub);
+  char *B = A + o_tc, *side = nullptr;
+  auto free_side = [&]() {
+    if (side) (void)hipFreeAsync(side, s);
+  };
+  uint64_t n_tiles = tiles_est;
+  uint64_t *tile_cnt = (uint64_t *)B;
+  void *cnt_scr = B + tiles_est * sizeof(uint64_t);
+  uint64_t words[3] = {0, 0, 0};  // tiles, inner rows, null rows
   if (outer) EO_TRY_HIP(fill_u32(bits, 0u, matched_words(nS), s), "match bitmap reset");
-  EO_TRY_HIP(span_count(P, hp.s_span, cap, (uint32_t)n_tiles, Rp, r_start, Sp, s_start, tile_start, bits, tile_cnt, s),
-             "count");
-  EO_TRY_HIP(scan_u64(tile_cnt, tile_cnt, n_tiles, small + 1, B + o_cscr, c->d_err, s), "count scan");
-  if (outer) {
-    EO_TRY_HIP(count_unmatched(nS, bits, ub, s), "unmatched count");
-    EO_TRY_HIP(scan_u64(ub, ub, ublocks, small + 2, A + o_ubs, c->d_err, s), "unmatched scan");
-  } else {
-    EO_TRY_HIP(fill_u64(small + 2, 0, 1, s), "fill");
+  for (;;) {
+    EO_TRY_HIP(span_count(P, hp.s_span, cap, (uint32_t)n_tiles, Rp, r_start, Sp, s_start, tile_start, bits, tile_cnt, s),
+               "count");
+    EO_TRY_HIP(scan_u64(tile_cnt, tile_cnt, n_tiles, cursor, cnt_scr, c->d_err, s), "count scan");
+    if (outer) {
+      EO_TRY_HIP(count_unmatched(nS, bits, ub, s), "unmatched count");
+      EO_TRY_HIP(scan_u64(ub, ub, ublocks, c->d_words + 2, A + o_ubs, c->d_err, s), "unmatched scan");
+    }
+    if (!side) clk.mark();  // 2
+    const uint64_t known = words[0];
+    st = end_results_checked(c, s, words, 3);
+    if (known) words[0] = known;
+    if (st == EO_OK && words[0] >= (1ull << 31)) {
+      set_last_error("too many join tiles");
+      st = EO_EINTERNAL;
+    }
+    if (st != EO_OK) {
+      free_side();
+      return st;
+    }
+    if (words[0] <= n_tiles) break;
+    n_tiles = words[0];
+    Layout L2;
+    const size_t o_cnt = L2.add(n_tiles * sizeof(uint64_t));
+    const size_t o_cscr = L2.add(scan_scratch_bytes_u64(n_tiles));
+    EO_TRY_HIP(hipMallocAsync((void **)&side, L2.total, s), "tile count buffer");
+    tile_cnt = (uint64_t *)(side + o_cnt);
+    cnt_scr = side + o_cscr;
   }
-  clk.mark();  // 2
-  uint64_t totals[2] = {0, 0};
-  st = read_u64(c, small + 1, totals, 2, s);
-  if (st == EO_OK) st = check_device_errors(c, s);
-  if (st != EO_OK) {
-    free_side();
-    return st;
-  }
+  n_tiles = words[0];
+  if (stats) stats->tiles = (uint32_t)n_tiles;
+  const uint64_t totals[2] = {words[1], words[2]};
   const uint64_t inner = totals[0];
   total = totals[0] + totals[1];
   *n_out = total;
@@ -856,7 +894,6 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   }
   free_side();
   EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  st = check_device_errors(c, s);
   if (stats) {
     stats->ms_partition = clk.ms(0, 1);
     stats->ms_count = clk.ms(1, 2);
@@ -864,7 +901,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     stats->ms_total = clk.ms(0, 3);
     tmr.finish();
   }
-  return st;
+  return EO_OK;
 }
 
 }  // namespace eo
@@ -897,28 +934,29 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
   Layout L;
   const size_t o_rin = L.add(host ? nR * sizeof(eo_tuple) : 0);
   const size_t o_sin = L.add(host ? nS * sizeof(eo_tuple) : 0);
-  const size_t o_cnt = L.add(slots * sizeof(uint64_t));
-  const size_t o_small = L.add(8 * sizeof(uint64_t));
+  const bool deterministic = o && (o->flags & EO_F_DETERMINISTIC);
+  const size_t o_cnt = L.add(deterministic ? slots * sizeof(uint64_t) : 0);
   const size_t o_bits = L.add(outer ? matched_words(nS) * sizeof(uint32_t) : 0);
   const uint64_t ublocks = outer ? unmatched_blocks(nS) : 0;  // deterministic outer rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);
-  const size_t o_scr = L.add(scan_scratch_bytes_u64(slots));
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  const size_t o_scr = L.add(deterministic ? scan_scratch_bytes_u64(slots) : 0);
+  eo_status st = ensure_arena(c, s, L.total);
+  if (st != EO_OK) return st;
   char *A = c->arena.base;
   const eo_tuple *dR = host ? (eo_tuple *)(A + o_rin) : R;
   const eo_tuple *dS = host ? (eo_tuple *)(A + o_sin) : S;
   uint64_t *cnt = (uint64_t *)(A + o_cnt);
-  uint64_t *small = (uint64_t *)(A + o_small);
+  uint64_t *const words_dev = c->d_words;  // rows (deterministic: inner rows, null rows)
   if (host) {
     EO_TRY_HIP(hipMemcpyAsync((void *)dR, R, nR * sizeof(eo_tuple), hipMemcpyHostToDevice, s), "h2d R");
     EO_TRY_HIP(hipMemcpyAsync((void *)dS, S, nS * sizeof(eo_tuple), hipMemcpyHostToDevice, s), "h2d S");
   }
+  if ((st = begin_results(c, s)) != EO_OK) return st;
   PhaseClock clk(c, s, stats != nullptr);
   ScopedTimer tmr(c, stats);
   clk.mark();
-  if (!(o && (o->flags & EO_F_DETERMINISTIC))) {
+  if (!deterministic) {
     // one fused pass; with out == NULL (or a too small buffer) it counts every
     // match and writes only the pairs that fit
     eo_pair *dout = out;
@@ -928,24 +966,26 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
       EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
-    EO_TRY_HIP(fill_u64(small, 0, 1, s), "cursor reset");
     uint32_t *matched = outer ? (uint32_t *)(A + o_bits) : nullptr;
     if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(nS), s), "match bitmap reset");
-    hipError_t e = nlj_fused(np, dR, dS, small, out ? dout : nullptr, cap_dev, wide, matched, s);
-    if (e == hipSuccess && outer) e = emit_unmatched(dS, nS, matched, small, out ? dout : nullptr, cap_dev, wide, s);
+    // every R block against every S block, the inner block looked up in an LDS
+    // hash table
+    hipError_t e = join_direct(plan_direct(nR, nS, nullptr, c->props.cus), dR, nR, dS, nS, cap_dev ? dout : nullptr,
+                               cap_dev, words_dev, wide, matched, false, out ? "nlj_fused" : "nlj_count", s);
+    if (e == hipSuccess && outer)
+      e = emit_unmatched(dS, nS, matched, words_dev, cap_dev ? dout : nullptr, cap_dev, wide, s);
     clk.mark();
     uint64_t total = 0;
-    eo_status st = EO_OK;
     if (e == hipSuccess) {
-      st = read_u64(c, small, &total, 1, s);
-      if (st == EO_OK && staged && total)  // on overflow: the out_cap rows that were written
+      st = end_results_checked(c, s, &total, 1);
+      if (st == EO_OK && staged && total) {  // on overflow: the out_cap rows that were written
         e = hipMemcpyAsync(out, dout, std::min(total, out_cap) * row, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+      }
     }
     if (staged) (void)hipFreeAsync(dout, s);
     if (e != hipSuccess) return hip_fail(e, "nlj");
     if (st != EO_OK) return st;
-    EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-    st = check_device_errors(c, s);
     *n_out = total;
     if (stats) {
       stats->n_out = total;
@@ -954,7 +994,6 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
       stats->ms_total = clk.ms(0, 1);
       tmr.finish();
     }
-    if (st != EO_OK) return st;
     return (out && total > out_cap) ? EO_ECAPACITY : EO_OK;
   }
   // Left outer: the count pass marks matched S tuples; the null rows follow
@@ -963,17 +1002,14 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
   uint64_t *ub = (uint64_t *)(A + o_ub);
   if (outer) EO_TRY_HIP(fill_u32(bits, 0u, matched_words(nS), s), "match bitmap reset");
   EO_TRY_HIP(nlj_count(np, dR, dS, cnt, s, bits), "nlj count");
-  EO_TRY_HIP(scan_u64(cnt, cnt, slots, small, A + o_scr, c->d_err, s), "nlj scan");
+  EO_TRY_HIP(scan_u64(cnt, cnt, slots, words_dev, A + o_scr, c->d_err, s), "nlj scan");
   if (outer) {
     EO_TRY_HIP(count_unmatched(nS, bits, ub, s), "unmatched count");
-    EO_TRY_HIP(scan_u64(ub, ub, ublocks, small + 1, A + o_ubs, c->d_err, s), "unmatched scan");
-  } else {
-    EO_TRY_HIP(fill_u64(small + 1, 0, 1, s), "fill");
+    EO_TRY_HIP(scan_u64(ub, ub, ublocks, words_dev + 1, A + o_ubs, c->d_err, s), "unmatched scan");
   }
   clk.mark();
   uint64_t totals[2] = {0, 0};
-  eo_status st = read_u64(c, small, totals, 2, s);
-  if (st == EO_OK) st = check_device_errors(c, s);
+  st = end_results_checked(c, s, totals, 2);
   if (st != EO_OK) return st;
   const uint64_t inner = totals[0], total = totals[0] + totals[1];
   *n_out = total;
@@ -999,7 +1035,7 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
     stats->ms_total = clk.ms(0, 2);
     tmr.finish();
   }
-  return check_device_errors(c, s);
+  return EO_OK;
 }
 
 eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_point3 *S, uint64_t nS,
@@ -1020,13 +1056,11 @@ eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_
   Layout L;
   const size_t o_rin = L.add(host ? nR * sizeof(eo_point3) : 0);
   const size_t o_sin = L.add(host ? nS * sizeof(eo_point3) : 0);
-  const size_t o_small = L.add(8 * sizeof(uint64_t));
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  eo_status st = ensure_arena(c, s, L.total);
+  if (st != EO_OK) return st;
   char *A = c->arena.base;
   const eo_point3 *dR = host ? (eo_point3 *)(A + o_rin) : R;
   const eo_point3 *dS = host ? (eo_point3 *)(A + o_sin) : S;
-  uint64_t *small = (uint64_t *)(A + o_small);
   if (host) {
     EO_TRY_HIP(hipMemcpyAsync((void *)dR, R, nR * sizeof(eo_point3), hipMemcpyHostToDevice, s), "h2d R");
     EO_TRY_HIP(hipMemcpyAsync((void *)dS, S, nS * sizeof(eo_point3), hipMemcpyHostToDevice, s), "h2d S");
@@ -1039,23 +1073,25 @@ eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_
     EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * sizeof(eo_pair), s), "output staging");
     staged = true;
   }
-  EO_TRY_HIP(fill_u64(small, 0, 1, s), "cursor reset");
+  if ((st = begin_results(c, s)) != EO_OK) {
+    if (staged) (void)hipFreeAsync(dout, s);
+    return st;
+  }
   clk.mark();
-  hipError_t e = nlj_dist(dR, nR, dS, nS, distance * distance, small, out ? dout : nullptr, out ? out_cap : 0,
+  hipError_t e = nlj_dist(dR, nR, dS, nS, distance * distance, c->d_words, out ? dout : nullptr, out ? out_cap : 0,
                           c->props.cus, s);
   clk.mark();
   uint64_t total = 0;
-  eo_status st = EO_OK;
   if (e == hipSuccess) {
-    st = read_u64(c, small, &total, 1, s);
-    if (st == EO_OK && staged && total)  // on overflow: the out_cap rows that were written
+    st = end_results_checked(c, s, &total, 1);
+    if (st == EO_OK && staged && total) {  // on overflow: the out_cap rows that were written
       e = hipMemcpyAsync(out, dout, std::min(total, out_cap) * sizeof(eo_pair), hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+    }
   }
   if (staged) (void)hipFreeAsync(dout, s);
   if (e != hipSuccess) return hip_fail(e, "distance join");
   if (st != EO_OK) return st;
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  st = check_device_errors(c, s);
   *n_out = total;
   if (stats) {
     stats->n_out = total;
@@ -1064,7 +1100,6 @@ eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_
     stats->ms_count = out ? 0.0 : clk.ms(0, 1);
     tmr.finish();
   }
-  if (st != EO_OK) return st;
   return (out && total > out_cap) ? EO_ECAPACITY : EO_OK;
 }
 

@@ -98,12 +98,13 @@ eo_status eo_hidx_build(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_join
   const size_t o_in = L.add(host ? nR * sizeof(eo_tuple) : 0);
   const size_t o_rank = L.add(nR * 4);
   const size_t o_scr = L.add(scan_scratch_bytes_u32(nb + 1));
-  hipError_t e = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = c->arena.reserve(L.total);
-  if (e != hipSuccess) {
+  st = ensure_arena(c, s, L.total);
+  if (st == EO_OK) st = begin_results(c, s);
+  if (st != EO_OK) {
     free_index(ix);
-    return hip_fail(e, "arena");
+    return st;
   }
+  hipError_t e = hipSuccess;
   char *A = c->arena.base;
   const eo_tuple *dR = stage_input(c, R, nR, host, A + o_in, s, &st);
   if (st != EO_OK) {
@@ -114,21 +115,22 @@ eo_status eo_hidx_build(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_join
   clk.mark();
   e = hidx_build(dR, nR, log2nb, ix->ent, ix->off, (uint32_t *)(A + o_rank), A + o_scr, c->d_err, s);
   clk.mark();
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);
     free_index(ix);
     return hip_fail(e, "hash index build");
+  }
+  st = end_results_checked(c, s, nullptr, 0);
+  if (st != EO_OK) {
+    (void)hipStreamSynchronize(s);
+    free_index(ix);
+    return st;
   }
   ix->build_ms = clk.ms(0, 1);
   if (o && o->stats) {
     std::memset(o->stats, 0, sizeof(*o->stats));
     o->stats->ms_build = ix->build_ms;
     o->stats->ms_total = ix->build_ms;
-  }
-  st = check_device_errors(c, s);
-  if (st != EO_OK) {
-    free_index(ix);
-    return st;
   }
   *out = ix;
   return EO_OK;
@@ -167,12 +169,13 @@ static eo_status sidx_build_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, int 
   const size_t o_leaf = L.add(learned ? nR * sizeof(uint16_t) : 0);
   const size_t o_scr = L.add(pscr);
   const size_t o_flag = L.add(sizeof(uint64_t));
-  hipError_t e = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = c->arena.reserve(L.total);
-  if (e != hipSuccess) {
+  st = ensure_arena(c, s, L.total);
+  if (st == EO_OK) st = begin_results(c, s);
+  if (st != EO_OK) {
     free_index(ix);
-    return hip_fail(e, "arena");
+    return st;
   }
+  hipError_t e = hipSuccess;
   char *A = c->arena.base;
   const eo_tuple *dR = stage_input(c, R, nR, host, A + o_in, s, &st);
   if (st != EO_OK) {
@@ -213,10 +216,16 @@ static eo_status sidx_build_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, int 
     if (e == hipSuccess && learned) e = learned_fit(ix->ent, nR, ix->model, (uint16_t *)(A + o_leaf), s);
   }
   clk.mark();
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);
     free_index(ix);
     return hip_fail(e, "sorted index build");
+  }
+  st = end_results_checked(c, s, nullptr, 0);
+  if (st != EO_OK) {
+    (void)hipStreamSynchronize(s);
+    free_index(ix);
+    return st;
   }
   ix->build_ms = clk.ms(0, 1);
   if (learned && nR) {
@@ -241,11 +250,6 @@ static eo_status sidx_build_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, int 
     std::memset(o->stats, 0, sizeof(*o->stats));
     o->stats->ms_build = ix->build_ms;
     o->stats->ms_total = ix->build_ms;
-  }
-  st = check_device_errors(c, s);
-  if (st != EO_OK) {
-    free_index(ix);
-    return st;
   }
   *out = ix;
   return EO_OK;
@@ -310,18 +314,16 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
   Layout L;
   const size_t o_in = L.add(host ? nS * sizeof(eo_tuple) : 0);
   const size_t o_cnt = L.add(tiles * sizeof(uint64_t));
-  const size_t o_small = L.add(64);
   const size_t o_scr = L.add(scan_scratch_bytes_u64(tiles));
   const bool empty_outer = outer && ix->n == 0;  // every probe unmatched
   const size_t o_bits = L.add(empty_outer ? matched_words(nS) * sizeof(uint32_t) : 0);
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  eo_status st = ensure_arena(c, s, L.total);
+  if (st != EO_OK) return st;
   char *A = c->arena.base;
-  eo_status st;
   const eo_tuple *dS = stage_input(c, S, nS, host, A + o_in, s, &st);
   if (st != EO_OK) return st;
   uint64_t *cnt = (uint64_t *)(A + o_cnt);
-  uint64_t *small = (uint64_t *)(A + o_small);
+  uint64_t *const rows_dev = c->d_words;
   PhaseClock clk(c, s, stats != nullptr);
   ScopedTimer tmr(c, stats);
   clk.mark();
@@ -329,6 +331,7 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
     set_last_error("EO_F_LEFT_OUTER on an empty index: default order only");
     return EO_EINVAL;
   }
+  if ((st = begin_results(c, s)) != EO_OK) return st;
   if (!(o && (o->flags & EO_F_DETERMINISTIC))) {
     // one lookup pass; each tile reserves its output range with one atomic
     // (with out == NULL, or a too small buffer, it counts every match)
@@ -338,28 +341,27 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
       EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
-    EO_TRY_HIP(fill_u64(small, 0, 1, s), "cursor reset");
     hipError_t e = hipSuccess;
     if (empty_outer) {
       uint32_t *none = (uint32_t *)(A + o_bits);
       e = fill_u32(none, 0u, matched_words(nS), s);
-      if (e == hipSuccess) e = emit_unmatched(dS, nS, none, small, out ? dout : nullptr, out ? out_cap : 0, wide, s);
+      if (e == hipSuccess) e = emit_unmatched(dS, nS, none, rows_dev, out ? dout : nullptr, out ? out_cap : 0, wide, s);
     } else {
       e = index_probe(kind, out != nullptr, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS,
-                      nullptr, small, out ? dout : nullptr, out ? out_cap : 0, nullptr, wide, outer, c->props.cus, s);
+                      nullptr, rows_dev, out ? dout : nullptr, out ? out_cap : 0, nullptr, wide, outer, c->props.cus, s);
     }
     clk.mark();
     uint64_t total = 0;
     if (e == hipSuccess) {
-      st = read_u64(c, small, &total, 1, s);
-      if (st == EO_OK && staged && total)  // on overflow: the out_cap rows that were written
+      st = end_results_checked(c, s, &total, 1);
+      if (st == EO_OK && staged && total) {  // on overflow: the out_cap rows that were written
         e = hipMemcpyAsync(out, dout, std::min(total, out_cap) * row, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+      }
     }
     if (staged) (void)hipFreeAsync(dout, s);
     if (e != hipSuccess) return hip_fail(e, "index join");
     if (st != EO_OK) return st;
-    EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-    st = check_device_errors(c, s);
     *n_out = total;
     if (stats) {
       stats->n_out = total;
@@ -368,17 +370,15 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
       stats->ms_total = clk.ms(0, 1);
       tmr.finish();
     }
-    if (st != EO_OK) return st;
     return (out && total > out_cap) ? EO_ECAPACITY : EO_OK;
   }
   EO_TRY_HIP(index_probe(kind, false, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS, cnt, nullptr,
                          nullptr, 0, nullptr, false, outer, c->props.cus, s),
              "index count");
-  EO_TRY_HIP(scan_u64(cnt, cnt, tiles, small, A + o_scr, c->d_err, s), "index scan");
+  EO_TRY_HIP(scan_u64(cnt, cnt, tiles, rows_dev, A + o_scr, c->d_err, s), "index scan");
   clk.mark();
   uint64_t total = 0;
-  st = read_u64(c, small, &total, 1, s);
-  if (st == EO_OK) st = check_device_errors(c, s);
+  st = end_results_checked(c, s, &total, 1);
   if (st != EO_OK) return st;
   *n_out = total;
   if (stats) stats->n_out = total;
@@ -403,7 +403,7 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
     stats->ms_total = clk.ms(0, 2);
     tmr.finish();
   }
-  return check_device_errors(c, s);
+  return EO_OK;
 }
 
 eo_status eo_index_lookup(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64_t nS, int method,
@@ -421,10 +421,9 @@ eo_status eo_index_lookup(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint
   Layout L;
   const size_t o_in = L.add(host ? nS * sizeof(eo_tuple) : 0);
   const size_t o_pos = L.add(host ? nS * sizeof(uint64_t) : 0);
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  eo_status st = ensure_arena(c, s, L.total);
+  if (st != EO_OK) return st;
   char *A = c->arena.base;
-  eo_status st;
   const eo_tuple *dS = stage_input(c, S, nS, host, A + o_in, s, &st);
   if (st != EO_OK) return st;
   uint64_t *dpos = host ? (uint64_t *)(A + o_pos) : pos;

@@ -66,6 +66,11 @@ struct eo_ctx {
   eo::Arena arena;
   uint32_t *d_err = nullptr;     // device-side error flags
   uint64_t *h_pinned = nullptr;  // 64 pinned words for small readbacks
+  // 8 device words of a call's results (counts, cursors), beside d_err: zero
+  // between calls (each call's publish clears them), reset by the next call
+  // when one ended early
+  uint64_t *d_words = nullptr;
+  bool words_dirty = false;
   uint64_t hbm_budget = 0;
   hipEvent_t ev[8] = {};
   eo::LaunchTimer timer;  // per-launch events, installed while a call collects stats
@@ -94,6 +99,17 @@ struct DeviceGuard {
 eo_status hip_fail(hipError_t e, const char *what);
 eo_status check_device_errors(eo_ctx *ctx, hipStream_t stream);
 eo_status read_u64(eo_ctx *ctx, const uint64_t *dev, uint64_t *host, int n, hipStream_t stream);
+
+// A call's result words: begin_results before its first kernel (ctx->d_words
+// then hold zeros in stream order), end_results after its last one reads back
+// words[0, n) and the device error flags with one launch and one wait.
+eo_status begin_results(eo_ctx *ctx, hipStream_t stream);
+eo_status end_results(eo_ctx *ctx, hipStream_t stream, uint64_t *words, int n, uint32_t *flags);
+// The same, failing with EO_EINTERNAL when a flag is set.
+eo_status end_results_checked(eo_ctx *ctx, hipStream_t stream, uint64_t *words, int n);
+// Grows the context's arena to `bytes`.  Growing frees the old one, so work on
+// `stream` ends first; an arena that is large enough is used in stream order.
+eo_status ensure_arena(eo_ctx *ctx, hipStream_t stream, size_t bytes);
 
 constexpr uint64_t kMaxRows = (1ull << 31) - 1;
 // Host-mode hash joins with at least this many S tuples run as streaming joins.

@@ -95,6 +95,29 @@ void k_join_fused(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
   }
 }
 
+// An unpartitioned join: tile t is R chunk t % chunks against S span t /
+// chunks, so nothing is planned on the device and the join is this launch.
+// WRITE = false counts only.
+template <typename C, bool WRITE>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
+void k_join_direct(const uint2 *__restrict__ R, uint64_t nR, const uint2 *__restrict__ S, uint64_t nS, uint32_t chunk,
+                   uint32_t chunks, uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor,
+                   int wide, uint32_t *matched, int swapped) {
+  __shared__ tile::ProbeShared<C> sh;
+  const uint32_t c = blockIdx.x % chunks, j = blockIdx.x / chunks;
+  SpanRef ref;
+  ref.r_beg = c * chunk;
+  ref.r_n = (uint32_t)min((uint64_t)chunk, nR - ref.r_beg);
+  ref.s_beg = j * span;
+  ref.s_n = (uint32_t)min((uint64_t)span, nS - ref.s_beg);
+  if (WRITE) {
+    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, cursor, wide != 0, matched, 0, swapped != 0);
+  } else {
+    const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr, false, matched);
+    if (threadIdx.x == 0 && n) atomic_add_agent(cursor, n);
+  }
+}
+
 // Deterministic order on the fused probe's tiles: a count pass (one count per
 // tile, and the matched bits of a left outer join), a scan of the counts, and
 // a write pass whose tiles write from their scanned offsets with a table
@@ -103,12 +126,15 @@ template <typename C>
 __global__ __launch_bounds__(kFNT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_span_count(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_start, const uint2 *__restrict__ S,
                   const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ tile_start, uint32_t P,
-                  uint32_t s_span, uint64_t *__restrict__ tile_count, uint32_t *matched) {
+                  uint32_t s_span, uint64_t *__restrict__ tile_count, uint32_t n, uint32_t *matched) {
   __shared__ tile::ProbeShared<C> sh;
-  for (uint32_t t = blockIdx.x;; t += gridDim.x) {  // a grid below the tile count loops
+  for (uint32_t t = blockIdx.x; t < n; t += gridDim.x) {  // a grid below the tile count loops
     if (t != blockIdx.x) __syncthreads();
     SpanRef ref;
-    if (!resolve_span(t, tile_start, P, r_start, r_start + 1, s_start, s_start + 1, s_span, C::Cap, &ref)) return;
+    if (!resolve_span(t, tile_start, P, r_start, r_start + 1, s_start, s_start + 1, s_span, C::Cap, &ref)) {
+      if (threadIdx.x == 0) tile_count[t] = 0;  // past the last tile (uniform)
+      continue;
+    }
     const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr, false, matched);
     if (threadIdx.x == 0) tile_count[t] = n;
   }
@@ -150,7 +176,8 @@ size_t join_plan_scratch_bytes(uint32_t parts) { return scan_scratch_bytes_u32((
 
 namespace eo {
 
-static_assert(tile::ProbeBig::Cap == kFusedTableFull && tile::ProbeSmall::Cap == kFusedTableHalf,
+static_assert(tile::ProbeBig::Cap == kFusedTableFull && tile::ProbeSmall::Cap == kFusedTableHalf &&
+                  tile::ProbeQuarter::Cap == kFusedTableQuarter,
               "the planner's table sizes are the probe's");
 
 uint32_t join_fused_cap(uint32_t lds_cap) {
@@ -213,6 +240,40 @@ hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t gr
   return hipGetLastError();
 }
 
+template <typename C>
+static hipError_t launch_direct(const DirectPlan &d, const uint2 *R, uint64_t nR, const uint2 *S, uint64_t nS,
+                                uint2 *out, uint64_t out_cap, uint64_t *cursor, bool wide, uint32_t *matched,
+                                bool swapped, const char *name, hipStream_t stream) {
+  const uint64_t grid = (uint64_t)d.chunks * d.spans;
+  if (grid > 0xffffffffull / C::NT) return hipErrorInvalidValue;  // 2^32 work-items a dispatch
+  if (out)
+    EO_TIMED(name, stream,
+             hipLaunchKernelGGL((k_join_direct<C, true>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
+                                d.chunk, d.chunks, d.span, out, out_cap, cursor, (int)wide, matched, (int)swapped));
+  else
+    EO_TIMED(name, stream,
+             hipLaunchKernelGGL((k_join_direct<C, false>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
+                                d.chunk, d.chunks, d.span, nullptr, 0ull, cursor, 0, matched, 0));
+  return hipGetLastError();
+}
+
+hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, const eo_tuple *S, uint64_t nS,
+                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched,
+                       bool swapped, const char *name, hipStream_t stream) {
+  if (nR == 0 || nS == 0) return hipSuccess;
+  const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
+  uint2 *vout = reinterpret_cast<uint2 *>(out);
+#define EO_DIRECT(C) \
+  launch_direct<tile::C>(d, vR, nR, vS, nS, vout, out_cap, out_cursor, wide, matched, swapped, name, stream)
+  switch (d.table) {
+    case kFusedTableFull: return EO_DIRECT(ProbeBig);
+    case kFusedTableHalf: return EO_DIRECT(ProbeSmall);
+    case kFusedTableQuarter: return EO_DIRECT(ProbeQuarter);
+    default: return hipErrorInvalidValue;
+  }
+#undef EO_DIRECT
+}
+
 hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const eo_tuple *R,
                       const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start, const uint32_t *tile_start,
                       uint32_t *matched, uint64_t *tile_count, hipStream_t stream) {
@@ -222,11 +283,11 @@ hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_
   if (cap == (uint32_t)tile::ProbeSmall::Cap)
     EO_TIMED("probe_count", stream,
              hipLaunchKernelGGL(k_span_count<tile::ProbeSmall>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, vS,
-                                s_start, tile_start, parts, s_span, tile_count, matched));
+                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched));
   else if (cap == (uint32_t)tile::ProbeBig::Cap)
     EO_TIMED("probe_count", stream,
              hipLaunchKernelGGL(k_span_count<tile::ProbeBig>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, vS,
-                                s_start, tile_start, parts, s_span, tile_count, matched));
+                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched));
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

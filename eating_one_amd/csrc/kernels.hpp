@@ -132,11 +132,19 @@ hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t gr
 // One launch of the integer VALU probe `kind` (EO_VALU_COMPARE / EO_VALU_ADD)
 // over `blocks` 256-thread blocks; *ops = the operations it performs.
 hipError_t valu_kernel(int kind, uint32_t blocks, uint32_t reps, uint64_t *sink, hipStream_t s, double *ops);
-// Copies the device error flags into *dst (one u64 word) and clears them, so
-// that one readback returns results and flags together.
-hipError_t take_error_flags(uint32_t *err, uint64_t *dst, hipStream_t stream);
+// The unpartitioned join on the host's tile plan, one launch.  *out_cursor must
+// be zero on entry; out == NULL counts only.  name: the launch timer's.
+struct DirectPlan;
+hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, const eo_tuple *S, uint64_t nS,
+                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched,
+                       bool swapped, const char *name, hipStream_t stream);
+// Ends a call's device work: writes words[0, n) (n <= 8) and, in host[n], the
+// error flags to pinned host memory, and clears both on the device, so that
+// the next call on the context needs no reset launch before its kernels.
+hipError_t publish_results(uint64_t *words, int n, uint32_t *err, uint64_t *host, hipStream_t stream);
 // Deterministic order on the fused tiles (join_fused_plan's tile_start):
-// span_count writes every tile's match count (and sets matched bits);
+// span_count writes the match counts of the first n_tiles tiles (0 past the
+// last one, so an estimate will do) and sets matched bits;
 // span_write writes every tile's rows from tile_off[t] on, in an order fixed
 // by the inputs.
 hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const eo_tuple *R,
@@ -337,11 +345,6 @@ uint64_t nlj_count_slots(const NljPlan &p);  // per-wave count entries
 // matched (optional): bitmap over S positions, bits set for S tuples with a match.
 hipError_t nlj_count(const NljPlan &p, const eo_tuple *R, const eo_tuple *S, uint64_t *wave_count,
                      hipStream_t stream, uint32_t *matched = nullptr);
-// One pass: every match counted into *cursor (zero on entry); with out != NULL
-// the pairs are written at positions reserved per wave (order unspecified,
-// positions >= out_cap counted only).
-hipError_t nlj_fused(const NljPlan &p, const eo_tuple *R, const eo_tuple *S, uint64_t *cursor, eo_pair *out,
-                     uint64_t out_cap, bool wide, uint32_t *matched, hipStream_t stream);
 // Distance-predicate NLJ over reference 3-D points: pairs (R id, S id) with
 // squared distance < d2, counted into *cursor (zero on entry), written when
 // out != NULL (positions >= out_cap counted only).

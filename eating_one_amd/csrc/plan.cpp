@@ -81,6 +81,48 @@ eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *o, HashPl
   return EO_OK;
 }
 
+DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus) {
+  // Time model of a tile in microseconds, fitted to joins of 300 to 131072 by
+  // 4000 to 2^24 tuples on each table: a workgroup's fixed cost, per R tuple
+  // built, per S tuple probed; and every S batch's output reservation, an
+  // atomic on one word of the whole device (about 100 million a second).
+  // 2^16 x 2^20: full tables 22 us, half 35, quarter 108; 1000 x 4000: 3.1,
+  // 1.8, 1.2 (each beside 18.5 of launches and the readback).
+  struct Table {
+    uint32_t cap, batch, per_cu;  // tuples, S tuples per batch, workgroups per CU
+    double fixed, build, probe;
+  };
+  constexpr double kAtomic = 0.010;
+  const Table tables[] = {{kFusedTableFull, 8192, 1, 2.0, 1.5e-4, 6e-4},
+                          {kFusedTableHalf, 4096, 2, 1.2, 2e-4, 1e-3},
+                          {kFusedTableQuarter, 2048, 4, 0.8, 2e-4, 7e-4}};
+  const int cap_opt = o ? o->lds_tuples : 0, span_opt = o ? o->s_tile : 0;
+  const uint64_t n_cu = (uint64_t)std::max(cus, 8);
+  DirectPlan best;
+  for (const Table &t : tables) {
+    if (cap_opt && fused_table_tuples((uint32_t)cap_opt, true) != t.cap) continue;
+    DirectPlan d;
+    d.table = t.cap;
+    d.chunks = (uint32_t)std::max<uint64_t>(1, (nR + t.cap - 1) / t.cap);
+    d.chunk = (uint32_t)std::max<uint64_t>(1, (nR + d.chunks - 1) / d.chunks);  // chunks of equal length
+    d.chunks = (uint32_t)std::max<uint64_t>(1, (nR + d.chunk - 1) / d.chunk);
+    const uint64_t slots = n_cu * t.per_cu, batches = std::max<uint64_t>(1, (nS + t.batch - 1) / t.batch);
+    // as many S spans as fill the chip once, of whole batches
+    uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / d.chunks));
+    uint64_t span = (batches + spans - 1) / spans * t.batch;
+    if (span_opt) span = std::max<uint64_t>(t.batch, (uint64_t)span_opt);
+    span = std::min<uint64_t>(span, 1u << 30);
+    spans = std::max<uint64_t>(1, (nS + span - 1) / span);
+    d.span = (uint32_t)span;
+    d.spans = (uint32_t)spans;
+    const double waves = (double)((d.chunks * spans + slots - 1) / slots);
+    d.us = waves * (t.fixed + t.build * d.chunk + t.probe * (double)std::min(span, nS)) +
+           kAtomic * (double)d.chunks * (double)batches;
+    if (!best.table || d.us < best.us) best = d;
+  }
+  return best;
+}
+
 uint32_t plan_span(uint64_t nR, uint64_t nS, uint32_t lds_cap, int bits, uint64_t s_pool, int cus) {
   // Fused probe: S spans short enough to give every CU a few tiles of the
   // s_pool S tuples that share the GPU (this join's, or a whole batch's), and

@@ -29,12 +29,30 @@ constexpr int kMaxJoinBits = 22;
 // R tuples one fused-probe LDS table holds for a planned lds_cap: the full
 // table (lds_cap 16384) 17408, the half table (lds_cap <= 8192) 8704.
 constexpr uint32_t kFusedTableFull = 17408, kFusedTableHalf = 8704;
-inline uint32_t fused_table_tuples(uint32_t lds_cap) { return lds_cap <= 8192 ? kFusedTableHalf : kFusedTableFull; }
 // An unpartitioned join (every S tile probes each R chunk of one LDS table)
 // when R fills at most this many tables and the S tuples read across them stay
 // within kUnpartitionedSReads.
 constexpr uint64_t kUnpartitionedChunks = 4;
 constexpr uint64_t kUnpartitionedSReads = 1ull << 22;
+
+// Tables of an unpartitioned join's tiles, by lds_cap: the full one (16384), the
+// half one (8192) and, in unpartitioned joins only, a quarter one (4096).
+constexpr uint32_t kFusedTableQuarter = 4352;
+inline uint32_t fused_table_tuples(uint32_t lds_cap, bool direct = false) {
+  if (direct && lds_cap <= 4096) return kFusedTableQuarter;
+  return lds_cap <= 8192 ? kFusedTableHalf : kFusedTableFull;
+}
+
+// The tiles of an unpartitioned join: `chunks` R chunks of `chunk` tuples (the
+// last one shorter) by `spans` S spans of `span` tuples.
+struct DirectPlan {
+  uint32_t table = 0;  // LDS table: kFusedTableFull, Half or Quarter
+  uint32_t chunk = 0, chunks = 0;
+  uint32_t span = 0, spans = 0;
+  double us = 0;  // the time model's estimate of the launch
+};
+// opts: lds_tuples and s_tile overrides (0: chosen here).
+DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *opts, int cus);
 
 // Returns EO_OK and fills *out, or EO_EINVAL for inconsistent overrides.
 eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *opts, HashPlan *out, int cus = 256);

@@ -196,7 +196,8 @@ struct Streamer {
                      r_start, r_start + 1, probe_side, s_start, s_start + 1, tile_start, dst, cap, small + 1, wide,
                      outer ? matched : nullptr, c->d_err, cs);
     } else {
-      e = nlj_fused(plan_nlj(nr, n), dR, dS[b], small + 1, dst, cap, wide, outer ? matched : nullptr, cs);
+      e = join_direct(plan_direct(nr, n, nullptr, c->props.cus), dR, nr, dS[b], n, cap ? dst : nullptr, cap, small + 1,
+                      wide, outer ? matched : nullptr, false, dst ? "nlj_fused" : "nlj_count", cs);
     }
     if (e == hipSuccess && outer) e = emit_unmatched(probe_side, n, matched, small + 1, dst, cap, wide, cs);
     if (e != hipSuccess) return hip_fail(e, hash ? "stream hash probe" : "stream nlj");

@@ -17,9 +17,11 @@ namespace tile {
 // CU with up to 128 VGPRs; ProbeSmall (8704 tuples, ~78 KB) lets two share a
 // CU, which leaves 64 VGPRs: 4 S tuples per thread keep its build (9 R tuples
 // per thread plus the first S batch in flight) within them.
-template <int CAP, int LOG2NB, int S_PER_THREAD>
+// ProbeQuarter (4352 tuples, 512 threads, four to a CU) cuts an unpartitioned
+// join into more, shorter tiles where the larger tables leave CUs idle.
+template <int CAP, int LOG2NB, int S_PER_THREAD, int THREADS = 1024>
 struct ProbeCfg {
-  static constexpr int NT = 1024;
+  static constexpr int NT = THREADS;
   static constexpr int Cap = CAP;
   static constexpr int Log2NB = LOG2NB;
   static constexpr int NB = 1 << LOG2NB;
@@ -30,6 +32,7 @@ struct ProbeCfg {
 };
 using ProbeBig = ProbeCfg<17408, 13, 8>;   // a 16K-tuple partition plus binomial spread
 using ProbeSmall = ProbeCfg<8704, 12, 4>;  // an 8K-tuple partition plus spread
+using ProbeQuarter = ProbeCfg<4352, 11, 4, 512>;
 constexpr int kFNT = 1024;
 constexpr int kFCap = ProbeBig::Cap;
 

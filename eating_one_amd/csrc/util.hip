@@ -168,17 +168,22 @@ __global__ __launch_bounds__(kValuNT) void k_valu_add(uint32_t seed, uint32_t re
   if (x == 0x9e3779b9u) sink[blockIdx.x] = x;
 }
 
-__global__ void k_take_flags(uint32_t *err, uint64_t *dst) {
-  if (threadIdx.x == 0) {
-    *dst = *err;
+__global__ void k_publish(uint64_t *words, int n, uint32_t *err, uint64_t *host) {
+  const int i = threadIdx.x;
+  if (i < n) {
+    host[i] = words[i];
+    words[i] = 0ull;
+  } else if (i == n) {
+    host[n] = *err;
     *err = 0u;
   }
 }
 
 }  // namespace
 
-hipError_t take_error_flags(uint32_t *err, uint64_t *dst, hipStream_t stream) {
-  hipLaunchKernelGGL(k_take_flags, dim3(1), dim3(64), 0, stream, err, dst);
+hipError_t publish_results(uint64_t *words, int n, uint32_t *err, uint64_t *host, hipStream_t stream) {
+  if (n < 0 || n > 8) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, stream, words, n, err, host);
   return hipGetLastError();
 }
 

@@ -1,0 +1,73 @@
+"""Unpartitioned joins (one launch of host-planned tiles: the hash join of a small build side and
+the block nested-loop join) at the edges of their tables and tiles, and the deterministic order
+when a skewed join has more tiles than the host estimated."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from eating_one_amd import _abi
+from common import brute_join, same_multiset
+
+pytestmark = pytest.mark.gpu
+
+
+def _relations(nR, nS, keys):
+    rng = np.random.default_rng(nR * 31 + nS)
+    R = np.stack([rng.integers(-keys // 2, keys // 2 + 1, nR), np.arange(nR)], 1).astype(np.int32)
+    S = np.stack([rng.integers(-keys // 2, keys // 2 + 1, nS), np.arange(nS) + 7], 1).astype(np.int32)
+    return R, S
+
+
+@pytest.mark.parametrize("lds", [0, 4096, 8192, 16384])
+@pytest.mark.parametrize("nR,nS", [(1, 1), (2, 2047), (4352, 2049), (4353, 4096), (8704, 4097), (8705, 3),
+                                   (17408, 8192), (17409, 8193), (52225, 20001)])
+def test_direct_tiles_equal_brute_force(ctx, lds, nR, nS):
+    R, S = _relations(nR, nS, max(nR, 4))
+    want = brute_join(R, S)
+    kw = dict(radix_bits=-1, lds_tuples=lds)
+    assert same_multiset(ctx.hash_join(R, S, **kw), want)
+    assert ctx.hash_join(R, S, count_only=True, **kw) == len(want)
+    outer = ctx.hash_join(R, S, left_outer=True, **kw)
+    null = outer[:, 0] == _abi.EO_NULL_PAYLOAD
+    assert same_multiset(outer[~null], want)
+    assert np.array_equal(np.sort(outer[null, 1]), np.sort(S[~np.isin(S[:, 0], R[:, 0]), 1]))
+    if lds == 0:
+        assert same_multiset(ctx.nlj_join(R, S), want)
+        assert ctx.nlj_join(R, S, count_only=True) == len(want)
+        rows = ctx.nlj_join(R, S, result16=True)
+        assert same_multiset(rows[:, [0, 2]], want) and np.array_equal(rows[:, 1], rows[:, 3])
+
+
+def test_direct_tiles_span_override_and_overflow(ctx):
+    """S spans from the caller, and an output too small for the rows: the count is whole and the
+    next call on the context starts from clean result words."""
+    R, S = _relations(9000, 70000, 6000)
+    want = brute_join(R, S)
+    assert same_multiset(ctx.hash_join(R, S, radix_bits=-1, s_tile=8192), want)
+    for fn in (ctx.lib.eo_hash_join, ctx.lib.eo_nlj_join):
+        o, n = ctx.opts(), ctypes.c_uint64()
+        out = np.full((100, 2), -5, dtype=np.int32)
+        st = fn(ctx.handle, R.ctypes.data, len(R), S.ctypes.data, len(S), out.ctypes.data, 90, ctypes.byref(n),
+                ctypes.byref(o))
+        assert st == _abi.EO_ECAPACITY and n.value == len(want)
+        assert (out[90:] == -5).all()
+        assert ctx.hash_join(R, S, count_only=True) == len(want)
+
+
+def test_deterministic_join_with_more_tiles_than_estimated(ctx):
+    """Every key in one of 64 partitions: 35 R chunks by 123 S spans there, far above the estimate
+    the count pass starts from."""
+    rng = np.random.default_rng(8)
+    nR, nS = 300_000, 1_000_000
+    R = np.stack([rng.permutation(nR) << 6, np.arange(nR)], 1).astype(np.int32)
+    S = np.stack([rng.integers(0, 2 * nR, nS) << 6, np.arange(nS)], 1).astype(np.int32)
+    kw = dict(radix_bits=6, passes=1, lds_tuples=8192, s_tile=8192)
+    hit = S[:, 0] >> 6 < nR
+    for outer in (False, True):
+        a = ctx.hash_join(R, S, deterministic=True, left_outer=outer, **kw)
+        assert np.array_equal(a, ctx.hash_join(R, S, deterministic=True, left_outer=outer, **kw))
+        inner = a[a[:, 0] != _abi.EO_NULL_PAYLOAD]
+        assert np.array_equal(np.sort(inner[:, 1]), np.flatnonzero(hit))
+        assert np.array_equal(R[inner[:, 0], 0], S[inner[:, 1], 0])
+        assert len(a) - len(inner) == (np.count_nonzero(~hit) if outer else 0)
