@@ -135,16 +135,24 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 
 // Lanes whose `digit` (BITS low bits) equals this lane's, among the lanes in
 // `active`.  BITS ballots; replaces a match_any instruction that CDNA lacks.
+// Collects the lanes that differ: with s the digit's bit sign-extended (0 or
+// ~0), ballot ^ s are the lanes whose bit is the other one.
 template <int BITS>
 __device__ __forceinline__ uint64_t match_peers(uint32_t digit, uint64_t active) {
-  uint64_t peers = active;
+  uint32_t lo = 0, hi = 0;
 #pragma unroll
   for (int b = 0; b < BITS; ++b) {
-    const bool bit = (digit >> b) & 1u;
-    const uint64_t m = __ballot(bit);
-    peers &= bit ? m : ~m;
+    const int32_t s = (int32_t)(digit << (31 - b)) >> 31;
+    const uint64_t m = __ballot(s != 0);
+    lo |= (uint32_t)m ^ (uint32_t)s;
+    hi |= (uint32_t)(m >> 32) ^ (uint32_t)s;
   }
-  return peers;
+  return active & ~(((uint64_t)hi << 32) | lo);
+}
+
+// Set bits of m below this lane.
+__device__ __forceinline__ uint32_t bits_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 // ---- workgroup scans --------------------------------------------------------

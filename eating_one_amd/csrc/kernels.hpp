@@ -41,6 +41,11 @@ hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *tot
                     void *scratch, uint32_t *err, hipStream_t stream);
 hipError_t scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total_dev,
                     void *scratch, uint32_t *err, hipStream_t stream);
+// scan_u32 on a scratch whose first scan_state_words_u32(n) u64 words an
+// earlier launch on the stream has cleared (one launch less).
+size_t scan_state_words_u32(uint64_t n);
+hipError_t scan_u32_clean(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
+                          uint32_t *err, hipStream_t stream);
 hipError_t fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t stream);
 hipError_t fill_u64(uint64_t *p, uint64_t v, uint64_t n, hipStream_t stream);
 

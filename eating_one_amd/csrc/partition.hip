@@ -16,6 +16,7 @@
 // Stripes are dealt so that consecutive stripes share an XCD, which makes
 // neighbouring runs of one digit meet in the same L2.
 #include <algorithm>
+#include <type_traits>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -29,6 +30,7 @@ using tile::kFastNT;
 using tile::kFastTile;
 
 constexpr int kPartNT = 512;
+constexpr uint64_t kStableStripes = 4096;  // stripes of a stable pass of up to 8 bits, at most
 constexpr int kMsdGroupsPerWg = 4;   // second-pass groups per persistent workgroup (exact partition)
 constexpr int kGapGroupsPerWg = 16;  // the same for the sampled partition
 
@@ -37,7 +39,7 @@ struct PartCfg {
   static constexpr int F = 1 << BITS;
   static constexpr int NT = kPartNT;
   static constexpr int NW = NT / kWave;
-  static constexpr int IPT = BITS <= 8 ? 16 : 8;   // tuples per thread per tile
+  static constexpr int IPT = 8;                    // tuples per thread per tile
   static constexpr int TILE = NT * IPT;
   static constexpr int WSPAN = TILE / NW;          // tuples per wave per tile
   static constexpr int DPT = (F + NT - 1) / NT;    // digits per thread
@@ -112,9 +114,12 @@ __device__ __forceinline__ bool stripe_of(const StripeGeo &geo, uint32_t g, uint
 // tuples), used when the input is 16-byte aligned.
 template <int BITS, bool V16>
 __global__ __launch_bounds__(kPartNT) void k_part_hist(const uint2 *__restrict__ in, StripeGeo geo, int shift,
-                                                       uint32_t xm, uint32_t *__restrict__ counts) {
+                                                       uint32_t xm, uint32_t *__restrict__ counts,
+                                                       uint64_t *__restrict__ zero, uint32_t nzero) {
   using C = PartCfg<BITS>;
   __shared__ uint32_t hist[C::F];
+  // the state of the scan that follows is cleared here instead of by a launch of its own
+  for (uint32_t i = blockIdx.x * C::NT + threadIdx.x; i < nzero; i += gridDim.x * C::NT) zero[i] = 0ull;
   uint32_t g, k;
   if (geo.seg_start) {
     g = blockIdx.x;  // grid is an upper bound: spread the real stripes over all XCDs
@@ -133,104 +138,168 @@ __global__ __launch_bounds__(kPartNT) void k_part_hist(const uint2 *__restrict__
   for (int d = threadIdx.x; d < C::F; d += C::NT) counts[sr.cidx0 + (uint64_t)d * sr.cstride] = hist[d];
 }
 
+// Stable scatter of one stripe (usually one tile).  A wave owns WSPAN
+// consecutive tuples of a tile, ranked 64 at a time in input order: the lanes
+// that share a digit find each other by ballots, and the group's first lane
+// takes the group's ranks from the wave's own LDS counter of that digit.  A
+// wave's LDS operations execute in order, so the counters of all its steps are
+// advanced back to back and their results awaited once (up to 9 bits; with
+// more digits the counters are 16-bit words, read and written step by step).
+// 8 tuples per thread (a tile of 4096): three workgroups of 512 threads share a
+// CU up to 8 bits, one's loads beside another's ranks.  Bound by VALU (the
+// ballots: 8 bits take about 50 instructions per 64 tuples) and memory alike: 5
+// M tuples by 8 bits 25 us (16 per thread 35 us, 12 26 us; 80 us with the
+// counters read and written step by step and idle XCDs); 2^26 by 8 bits with
+// the histogram 0.83 -> 0.51 ms.
 template <int BITS>
-__global__ __launch_bounds__(kPartNT) void k_part_scatter(const uint2 *__restrict__ in, uint64_t n, int shift,
+struct StableShared {
+  using C = PartCfg<BITS>;
+  static constexpr bool kAdd = BITS <= 9;
+  using Cnt = typename std::conditional<kAdd, uint32_t, uint16_t>::type;
+  uint2 stage[C::TILE];
+  Cnt wc[C::NW][C::F];       // per-wave digit counts, then each wave's offset within its digit
+  uint32_t tbase[C::F];      // the tile's digit counts, then its digit starts in stage
+  uint32_t pbase[C::F];      // output position of stage slot i (digit d) = pbase[d] + i (mod 2^32)
+  uint32_t cursor[C::F];     // next output position of each digit
+  uint32_t scan_tmp[C::NW + 1];
+};
+
+template <int BITS>
+__global__ __launch_bounds__(kPartNT) __attribute__((amdgpu_waves_per_eu(4))) void k_part_scatter(const uint2 *__restrict__ in, uint64_t n, int shift,
                                                           uint32_t xm, uint32_t G, uint64_t stripe_len,
                                                           uint32_t K, const uint32_t *__restrict__ offsets,
                                                           uint2 *__restrict__ out, uint32_t *err) {
   using C = PartCfg<BITS>;
+  using SH = StableShared<BITS>;
   constexpr int F = C::F;
-  __shared__ uint32_t cursor[F];
-  __shared__ uint32_t tbase[F + 1];
-  __shared__ uint16_t wcnt[C::NW][F];
-  __shared__ uint2 stage[C::TILE];
-  __shared__ uint32_t scan_tmp[C::NW + 1];
-
+  __shared__ SH sh;
   const uint32_t g = xcd_local_index(blockIdx.x, G);
-  for (int d = threadIdx.x; d < F; d += C::NT) cursor[d] = offsets[((uint64_t)d * G + g) * K];
   const uint64_t beg = (uint64_t)g * stripe_len;
   const uint64_t end = beg + stripe_len < n ? beg + stripe_len : n;
+  if (beg >= end) return;
+  for (int d = threadIdx.x; d < F; d += C::NT) sh.cursor[d] = offsets[((uint64_t)d * G + g) * K];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
-  const uint64_t lt = lanemask_lt();
-
+  uint2 v[C::IPT];
+  // through a buffer resource over the tile: lanes past the end read zero, and
+  // all loads share one offset register
+  auto load = [&](uint64_t t0) {
+    const uint64_t left = t0 < end ? end - t0 : 0;
+    const uint32_t bytes = (uint32_t)min<uint64_t>(left, C::TILE) * 8u;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(in + min(t0, end)), 0, (int)bytes, tile::kBufferRsrcWord3);
+    const int at = (w * C::WSPAN + lane) * 8;
+#pragma unroll
+    for (int it = 0; it < C::IPT; ++it) {
+      typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+      const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(rs, at + it * kWave * 8, 0, 0);
+      v[it] = make_uint2(x.x, x.y);
+    }
+  };
+  load(beg);
   for (uint64_t t0 = beg; t0 < end; t0 += C::TILE) {
     const uint32_t tn = (uint32_t)((end - t0) < (uint64_t)C::TILE ? (end - t0) : (uint64_t)C::TILE);
-    for (int i = threadIdx.x; i < C::NW * F / 2; i += C::NT) reinterpret_cast<uint32_t *>(&wcnt[0][0])[i] = 0;
+    for (int i = threadIdx.x; i < (int)(sizeof(sh.wc) / 4); i += C::NT) reinterpret_cast<uint32_t *>(sh.wc)[i] = 0;
     __syncthreads();
-
-    uint2 v[C::IPT];
-    uint32_t dg[C::IPT];
     uint32_t rk[C::IPT];
+    if constexpr (SH::kAdd) {
+      uint32_t pk[C::IPT];  // lanes before this one in its group | the group's first lane << 8
 #pragma unroll
-    for (int it = 0; it < C::IPT; ++it) {
-      const uint32_t li = (uint32_t)(w * C::WSPAN + it * kWave + lane);
-      const bool valid = li < tn;
-      v[it] = valid ? in[t0 + li] : make_uint2(0u, 0u);
-      dg[it] = digit_of(v[it].x, xm, shift, F - 1);
-    }
+      for (int it = 0; it < C::IPT; ++it) {
+        const bool valid = (uint32_t)(w * C::WSPAN + it * kWave + lane) < tn;
+        const uint32_t d = digit_of(v[it].x, xm, shift, F - 1);
+        const uint64_t peers = match_peers<BITS>(d, __ballot(valid));
+        const uint32_t before = bits_below(peers);
+        const uint32_t lead = valid ? (uint32_t)__ffsll((unsigned long long)peers) - 1u : (uint32_t)lane;
+        pk[it] = before | lead << 8;
+        rk[it] = 0;
+        if (valid && before == 0) rk[it] = atomicAdd(&sh.wc[w][d], (uint32_t)__popcll(peers));
+        __builtin_amdgcn_sched_barrier(0);  // one step's masks at a time: interleaved, they spill
+      }
 #pragma unroll
-    for (int it = 0; it < C::IPT; ++it) {
-      const uint32_t li = (uint32_t)(w * C::WSPAN + it * kWave + lane);
-      const bool valid = li < tn;
-      const uint64_t peers = match_peers<BITS>(dg[it], __ballot(valid));
-      const uint32_t before = (uint32_t)__popcll(peers & lt);
-      uint32_t old = 0;
-      if (valid) old = wcnt[w][dg[it]];
-      rk[it] = old + before;
-      if (valid && before == 0) wcnt[w][dg[it]] = (uint16_t)(old + (uint32_t)__popcll(peers));
+      for (int it = 0; it < C::IPT; ++it)
+        rk[it] = (uint32_t)__shfl((int)rk[it], (int)(pk[it] >> 8)) + (pk[it] & 0xffu);
+    } else {
+#pragma unroll
+      for (int it = 0; it < C::IPT; ++it) {
+        const bool valid = (uint32_t)(w * C::WSPAN + it * kWave + lane) < tn;
+        const uint32_t d = digit_of(v[it].x, xm, shift, F - 1);
+        const uint64_t peers = match_peers<BITS>(d, __ballot(valid));
+        const uint32_t before = bits_below(peers);
+        const uint32_t old = valid ? sh.wc[w][d] : 0u;
+        rk[it] = old + before;
+        if (valid && before == 0) sh.wc[w][d] = (typename SH::Cnt)(old + (uint32_t)__popcll(peers));
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     __syncthreads();
-
-    // Per digit: exclusive offsets over waves (in place) and the tile total.
+    // per digit: exclusive offsets over waves (in place) and the tile's count
     for (int d = threadIdx.x; d < F; d += C::NT) {
       uint32_t run = 0;
 #pragma unroll
       for (int ww = 0; ww < C::NW; ++ww) {
-        const uint32_t c = wcnt[ww][d];
-        wcnt[ww][d] = (uint16_t)run;
+        const uint32_t c = sh.wc[ww][d];
+        sh.wc[ww][d] = (typename SH::Cnt)run;
         run += c;
       }
-      tbase[d] = run;
+      sh.tbase[d] = run;
     }
     __syncthreads();
+    // the digits' starts in stage, their output bases, the cursors past this
+    // tile: by wave 0 up to 9 bits (no barriers), by all threads beyond (a
+    // lane's consecutive digits would all meet in a few LDS banks)
     {
-      uint32_t loc[C::DPT];
-      uint32_t sum = 0;
+      constexpr int PER = BITS <= 9 ? (F + kWave - 1) / kWave : C::DPT;
+      if (BITS > 9 || threadIdx.x < kWave) {
+        uint32_t loc[PER];
+        uint32_t sum = 0;
 #pragma unroll
-      for (int j = 0; j < C::DPT; ++j) {
-        const int d = threadIdx.x * C::DPT + j;
-        loc[j] = d < F ? tbase[d] : 0u;
-        sum += loc[j];
-      }
-      uint32_t tot;
-      uint32_t ex = block_excl_scan<C::NT, uint32_t>(sum, scan_tmp, &tot);
+        for (int k = 0; k < PER; ++k) {
+          const int d = (int)threadIdx.x * PER + k;
+          loc[k] = d < F ? sh.tbase[d] : 0u;
+          sum += loc[k];
+        }
+        uint32_t ex;
+        if constexpr (BITS <= 9) {
+          ex = wave_incl_scan(sum) - sum;
+        } else {
+          uint32_t tot;
+          ex = block_excl_scan<C::NT, uint32_t>(sum, sh.scan_tmp, &tot);
+        }
 #pragma unroll
-      for (int j = 0; j < C::DPT; ++j) {
-        const int d = threadIdx.x * C::DPT + j;
-        if (d < F) tbase[d] = ex;
-        ex += loc[j];
+        for (int k = 0; k < PER; ++k) {
+          const int d = (int)threadIdx.x * PER + k;
+          if (d < F) {
+            const uint32_t c = sh.cursor[d];
+            sh.tbase[d] = ex;
+            sh.pbase[d] = c - ex;
+            sh.cursor[d] = c + loc[k];
+          }
+          ex += loc[k];
+        }
       }
-      if (threadIdx.x == 0) tbase[F] = tn;
     }
     __syncthreads();
-
 #pragma unroll
     for (int it = 0; it < C::IPT; ++it) {
-      const uint32_t li = (uint32_t)(w * C::WSPAN + it * kWave + lane);
-      if (li < tn) stage[tbase[dg[it]] + wcnt[w][dg[it]] + rk[it]] = v[it];
+      if ((uint32_t)(w * C::WSPAN + it * kWave + lane) < tn) {
+        const uint32_t d = digit_of(v[it].x, xm, shift, F - 1);
+        sh.stage[sh.tbase[d] + sh.wc[w][d] + rk[it]] = v[it];
+      }
     }
+    load(t0 + C::TILE);  // the next tile's loads beside this one's writes (past the end: none)
     __syncthreads();
-
-    for (uint32_t i = threadIdx.x; i < tn; i += C::NT) {
-      const uint2 t = stage[i];
-      const uint32_t d = digit_of(t.x, xm, shift, F - 1);
-      const uint64_t pos = (uint64_t)cursor[d] + (i - tbase[d]);
-      if (pos < n) out[pos] = t;
-      else atomic_or_agent(err, kErrOverflow);
+#pragma unroll
+    for (int k = 0; k < C::IPT; ++k) {
+      const uint32_t i = (uint32_t)(k * C::NT) + threadIdx.x;
+      if (i < tn) {
+        const uint2 t = sh.stage[i];
+        const uint32_t pos = sh.pbase[digit_of(t.x, xm, shift, F - 1)] + i;
+        if (pos < n) out[pos] = t;
+        else atomic_or_agent(err, kErrOverflow);
+      }
     }
-    __syncthreads();
-    for (int d = threadIdx.x; d < F; d += C::NT) cursor[d] += tbase[d + 1] - tbase[d];
+    // (the next tile's first barrier follows its wc reset, which no flush reads)
   }
 }
 
@@ -282,16 +351,18 @@ hipError_t launch_pass(const PartPassPlan &p, const eo_tuple *in, eo_tuple *out,
   const bool aligned = ((uintptr_t)in & 7) == 0;
   StripeGeo geo{p.n, p.stripe_len, p.stripes, p.hist_split, nullptr, nullptr, 0};
   const uint32_t hist_grid = p.stripes * p.hist_split;
+  const uint64_t m = ((uint64_t)p.stripes * p.hist_split) << BITS;
+  uint64_t *zero = (uint64_t *)scan_scratch;
+  const uint32_t nzero = (uint32_t)scan_state_words_u32(m);
   if (aligned)
     EO_TIMED("part_hist", stream, hipLaunchKernelGGL((k_part_hist<BITS, true>), dim3(hist_grid), dim3(kPartNT), 0, stream, vin, geo, p.shift,
-                       p.xor_mask, counts));
+                       p.xor_mask, counts, zero, nzero));
   else
     EO_TIMED("part_hist", stream, hipLaunchKernelGGL((k_part_hist<BITS, false>), dim3(hist_grid), dim3(kPartNT), 0, stream, vin, geo, p.shift,
-                       p.xor_mask, counts));
+                       p.xor_mask, counts, zero, nzero));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const uint64_t m = ((uint64_t)p.stripes * p.hist_split) << BITS;
-  e = scan_u32(counts, counts, m, nullptr, scan_scratch, err, stream);
+  e = scan_u32_clean(counts, counts, m, nullptr, scan_scratch, err, stream);
   if (e != hipSuccess) return e;
   if (p.fast) {
     if ((uintptr_t)in & 15) return hipErrorInvalidValue;  // stripe 0 starts at the array start
@@ -358,7 +429,7 @@ hipError_t launch_seg_pass(const SegPassPlan &p, const eo_tuple *in, eo_tuple *o
   const uint2 *vin = reinterpret_cast<const uint2 *>(in);
   const uint32_t grid = (p.max_stripes + kXcds - 1) / kXcds * kXcds;
   EO_TIMED("seg_hist", stream, hipLaunchKernelGGL((k_part_hist<BITS, true>), dim3(grid), dim3(kPartNT), 0, stream, vin, geo, p.shift, 0u,
-                     counts));
+                     counts, nullptr, 0u));
   e = hipGetLastError();
   if (e == hipSuccess) e = scan_u32(counts, counts, m, nullptr, scan_scratch, err, stream);
   if (e != hipSuccess) return e;
@@ -1160,12 +1231,22 @@ PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_m
   cus = std::max(cus, kXcds);
   const uint64_t tile = fast ? (uint64_t)kFastTile : tile_of_bits(bits);
   const uint64_t tiles = std::max<uint64_t>(1, (n + tile - 1) / tile);
-  // fast: kFastWgPerCu 64 KB-LDS workgroups per CU, one stripe each; stable: two per CU.
-  uint64_t g = std::min<uint64_t>(tiles, (uint64_t)cus * (fast ? tile::kFastWgPerCu : 2));
-  g = (g + kXcds - 1) / kXcds * kXcds;
-  uint64_t len = (n + g - 1) / g;
-  len = std::max<uint64_t>(tile, (len + 1) & ~1ull);
-  if (!fast) len = (len + tile - 1) / tile * tile;
+  // fast: kFastWgPerCu workgroups per CU, one stripe each.  Stable: a tile per
+  // workgroup, handed out by the hardware (5 M tuples as 8192-tuple tiles were
+  // 306 stripes of two on 512 workgroups: three of the eight XCDs had none),
+  // and longer stripes once their counts would pass 2^20 (4096 tiles of 8 bits).
+  uint64_t g, len;
+  if (fast) {
+    g = std::min<uint64_t>(tiles, (uint64_t)cus * tile::kFastWgPerCu);
+    g = (g + kXcds - 1) / kXcds * kXcds;
+    len = (n + g - 1) / g;
+    len = std::max<uint64_t>(tile, (len + 1) & ~1ull);
+  } else {
+    const uint64_t most = kStableStripes >> std::max(0, bits - 8);
+    const uint64_t per = (tiles + most - 1) / most;
+    len = per * tile;
+    g = ((tiles + per - 1) / per + kXcds - 1) / kXcds * kXcds;
+  }
   p.stripes = (uint32_t)g;
   p.stripe_len = len;
   // the histogram reads with ~4 workgroups per CU

@@ -126,7 +126,7 @@ size_t scan_scratch(uint64_t n) {  // sized for the short tiles: covers both lau
 
 template <typename T, int IPT>
 hipError_t scan_impl(const T *in, T *out, uint64_t n, uint64_t *total_dev, void *scratch, uint32_t *err,
-                     hipStream_t stream) {
+                     hipStream_t stream, bool clean = false) {
   if (n == 0) {
     if (total_dev) return fill_u64(total_dev, 0, 1, stream);
     return hipSuccess;
@@ -137,8 +137,10 @@ hipError_t scan_impl(const T *in, T *out, uint64_t n, uint64_t *total_dev, void 
   if (tiles >= (1ull << 31)) return hipErrorInvalidValue;
   uint64_t *status = (uint64_t *)scratch;
   uint32_t *ticket = (uint32_t *)(status + tiles);
-  hipError_t e = fill_u64(status, 0, tiles + 1, stream);
-  if (e != hipSuccess) return e;
+  if (!clean) {
+    hipError_t e = fill_u64(status, 0, tiles + 1, stream);
+    if (e != hipSuccess) return e;
+  }
   if (big)
     hipLaunchKernelGGL((k_scan<T, kScanNTBig, IPT>), dim3((uint32_t)tiles), dim3(kScanNTBig), 0, stream, in, out, n,
                        status, ticket, total_dev, err);
@@ -156,6 +158,14 @@ size_t scan_scratch_bytes_u64(uint64_t n) { return scan_scratch<uint64_t, kScanI
 hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
                     uint32_t *err, hipStream_t stream) {
   return scan_impl<uint32_t, kScanIPT32>(in, out, n, total_dev, scratch, err, stream);
+}
+size_t scan_state_words_u32(uint64_t n) {
+  const uint64_t tile = (uint64_t)(n >= kScanBigMin ? kScanNTBig : kScanNT) * kScanIPT32;
+  return (size_t)((n + tile - 1) / tile) + 1;
+}
+hipError_t scan_u32_clean(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
+                          uint32_t *err, hipStream_t stream) {
+  return scan_impl<uint32_t, kScanIPT32>(in, out, n, total_dev, scratch, err, stream, true);
 }
 hipError_t scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
                     uint32_t *err, hipStream_t stream) {

@@ -719,8 +719,18 @@ __device__ __forceinline__ void hist_stripe(uint32_t *hist, const uint2 *__restr
         for (int u = 0; u < 4; ++u) q[u] = ld_stream(in4 + i + u * NT);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          atomicAdd(&hist[digit_of(q[u].x, xm, shift, F - 1)], 1u);
-          atomicAdd(&hist[digit_of(q[u].z, xm, shift, F - 1)], 1u);
+          const uint32_t d0 = digit_of(q[u].x, xm, shift, F - 1), d1 = digit_of(q[u].z, xm, shift, F - 1);
+          // a wave whose active lanes share one digit (sorted input, the high
+          // digit of skewed keys) counts with one atomic instead of 128 on
+          // one word (the last pass of 5 M lognormal keys 23.8 -> 14.7 us)
+          const uint32_t dr = __builtin_amdgcn_readfirstlane(d0);
+          if (__ballot(d0 != dr || d1 != dr) == 0) {  // wave-uniform
+            const uint64_t act = __ballot(true);
+            if (bits_below(act) == 0) atomicAdd(&hist[dr], 2u * (uint32_t)__popcll(act));
+          } else {
+            atomicAdd(&hist[d0], 1u);
+            atomicAdd(&hist[d1], 1u);
+          }
         }
       }
       for (; i < npairs; i += NT) {

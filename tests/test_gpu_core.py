@@ -60,6 +60,21 @@ def test_partition_stable_bits(ctx, bits, shift):
     assert np.array_equal(out, want)
 
 
+@pytest.mark.parametrize("bits", [1, 8, 9, 10, 11])
+@pytest.mark.parametrize("n", [63, 4095, 4096, 4097, 40961, (1 << 21) + 4097])
+def test_partition_stable_tile_edges(ctx, bits, n):
+    """Sizes at the edges of the scatter's 4096-tuple tiles, and stripes of several tiles (more
+    than 2^21 tuples at 11 bits); a third of the keys share one digit."""
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(-(1 << 31), 1 << 31, n)
+    keys[rng.random(n) < 0.33] = 5
+    T = np.stack([keys, np.arange(n)], 1).astype(np.int32)
+    out, off = ctx.radix_partition(T, bits, 3)
+    digit = (T[:, 0].view(np.uint32) >> 3) & ((1 << bits) - 1)
+    assert np.array_equal(out, T[np.argsort(digit, kind="stable")])
+    assert np.array_equal(np.diff(off), np.bincount(digit, minlength=1 << bits))
+
+
 def test_partition_skewed_and_tiny(ctx):
     for n in (0, 1, 5, 4096, 4097):
         T = np.stack([np.full(n, 7, dtype=np.int32), np.arange(n, dtype=np.int32)], 1)
