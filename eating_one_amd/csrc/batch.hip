@@ -246,7 +246,7 @@ __global__ __launch_bounds__(1024) void k_blayout(const BatchSeg *__restrict__ s
     if (b0 + k < F) {
       const uint64_t a = min(at, sg.budget), e = min(at + c[k], sg.budget);
       sg.part_start[b0 + k] = (uint32_t)a;
-      sg.cur[b0 + k] = (uint32_t)a;
+      sg.cur[tile::cursor_slot<BITS>(b0 + k)] = (uint32_t)a;
       sg.re[b0 + k] = (uint32_t)e;
     }
     at += c[k];
@@ -262,7 +262,7 @@ __global__ void k_bends(const BatchSeg *__restrict__ segs, uint32_t nseg) {
   if (i >= (uint64_t)nseg * F) return;
   const BatchSeg sg = load_seg(segs, (uint32_t)(i / F));
   const uint32_t d = (uint32_t)(i % F);
-  sg.part_end[d] = min(sg.cur[d], sg.re[d]);
+  sg.part_end[d] = min(sg.cur[tile::cursor_slot<BITS>(d)], sg.re[d]);
 }
 
 // pair_join[pair_base + p] = j for every partition p of join j (one workgroup per join).

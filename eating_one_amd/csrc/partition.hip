@@ -890,6 +890,13 @@ __global__ __launch_bounds__(256) void k_gap_reduce(const uint32_t *__restrict__
 // the buffers (budget1, budget2 tuples) for any sample of unclumped input; a
 // total beyond them (clumped input, or an empty sample) raises kErrCapacity
 // before any tuple moves, and every region is clipped to its buffer.
+// Place of final partition b's cursor: its high digit's 2^BL cursors, each in
+// the scatter's order.
+template <int BL>
+__device__ __forceinline__ uint32_t gap_cur2(uint32_t b) {
+  return (b >> BL << BL) + tile::cursor_slot<BL>(b & ((1u << BL) - 1));
+}
+
 template <int BH, int BL>
 __global__ __launch_bounds__(kGapLayoutNT) void k_gap_layout(const uint32_t *__restrict__ hs, uint64_t n,
                                                               uint32_t T, uint32_t Tg, uint64_t budget1,
@@ -966,7 +973,6 @@ __global__ __launch_bounds__(kGapLayoutNT) void k_gap_layout(const uint32_t *__r
     for (uint32_t k = 0; k < BPT; k += 4) {
       const uint4 a4 = make_uint4(va[k], va[k + 1], va[k + 2], va[k + 3]);
       *reinterpret_cast<uint4 *>(part_start + b0 + k) = a4;
-      *reinterpret_cast<uint4 *>(cur2 + b0 + k) = a4;
       *reinterpret_cast<uint4 *>(re2 + b0 + k) = make_uint4(ve[k], ve[k + 1], ve[k + 2], ve[k + 3]);
     }
   } else {
@@ -974,11 +980,13 @@ __global__ __launch_bounds__(kGapLayoutNT) void k_gap_layout(const uint32_t *__r
     for (uint32_t k = 0; k < BPT; ++k) {
       if (b0 + k < FT) {
         part_start[b0 + k] = va[k];
-        cur2[b0 + k] = va[k];
         re2[b0 + k] = ve[k];
       }
     }
   }
+#pragma unroll
+  for (uint32_t k = 0; k < BPT; ++k)
+    if (b0 + k < FT) cur2[gap_cur2<BL>(b0 + k)] = va[k];
   if (threadIdx.x == 0) part_start[FT] = (uint32_t)min(tot2, budget2);
   // first-pass regions: thread i = h * 8 + x
   const uint32_t i = threadIdx.x, h = i / kGapRanges, x = i % kGapRanges;
@@ -1016,7 +1024,7 @@ __global__ __launch_bounds__(kGapLayoutNT) void k_gap_layout(const uint32_t *__r
   if (i < NSEG) {
     const uint32_t k = x * F1 + h;
     rs1[k] = (uint32_t)min(a1, budget1);
-    cur1[k] = (uint32_t)min(a1, budget1);
+    cur1[x * F1 + tile::cursor_slot<BH>(h)] = (uint32_t)min(a1, budget1);
     re1[k] = (uint32_t)min(a1 + c1, budget1);
   }
 }
@@ -1038,17 +1046,20 @@ __device__ __forceinline__ uint32_t gap_seg_digit(uint32_t i, uint32_t F1) {
 // receives their exclusive prefix over the segments in queue order
 // (grp[nseg] = total), and grp[nseg + 1 + q], the ticket of queue q, is
 // cleared.  Also raises kErrCapacity for a region that overflowed.
+template <int BH>
 __global__ __launch_bounds__(kGapLayoutNT) void k_gap_groups(const uint32_t *__restrict__ rs1,
                                                              const uint32_t *__restrict__ cur1,
-                                                             const uint32_t *__restrict__ re1, uint32_t F1,
-                                                             uint64_t L, uint32_t *__restrict__ grp, uint32_t *err) {
+                                                             const uint32_t *__restrict__ re1, uint64_t L,
+                                                             uint32_t *__restrict__ grp, uint32_t *err) {
+  constexpr uint32_t F1 = 1u << BH;
   __shared__ uint32_t red[kGapLayoutNT / kWave + 1];
   const uint32_t i = threadIdx.x, nseg = F1 * kGapRanges;
   uint32_t J = 0;
   if (i < nseg) {
-    const uint32_t k = (i % kGapRanges) * F1 + gap_seg_digit(i, F1);
-    if (cur1[k] > re1[k]) atomic_or_agent(err, kErrCapacity);
-    const uint64_t len = (uint64_t)min(cur1[k], re1[k]) - rs1[k];
+    const uint32_t h = gap_seg_digit(i, F1), k = (i % kGapRanges) * F1 + h;
+    const uint32_t c = cur1[(i % kGapRanges) * F1 + tile::cursor_slot<BH>(h)];
+    if (c > re1[k]) atomic_or_agent(err, kErrCapacity);
+    const uint64_t len = (uint64_t)min(c, re1[k]) - rs1[k];
     const uint64_t j = (len + L / 2) / L;
     J = (uint32_t)(j < 1 ? 1 : (j > 65536 ? 65536 : j));
   }
@@ -1063,15 +1074,15 @@ __global__ __launch_bounds__(kGapLayoutNT) void k_gap_groups(const uint32_t *__r
 // one work queue per XCD (above): group w of segment (h, x) is the j-th of its
 // J equal parts (even bounds: 16-byte loads), scattered by the low digit with
 // runs reserved from cur2[h F2 + d].
-template <int BL>
+template <int BH, int BL>
 __global__ __launch_bounds__(kFastNT) void k_gap_scatter(const uint2 *__restrict__ in,
                                                          const uint32_t *__restrict__ rs1,
                                                          const uint32_t *__restrict__ cur1,
-                                                         const uint32_t *__restrict__ re1, uint32_t F1,
+                                                         const uint32_t *__restrict__ re1,
                                                          const uint32_t *__restrict__ grp, uint32_t *tickets,
                                                          const uint32_t *__restrict__ re2, uint32_t *cur2,
                                                          uint2 *__restrict__ out, uint32_t *err) {
-  constexpr uint32_t F2 = 1u << BL;
+  constexpr uint32_t F1 = 1u << BH, F2 = 1u << BL;
   __shared__ tile::ScatterShared<BL, false> sh;
   __shared__ uint32_t s_w;
   const uint32_t nseg = F1 * kGapRanges, Q = gap_queues(F1), spq = nseg / Q;  // segments per queue
@@ -1095,7 +1106,7 @@ __global__ __launch_bounds__(kFastNT) void k_gap_scatter(const uint2 *__restrict
     const uint32_t h = gap_seg_digit(i, F1), k = (i % kGapRanges) * F1 + h;
     const uint32_t J = grp[i + 1] - grp[i], j = w - grp[i];
     const uint64_t b0 = rs1[k];
-    const uint64_t len = (uint64_t)min(cur1[k], re1[k]) - b0;
+    const uint64_t len = (uint64_t)min(cur1[(i % kGapRanges) * F1 + tile::cursor_slot<BH>(h)], re1[k]) - b0;
     const uint64_t beg = b0 + (((uint64_t)j * len / J) & ~1ull);
     const uint64_t end = j + 1 == J ? b0 + len : b0 + (((uint64_t)(j + 1) * len / J) & ~1ull);
     for (uint32_t d = threadIdx.x; d < F2; d += kFastNT) {
@@ -1109,10 +1120,11 @@ __global__ __launch_bounds__(kFastNT) void k_gap_scatter(const uint2 *__restrict
 }
 
 // part_end[b] = the filled end of final partition b.
+template <int BL>
 __global__ void k_gap_ends(const uint32_t *__restrict__ cur2, const uint32_t *__restrict__ re2, uint32_t FT,
                            uint32_t *__restrict__ part_end) {
   const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < FT) part_end[b] = min(cur2[b], re2[b]);
+  if (b < FT) part_end[b] = min(cur2[gap_cur2<BL>(b)], re2[b]);
 }
 
 // Tuples a relation of n needs in a buffer of P sampled regions (the first
@@ -1193,16 +1205,16 @@ hipError_t launch_gap(uint64_t n, uint64_t group_len, uint32_t workers, const eo
                               reinterpret_cast<const uint2 *>(in), n, BL, re1, reinterpret_cast<uint2 *>(tmp), err,
                               cur1));
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_gap_groups, dim3(1), dim3(kGapLayoutNT), 0, stream, rs1, cur1, re1, F1, group_len, grp, err);
+  hipLaunchKernelGGL(k_gap_groups<BH>, dim3(1), dim3(kGapLayoutNT), 0, stream, rs1, cur1, re1, group_len, grp, err);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const uint64_t max_groups = NSEG + n / group_len + 1;
   const uint32_t grid = (uint32_t)std::min<uint64_t>(max_groups, std::max<uint32_t>(workers, 1));
   EO_TIMED("seg_scatter", stream,
-           hipLaunchKernelGGL((k_gap_scatter<BL>), dim3(grid), dim3(kFastNT), 0, stream,
-                              reinterpret_cast<const uint2 *>(tmp), rs1, cur1, re1, F1, grp, grp + NSEG + 1, re2,
+           hipLaunchKernelGGL((k_gap_scatter<BH, BL>), dim3(grid), dim3(kFastNT), 0, stream,
+                              reinterpret_cast<const uint2 *>(tmp), rs1, cur1, re1, grp, grp + NSEG + 1, re2,
                               cur2, reinterpret_cast<uint2 *>(out), err));
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_gap_ends, dim3((FT + 255) / 256), dim3(256), 0, stream, cur2, re2, FT, part_end);
+  hipLaunchKernelGGL(k_gap_ends<BL>, dim3((FT + 255) / 256), dim3(256), 0, stream, cur2, re2, FT, part_end);
   return hipGetLastError();
 }
 
