@@ -22,6 +22,7 @@ CLI = os.path.join(PKG, "eo_join")
 SOURCES = [
     "scan.hip",
     "partition.hip",
+    "onepass.hip",
     "hashjoin.hip",
     "nlj.hip",
     "index.hip",

@@ -82,7 +82,8 @@ eo_status read_u64(eo_ctx *ctx, const uint64_t *dev, uint64_t *host, int n, hipS
 }
 
 eo_status begin_results(eo_ctx *ctx, hipStream_t stream) {
-  if (ctx->words_dirty) EO_TRY_HIP(fill_u64(ctx->d_words, 0, 8, stream), "result reset");
+  if (ctx->words_dirty)
+    EO_TRY_HIP(fill_u64(ctx->d_words, 0, 8 + kCountWords / 2, stream), "result reset");
   ctx->words_dirty = true;
   return EO_OK;
 }
@@ -242,9 +243,14 @@ eo_status eo_ctx_create(eo_ctx **out, int device, const eo_ctx_opts *opts) {
   c->props.l2 = pr.l2CacheSize;
   c->hbm_budget = (opts && opts->hbm_budget) ? opts->hbm_budget : 200ull * 1000 * 1000 * 1000;
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc((void **)&c->d_err, 256);
-  if (e == hipSuccess) e = hipMemset(c->d_err, 0, 256);
-  if (e == hipSuccess) c->d_words = (uint64_t *)c->d_err + 8;
+  // error flags, result words, counts: one allocation, zero from the start
+  const size_t small_bytes = 128 + kCountWords * sizeof(uint32_t);
+  if (e == hipSuccess) e = hipMalloc((void **)&c->d_err, small_bytes);
+  if (e == hipSuccess) e = hipMemset(c->d_err, 0, small_bytes);
+  if (e == hipSuccess) {
+    c->d_words = (uint64_t *)c->d_err + 8;
+    c->d_counts = (uint32_t *)(c->d_words + 8);
+  }
   if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_pinned, 64 * sizeof(uint64_t), hipHostMallocDefault);
   for (int i = 0; i < 8 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
   for (int i = 0; i < 2 * kMaxTimedLaunches && e == hipSuccess; ++i) e = hipEventCreate(&c->timer.ev[i]);
@@ -609,6 +615,23 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     apply_tuned(c, nR, nS, &eff);
     if ((st = plan_hash_join(nR, nS, &eff, &hp, c->props.cus)) != EO_OK) return st;
   }
+  // Fused joins planned here (no plan fields given or tuned) of up to one pass:
+  // unpartitioned or both relations partitioned together, as the time model
+  // has it.  The fixed-scratch entry point and the exact partitions keep the
+  // plan above.
+  const bool aligned = host || (aligned16(R) && aligned16(S));
+  const bool fused_auto = !fx && !(eff.flags & (EO_F_DETERMINISTIC | EO_F_EXACT_PARTITIONS)) && !eff.radix_bits &&
+                          !eff.passes && !eff.lds_tuples && !eff.s_tile && hp.passes <= 1;
+  if (fused_auto && aligned && nR) {
+    HashPlan one = hp;
+    const double us = plan_one_pass(nR, nS, c->props.cus, &one);
+    // (the model of the unpartitioned join is some 15 % low: 2^16 x 2^20 22.5
+    // us for 19.4, 100000 x 2^20 38.5 for 32, partitioned 31)
+    if (us < 1.2 * plan_direct(nR, nS, nullptr, c->props.cus, outer).us && one_pass_supported(nR, nS, one.bits))
+      hp = one;
+    else
+      hp.bits = hp.bits_pass1 = hp.passes = 0;
+  }
   DeviceGuard g(c->device);
   hipStream_t s = pick_stream(c, o);
   const uint32_t P = 1u << hp.bits;
@@ -620,8 +643,11 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const bool gapR = gap_try && gap_supported(nR, hp.bits_pass2, hp.bits_pass1);
   const bool gapS = gap_try && gap_supported(nS, hp.bits_pass2, hp.bits_pass1);
   const bool direct = !deterministic && hp.passes == 0;  // unpartitioned: the tiles are planned here
-  const uint64_t rp_rows = gapR ? gap_out_rows(nR, hp.bits_pass2, hp.bits_pass1) : nR;
-  const uint64_t sp_rows = gapS ? gap_out_rows(nS, hp.bits_pass2, hp.bits_pass1) : nS;
+  // fused joins of one pass partition both relations together
+  const bool one = !fx && !deterministic && hp.passes == 1 && !(o && (o->flags & EO_F_EXACT_PARTITIONS)) &&
+                   aligned && one_pass_supported(nR, nS, hp.bits);
+  const uint64_t rp_rows = one ? one_pass_rows(nR, hp.bits) : gapR ? gap_out_rows(nR, hp.bits_pass2, hp.bits_pass1) : nR;
+  const uint64_t sp_rows = one ? one_pass_rows(nS, hp.bits) : gapS ? gap_out_rows(nS, hp.bits_pass2, hp.bits_pass1) : nS;
   const uint64_t tmp_rows = std::max(gapR ? gap_tmp_rows(nR, hp.bits_pass2, hp.bits_pass1) : nR,
                                      gapS ? gap_tmp_rows(nS, hp.bits_pass2, hp.bits_pass1) : nS);
 
@@ -633,11 +659,17 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_tmp = L.add(hp.passes == 2 ? tmp_rows * sizeof(eo_tuple) : 0);
   const size_t o_rs = L.add((P + 1) * sizeof(uint32_t));
   const size_t o_ss = L.add((P + 1) * sizeof(uint32_t));
-  const size_t o_re = L.add(gapR ? P * sizeof(uint32_t) : 0);
-  const size_t o_se = L.add(gapS ? P * sizeof(uint32_t) : 0);
+  const size_t o_re = L.add(gapR || one ? P * sizeof(uint32_t) : 0);
+  const size_t o_se = L.add(gapS || one ? P * sizeof(uint32_t) : 0);
+  const size_t o_rc = L.add(one ? P * sizeof(uint32_t) : 0);
+  const size_t o_sc = L.add(one ? P * sizeof(uint32_t) : 0);
   const size_t o_ts = L.add((P + 1) * sizeof(uint32_t));
-  const size_t o_bits = L.add(outer ? matched_words(nS) * sizeof(uint32_t) : 0);
-  const uint64_t ublocks = outer ? unmatched_blocks(nS) : 0;  // deterministic outer rows: block offsets
+  const DirectPlan dp = direct ? plan_direct(nR, nS, &eff, c->props.cus, outer) : DirectPlan{};
+  const uint64_t spans = direct ? dp.spans : (uint64_t)P + nS / hp.s_span + 1;
+  const size_t o_bits = L.add(!outer ? 0
+                              : deterministic ? matched_words(nS) * sizeof(uint32_t)
+                                              : outer_words(hp.passes ? sp_rows : nS, spans) * sizeof(uint32_t));
+  const uint64_t ublocks = outer && deterministic ? unmatched_blocks(nS) : 0;  // null rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);
   const size_t o_pscr = L.add(std::max(partition_scratch(nR, hp, c->props.cus), partition_scratch(nS, hp, c->props.cus)));
@@ -679,8 +711,26 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   ScopedTimer tmr(c, stats);
   clk.mark();  // 0
   const eo_tuple *Rp = dR, *Sp = dS;
-  bool used_gap = false;
-  if (hp.passes) {
+  bool used_gap = false, sampled = false;
+  const uint32_t cap = join_fused_cap(hp.lds_cap);
+  // result words: the tile count, the match count, (deterministic) the null rows
+  uint64_t *const n_tiles_dev = c->d_words, *const cursor = c->d_words + 1;
+  if (one) {
+    OneArgs a{};
+    eo_tuple *rp = (eo_tuple *)(A + o_rp), *sp = (eo_tuple *)(A + o_sp);
+    r_end = (uint32_t *)(A + o_re);
+    s_end = (uint32_t *)(A + o_se);
+    a.rel[0] = one_pass_rel(dR, nR, hp.bits, rp, r_start, (uint32_t *)(A + o_re), (uint32_t *)(A + o_rc));
+    a.rel[1] = one_pass_rel(dS, nS, hp.bits, sp, s_start, (uint32_t *)(A + o_se), (uint32_t *)(A + o_sc));
+    a.hs = c->d_counts;
+    a.ticket = c->d_counts + kCountWords - 2;
+    EO_TRY_HIP(one_pass_partition(a, hp.bits, hp.s_span, cap, outer, tile_start, n_tiles_dev, c->d_err, s),
+               "one-pass partition");
+    used_gap = true;
+    sampled = a.rel[0].sampled || a.rel[1].sampled;
+    Rp = rp;
+    Sp = sp;
+  } else if (hp.passes) {
     eo_tuple *rp = (eo_tuple *)(A + o_rp), *sp = (eo_tuple *)(A + o_sp), *tmp = (eo_tuple *)(A + o_tmp);
     // deterministic order needs partitions whose positions the inputs fix
     // (the fast passes rank by atomics): the ordered two-pass partition, or
@@ -713,7 +763,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
       st = partition_relation(c, dS, nS, hp, tmp, sp, s_start, A + o_pscr, s, stable, fixed);
       if (st != EO_OK) return st;
     }
-    used_gap = gr || gs;
+    used_gap = sampled = gr || gs;
     Rp = rp;
     Sp = sp;
   } else if (!direct) {
@@ -725,19 +775,15 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   clk.mark();  // 1
 
   // both orders use the fused probe's tiles: (partition, R chunk, S span)
-  const uint32_t cap = join_fused_cap(hp.lds_cap);
-  // result words: the tile count, the match count, (deterministic) the null rows
-  uint64_t *const n_tiles_dev = c->d_words, *const cursor = c->d_words + 1;
-  const DirectPlan dp = direct ? plan_direct(nR, nS, &eff, c->props.cus) : DirectPlan{};
-  if (!direct)
+  if (!direct && !one)
     EO_TRY_HIP(join_fused_plan(P, hp.s_span, cap, r_start, r_end, s_start, s_end, tile_start, n_tiles_dev, A + o_jscr,
-                               c->d_err, s),
+                               c->d_err, s, outer && !deterministic),
                "tile plan");
   if (stats) {
     stats->radix_bits = (uint32_t)hp.bits;
     stats->passes = (uint32_t)hp.passes;
     stats->lds_tuples = hp.lds_cap;
-    stats->sampled = used_gap ? 1u : 0u;
+    stats->sampled = sampled ? 1u : 0u;
   }
   eo_pair *dout = out;
   bool staged = false;
@@ -753,22 +799,20 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
       EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
-    uint32_t *matched = outer ? (uint32_t *)(A + o_bits) : nullptr;
-    if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(nS), s), "match bitmap reset");
+    uint32_t *ow = outer ? (uint32_t *)(A + o_bits) : nullptr;
     clk.mark();  // 2
     hipError_t e;
     if (direct)
-      e = join_direct(dp, Rp, nR, Sp, nS, cap_dev ? dout : nullptr, cap_dev, cursor, wide, matched, swapped, "probe", s);
+      e = join_direct(dp, Rp, nR, Sp, nS, cap_dev ? dout : nullptr, cap_dev, cursor, wide, ow, swapped, "probe", s);
     else
       e = join_fused(P, hp.s_span, cap, join_fused_grid(P, nR, nS, tiles_est, c->props.cus), n_tiles_dev, Rp, r_start,
-                     r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, cursor, wide, matched, c->d_err, s, swapped);
-    if (e == hipSuccess && outer) e = emit_unmatched(Sp, nS, matched, cursor, dout, cap_dev, wide, s);
+                     r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, cursor, wide, ow, c->d_err, s, swapped);
     clk.mark();  // 3
     uint64_t words[2] = {0, 0};  // tiles, matches
     uint32_t flags = 0;
     if (e == hipSuccess) {
       st = end_results(c, s, words, 2, &flags);
-      if (direct) words[0] = (uint64_t)dp.chunks * dp.spans;
+      if (direct) words[0] = (uint64_t)(outer ? 1u : dp.chunks) * dp.spans;
       total = words[1];
       if (st == EO_OK && used_gap && flags == kErrCapacity) {
         // a sampled region was too small: the rows are incomplete, so the
@@ -936,8 +980,11 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
   const size_t o_sin = L.add(host ? nS * sizeof(eo_tuple) : 0);
   const bool deterministic = o && (o->flags & EO_F_DETERMINISTIC);
   const size_t o_cnt = L.add(deterministic ? slots * sizeof(uint64_t) : 0);
-  const size_t o_bits = L.add(outer ? matched_words(nS) * sizeof(uint32_t) : 0);
-  const uint64_t ublocks = outer ? unmatched_blocks(nS) : 0;  // deterministic outer rows: block offsets
+  const DirectPlan dp = plan_direct(nR, nS, nullptr, c->props.cus, outer);
+  const size_t o_bits = L.add(!outer ? 0
+                              : deterministic ? matched_words(nS) * sizeof(uint32_t)
+                                              : outer_words(nS, dp.spans) * sizeof(uint32_t));
+  const uint64_t ublocks = outer && deterministic ? unmatched_blocks(nS) : 0;  // null rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);
   const size_t o_scr = L.add(deterministic ? scan_scratch_bytes_u64(slots) : 0);
@@ -966,14 +1013,10 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
       EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
-    uint32_t *matched = outer ? (uint32_t *)(A + o_bits) : nullptr;
-    if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(nS), s), "match bitmap reset");
     // every R block against every S block, the inner block looked up in an LDS
     // hash table
-    hipError_t e = join_direct(plan_direct(nR, nS, nullptr, c->props.cus), dR, nR, dS, nS, cap_dev ? dout : nullptr,
-                               cap_dev, words_dev, wide, matched, false, out ? "nlj_fused" : "nlj_count", s);
-    if (e == hipSuccess && outer)
-      e = emit_unmatched(dS, nS, matched, words_dev, cap_dev ? dout : nullptr, cap_dev, wide, s);
+    hipError_t e = join_direct(dp, dR, nR, dS, nS, cap_dev ? dout : nullptr, cap_dev, words_dev, wide,
+                               outer ? (uint32_t *)(A + o_bits) : nullptr, false, out ? "nlj_fused" : "nlj_count", s);
     clk.mark();
     uint64_t total = 0;
     if (e == hipSuccess) {

@@ -67,9 +67,10 @@ struct eo_ctx {
   uint32_t *d_err = nullptr;     // device-side error flags
   uint64_t *h_pinned = nullptr;  // 64 pinned words for small readbacks
   // 8 device words of a call's results (counts, cursors), beside d_err: zero
-  // between calls (each call's publish clears them), reset by the next call
+  // between calls (each call's kernels clear them), reset by the next call
   // when one ended early
   uint64_t *d_words = nullptr;
+  uint32_t *d_counts = nullptr;  // kCountWords words of a one-pass partition's counts and tickets, likewise zero
   bool words_dirty = false;
   uint64_t hbm_budget = 0;
   hipEvent_t ev[8] = {};
@@ -99,6 +100,8 @@ struct DeviceGuard {
 eo_status hip_fail(hipError_t e, const char *what);
 eo_status check_device_errors(eo_ctx *ctx, hipStream_t stream);
 eo_status read_u64(eo_ctx *ctx, const uint64_t *dev, uint64_t *host, int n, hipStream_t stream);
+
+constexpr uint32_t kCountWords = 2 * kOneCopies * ((1u << kOneMaxBits) + 2) + 64;  // (the last two: tickets)
 
 // A call's result words: begin_results before its first kernel (ctx->d_words
 // then hold zeros in stream order), end_results after its last one reads back

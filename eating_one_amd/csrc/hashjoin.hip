@@ -76,7 +76,7 @@ void k_join_fused(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
                   const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ s_end,
                   const uint32_t *__restrict__ tile_start, uint32_t P,
                                                      uint32_t s_span, uint2 *__restrict__ out, uint64_t out_cap,
-                                                     uint64_t *out_cursor, int wide, uint32_t *matched,
+                                                     uint64_t *out_cursor, int wide,
                                                      const uint64_t *__restrict__ n_tiles, uint32_t *err,
                                                      int swapped) {
   __shared__ tile::ProbeShared<C> sh;
@@ -91,8 +91,66 @@ void k_join_fused(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
     if (t != blockIdx.x) __syncthreads();  // the previous tile's LDS reads are done
     SpanRef ref;
     if (!resolve_span(t, tile_start, P, r_start, r_end, s_start, s_end, s_span, C::Cap, &ref)) return;
-    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, out_cursor, wide != 0, matched, 0, swapped != 0);
+    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, out_cursor, wide != 0, nullptr, 0, swapped != 0);
   }
+}
+
+// Left outer join of one S span against R chunks [0, chunks) of one partition
+// (R[rb, rb + rn), equal chunks of at most C::Cap): the rows of every chunk,
+// and with the last one the null rows.  A span whose partition is one chunk
+// (the usual case) needs no bitmap; otherwise its words start at mw.
+template <typename C>
+__device__ __forceinline__ void outer_span(tile::ProbeShared<C> &sh, const uint2 *__restrict__ R, uint32_t rb,
+                                           uint32_t rn, const uint2 *__restrict__ S, uint32_t s_beg, uint32_t s_n,
+                                           uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor, bool wide,
+                                           uint32_t *mw) {
+  const uint32_t nc = max(1u, (rn + C::Cap - 1) / C::Cap), chunk = (rn + nc - 1) / nc;
+  for (uint32_t c = 0; c < nc; ++c) {
+    SpanRef ref;
+    ref.r_beg = rb + c * chunk;
+    ref.r_n = min(chunk, rn - c * chunk);
+    ref.s_beg = s_beg;
+    ref.s_n = s_n;
+    tile::probe_tile<C, tile::kProbeFused, true>(sh, R, S, ref, out, out_cap, cursor, wide, nullptr, 0, false,
+                                                 nc > 1 ? mw : nullptr, c == 0, c + 1 == nc);
+  }
+}
+
+// Left outer joins: tile t is S span t - tile_start[p] of its partition p.
+// words: the spans' bitmaps, span t's from s_beg / 32 + 2 t on.
+template <typename C>
+__global__ __launch_bounds__(kFNT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
+void k_join_outer(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_start,
+                  const uint32_t *__restrict__ r_end, const uint2 *__restrict__ S,
+                  const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ s_end,
+                  const uint32_t *__restrict__ tile_start, uint32_t P, uint32_t s_span, uint2 *__restrict__ out,
+                  uint64_t out_cap, uint64_t *cursor, int wide, uint32_t *words,
+                  const uint64_t *__restrict__ n_tiles, uint32_t *err) {
+  __shared__ tile::ProbeShared<C> sh;
+  const uint64_t nt = *n_tiles;
+  if (nt >= (1ull << 31)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomic_or_agent(err, kErrOverflow);
+    return;
+  }
+  for (uint32_t t = blockIdx.x; t < (uint32_t)nt; t += gridDim.x) {
+    if (t != blockIdx.x) __syncthreads();
+    const uint32_t p = wave_find(tile_start, P, t);
+    const uint32_t rb = r_start[p], rn = r_end[p] - rb;
+    const uint32_t j = t - tile_start[p], sb = s_start[p] + j * s_span;
+    outer_span<C>(sh, R, rb, rn, S, sb, min(s_span, s_end[p] - sb), out, out_cap, cursor, wide != 0,
+                  words + sb / 32 + 2ull * t);
+  }
+}
+
+template <typename C>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
+void k_join_direct_outer(const uint2 *__restrict__ R, uint32_t nR, const uint2 *__restrict__ S, uint32_t nS,
+                         uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor, int wide,
+                         uint32_t *words) {
+  __shared__ tile::ProbeShared<C> sh;
+  const uint32_t sb = blockIdx.x * span;
+  outer_span<C>(sh, R, 0, nR, S, sb, min(span, nS - sb), out, out_cap, cursor, wide != 0,
+                words + sb / 32 + 2ull * blockIdx.x);
 }
 
 // An unpartitioned join: tile t is R chunk t % chunks against S span t /
@@ -102,7 +160,7 @@ template <typename C, bool WRITE>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_join_direct(const uint2 *__restrict__ R, uint64_t nR, const uint2 *__restrict__ S, uint64_t nS, uint32_t chunk,
                    uint32_t chunks, uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor,
-                   int wide, uint32_t *matched, int swapped) {
+                   int wide, int swapped) {
   __shared__ tile::ProbeShared<C> sh;
   const uint32_t c = blockIdx.x % chunks, j = blockIdx.x / chunks;
   SpanRef ref;
@@ -111,9 +169,9 @@ void k_join_direct(const uint2 *__restrict__ R, uint64_t nR, const uint2 *__rest
   ref.s_beg = j * span;
   ref.s_n = (uint32_t)min((uint64_t)span, nS - ref.s_beg);
   if (WRITE) {
-    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, cursor, wide != 0, matched, 0, swapped != 0);
+    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, cursor, wide != 0, nullptr, 0, swapped != 0);
   } else {
-    const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr, false, matched);
+    const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr);
     if (threadIdx.x == 0 && n) atomic_add_agent(cursor, n);
   }
 }
@@ -156,7 +214,8 @@ void k_span_write(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
 }
 
 __global__ void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end, const uint32_t *s_start,
-                             const uint32_t *s_end, uint32_t P, uint32_t s_span, uint32_t cap, uint32_t *tiles) {
+                             const uint32_t *s_end, uint32_t P, uint32_t s_span, uint32_t cap, int outer,
+                             uint32_t *tiles) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p > P) return;
   if (p == P) {
@@ -165,10 +224,13 @@ __global__ void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end, con
   }
   const uint32_t rn = r_end[p] - r_start[p];
   const uint32_t sn = s_end[p] - s_start[p];
-  tiles[p] = (rn && sn) ? ((rn + cap - 1) / cap) * ((sn + s_span - 1) / s_span) : 0u;
+  const uint32_t spans = (sn + s_span - 1) / s_span;
+  tiles[p] = outer ? spans : rn ? (rn + cap - 1) / cap * spans : 0u;
 }
 
 }  // namespace
+
+size_t outer_words(uint64_t s_rows, uint64_t spans) { return s_rows / 32 + 2 * spans + 4; }
 
 size_t join_plan_scratch_bytes(uint32_t parts) { return scan_scratch_bytes_u32((uint64_t)parts + 1); }
 
@@ -187,10 +249,10 @@ uint32_t join_fused_cap(uint32_t lds_cap) {
 hipError_t join_fused_plan(uint32_t parts, uint32_t s_span, uint32_t cap, const uint32_t *r_start,
                            const uint32_t *r_end, const uint32_t *s_start, const uint32_t *s_end,
                            uint32_t *tile_start, uint64_t *n_tiles_dev, void *scan_scratch, uint32_t *err,
-                           hipStream_t stream) {
+                           hipStream_t stream, bool outer) {
   const uint32_t n = parts + 1;
   hipLaunchKernelGGL(k_plan_spans, dim3((n + 255) / 256), dim3(256), 0, stream, r_start, r_end, s_start, s_end,
-                     parts, s_span, cap, tile_start);
+                     parts, s_span, cap, (int)outer, tile_start);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return scan_u32(tile_start, tile_start, n, n_tiles_dev, scan_scratch, err, stream);
@@ -220,51 +282,60 @@ uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tile
 hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
                       const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
                       const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
-                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched, uint32_t *err,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer, uint32_t *err,
                       hipStream_t stream, bool swapped) {
   if (grid == 0) return hipSuccess;
   const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
   uint2 *vout = reinterpret_cast<uint2 *>(out);
-  if (cap == (uint32_t)tile::ProbeSmall::Cap)
-    EO_TIMED("probe", stream,
-             hipLaunchKernelGGL(k_join_fused<tile::ProbeSmall>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end,
-                                vS, s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,
-                                matched, n_tiles_dev, err, (int)swapped));
-  else if (cap == (uint32_t)tile::ProbeBig::Cap)
-    EO_TIMED("probe", stream,
-             hipLaunchKernelGGL(k_join_fused<tile::ProbeBig>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end,
-                                vS, s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,
-                                matched, n_tiles_dev, err, (int)swapped));
-  else
-    return hipErrorInvalidValue;
+#define EO_FUSED(C)                                                                                                  \
+  do {                                                                                                               \
+    if (outer)                                                                                                       \
+      EO_TIMED("probe", stream,                                                                                      \
+               hipLaunchKernelGGL(k_join_outer<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,   \
+                                  s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,   \
+                                  outer, n_tiles_dev, err));                                                         \
+    else                                                                                                             \
+      EO_TIMED("probe", stream,                                                                                      \
+               hipLaunchKernelGGL(k_join_fused<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,   \
+                                  s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,   \
+                                  n_tiles_dev, err, (int)swapped));                                                  \
+  } while (0)
+  if (cap == (uint32_t)tile::ProbeSmall::Cap) EO_FUSED(ProbeSmall);
+  else if (cap == (uint32_t)tile::ProbeBig::Cap) EO_FUSED(ProbeBig);
+  else return hipErrorInvalidValue;
+#undef EO_FUSED
   return hipGetLastError();
 }
 
 template <typename C>
 static hipError_t launch_direct(const DirectPlan &d, const uint2 *R, uint64_t nR, const uint2 *S, uint64_t nS,
-                                uint2 *out, uint64_t out_cap, uint64_t *cursor, bool wide, uint32_t *matched,
+                                uint2 *out, uint64_t out_cap, uint64_t *cursor, bool wide, uint32_t *outer,
                                 bool swapped, const char *name, hipStream_t stream) {
-  const uint64_t grid = (uint64_t)d.chunks * d.spans;
+  const uint64_t grid = outer ? d.spans : (uint64_t)d.chunks * d.spans;
   if (grid > 0xffffffffull / C::NT) return hipErrorInvalidValue;  // 2^32 work-items a dispatch
-  if (out)
+  if (outer)
+    EO_TIMED(name, stream,
+             hipLaunchKernelGGL(k_join_direct_outer<C>, dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, (uint32_t)nR,
+                                S, (uint32_t)nS, d.span, out, out_cap, cursor, (int)wide, outer));
+  else if (out)
     EO_TIMED(name, stream,
              hipLaunchKernelGGL((k_join_direct<C, true>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
-                                d.chunk, d.chunks, d.span, out, out_cap, cursor, (int)wide, matched, (int)swapped));
+                                d.chunk, d.chunks, d.span, out, out_cap, cursor, (int)wide, (int)swapped));
   else
     EO_TIMED(name, stream,
              hipLaunchKernelGGL((k_join_direct<C, false>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
-                                d.chunk, d.chunks, d.span, nullptr, 0ull, cursor, 0, matched, 0));
+                                d.chunk, d.chunks, d.span, nullptr, 0ull, cursor, 0, 0));
   return hipGetLastError();
 }
 
 hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, const eo_tuple *S, uint64_t nS,
-                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched,
+                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer,
                        bool swapped, const char *name, hipStream_t stream) {
-  if (nR == 0 || nS == 0) return hipSuccess;
+  if (nS == 0 || (nR == 0 && !outer)) return hipSuccess;
   const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
   uint2 *vout = reinterpret_cast<uint2 *>(out);
 #define EO_DIRECT(C) \
-  launch_direct<tile::C>(d, vR, nR, vS, nS, vout, out_cap, out_cursor, wide, matched, swapped, name, stream)
+  launch_direct<tile::C>(d, vR, nR, vS, nS, vout, out_cap, out_cursor, wide, outer, swapped, name, stream)
   switch (d.table) {
     case kFusedTableFull: return EO_DIRECT(ProbeBig);
     case kFusedTableHalf: return EO_DIRECT(ProbeSmall);

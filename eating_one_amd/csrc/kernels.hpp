@@ -102,6 +102,36 @@ hipError_t partition_seg_pass(const SegPassPlan &p, const eo_tuple *in, eo_tuple
 hipError_t partition_bounds(const eo_tuple *sorted, uint64_t n, int bits, int shift,
                             uint32_t xor_mask, uint32_t *part_start, hipStream_t stream);
 
+// ---- onepass.hip -------------------------------------------------------------
+// One-pass partition of both relations of a fused join in three launches, the
+// last of them the probe's tile plan.  Up to 10 bits (at 11 the scatter's
+// staging tile and digit arrays fill the LDS, and two passes are faster).
+constexpr int kOneMaxBits = 10;
+constexpr uint32_t kOneCopies = 8;
+struct OneRel {
+  const uint2 *in;  // 16-byte aligned
+  uint2 *out;       // one_pass_rows tuples
+  uint64_t n, budget;
+  uint32_t units, tiles;  // counting workgroups, scatter tiles
+  uint32_t sampled;
+  uint32_t *start, *end, *cur;  // 2^bits each: partition p is out[start[p], end[p])
+};
+struct OneArgs {
+  OneRel rel[2];     // R, S
+  uint32_t *hs;      // 2 kOneCopies one_hs_words(bits) words, zero on entry and again on completion
+  uint32_t *ticket;  // 2 words, likewise
+};
+__host__ __device__ inline constexpr uint32_t one_hs_words(int bits) { return (1u << bits) + 2u; }
+uint64_t one_pass_rows(uint64_t n, int bits);
+bool one_pass_supported(uint64_t nR, uint64_t nS, int bits);
+OneRel one_pass_rel(const eo_tuple *in, uint64_t n, int bits, eo_tuple *out, uint32_t *start, uint32_t *end,
+                    uint32_t *cur);
+// tile_start: 2^bits + 1; *n_tiles: their number.  cap: R tuples per probe
+// tile; outer: the tiles of join_fused's left outer joins.  A partition that
+// proves too small raises kErrCapacity in *err.
+hipError_t one_pass_partition(const OneArgs &a, int bits, uint32_t s_span, uint32_t cap, bool outer,
+                              uint32_t *tile_start, uint64_t *n_tiles, uint32_t *err, hipStream_t stream);
+
 // ---- hashjoin.hip -----------------------------------------------------------
 // Scratch of join_fused_plan's scan over the P + 1 tile counts.
 size_t join_plan_scratch_bytes(uint32_t parts);
@@ -118,7 +148,7 @@ uint32_t join_fused_cap(uint32_t lds_cap);
 hipError_t join_fused_plan(uint32_t parts, uint32_t s_span, uint32_t cap, const uint32_t *r_start,
                            const uint32_t *r_end, const uint32_t *s_start, const uint32_t *s_end,
                            uint32_t *tile_start, uint64_t *n_tiles_dev, void *scan_scratch, uint32_t *err,
-                           hipStream_t stream);
+                           hipStream_t stream, bool outer = false);
 // Grid of join_fused for `parts` partitions of nR x nS tuples, sized without
 // the tile count (tiles_est: the host's estimate of it).
 uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tiles_est, int cus);
@@ -126,22 +156,27 @@ uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tile
 // is correct; a tile count of 2^31 or more raises kErrOverflow in *err and
 // probes nothing).
 // wide: out holds 16-byte RESULT rows {R payload, key, S payload, key};
-// matched (optional): bitmap over S positions of the tuples that matched.
+// outer (optional): a left outer join — a null row per S tuple without a match
+// comes with the other rows, the plan is join_fused_plan's for outer joins, and
+// `outer` is scratch of outer_words(rows of the S buffer, spans) words (no
+// contents expected) for partitions whose R side takes several tables.
 // swapped: R is the caller's S and S its R (the smaller relation built into
 // the tables); the rows are written with the payloads exchanged.
 hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
                       const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
                       const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
-                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched, uint32_t *err,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer, uint32_t *err,
                       hipStream_t stream, bool swapped = false);
+size_t outer_words(uint64_t s_rows, uint64_t spans);
 // One launch of the integer VALU probe `kind` (EO_VALU_COMPARE / EO_VALU_ADD)
 // over `blocks` 256-thread blocks; *ops = the operations it performs.
 hipError_t valu_kernel(int kind, uint32_t blocks, uint32_t reps, uint64_t *sink, hipStream_t s, double *ops);
 // The unpartitioned join on the host's tile plan, one launch.  *out_cursor must
-// be zero on entry; out == NULL counts only.  name: the launch timer's.
+// be zero on entry; out == NULL counts only; outer: as join_fused's.  name: the
+// launch timer's.
 struct DirectPlan;
 hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, const eo_tuple *S, uint64_t nS,
-                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched,
+                       eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer,
                        bool swapped, const char *name, hipStream_t stream);
 // Ends a call's device work: writes words[0, n) (n <= 8) and, in host[n], the
 // error flags to pinned host memory, and clears both on the device, so that
@@ -229,8 +264,9 @@ hipError_t partition_msd2(uint64_t n, int bits_hi, int bits_lo, const eo_tuple *
 constexpr uint64_t kGapMinRows = 1ull << 20;
 bool gap_supported(uint64_t n, int bits_hi, int bits_lo);
 // Tuples of a buffer that holds `parts` sampled regions of a relation of n
-// (for n >= kGapMinRows: enough for any sample).
-uint64_t gap_rows(uint64_t n, uint64_t parts);
+// (for n >= kGapMinRows: enough for any sample whose variance is at most kappa
+// times a random one's).
+uint64_t gap_rows(uint64_t n, uint64_t parts, double kappa = 2.0);
 uint64_t gap_tmp_rows(uint64_t n, int bits_hi, int bits_lo);
 uint64_t gap_out_rows(uint64_t n, int bits_hi, int bits_lo);
 size_t gap_scratch_bytes(uint64_t n, int bits_hi, int bits_lo);

@@ -1398,7 +1398,7 @@ bool gap_supported(uint64_t n, int bits_hi, int bits_lo) {
          gap_bound(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax) + n < (1ull << 32);
 }
 
-uint64_t gap_rows(uint64_t n, uint64_t parts) { return gap_bound(n, parts, kGapKappaMax); }
+uint64_t gap_rows(uint64_t n, uint64_t parts, double kappa) { return gap_bound(n, parts, kappa); }
 
 uint64_t gap_tmp_rows(uint64_t n, int bits_hi, int /*bits_lo*/) {
   return gap_bound(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax);

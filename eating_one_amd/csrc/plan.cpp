@@ -27,8 +27,14 @@ eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *o, HashPl
   // extra radix bit lands in the second pass (which moves the same bytes),
   // and two probe workgroups per CU hide each other's barrier and atomic
   // round trips (C2, 2^27 x 2^28: probe 1.32 -> 1.08 ms, join 5.09 -> 4.93 ms;
-  // deterministic order 7.35 -> 6.86 ms).
-  if (!cap_opt && !bits_opt && nR > 16384 && ceil_log2((nR + 16383) / 16384) > kMaxPassBits) p.lds_cap = 8192u;
+  // deterministic order 7.35 -> 6.86 ms).  The fused order takes two passes
+  // from 11 bits on: a tile's runs of 2048 digits are 64 bytes (30 M x 60 M
+  // tuples: 1.14 ms in one pass of 11 bits, 0.99 in two of 6; 2^24 x 2^25: 0.57
+  // in one of 10, 0.64 in two).
+  const bool det = o && (o->flags & EO_F_DETERMINISTIC);
+  if (!cap_opt && !bits_opt && nR > 16384 &&
+      ceil_log2((nR + 16383) / 16384) > (det ? kMaxPassBits : kOneMaxBits))
+    p.lds_cap = 8192u;
   if (bits_opt == -1) {
     p.bits = 0;
   } else if (bits_opt > 0) {
@@ -81,25 +87,29 @@ eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *o, HashPl
   return EO_OK;
 }
 
-DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus) {
-  // Time model of a tile in microseconds, fitted to joins of 300 to 131072 by
-  // 4000 to 2^24 tuples on each table: a workgroup's fixed cost, per R tuple
-  // built, per S tuple probed; and every S batch's output reservation, an
-  // atomic on one word of the whole device (about 100 million a second).
-  // 2^16 x 2^20: full tables 22 us, half 35, quarter 108; 1000 x 4000: 3.1,
-  // 1.8, 1.2 (each beside 18.5 of launches and the readback).
-  struct Table {
-    uint32_t cap, batch, per_cu;  // tuples, S tuples per batch, workgroups per CU
-    double fixed, build, probe;
-  };
-  constexpr double kAtomic = 0.010;
-  const Table tables[] = {{kFusedTableFull, 8192, 1, 2.0, 1.5e-4, 6e-4},
-                          {kFusedTableHalf, 4096, 2, 1.2, 2e-4, 1e-3},
-                          {kFusedTableQuarter, 2048, 4, 0.8, 2e-4, 7e-4}};
+namespace {
+// Time model of a probe tile in microseconds, fitted to joins of 300 to 131072
+// by 4000 to 2^24 tuples on each table: a workgroup's fixed cost, per R tuple
+// built, per S tuple probed; and every S batch's output reservation, an
+// atomic on one word of the whole device (about 100 million a second).
+// 2^16 x 2^20 unpartitioned: full tables 22 us, half 35, quarter 108; 1000 x
+// 4000: 3.1, 1.8, 1.2 (each beside 18.5 of launches and the readback).
+struct ProbeTable {
+  uint32_t cap, batch, per_cu;  // tuples, S tuples per batch, workgroups per CU
+  double fixed, build, probe;
+  double tile(double r, double s) const { return fixed + build * r + probe * s; }
+};
+constexpr double kAtomicUs = 0.010;
+constexpr ProbeTable kProbeTables[] = {{kFusedTableFull, 8192, 1, 2.0, 1.5e-4, 6e-4},
+                                       {kFusedTableHalf, 4096, 2, 1.2, 2e-4, 1e-3},
+                                       {kFusedTableQuarter, 2048, 4, 0.8, 2e-4, 7e-4}};
+}  // namespace
+
+DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus, bool outer) {
   const int cap_opt = o ? o->lds_tuples : 0, span_opt = o ? o->s_tile : 0;
   const uint64_t n_cu = (uint64_t)std::max(cus, 8);
   DirectPlan best;
-  for (const Table &t : tables) {
+  for (const ProbeTable &t : kProbeTables) {
     if (cap_opt && fused_table_tuples((uint32_t)cap_opt, true) != t.cap) continue;
     DirectPlan d;
     d.table = t.cap;
@@ -108,17 +118,54 @@ DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus)
     d.chunks = (uint32_t)std::max<uint64_t>(1, (nR + d.chunk - 1) / d.chunk);
     const uint64_t slots = n_cu * t.per_cu, batches = std::max<uint64_t>(1, (nS + t.batch - 1) / t.batch);
     // as many S spans as fill the chip once, of whole batches
-    uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / d.chunks));
+    const uint64_t side = outer ? 1 : d.chunks;  // chunks of a span that run beside each other
+    uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / side));
     uint64_t span = (batches + spans - 1) / spans * t.batch;
     if (span_opt) span = std::max<uint64_t>(t.batch, (uint64_t)span_opt);
     span = std::min<uint64_t>(span, 1u << 30);
     spans = std::max<uint64_t>(1, (nS + span - 1) / span);
     d.span = (uint32_t)span;
     d.spans = (uint32_t)spans;
-    const double waves = (double)((d.chunks * spans + slots - 1) / slots);
-    d.us = waves * (t.fixed + t.build * d.chunk + t.probe * (double)std::min(span, nS)) +
-           kAtomic * (double)d.chunks * (double)batches;
+    const double waves = (double)((side * spans + slots - 1) / slots) * (double)(d.chunks / side);
+    d.us = waves * t.tile(d.chunk, (double)std::min(span, nS)) + kAtomicUs * (double)d.chunks * (double)batches;
     if (!best.table || d.us < best.us) best = d;
+  }
+  return best;
+}
+
+double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p) {
+  // launches: counts, scatter, tile plan (measured at 3.4 M to 50 M tuples of 5
+  // to 10 bits: 9 to 21 us, 18 to 227 us, 5 us); more digits cut the scatter's
+  // runs short
+  const double n = (double)nR + (double)nS, fixed = 9 + 0.25e-6 * n + 5;
+  const uint64_t n_cu = (uint64_t)std::max(cus, 8);
+  double best = 0;
+  for (const ProbeTable &t : kProbeTables) {
+    if (t.cap == kFusedTableQuarter) continue;  // unpartitioned joins only
+    const uint32_t lds = t.cap == kFusedTableFull ? 16384 : 8192;
+    const int b0 = std::max(1, ceil_log2((nR + lds - 1) / lds));
+    for (int b = b0; b <= std::min(b0 + 5, kOneMaxBits); ++b) {
+      const double scatter = 8 + 3.7e-6 * n * (b <= 8 ? 1.0 : b == 9 ? 1.07 : 1.22);
+      const uint64_t P = 1ull << b, slots = n_cu * t.per_cu;
+      const double r = (double)nR / P, s = (double)nS / P;
+      for (uint64_t k = 1; k <= 16; k *= 2) {  // spans per partition
+        if (k > 1 && s / k < t.batch) break;
+        // tiles a little over the mean: a partition's length varies
+        const double us = fixed + scatter + (double)((P * k + slots - 1) / slots) * t.tile(r, s / k) +
+                          kAtomicUs * P * k * std::max(1.0, s / k / t.batch);
+        if (best == 0 || us < best) {
+          best = us;
+          p->bits = p->bits_pass1 = b;
+          p->bits_pass2 = 0;
+          p->passes = 1;
+          p->lds_cap = lds;
+          // half as long again as the mean share, so that ordinary partitions
+          // stay k tiles and one grown by skewed keys still splits
+          const uint64_t span = (uint64_t)(1.5 * s / k) + t.batch - 1;
+          p->s_span = (uint32_t)std::min<uint64_t>(span / t.batch * t.batch, 1u << 20);
+        }
+      }
+    }
   }
   return best;
 }

@@ -51,8 +51,14 @@ struct DirectPlan {
   uint32_t span = 0, spans = 0;
   double us = 0;  // the time model's estimate of the launch
 };
-// opts: lds_tuples and s_tile overrides (0: chosen here).
-DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *opts, int cus);
+// opts: lds_tuples and s_tile overrides (0: chosen here).  outer: a left outer
+// join, whose spans take the chunks one after the other.
+DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *opts, int cus, bool outer = false);
+
+// The plan of a fused join of one pass that partitions both relations together
+// (kernels.hpp, OneArgs): fills bits, table and span of *p and returns the time
+// model's estimate of the whole join in microseconds.
+double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p);
 
 // Returns EO_OK and fills *out, or EO_EINVAL for inconsistent overrides.
 eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *opts, HashPlan *out, int cus = 256);

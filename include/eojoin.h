@@ -137,10 +137,10 @@ typedef struct eo_join_opts {
  * in S order (the hash join's S order is its stable partition's). */
 #define EO_F_LEFT_OUTER 16
 /* Hash join: always partition from a full histogram pass.  By default a
- * fused inner join of two passes and at least 2^20 tuples per relation sizes
- * its partitions from a 1/16 sample instead (one read of the input less) and
- * redoes the join exactly if the sample underestimated a partition; the rows
- * are the same either way. */
+ * fused join of one pass (inner or left outer), or an inner one of two, sizes
+ * the partitions of a relation of at least 2^20 tuples from a 1/16 sample
+ * instead (one read of the input less) and redoes the join exactly if the
+ * sample underestimated a partition; the rows are the same either way. */
 #define EO_F_EXACT_PARTITIONS 32
 #define EO_NULL_PAYLOAD ((int32_t)0x80000000)
 
