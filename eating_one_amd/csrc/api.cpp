@@ -163,7 +163,7 @@ eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const 
   if (hp.passes == 1) {
     // fixed order: the ordered fast scatter up to 7 bits, else the stable one
     const bool fast = aligned16(in) && !stable && (!fixed || hp.bits_pass1 <= 7);
-    PartPassPlan pp = plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, fast);
+    PartPassPlan pp = plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, fast, hp.stable_stripes);
     pp.ordered = fast && fixed;
     EO_TRY_HIP(partition_pass(pp, in, out, part_start, scratch, ctx->d_err, s), "partition pass");
     return EO_OK;
@@ -186,8 +186,8 @@ eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const 
     EO_TRY_HIP(partition_seg_pass(p2, tmp, out, start1, part_start, rest, ctx->d_err, s), "partition pass 2");
     return EO_OK;
   }
-  PartPassPlan p1 = plan_partition_pass(n, b_lo, 0, 0u, cus);
-  PartPassPlan p2 = plan_partition_pass(n, b_hi, b_lo, 0u, cus);
+  PartPassPlan p1 = plan_partition_pass(n, b_lo, 0, 0u, cus, false, hp.stable_stripes);
+  PartPassPlan p2 = plan_partition_pass(n, b_hi, b_lo, 0u, cus, false, hp.stable_stripes);
   EO_TRY_HIP(partition_pass(p1, in, tmp, nullptr, scratch, ctx->d_err, s), "partition pass 1");
   EO_TRY_HIP(partition_pass(p2, tmp, out, nullptr, scratch, ctx->d_err, s), "partition pass 2");
   EO_TRY_HIP(partition_bounds(out, n, hp.bits, 0, 0u, part_start, s), "partition bounds");
@@ -195,15 +195,16 @@ eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const 
 }
 
 size_t partition_scratch(uint64_t n, const HashPlan &hp, int cus) {
+  const uint32_t most = hp.stable_stripes;
   size_t b = 0;
   if (hp.passes == 1) {
     b = std::max(partition_pass_scratch_bytes(plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, true)),
-                 partition_pass_scratch_bytes(plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, false)));
+                 partition_pass_scratch_bytes(plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, false, most)));
   } else if (hp.passes == 2) {
     const int b_lo = hp.bits_pass1, b_hi = hp.bits_pass2;
     const size_t head = (((1u << b_hi) + 1) * sizeof(uint32_t) + 255) / 256 * 256;
-    b = std::max(partition_pass_scratch_bytes(plan_partition_pass(n, b_lo, 0, 0u, cus)),
-                 partition_pass_scratch_bytes(plan_partition_pass(n, b_hi, b_lo, 0u, cus)));
+    b = std::max(partition_pass_scratch_bytes(plan_partition_pass(n, b_lo, 0, 0u, cus, false, most)),
+                 partition_pass_scratch_bytes(plan_partition_pass(n, b_hi, b_lo, 0u, cus, false, most)));
     b = std::max(b, head + partition_pass_scratch_bytes(plan_partition_pass(n, b_hi, b_lo, 0u, cus, true)));
     b = std::max(b, head + seg_pass_scratch_bytes(plan_seg_pass(n, 1u << b_hi, b_lo, 0, cus)));
     if (msd2_supported(b_hi, b_lo)) b = std::max(b, msd2_scratch_bytes(n, b_hi, b_lo, cus));
@@ -632,6 +633,9 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     else
       hp.bits = hp.bits_pass1 = hp.passes = 0;
   }
+  // the fixed scratch holds the counts of this many stripes of a stable pass
+  // (inputs that are not 16-byte aligned)
+  if (fx) hp.stable_stripes = kNoAllocStripes;
   DeviceGuard g(c->device);
   hipStream_t s = pick_stream(c, o);
   const uint32_t P = 1u << hp.bits;
@@ -666,9 +670,8 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_ts = L.add((P + 1) * sizeof(uint32_t));
   const DirectPlan dp = direct ? plan_direct(nR, nS, &eff, c->props.cus, outer) : DirectPlan{};
   const uint64_t spans = direct ? dp.spans : (uint64_t)P + nS / hp.s_span + 1;
-  const size_t o_bits = L.add(!outer ? 0
-                              : deterministic ? matched_words(nS) * sizeof(uint32_t)
-                                              : outer_words(hp.passes ? sp_rows : nS, spans) * sizeof(uint32_t));
+  const size_t outer_bytes = outer ? outer_words(hp.passes ? sp_rows : nS, spans) * sizeof(uint32_t) : 0;
+  const size_t o_bits = L.add(outer && deterministic ? matched_words(nS) * sizeof(uint32_t) : outer_bytes);
   const uint64_t ublocks = outer && deterministic ? unmatched_blocks(nS) : 0;  // null rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);
@@ -682,7 +685,10 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_tc = L.add(tiles_est * sizeof(uint64_t) + scan_scratch_bytes_u64(tiles_est));
   char *A = nullptr;
   if (fx) {  // the caller's fixed scratch: no allocation, no synchronisation
-    if (L.total > fx->cap) {
+    // (the spans' bitmaps take a little more than one bit a row: the buffer has
+    // room for that beyond its nominal size, so the sizes that fit stay the same)
+    const size_t over = std::min<size_t>(fx->slack, outer ? 8 * spans + 16 : 0);
+    if (L.total > fx->cap + over) {
       set_last_error("hash join needs " + std::to_string(L.total) + " bytes of scratch, the fixed buffer holds " +
                      std::to_string(fx->cap));
       return EO_EINVAL;

@@ -144,7 +144,11 @@ void fold_timer(const LaunchTimer &t, eo_join_stats *stats);
 struct FixedScratch {
   char *base;
   size_t cap;
+  size_t slack;  // bytes past cap, for left outer joins' bitmaps only
 };
+// Stripes of a stable partition pass in fixed scratch: 4 bytes per stripe and
+// digit (4096 stripes of 9 bits would take 8 MiB of it).
+constexpr uint32_t kNoAllocStripes = 1024;
 // eo_hash_join; with fx, its scratch comes from [fx->base, fx->base + cap)
 // (a join that needs more is refused with EO_EINVAL) and nothing is
 // allocated or synchronised before the kernels are enqueued.

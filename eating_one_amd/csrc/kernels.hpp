@@ -72,7 +72,9 @@ struct PartPassPlan {
   bool ordered = false;  // fast, <= 7 bits: ranks fixed by the input (the same positions on every run)
 };
 // fast = false: stable scatter (ballot-ranked), equal to the CPU_JOIN partition.
-PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_mask, int cus, bool fast = false);
+// most: a stable pass's stripes at most (0 = the pass's own bound).
+PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_mask, int cus, bool fast = false,
+                                 uint32_t most = 0);
 size_t partition_pass_scratch_bytes(const PartPassPlan &p);
 // counts -> scan -> scatter.  part_start (optional, 2^bits+1 u32 entries, device)
 // receives the partition start offsets of this pass.

@@ -1233,7 +1233,8 @@ uint32_t tile_of_bits(int bits) {
 
 }  // namespace
 
-PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_mask, int cus, bool fast) {
+PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_mask, int cus, bool fast,
+                                 uint32_t most_stripes) {
   PartPassPlan p{};
   p.n = n;
   p.bits = bits;
@@ -1254,7 +1255,8 @@ PartPassPlan plan_partition_pass(uint64_t n, int bits, int shift, uint32_t xor_m
     len = (n + g - 1) / g;
     len = std::max<uint64_t>(tile, (len + 1) & ~1ull);
   } else {
-    const uint64_t most = kStableStripes >> std::max(0, bits - 8);
+    uint64_t most = kStableStripes >> std::max(0, bits - 8);
+    if (most_stripes) most = std::min<uint64_t>(most, most_stripes);
     const uint64_t per = (tiles + most - 1) / most;
     len = per * tile;
     g = ((tiles + per - 1) / per + kXcds - 1) / kXcds * kXcds;

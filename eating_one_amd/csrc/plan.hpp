@@ -22,6 +22,7 @@ struct HashPlan {
   uint32_t lds_cap = 0;
   uint32_t s_tile = 0;  // S tuples per tile of the deterministic count/write path
   uint32_t s_span = 0;  // S tuples per tile of the fused probe
+  uint32_t stable_stripes = 0;  // stripes of a stable partition pass at most (0 = the pass's bound)
 };
 
 constexpr int kMaxJoinBits = 22;

@@ -74,3 +74,20 @@ def test_noalloc_refuses_what_needs_allocation(ctx):
     assert st == 0 and n_ok == ctx.hash_join_device(dR, 1000, dS, 2000, None, 0)[0]
     for d in (dbig, dout, dS, dR):
         d.close()
+
+
+def test_noalloc_unaligned_near_its_limit(ctx):
+    """7.95 M tuples of 9 radix bits, R and S off 16-byte alignment: their partition pass must not
+    ask for more counts than the fixed buffer has beside the tuples (2 MiB: 1024 stripes)."""
+    nR, nS = 7_650_000, 300_000
+    dR, dS = DeviceArray(ctx, 8 * (nR + 1)), DeviceArray(ctx, 8 * (nS + 1))
+    ctx.gen_build(dR, nR + 1, seed=5)
+    ctx.gen_probe(dS, nS + 1, nR, 0.5, seed=6)
+    n, m = ctypes.c_uint64(), ctypes.c_uint64()
+    o = ctx.opts(where=_abi.EO_DEVICE, left_outer=True)
+    args = (dR.ptr + 8, nR, dS.ptr + 8, nS, None, 0)
+    assert ctx.lib.eo_hash_join_noalloc(ctx.handle, *args, ctypes.byref(n), ctypes.byref(o)) == _abi.EO_OK
+    assert ctx.lib.eo_hash_join(ctx.handle, *args, ctypes.byref(m), ctypes.byref(o)) == _abi.EO_OK
+    assert n.value == m.value >= nS
+    dR.close()
+    dS.close()
