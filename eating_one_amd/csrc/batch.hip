@@ -113,14 +113,14 @@ __global__ __launch_bounds__(kFastNT) void k_bseg_scatter(const BatchSeg *__rest
     if (threadIdx.x == 0) s_err = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
       sh.cursor[d] = sg.re[d];
-      sh.cnt[d] = 0;
+      sh.clear_count(d);
     }
   } else {
     const uint64_t base = offsets[sg.count_base];  // tuples of the group's earlier relations
     for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
       const uint32_t c = (uint32_t)(offsets[sg.count_base + (uint64_t)d * sg.nstripes + s] - base);
       sh.cursor[d] = c;
-      sh.cnt[d] = 0;
+      sh.clear_count(d);
       // the relation's first stripe starts every digit: its offsets are the
       // partition starts (relative to the relation)
       if (s == 0) sg.part_start[d] = c;

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kFastNT) void k_one_scatter(OneArgs a, uint32_t *er
   if (threadIdx.x == 0) s_err = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
     sh.cursor[d] = r.end[d];
-    sh.cnt[d] = 0;
+    sh.clear_count(d);
   }
   tile::scatter_stripe<BITS, false, true>(sh, r.in, beg, end, r.n, 0, 0u, r.out, err, r.cur, &s_err);
 }

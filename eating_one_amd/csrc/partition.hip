@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kFastNT) void k_part_scatter_fast(const uint2 *__re
   if (!stripe_of<(1 << BITS)>(geo, g, 0, &sr, true)) return;
   for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
     sh.cursor[d] = offsets[sr.cidx0 + (uint64_t)d * sr.cstride];
-    sh.cnt[d] = 0;
+    sh.clear_count(d);
   }
   tile::scatter_stripe<BITS, ORDERED>(sh, in, sr.beg, sr.end, geo.n, shift, xm, out, err);
 }
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(kFastNT) void k_tile_scatter(const uint2 *__restric
   if (RES && threadIdx.x == 0) s_err = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
     sh.cursor[d] = RES ? offsets[((uint64_t)rx << BITS) + d] : offsets[(uint64_t)d * T + t];
-    sh.cnt[d] = 0;
+    sh.clear_count(d);
   }
   tile::scatter_stripe<BITS, ORDERED, RES>(sh, in, beg, end, n, shift, 0u, out, err,
                                            RES ? res + ((uint64_t)rx << BITS) : nullptr, RES ? &s_err : nullptr);
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(kFastNT) void k_msd_scatter(const uint2 *__restrict
     const uint64_t end = c1 == (uint64_t)F1 * G ? n : off1[c1 * K];
     for (uint32_t d = threadIdx.x; d < F2; d += kFastNT) {
       sh.cursor[d] = off2[((uint64_t)dh * F2 + d) * G + g0];
-      sh.cnt[d] = 0;
+      sh.clear_count(d);
     }
     __syncthreads();
     tile::scatter_stripe<BL, ORDERED>(sh, in, beg, end, n, 0, 0u, out, err);
@@ -1111,7 +1111,7 @@ __global__ __launch_bounds__(kFastNT) void k_gap_scatter(const uint2 *__restrict
     const uint64_t end = j + 1 == J ? b0 + len : b0 + (((uint64_t)(j + 1) * len / J) & ~1ull);
     for (uint32_t d = threadIdx.x; d < F2; d += kFastNT) {
       sh.cursor[d] = re2[(uint64_t)h * F2 + d];
-      sh.cnt[d] = 0;
+      sh.clear_count(d);
     }
     __syncthreads();
     tile::scatter_stripe<BL, false, true>(sh, in, beg, end, 0, 0, 0u, out, err, cur2 + (uint64_t)h * F2);

@@ -91,3 +91,20 @@ def test_sample_too_small_redoes_the_join(ctx):
     R = np.stack([rng.permutation(200_000), np.arange(200_000)], 1).astype(np.int32)
     _check(ctx, R, S, 2, radix_bits=6, passes=1)
     assert same_multiset(ctx.hash_join(R[:5000], S[:9000]), brute_join(R[:5000], S[:9000]))
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("order", ["random", "sorted", "one digit"])
+@pytest.mark.parametrize("flags", [0, _abi.EO_F_EXACT_PARTITIONS])
+def test_few_digits(ctx, bits, order, flags):
+    """Few digits are counted in several copies each: waves of mixed and of single digits, tiles
+    that end anywhere, in the reserving scatter (flags = 0) and the counted one."""
+    nR, nS = 16384 + 129, 3 * 16384 + 77
+    R, S = _relations(nR, nS, nR, bits)
+    if order == "sorted":
+        R, S = R[np.argsort(R[:, 0])], S[np.argsort(S[:, 0])]
+        R[:, 0] >>= 1  # runs of equal digits
+    elif order == "one digit":
+        R[:, 0] &= -64
+        S[:, 0] &= -64
+    _check(ctx, R, S, 0, outer=False, radix_bits=bits, passes=1, flags=flags)
