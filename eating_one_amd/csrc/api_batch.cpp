@@ -66,7 +66,7 @@ struct eo_batch {
   eo::Arena arena;
   char *h_blob = nullptr;  // pinned descriptor staging
   size_t h_blob_cap = 0;
-  uint64_t *h_counts = nullptr;  // pinned per-join counts
+  uint64_t *h_counts = nullptr;  // pinned per-join counts, capacity flag, error flags
   size_t h_counts_cap = 0;
   hipEvent_t done = nullptr;
   hipEvent_t t0 = nullptr, t1 = nullptr;  // batch start / end (stats only)
@@ -87,7 +87,7 @@ struct eo_batch {
     size_t o_hs = 0;  // sampled groups: the relations' sampled counts (arena)
   };
   std::vector<Group> groups;
-  size_t o_blob = 0, blob_bytes = 0, o_cursor = 0, o_head = 0, o_counts = 0, o_cscr = 0, o_tmp = 0, o_pscr = 0,
+  size_t o_blob = 0, blob_bytes = 0, o_cursor = 0, o_counts = 0, o_cscr = 0, o_tmp = 0, o_pscr = 0,
          o_pair = 0, o_tiles = 0, o_tscr = 0, o_tdesc = 0;
   uint32_t tiles_cap = 0;  // probe tile descriptors written ahead of the probe
   size_t o_joins_blob = 0;
@@ -131,6 +131,7 @@ eo_status plan_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo_j
   b->joins.clear();
   b->req_join.assign(n, -1);
   group_members.assign(2 * (kMaxGroupBits + 1), {});  // [bits]: exact groups, [kMaxGroupBits + 1 + bits]: sampled
+  // (exact relations of up to kBatchSmallBits share that group)
   b->any_sampled = false;
   uint64_t max_tmp = 0;
   size_t max_pscr = 0;
@@ -219,7 +220,7 @@ eo_status plan_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo_j
       }
       if (group) {
         sd.mode = 1;
-        group_members[J.hp.bits + (sd.sampled ? kMaxGroupBits + 1 : 0)].push_back({(uint32_t)b->joins.size(), which});
+        group_members[sd.sampled ? kMaxGroupBits + 1 + J.hp.bits : std::max(J.hp.bits, kBatchSmallBits)].push_back({(uint32_t)b->joins.size(), which});
       } else {
         sd.mode = 2;
         if (J.hp.passes == 2) max_tmp = std::max(max_tmp, cnt);
@@ -271,7 +272,7 @@ eo_status plan_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo_j
       const uint64_t ns = (sd.n + len - 1) / len;
       stripes += ns;
       if (sampled) samp += (sd.n + kPartTile * kBatchSampleTiles - 1) / (kPartTile * kBatchSampleTiles);
-      else counts += ns << bits;
+      else counts += ns << b->joins[m.first].hp.bits;
     }
     if (stripes >= (1ull << 31) || samp >= (1ull << 31)) return EO_EINVAL;
     G.g.total_stripes = (uint32_t)stripes;
@@ -295,8 +296,7 @@ eo_status plan_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo_j
   blob_bytes = (blob + 15) / 16 * 16;
   b->o_blob = L.add(blob_bytes);
   b->o_bits = L.add(b->bits_words * sizeof(uint32_t));
-  b->o_cursor = L.add(((size_t)nj + 1) * sizeof(uint64_t));  // per-join counts, then the capacity flag
-  b->o_head = L.add(sizeof(uint64_t));
+  b->o_cursor = L.add(((size_t)nj + 2) * sizeof(uint64_t));  // per-join counts, the capacity flag, the queue head
   b->o_counts = L.add(max_counts * sizeof(uint64_t));
   b->o_cscr = L.add(max_counts ? scan_scratch_bytes_u64(max_counts) : 0);
   b->o_tmp = L.add(part_bytes(max_tmp));
@@ -382,6 +382,7 @@ void fill_blob(eo_batch *b, const std::vector<std::vector<std::pair<uint32_t, in
       sg.in = reinterpret_cast<const uint2 *>(sd.in);
       sg.out = reinterpret_cast<uint2 *>(A + sd.o_part);
       sg.n = sd.n;
+      sg.bits = (uint32_t)b->joins[mem[k].first].hp.bits;
       sg.stripe_base = stripe_base;
       sg.nstripes = (uint32_t)((sd.n + len - 1) / len);
       sg.count_base = count_base;
@@ -397,7 +398,7 @@ void fill_blob(eo_batch *b, const std::vector<std::vector<std::pair<uint32_t, in
         sg.budget = sd.budget;
         samp_base += sg.nsamp;
       } else {
-        count_base += (uint64_t)sg.nstripes << bits;
+        count_base += (uint64_t)sg.nstripes << sg.bits;
       }
       stripe_base += sg.nstripes;
       hs[k] = sg;
@@ -414,11 +415,10 @@ eo_status enqueue_batch(eo_batch *b, hipStream_t s) {
   char *A = b->arena.base;
   const uint32_t nj = (uint32_t)b->joins.size();
   uint64_t *cursor = reinterpret_cast<uint64_t *>(A + b->o_cursor);
-  uint32_t *head = reinterpret_cast<uint32_t *>(A + b->o_head);
   if (nj == 0) return EO_OK;
-  EO_TRY_HIP(fill_u64(cursor, 0, (uint64_t)nj + 1, s), "cursor reset");  // counts and the capacity flag
+  EO_TRY_HIP(fill_u64(cursor, 0, (uint64_t)nj + 2, s), "cursor reset");  // counts, capacity flag, queue head
   uint32_t *cap_flag = reinterpret_cast<uint32_t *>(cursor + nj);
-  EO_TRY_HIP(fill_u32(head, 0u, 1, s), "queue reset");
+  uint32_t *head = reinterpret_cast<uint32_t *>(cursor + nj + 1);
   if (b->outer)
     EO_TRY_HIP(fill_u32(reinterpret_cast<uint32_t *>(A + b->o_bits), 0u, b->bits_words, s), "match bitmap reset");
   uint64_t *counts = reinterpret_cast<uint64_t *>(A + b->o_counts);
@@ -446,8 +446,7 @@ eo_status enqueue_batch(eo_batch *b, hipStream_t s) {
     EO_TRY_HIP(batch_emit_unmatched(dj, nj, reinterpret_cast<const uint32_t *>(A + b->o_blob + b->o_emit),
                                     b->emit_blocks, s),
                "outer rows");
-  EO_TRY_HIP(hipMemcpyAsync(b->h_counts, cursor, ((size_t)nj + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s),
-             "count readback");
+  EO_TRY_HIP(batch_publish(cursor, nj + 1, c->d_err, b->h_counts, s), "count readback");
   return EO_OK;
 }
 
@@ -644,7 +643,7 @@ eo_status submit_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo
                "blob staging");
     b->h_blob_cap = std::max<size_t>(blob_bytes, 4096);
   }
-  const size_t ncnt = b->joins.size() + 1;  // the counts and the capacity flag
+  const size_t ncnt = b->joins.size() + 2;  // the counts, the capacity flag and the error flags
   if (ncnt > b->h_counts_cap) {
     if (b->h_counts) (void)hipHostFree(b->h_counts);
     b->h_counts = nullptr;
@@ -753,9 +752,17 @@ eo_status eo_batch_wait(eo_batch *b, eo_result *res, uint32_t n) {
   for (;;) {
     b->in_flight = false;
     EO_TRY_HIP(hipEventSynchronize(b->done), "batch wait");
-    eo_status st = check_device_errors(c, b->stream);
-    if (st != EO_OK) return st;
+    // (the error flags came with the counts; a copy of their own cost 36 us)
     const size_t nj = b->joins.size();
+    eo_status st = EO_OK;
+    if (nj == 0 || b->h_counts[nj + 1]) {
+      st = check_device_errors(c, b->stream);  // and clears them
+      if (st == EO_OK && nj) {  // cleared by another call meanwhile: this batch still failed
+        set_last_error("device error flags 0x" + std::to_string(b->h_counts[nj + 1]));
+        st = EO_EINTERNAL;
+      }
+    }
+    if (st != EO_OK) return st;
     if (!(b->any_sampled && nj && (b->h_counts[nj] & kErrCapacity))) break;
     // a sampled partition was too small: its join's rows are incomplete, so
     // the whole batch runs again with exact partitions (same requests and

@@ -5,10 +5,10 @@
 // of small and medium joins those launch and sync gaps dominate.  Here a batch
 // of joins runs as a fixed, host-sync-free sequence:
 //   1. partition: the relations of all joins that need the same number of
-//      radix bits form one group; one histogram launch, one u64 scan and one
+//      radix bits (or up to kBatchSmallBits) form one group; one histogram launch, one u64 scan and one
 //      scatter launch partition every relation of the group (each stripe
 //      finds its relation by binary search in a descriptor table);
-//   2. plan: one thread per (join, partition) pair counts its probe tiles,
+//   2. plan: a thread per (join, partition) pair counts its probe tiles,
 //      a scan numbers them, and one thread per tile (up to an estimate of
 //      the count) writes the tile's descriptor;
 //   3. probe: a persistent kernel (one workgroup per CU) drains a device work
@@ -18,6 +18,7 @@
 // The only host interaction is reading the per-join counts at the end, so
 // the whole sequence can also be captured once into a hipGraph and replayed.
 #include <algorithm>
+#include <type_traits>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -72,27 +73,72 @@ __device__ __forceinline__ BatchJoin load_join(const BatchJoin *joins, uint32_t 
   return J;
 }
 
+// f(std::integral_constant<int, b>) for the relation's bits b.  The small
+// group's relations differ in theirs: one launch holds the code of each.  (In
+// a batch of 1024 joins of 2^10 to 2^16 tuples a histogram, scan and scatter
+// for each of three numbers of bits were 9 launches, each with the tail of a
+// few hundred workgroups: 35 + 63 us of histograms and scatters, now 20 + 50;
+// the batch, with its plan in fewer launches too, 375 -> 296 us.)
+template <int BITS, typename Fn>
+__device__ __forceinline__ void with_bits(uint32_t bits, Fn &&f) {
+  if constexpr (BITS == kBatchSmallBits) {
+    static_assert(kBatchSmallBits == 5, "one case per number of bits");
+    switch (__builtin_amdgcn_readfirstlane((int)bits)) {
+      case 1: return f(std::integral_constant<int, 1>{});
+      case 2: return f(std::integral_constant<int, 2>{});
+      case 3: return f(std::integral_constant<int, 3>{});
+      case 4: return f(std::integral_constant<int, 4>{});
+      default: return f(std::integral_constant<int, 5>{});
+    }
+  } else {
+    f(std::integral_constant<int, BITS>{});
+  }
+}
+
+// Also clears the state of the scan that follows (nzero words).
 template <int BITS>
 __global__ __launch_bounds__(kBHistNT) void k_bseg_hist(const BatchSeg *__restrict__ segs, uint32_t nseg,
                                                         uint32_t total_stripes, uint64_t len,
-                                                        uint64_t *__restrict__ counts) {
-  constexpr int F = 1 << BITS;
-  __shared__ uint32_t hist[F];
+                                                        uint64_t *__restrict__ counts, uint64_t *__restrict__ zero,
+                                                        uint32_t nzero) {
+  __shared__ uint32_t hist[1 << BITS];
+  for (uint32_t i = blockIdx.x * kBHistNT + threadIdx.x; i < nzero; i += gridDim.x * kBHistNT) zero[i] = 0ull;
   const uint32_t g = xcd_local_index(blockIdx.x, gridDim.x);
   if (g >= total_stripes) return;
   const BatchSeg sg = load_seg(segs, find_seg(segs, nseg, g));
   const uint32_t s = g - sg.stripe_base;
   const uint64_t beg = (uint64_t)s * len;
   const uint64_t end = beg + len < sg.n ? beg + len : sg.n;
-  for (int d = threadIdx.x; d < F; d += kBHistNT) hist[d] = 0;
-  __syncthreads();
-  tile::hist_stripe<BITS, kBHistNT, true>(hist, sg.in, beg, end, 0, 0u);
-  __syncthreads();
-  for (int d = threadIdx.x; d < F; d += kBHistNT) counts[sg.count_base + (uint64_t)d * sg.nstripes + s] = hist[d];
+  with_bits<BITS>(sg.bits, [&](auto bits) {
+    constexpr int B = decltype(bits)::value, F = 1 << B;
+    for (int d = threadIdx.x; d < F; d += kBHistNT) hist[d] = 0;
+    __syncthreads();
+    tile::hist_stripe<B, kBHistNT, true>(hist, sg.in, beg, end, 0, 0u);
+    __syncthreads();
+    for (int d = threadIdx.x; d < F; d += kBHistNT) counts[sg.count_base + (uint64_t)d * sg.nstripes + s] = hist[d];
+  });
+}
+
+// The exact scatter of one stripe: its offsets come from the scanned counts.
+template <int BITS>
+__device__ __forceinline__ void seg_scatter(tile::ScatterShared<BITS> &sh, const BatchSeg &sg, uint32_t s,
+                                            uint64_t beg, uint64_t end, const uint64_t *__restrict__ offsets,
+                                            uint32_t *err) {
+  const uint64_t base = offsets[sg.count_base];  // tuples of the group's earlier relations
+  for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
+    const uint32_t c = (uint32_t)(offsets[sg.count_base + (uint64_t)d * sg.nstripes + s] - base);
+    sh.cursor[d] = c;
+    sh.clear_count(d);
+    // the relation's first stripe starts every digit: its offsets are the
+    // partition starts (relative to the relation)
+    if (s == 0) sg.part_start[d] = c;
+  }
+  if (s == 0 && threadIdx.x == 0) sg.part_start[1 << BITS] = (uint32_t)sg.n;
+  tile::scatter_stripe<BITS>(sh, sg.in, beg, end, sg.n, 0, 0u, sg.out, err);
 }
 
 // RES (sampled groups): the stripe reserves its runs from the relation's
-// region cursors; otherwise its offsets come from the scanned counts.
+// region cursors; otherwise seg_scatter, in the LDS of the group's most bits.
 template <int BITS, bool RES = false>
 __global__ __launch_bounds__(kFastNT) void k_bseg_scatter(const BatchSeg *__restrict__ segs, uint32_t nseg,
                                                           uint32_t total_stripes, uint64_t len,
@@ -104,31 +150,25 @@ __global__ __launch_bounds__(kFastNT) void k_bseg_scatter(const BatchSeg *__rest
   const uint32_t s = g - sg.stripe_base;
   const uint64_t beg = (uint64_t)s * len;
   const uint64_t end = beg + len < sg.n ? beg + len : sg.n;
+  if constexpr (!RES) {
+    with_bits<BITS>(sg.bits, [&](auto bits) {
+      constexpr int B = decltype(bits)::value;
+      static_assert(sizeof(tile::ScatterShared<B>) <= sizeof(sh), "fewer bits take less LDS");
+      seg_scatter<B>(reinterpret_cast<tile::ScatterShared<B> &>(sh), sg, s, beg, end, offsets, err);
+    });
+    return;
+  }
   // RES (sampled groups; err is the batch's own capacity flag): once a layout
   // has found a relation's regions too large for its buffer, or a region
   // overflowed, the batch is redone exactly, so the stripes still to come
   // move nothing (read beside the cursors, tested after the first barrier)
   __shared__ uint32_t s_err;
-  if constexpr (RES) {
-    if (threadIdx.x == 0) s_err = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
-      sh.cursor[d] = sg.re[d];
-      sh.clear_count(d);
-    }
-  } else {
-    const uint64_t base = offsets[sg.count_base];  // tuples of the group's earlier relations
-    for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
-      const uint32_t c = (uint32_t)(offsets[sg.count_base + (uint64_t)d * sg.nstripes + s] - base);
-      sh.cursor[d] = c;
-      sh.clear_count(d);
-      // the relation's first stripe starts every digit: its offsets are the
-      // partition starts (relative to the relation)
-      if (s == 0) sg.part_start[d] = c;
-    }
-    if (s == 0 && threadIdx.x == 0) sg.part_start[1 << BITS] = (uint32_t)sg.n;
+  if (threadIdx.x == 0) s_err = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int d = threadIdx.x; d < (1 << BITS); d += kFastNT) {
+    sh.cursor[d] = sg.re[d];
+    sh.clear_count(d);
   }
-  tile::scatter_stripe<BITS, false, RES>(sh, sg.in, beg, end, sg.n, 0, 0u, sg.out, err, RES ? sg.cur : nullptr,
-                                         RES ? &s_err : nullptr);
+  tile::scatter_stripe<BITS, false, true>(sh, sg.in, beg, end, sg.n, 0, 0u, sg.out, err, sg.cur, &s_err);
 }
 
 // ---- sampled groups ----------------------------------------------------------------
@@ -265,27 +305,28 @@ __global__ void k_bends(const BatchSeg *__restrict__ segs, uint32_t nseg) {
   sg.part_end[d] = min(sg.cur[tile::cursor_slot<BITS>(d)], sg.re[d]);
 }
 
-// pair_join[pair_base + p] = j for every partition p of join j (one workgroup per join).
-__global__ void k_bpairs(const BatchJoin *__restrict__ joins, uint32_t *__restrict__ pair_join) {
-  const uint32_t j = blockIdx.x;
+// Join blockIdx.x: its number and its tile count for each of its (join,
+// partition) pairs q; tiles[npairs] = 0; the state of the scan that follows
+// cleared.  gridDim.y workgroups share a join's partitions.
+__global__ void k_bplan(const BatchJoin *__restrict__ joins, uint32_t *__restrict__ pair_join, uint32_t npairs,
+                        uint32_t *__restrict__ tiles, uint64_t *__restrict__ zero, uint32_t nzero) {
+  const uint32_t j = blockIdx.x, t = blockIdx.y * blockDim.x + threadIdx.x, nt = gridDim.y * blockDim.x;
+  for (uint32_t i = j * nt + t; i < nzero; i += gridDim.x * nt) zero[i] = 0ull;
+  if (j == 0 && t == 0) tiles[npairs] = 0;
   const BatchJoin J = load_join(joins, j);
-  for (uint32_t p = threadIdx.x; p < J.P; p += blockDim.x) pair_join[J.pair_base + p] = j;
+  for (uint32_t p = t; p < J.P; p += nt) {
+    const uint32_t rn = J.r_end[p] - J.r_start[p];
+    const uint32_t sn = J.s_end[p] - J.s_start[p];
+    pair_join[J.pair_base + p] = j;
+    tiles[J.pair_base + p] = (rn && sn) ? ((rn + kFCap - 1) / kFCap) * ((sn + J.s_span - 1) / J.s_span) : 0u;
+  }
 }
 
-// tiles[q] for every (join, partition) pair q; tiles[npairs] = 0.
-__global__ void k_bplan(const BatchJoin *__restrict__ joins, const uint32_t *__restrict__ pair_join, uint32_t npairs,
-                        uint32_t *tiles) {
-  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q > npairs) return;
-  if (q == npairs) {
-    tiles[npairs] = 0;
-    return;
-  }
-  const BatchJoin J = load_join(joins, pair_join[q]);
-  const uint32_t p = q - J.pair_base;
-  const uint32_t rn = J.r_end[p] - J.r_start[p];
-  const uint32_t sn = J.s_end[p] - J.s_start[p];
-  tiles[q] = (rn && sn) ? ((rn + kFCap - 1) / kFCap) * ((sn + J.s_span - 1) / J.s_span) : 0u;
+// Pinned host memory: visible once the batch's event is.
+__global__ void k_bpublish(const uint64_t *__restrict__ words, uint32_t n, const uint32_t *__restrict__ err,
+                           uint64_t *__restrict__ host) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n) host[i] = i < n ? words[i] : (uint64_t)*err;
 }
 
 // Descriptor of probe tile t of pair q (tile_start[q] <= t < tile_start[q + 1]):
@@ -441,16 +482,22 @@ hipError_t launch_group(const BatchGroup &g, uint64_t *counts, void *scan_scratc
       return hipGetLastError();
     }
   }
-  EO_TIMED("batch_hist", stream,
-           hipLaunchKernelGGL(k_bseg_hist<BITS>, dim3(grid), dim3(kBHistNT), 0, stream, g.segs, g.nseg,
-                              g.total_stripes, g.stripe_len, counts));
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = scan_u64(counts, counts, g.ncounts, nullptr, scan_scratch, err, stream);
-  if (e != hipSuccess) return e;
-  EO_TIMED("batch_scatter", stream,
-           hipLaunchKernelGGL(k_bseg_scatter<BITS>, dim3(grid), dim3(kFastNT), 0, stream, g.segs, g.nseg,
-                              g.total_stripes, g.stripe_len, counts, err));
-  return hipGetLastError();
+  if constexpr (BITS < kBatchSmallBits) {  // (the small group's relations)
+    return hipErrorInvalidValue;
+  } else {
+    const size_t nzero = scan_state_words_u64(g.ncounts);
+    if (nzero >= (1ull << 32)) return hipErrorInvalidValue;
+    EO_TIMED("batch_hist", stream,
+             hipLaunchKernelGGL(k_bseg_hist<BITS>, dim3(grid), dim3(kBHistNT), 0, stream, g.segs, g.nseg,
+                                g.total_stripes, g.stripe_len, counts, (uint64_t *)scan_scratch, (uint32_t)nzero));
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = scan_u64_clean(counts, counts, g.ncounts, nullptr, scan_scratch, err, stream);
+    if (e != hipSuccess) return e;
+    EO_TIMED("batch_scatter", stream,
+             hipLaunchKernelGGL(k_bseg_scatter<BITS>, dim3(grid), dim3(kFastNT), 0, stream, g.segs, g.nseg,
+                                g.total_stripes, g.stripe_len, counts, err));
+    return hipGetLastError();
+  }
 }
 
 }  // namespace
@@ -482,12 +529,12 @@ hipError_t batch_plan(const BatchJoin *joins, uint32_t njoins, uint32_t *pair_jo
                       uint32_t *tile_start, BatchTile *tiles, uint32_t tiles_cap, void *scan_scratch, uint32_t *err,
                       hipStream_t stream) {
   if (njoins == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_bpairs, dim3(njoins), dim3(256), 0, stream, joins, pair_join);
-  hipLaunchKernelGGL(k_bplan, dim3((npairs + 1 + 255) / 256), dim3(256), 0, stream, joins, pair_join, npairs,
-                     tile_start);
+  const uint32_t share = std::min<uint32_t>(1024, npairs / njoins / 256 + 1);
+  hipLaunchKernelGGL(k_bplan, dim3(njoins, share), dim3(256), 0, stream, joins, pair_join, npairs, tile_start,
+                     (uint64_t *)scan_scratch, (uint32_t)scan_state_words_u32((uint64_t)npairs + 1));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  e = scan_u32(tile_start, tile_start, (uint64_t)npairs + 1, nullptr, scan_scratch, err, stream);
+  e = scan_u32_clean(tile_start, tile_start, (uint64_t)npairs + 1, nullptr, scan_scratch, err, stream);
   if (e != hipSuccess || tiles_cap == 0 || npairs == 0) return e;
   const uint32_t blocks = (uint32_t)std::min<uint64_t>(((uint64_t)tiles_cap + 255) / 256, 4096);
   hipLaunchKernelGGL(k_btiles, dim3(blocks), dim3(256), 0, stream, joins, pair_join, tile_start, npairs, tiles,
@@ -500,6 +547,11 @@ hipError_t batch_emit_unmatched(const BatchJoin *joins, uint32_t njoins, const u
   if (njoins == 0 || blocks == 0) return hipSuccess;
   EO_TIMED("outer_rows", stream,
            hipLaunchKernelGGL(k_bemit, dim3(blocks), dim3(256), 0, stream, joins, njoins, emit_start));
+  return hipGetLastError();
+}
+
+hipError_t batch_publish(const uint64_t *words, uint32_t n, const uint32_t *err, uint64_t *host, hipStream_t stream) {
+  hipLaunchKernelGGL(k_bpublish, dim3(n / 256 + 1), dim3(256), 0, stream, words, n, err, host);
   return hipGetLastError();
 }
 

@@ -46,6 +46,9 @@ hipError_t scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *tot
 size_t scan_state_words_u32(uint64_t n);
 hipError_t scan_u32_clean(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
                           uint32_t *err, hipStream_t stream);
+size_t scan_state_words_u64(uint64_t n);
+hipError_t scan_u64_clean(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
+                          uint32_t *err, hipStream_t stream);
 hipError_t fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t stream);
 hipError_t fill_u64(uint64_t *p, uint64_t v, uint64_t n, hipStream_t stream);
 
@@ -285,12 +288,15 @@ hipError_t partition_gapped(uint64_t n, int bits_hi, int bits_lo, const eo_tuple
 // ---- batch.hip --------------------------------------------------------------
 // One relation of one join to partition in a batch group (all of a group's
 // relations use the same number of radix bits, digit = key & (2^bits - 1)).
+// Relations of up to this many radix bits form one exact group.
+constexpr int kBatchSmallBits = 5;
 struct BatchSeg {
   const uint2 *in;           // 16-byte aligned
   uint2 *out;
   uint64_t n;
   uint32_t stripe_base;      // first stripe of this relation in the group
   uint32_t nstripes;
+  uint32_t bits;             // the relation's radix bits (the group's, or fewer in the small group)
   uint64_t count_base;       // first count of this relation: counts laid out [rel][digit][stripe]
   uint32_t *part_start;      // 2^bits + 1 partition starts (output)
   // sampled groups: partitions sized from a 1/16 sample (gaps between them)
@@ -303,7 +309,7 @@ struct BatchSeg {
   uint64_t budget;           // tuples of out
 };
 struct BatchGroup {
-  int bits;
+  int bits;                  // exact groups: kBatchSmallBits holds relations of 1 to kBatchSmallBits bits
   int sampled;               // partitions sized from a sample, runs reserved with atomics
   const BatchSeg *segs;      // device table, ordered by stripe_base (and samp_base)
   uint32_t nseg;
@@ -366,6 +372,9 @@ hipError_t batch_plan(const BatchJoin *joins, uint32_t njoins, uint32_t *pair_jo
 // join's unmatched_blocks(nS), emit_start[njoins] the grid.
 hipError_t batch_emit_unmatched(const BatchJoin *joins, uint32_t njoins, const uint32_t *emit_start,
                                 uint32_t blocks, hipStream_t stream);
+// The per-join counts, the capacity flag and the context's error flags to the
+// pinned host words [0, n) and n.
+hipError_t batch_publish(const uint64_t *words, uint32_t n, const uint32_t *err, uint64_t *host, hipStream_t stream);
 // *queue_head must be zero on entry; grid = one workgroup per CU.  Tiles
 // below tiles_cap read their descriptor; later ones resolve their pair by
 // search.

@@ -159,10 +159,12 @@ hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *tot
                     uint32_t *err, hipStream_t stream) {
   return scan_impl<uint32_t, kScanIPT32>(in, out, n, total_dev, scratch, err, stream);
 }
-size_t scan_state_words_u32(uint64_t n) {
-  const uint64_t tile = (uint64_t)(n >= kScanBigMin ? kScanNTBig : kScanNT) * kScanIPT32;
+static size_t scan_state_words(uint64_t n, int ipt) {
+  const uint64_t tile = (uint64_t)(n >= kScanBigMin ? kScanNTBig : kScanNT) * ipt;
   return (size_t)((n + tile - 1) / tile) + 1;
 }
+size_t scan_state_words_u32(uint64_t n) { return scan_state_words(n, kScanIPT32); }
+size_t scan_state_words_u64(uint64_t n) { return scan_state_words(n, kScanIPT64); }
 hipError_t scan_u32_clean(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
                           uint32_t *err, hipStream_t stream) {
   return scan_impl<uint32_t, kScanIPT32>(in, out, n, total_dev, scratch, err, stream, true);
@@ -170,6 +172,10 @@ hipError_t scan_u32_clean(const uint32_t *in, uint32_t *out, uint64_t n, uint64_
 hipError_t scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
                     uint32_t *err, hipStream_t stream) {
   return scan_impl<uint64_t, kScanIPT64>(in, out, n, total_dev, scratch, err, stream);
+}
+hipError_t scan_u64_clean(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total_dev, void *scratch,
+                          uint32_t *err, hipStream_t stream) {
+  return scan_impl<uint64_t, kScanIPT64>(in, out, n, total_dev, scratch, err, stream, true);
 }
 
 hipError_t fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t stream) {

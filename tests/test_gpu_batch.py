@@ -425,3 +425,24 @@ def test_batch_sampled_clumping(ctx, run, sampled):
             assert same_multiset(r.pairs(n_out), r.want), i
     finally:
         b.free()
+
+
+def test_relations_of_different_bits_partition_together(ctx):
+    """Relations of 1 to 5 radix bits share their partition launches, those of 6 bits have their own;
+    sizes at the edges of tiles, a relation smaller than its partner on either side."""
+    rng = np.random.default_rng(11)
+    b = ctx.batch()
+    reqs, want, keep = [], [], []
+    for i, nR in enumerate([9001, 16384, 16385, 33001, 66001, 131073, 262145, 400001, 8705, 70001]):
+        nS = [2 * nR + 1, 16384, nR // 2 + 1][i % 3]
+        R = np.stack([rng.integers(-nR, nR, nR), np.arange(nR)], 1).astype(np.int32)
+        S = np.stack([rng.integers(-nR, nR, nS), np.arange(nS)], 1).astype(np.int32)
+        want.append(brute_join(R, S))
+        cap = len(want[-1]) + 1
+        bufs = DeviceArray.from_host(ctx, R), DeviceArray.from_host(ctx, S), DeviceArray(ctx, 8 * cap)
+        keep.append(bufs)
+        reqs.append(eo.request(R=bufs[0], nR=nR, S=bufs[1], nS=nS, out=bufs[2], out_cap=cap))
+    for again in range(2):
+        for k, (_, n, status) in enumerate(b.run(reqs)):
+            assert status == 0 and n == len(want[k])
+            assert same_multiset(keep[k][2].to_host(np.int32, (n, 2)), want[k])
