@@ -148,32 +148,63 @@ __global__ __launch_bounds__(kNljNT) void k_nlj(const uint2 *__restrict__ R, uin
 // that order with every subtraction, product and sum rounded on its own
 // (__dsub_rn / __dmul_rn / __dadd_rn: no fused multiply-add), which makes each
 // decision bit-identical to the reference's unfused x86-64 arithmetic.  One
-// fused pass: an R tile (up to 1024 points) in LDS, 8 S points per lane, OR-accumulated ballots per group of 8 R points,
-// per-wave hit-group list, one output reservation per wave.
+// fused pass: R tiles of up to 1024 points in LDS against the workgroup's 2048 S points in
+// registers, rows reserved per workgroup.
 //
 // The exact predicate takes 9 FP64 instructions per pair.  Every pair first
-// passes a filter of 4 (three FMAs and a compare) that never rejects a match:
+// passes a filter that never rejects a match:
+//   |r|^2 - 2 r.s + |s|^2 - d2 < 0,  lowered by a bound on the filter's error
+// and only pairs that pass it evaluate the predicate, on the coordinates as
+// given.  There are two filters, chosen by a workgroup for each of its R tiles
+// by the points in it.
+//
+// Matrix filter (dist_matrix).  The sum is a contraction: coordinates about a
+// common origin o (a mean of the S tile's points, subtracted in FP64) as two
+// bf16 words, h = bf16(x), m = bf16(x - h), and the squared lengths as three:
+//   hh' + hm' + mh' for each coordinate (9 products), c_r 1 (3), 1 t_s (3)
+// 15 of the 16 products that one 32x32x16 MFMA sums per pair; a sign test of
+// its 32-bit result is the filter.  Error, with N = |r - o|^2 + |s - o|^2: a
+// bf16 word rounds off at most 2^-8 of its number, so hh' + hm' + mh' misses
+// 3.03 2^-16 2 |x x'| per coordinate, in all 12.1 2^-18 N; 16 additions of terms
+// whose magnitudes sum to 2 N + d2, each off by 2^-22 of that sum at most even
+// if the unit cuts instead of rounding: 2^-18 (2 N + d2); the third words of c
+// and t and the FP64 steps stay below 2^-22 (N + d2).  Together under 14.2
+// 2^-18 (N + d2); kMatSlack is 16 2^-18.  (Measured over 2^24 pairs each in
+// boxes of 4 to 100, near each other or not: 6.9 2^-18 (N + d2) at most; 0.04
+// where the coordinates are bf16 numbers.)  It is used where every N stays within 2^15 d2, so that
+// the slack is 2 d2 at the corners and few pairs pass that do not match, and
+// d2 is within 2^-60 .. 2^60 (no bf16 or 32-bit word overflows, and what is
+// flushed to zero is far below the slack).
+//
+// FP64 filter (dist_fp64), else: three FMAs and a compare,
 //   |r|^2 - 2 r.s < d2 - |s|^2,   both sides widened by kDistSlack of the terms
-// and only the S registers of a group in which it holds for some pair evaluate
-// the predicate (on coordinates read again, so that the loop keeps only the
-// filter's registers).  8 S points per lane, because the R point that they
-// share is a 32-byte LDS broadcast: with 4 the CU's LDS port is as busy as its
-// four FP64 pipes.
+// 8 S points per lane, because the R point that they share is a 32-byte LDS
+// broadcast: with 4 the CU's LDS port is as busy as its four FP64 pipes.
 // Rounding: with u = 2^-53 the filter's left side is off by at most 3u |r|^2
 // (the squares' sum) + 3u (|r|^2 + 2 |r||s|) (the FMAs) <= 9u (|r|^2 + |s|^2),
 // the right side by 4u (|s|^2 + d2), and the reference's own sum is within 8u
 // of the real squared distance, at most 8u d2 at the threshold: together
 // under 16u (|r|^2 + |s|^2 + d2); kDistSlack is 128u.  A point whose squared
 // length is not below 2^1000 (infinities and NaN included) makes every pair
-// of it pass.  FP64 issue bound (0.89 of the VALU's cycles): 2^17 x 2^17 points
-// in 3.69 ms with the exact predicate on every pair, 2.27 ms with the filter
-// (4 S points per lane 2.35, a running minimum instead of the compares 2.33).
+// of it pass.
+//
+// 2^17 x 2^17 points: 3.69 ms with the exact predicate on every pair, 2.27 ms
+// with the FP64 filter (issue bound, 0.89 of the VALU's cycles), 0.53 ms with
+// the matrix filter: a SIMD's MFMAs (0.44 of its cycles) and VALU (0.62) do not
+// run beside each other, so the signs cost as much as the products.  (Each MFMA
+// issued before the signs of the tile before it, four tiles to a test: 0.66
+// ms, registers spilled.)
 constexpr int kDistNT = 256;
 constexpr int kDistNW = kDistNT / kWave;
 constexpr int kDistK = 8;
 constexpr int kDistSTile = kDistNT * kDistK;  // 2048
-constexpr int kDistRTile = 1024;
+constexpr int kDistRTile = 1024;                // R points in LDS at a time
+constexpr int kDistRFull = 8 * kDistRTile;      // R points of a workgroup, at most: its S side is prepared once
 constexpr int kDistGroup = 8;
+constexpr int kMatTiles = kDistSTile / kDistNW / 32;  // 32-point S tiles per wave
+constexpr int kMatList = 384;                         // rows a wave collects before it writes them
+constexpr double kMatSlack = 0x1p-14;
+constexpr double kMatMaxN = 0x1p14;  // squared length of a point, in units of d2
 constexpr double kDistSlack = 0x1p-46;
 constexpr double kDistHuge = 0x1p1000;
 constexpr double kDistTiny = 0x1p-1060;  // covers squares that round to a multiple of 2^-1074
@@ -196,17 +227,12 @@ struct alignas(16) DistPoint {
   double x, y, z, c;
 };
 
+// Rows of one R tile in LDS with the FP64 filter.
 template <bool WRITE>
-__global__ __launch_bounds__(kDistNT) __attribute__((amdgpu_waves_per_eu(4))) void k_nlj_dist(const Point3 *__restrict__ R, uint64_t nR,
-                                                      const Point3 *__restrict__ S, uint64_t nS, uint32_t s_tiles,
-                                                      uint32_t r_tile, double d2, uint64_t *cursor,
-                                                      uint2 *__restrict__ out, uint64_t out_cap) {
-  __shared__ DistPoint rp[kDistRTile];
-  __shared__ uint16_t hits[WRITE ? kDistNW : 1][WRITE ? kDistRTile / kDistGroup : 1];
-  const uint32_t b = blockIdx.x;
-  const uint32_t st = b % s_tiles, rt = b / s_tiles;
-  const uint64_t r0 = (uint64_t)rt * r_tile;
-  const uint32_t rn = (uint32_t)std::min<uint64_t>(r_tile, nR - r0);
+__device__ __forceinline__ void dist_fp64(DistPoint *rp, uint16_t (*hits)[WRITE ? kDistRTile / kDistGroup : 1],
+                                          const Point3 *__restrict__ R, uint64_t r0, uint32_t rn,
+                                          const Point3 *__restrict__ S, uint64_t nS, uint32_t st, double d2,
+                                          uint64_t *cursor, uint2 *__restrict__ out, uint64_t out_cap) {
   for (uint32_t i = threadIdx.x; i < rn; i += kDistNT) {
     const Point3 &p = R[r0 + i];
     const double x = p.v[0], y = p.v[1], z = p.v[2], q = x * x + y * y + z * z;
@@ -313,6 +339,168 @@ __global__ __launch_bounds__(kDistNT) __attribute__((amdgpu_waves_per_eu(4))) vo
   }
 }
 
+// A number as the sum of its first two or three bf16 words (round to nearest).
+struct Bf16Words {
+  __bf16 h, m, l;
+};
+__device__ __forceinline__ Bf16Words bf16_words(double v) {
+  const float f = (float)v;
+  Bf16Words r;
+  r.h = (__bf16)f;
+  const float f1 = f - (float)r.h;
+  r.m = (__bf16)f1;
+  r.l = (__bf16)(f1 - (float)r.m);
+  return r;
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Collected rows of a wave, (R point of the workgroup) << 11 | (S point of its
+// tile), to out.
+__device__ __forceinline__ void dist_flush(const uint32_t *list, uint32_t n, uint64_t base, const Point3 *__restrict__ R,
+                                           uint64_t r_base, const Point3 *__restrict__ S, uint64_t s_base,
+                                           uint2 *__restrict__ out, uint64_t out_cap) {
+  for (uint32_t k = lane_id(); k < n; k += kWave) {
+    const uint32_t e = list[k];
+    if (base + k < out_cap)
+      out[base + k] = make_uint2((uint32_t)R[r_base + (e >> 11)].id, (uint32_t)S[s_base + (e & 2047u)].id);
+  }
+}
+
+// A workgroup: S points [2048 st, + 2048) against r_tile R points, 1024 at a
+// time in LDS (as bf16 words, 32 bytes each, or as DistPoints).  A wave's 512 S
+// points stay in registers as 16 MFMA operands; each 32 R points are read once
+// (16 bytes per lane) for 16 MFMAs.  Per 1024 pairs one MFMA of 8 passes (32
+// cycles) and 8 three-operand ORs (32 cycles of VALU) on the signs of its
+// results.
+template <bool WRITE>
+__global__ __launch_bounds__(kDistNT) __attribute__((amdgpu_waves_per_eu(4))) void k_nlj_dist(
+    const Point3 *__restrict__ R, uint64_t nR, const Point3 *__restrict__ S, uint64_t nS, uint32_t s_tiles,
+    uint32_t r_tile, double d2, uint64_t *cursor, uint2 *__restrict__ out, uint64_t out_cap) {
+  __shared__ DistPoint rp[kDistRTile];
+  __shared__ uint16_t hits[WRITE ? kDistNW : 1][WRITE ? kDistRTile / kDistGroup : 1];
+  __shared__ uint32_t list[WRITE ? kDistNW : 1][WRITE ? kMatList : 1];
+  __shared__ uint32_t unfit;  // some point so far is outside the matrix filter's range
+  __shared__ uint32_t wave_rows[kDistNW];
+  __shared__ uint64_t wg_base;
+  bf16x8 *const frag = reinterpret_cast<bf16x8 *>(rp);  // [half][point]: products 0..7 and 8..15
+  static_assert(sizeof(rp) == 2 * kDistRTile * sizeof(bf16x8), "the two forms of an R tile take the same LDS");
+  const uint32_t st = blockIdx.x % s_tiles, rt = blockIdx.x / s_tiles;
+  const uint64_t r_base = (uint64_t)rt * r_tile, s_base = (uint64_t)st * kDistSTile;
+  const uint64_t r_last = std::min<uint64_t>(nR, r_base + r_tile);
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  const uint32_t half = lane >> 5, col = lane & 31;
+  if (threadIdx.x == 0) unfit = d2 >= 0x1p-60 && d2 <= 0x1p60 ? 0u : 1u;
+  // the origin: the mean of 64 points spread over the S tile (the same in
+  // every wave: the same loads and sums)
+  const uint64_t sn = std::min<uint64_t>(kDistSTile, nS - s_base);
+  const Point3 &op = S[s_base + (uint64_t)lane * sn / kWave];
+  const double ox = wave_sum<double>(op.v[0]) / kWave, oy = wave_sum<double>(op.v[1]) / kWave,
+               oz = wave_sum<double>(op.v[2]) / kWave;
+  const double max_n = kMatMaxN * d2;
+  const __bf16 zero = (__bf16)0.0f, one = (__bf16)1.0f;
+  __syncthreads();
+  bf16x8 b[kMatTiles];
+#pragma unroll
+  for (int t = 0; t < kMatTiles; ++t) {
+    const uint32_t i = (uint32_t)(w * kMatTiles + t) * 32 + col;
+    const bool ok = i < sn;
+    const Point3 &p = S[s_base + (ok ? i : 0u)];
+    const double x = p.v[0] - ox, y = p.v[1] - oy, z = p.v[2] - oz, n = x * x + y * y + z * z;
+    if (!(n <= max_n)) unfit = 1;
+    const Bf16Words bx = bf16_words(-2.0 * x), by = bf16_words(-2.0 * y), bz = bf16_words(-2.0 * z);
+    // (a lane past the end of S passes nothing)
+    const Bf16Words bt = bf16_words(ok ? n - d2 - kMatSlack * (n + d2) : 4.0 * max_n);
+    b[t] = half ? bf16x8{bz.h, one, one, one, bt.h, bt.m, bt.l, zero}
+                : bf16x8{bx.h, bx.m, bx.h, by.h, by.m, by.h, bz.h, bz.m};
+  }
+  uint64_t total = 0;
+  uint32_t nl = 0;  // rows in this wave's list
+  uint64_t r0 = r_base;
+  for (; r0 < r_last; r0 += kDistRTile) {
+    const uint32_t rn = (uint32_t)std::min<uint64_t>(kDistRTile, r_last - r0), rows = (rn + 31) / 32 * 32;
+    __syncthreads();  // the last R tile is read, every S point tested
+    if (!unfit) {
+      for (uint32_t i = threadIdx.x; i < rows; i += kDistNT) {
+        const bool ok = i < rn;
+        const Point3 &p = R[r0 + (ok ? i : 0u)];
+        const double x = p.v[0] - ox, y = p.v[1] - oy, z = p.v[2] - oz, n = x * x + y * y + z * z;
+        if (!(n <= max_n)) unfit = 1;
+        const Bf16Words ax = bf16_words(x), ay = bf16_words(y), az = bf16_words(z);
+        const Bf16Words ac = bf16_words(ok ? n - kMatSlack * n : 8.0 * max_n);  // (a row past the end: no pair)
+        frag[i] = bf16x8{ax.h, ax.h, ax.m, ay.h, ay.h, ay.m, az.h, az.h};
+        frag[kDistRTile + i] = bf16x8{az.m, ac.h, ac.m, ac.l, one, one, one, zero};
+      }
+    }
+    __syncthreads();
+    if (unfit) break;
+    for (uint32_t g = 0; g < rows; g += 32) {
+      const bf16x8 a = frag[half * kDistRTile + g + col];
+#pragma unroll
+      for (int t = 0; t < kMatTiles; t += 2) {
+        const f32x16 c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[t], f32x16{}, 0, 0, 0);
+        const f32x16 c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[t + 1], f32x16{}, 0, 0, 0);
+        uint32_t sign = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sign |= __float_as_uint(c0[i]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sign |= __float_as_uint(c1[i]);
+        if (__ballot((int32_t)sign < 0) == 0) continue;
+        uint32_t cand = 0;  // bit i: result i of the first S tile, bit 16 + i: of the second
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          cand |= (__float_as_uint(c0[i]) >> 31) << i | (__float_as_uint(c1[i]) >> 31) << (16 + i);
+        while (__ballot(cand != 0)) {
+          // result i: R point (i & 3) + 8 (i >> 2 & 3) + 4 half of the 32, S point col of tile t or t + 1
+          const uint32_t i = (uint32_t)__ffs(cand) - 1u;
+          const uint32_t r = g + (i & 3u) + 8u * (i >> 2 & 3u) + 4u * half;
+          const uint32_t sp = (uint32_t)(w * kMatTiles + t + (i >> 4 & 1u)) * 32 + col;
+          bool eq = cand != 0 && r < rn && sp < sn;
+          if (eq) {
+            const Point3 &p = R[r0 + r], &q = S[s_base + sp];
+            eq = dist_lt(q.v[0], q.v[1], q.v[2], p.v[0], p.v[1], p.v[2], d2);
+          }
+          cand &= cand - 1u;
+          const uint64_t m = __ballot(eq);
+          const uint32_t n = (uint32_t)__popcll(m);
+          if (!n) continue;
+          total += n;
+          if (!WRITE) continue;
+          if (eq) list[w][nl + (uint32_t)__popcll(m & lanemask_lt())] = (uint32_t)(r0 - r_base + r) << 11 | sp;
+          nl += n;
+          if (nl > kMatList - kWave) {
+            uint64_t base = 0;
+            if (lane == 0) base = atomic_add_agent(cursor, (uint64_t)nl);
+            dist_flush(list[w], nl, read_lane(base, 0), R, r_base, S, s_base, out, out_cap);
+            total -= nl;
+            nl = 0;
+          }
+        }
+      }
+    }
+  }
+  for (; r0 < r_last; r0 += kDistRTile) {  // from the first R tile outside the matrix filter's range on
+    __syncthreads();
+    dist_fp64<WRITE>(rp, hits, R, r0, (uint32_t)std::min<uint64_t>(kDistRTile, r_last - r0), S, nS, st, d2, cursor,
+                     out, out_cap);
+  }
+  // the rows not yet counted, with one reservation per workgroup
+  if (lane == 0) wave_rows[w] = (uint32_t)total;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t n = 0;
+    for (int v = 0; v < kDistNW; ++v) n += wave_rows[v];
+    wg_base = n ? atomic_add_agent(cursor, n) : 0ull;
+  }
+  if (!WRITE) return;
+  __syncthreads();
+  uint64_t base = wg_base;
+  for (int v = 0; v < w; ++v) base += wave_rows[v];
+  dist_flush(list[w], nl, base, R, r_base, S, s_base, out, out_cap);
+}
+
+static_assert(kDistRFull << 11 > 0 && kDistSTile == 2048, "a collected row: R point << 11 | S point");
 static_assert(kDistK <= 8 && kDistRTile / kDistGroup <= 256, "a hit record: group << 8 | S registers");
 
 }  // namespace
@@ -355,7 +543,7 @@ hipError_t nlj_write(const NljPlan &p, const eo_tuple *R, const eo_tuple *S, con
 // R tuples per tile: `full`, or fewer (whole groups, at least 64) while the
 // grid has less than four workgroups of 256 threads per CU: a small join is
 // bound by the length of one workgroup's loop (2^12 x 2^12 points in 16 tile
-// pairs of 1024 x 1024: 279 us; in 128 of 64 x 2048, with the filter: 58 us).
+// pairs of 1024 x 1024: 279 us; in 128 of 64 x 2048 58 us, with the matrix filter 25 us a call).
 static uint32_t nlj_r_tile(uint64_t nR, uint64_t s_tiles, uint32_t full, uint32_t group, int cus) {
   const uint64_t want = 4ull * (uint64_t)std::max(cus, 8) / std::max<uint64_t>(s_tiles, 1);  // R tiles
   uint64_t t = want > 1 ? (nR + want - 1) / want : full;
@@ -366,7 +554,7 @@ static uint32_t nlj_r_tile(uint64_t nR, uint64_t s_tiles, uint32_t full, uint32_
 hipError_t nlj_dist(const eo_point3 *R, uint64_t nR, const eo_point3 *S, uint64_t nS, double d2, uint64_t *cursor,
                     eo_pair *out, uint64_t out_cap, int cus, hipStream_t stream) {
   const uint64_t s_tiles = (nS + kDistSTile - 1) / kDistSTile;
-  const uint32_t r_tile = nlj_r_tile(nR, s_tiles, kDistRTile, kDistGroup, cus);
+  const uint32_t r_tile = nlj_r_tile(nR, s_tiles, kDistRFull, 32, cus);
   const uint64_t grid = (nR + r_tile - 1) / r_tile * s_tiles;
   if (grid == 0) return hipSuccess;
   if (grid >= (1ull << 31)) return hipErrorInvalidValue;

@@ -414,6 +414,31 @@ def test_nlj_dist_filter_keeps_every_match(ctx, nR, nS, scale, offset, dist):
     assert len(got) == len(want) and same_multiset(got, want)
 
 
+@pytest.mark.parametrize("nR,nS", [(1, 1), (31, 2047), (33, 2049), (1024, 513), (1025, 2048), (9000, 70)])
+@pytest.mark.parametrize("box,offset,dist", [(9.0, 0.0, 1.0), (100.0, 0.0, 1.0), (2.0, -1e7, 1.0), (30.0, 5e5, 0.25),
+                                             (500.0, 0.0, 1.0)])
+@pytest.mark.parametrize("outlier", [False, True])
+def test_nlj_dist_matrix_filter(ctx, nR, nS, box, offset, dist, outlier):
+    """Both filters of the distance join and the change from one to the other (an outlier in the
+    last R tile), tile remainders, dense rows, and pairs one rounding inside and outside."""
+    rng = np.random.default_rng(nR * 7 + nS)
+    R = np.zeros(nR, dtype=oracle.POINT3)
+    S = np.zeros(nS, dtype=oracle.POINT3)
+    R["id"], S["id"] = np.arange(nR), np.arange(nS) + 10 ** 6
+    R["v"] = rng.uniform(0, box, size=(nR, 3)) + offset
+    S["v"] = rng.uniform(0, box, size=(nS, 3)) + offset
+    k = min(nR, nS) // 3
+    for i, away in enumerate([dist, np.nextafter(dist, 0.0), np.nextafter(dist, 9.0)]):
+        S["v"][i * k:(i + 1) * k] = R["v"][i * k:(i + 1) * k]
+        S["v"][i * k:(i + 1) * k, i] += away
+    if outlier:
+        R["v"][-1] = offset + 1e6
+    want = oracle.nlj_dist_join(R, S, dist)
+    got = ctx.nlj_dist_join(R, S, dist)
+    assert len(got) == len(want) and same_multiset(got, want)
+    assert ctx.nlj_dist_join(R, S, dist, count_only=True) == len(want)
+
+
 @pytest.mark.parametrize("hot", [0.3, 0.7, 1.0])
 def test_two_pass_hot_key(ctx, hot):
     """One key holding up to all of S: one first-pass segment far larger than the
