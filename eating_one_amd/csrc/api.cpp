@@ -279,6 +279,7 @@ eo_status eo_ctx_destroy(eo_ctx *c) {
   for (eo_batch *b : c->serve_pool) eo_batch_free(b);
   c->serve_pool.clear();
   c->arena.release();
+  (void)c->index_block.release();
   for (hipStream_t &x : c->xfer)
     if (x) {
       (void)hipStreamSynchronize(x);

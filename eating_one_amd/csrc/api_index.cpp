@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "ctx.hpp"
@@ -24,6 +25,7 @@ struct eo_index {
   uint32_t *off = nullptr;  // hash: bucket offsets; sorted: the directory
   void *model = nullptr;
   uint64_t bytes = 0;
+  size_t mem_bytes = 0;  // of mem: bytes, or more in a block kept from another index
   double build_ms = 0.0;
   int32_t max_err = 0;
   double mean_err = 0.0;
@@ -33,13 +35,35 @@ namespace {
 
 using namespace eo;
 
+// Bytes of a freed index's memory that its context keeps for the next one, at
+// most: hipMalloc and hipFree take 11 us each, a sixth of building an index of
+// 2^18 tuples and joining it.
+constexpr size_t kIndexKeepBytes = 256u << 20;
+
 // Allocates the index's memory: its entries, `words` u32 and `model` bytes.
 eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
   Layout L;
   const size_t o_ent = L.add(index_entries(ix->n) * sizeof(eo_tuple));
   const size_t o_off = L.add(words * sizeof(uint32_t));
   const size_t o_model = L.add(model);
-  EO_TRY_HIP(hipMalloc((void **)&ix->mem, L.total), "index allocation");
+  KeptBlock &k = ix->ctx->index_block;
+  {
+    std::lock_guard<std::mutex> lk(k.mu);
+    if (k.mem && k.bytes >= L.total && k.bytes / 2 <= L.total) {  // (a small index takes no large block)
+      ix->mem = k.mem;
+      ix->mem_bytes = k.bytes;
+      k.mem = nullptr;
+    }
+  }
+  if (!ix->mem) {
+    hipError_t e = hipMalloc((void **)&ix->mem, L.total);
+    if (e == hipErrorOutOfMemory && k.release()) e = hipMalloc((void **)&ix->mem, L.total);
+    if (e != hipSuccess) {
+      ix->mem = nullptr;
+      return hip_fail(e, "index allocation");
+    }
+    ix->mem_bytes = L.total;
+  }
   ix->bytes = L.total;
   ix->ent = (eo_tuple *)(ix->mem + o_ent);
   ix->off = (uint32_t *)(ix->mem + o_off);
@@ -49,7 +73,18 @@ eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
 
 void free_index(eo_index *ix) {
   if (!ix) return;
-  if (ix->mem) (void)hipFree(ix->mem);
+  char *mem = ix->mem;
+  if (mem && ix->mem_bytes <= kIndexKeepBytes) {
+    // the last block stays with the context, once no stream uses it any more
+    // (hipFree waits for that too)
+    KeptBlock &k = ix->ctx->index_block;
+    if (hipDeviceSynchronize() == hipSuccess) {
+      std::lock_guard<std::mutex> lk(k.mu);
+      std::swap(mem, k.mem);
+      k.bytes = ix->mem_bytes;
+    }
+  }
+  if (mem) (void)hipFree(mem);
   delete ix;
 }
 

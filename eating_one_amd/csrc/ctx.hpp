@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -59,6 +60,22 @@ struct DeviceProps {
 
 }  // namespace eo
 
+namespace eo {
+// One freed device block kept for the next allocation of its size.
+struct KeptBlock {
+  std::mutex mu;
+  char *mem = nullptr;
+  size_t bytes = 0;
+  bool release() {  // gives it back; whether there was one
+    std::lock_guard<std::mutex> lk(mu);
+    if (!mem) return false;
+    (void)hipFree(mem);
+    mem = nullptr;
+    return true;
+  }
+};
+}  // namespace eo
+
 struct eo_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -80,6 +97,7 @@ struct eo_ctx {
   std::map<uintptr_t, size_t> pinned;           // eo_host_alloc blocks: start -> bytes
   hipStream_t xfer[2] = {};                     // copy streams of eo_stream_join (H2D, D2H)
   eo::PinnedBuf stage;                          // its pinned staging
+  eo::KeptBlock index_block;                    // the last freed index's memory
 };
 
 namespace eo {

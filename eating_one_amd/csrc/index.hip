@@ -67,8 +67,10 @@ constexpr uint32_t kPadKey = 0x7fffffffu;     // fills the last line of every le
 
 // cnt[b] = tuples of bucket b; rank[i] = tuple i's place among them (the count
 // its own increment found, so that the placement needs no second atomic).
+// Also clears the state of the scan that follows (nzero words).
 __global__ void k_hidx_count(const uint2 *__restrict__ R, uint64_t n, int log2nb, uint32_t *cnt,
-                             uint32_t *__restrict__ rank) {
+                             uint32_t *__restrict__ rank, uint64_t *__restrict__ zero, uint32_t nzero) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nzero; i += gridDim.x * blockDim.x) zero[i] = 0ull;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
     rank[i] = atomicAdd(&cnt[bucket_hash((int32_t)R[i].x, log2nb)], 1u);
 }
@@ -598,9 +600,10 @@ hipError_t hidx_build(const eo_tuple *R, uint64_t n, int log2nb, eo_tuple *ent, 
   hipError_t e = fill_u32(off, 0u, nb + 1, stream);
   if (e != hipSuccess) return e;
   const uint2 *vR = reinterpret_cast<const uint2 *>(R);
-  hipLaunchKernelGGL(k_hidx_count, dim3(grid_for(n)), dim3(256), 0, stream, vR, n, log2nb, off, rank);
+  hipLaunchKernelGGL(k_hidx_count, dim3(grid_for(n)), dim3(256), 0, stream, vR, n, log2nb, off, rank,
+                     (uint64_t *)scan_scratch, (uint32_t)scan_state_words_u32(nb + 1));
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = scan_u32(off, off, nb + 1, nullptr, scan_scratch, err, stream)) != hipSuccess) return e;
+  if ((e = scan_u32_clean(off, off, nb + 1, nullptr, scan_scratch, err, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(k_hidx_place, dim3(grid_for(n)), dim3(256), 0, stream, vR, n, log2nb, off, rank,
                      reinterpret_cast<uint2 *>(ent));
   return hipGetLastError();

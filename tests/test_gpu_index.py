@@ -193,3 +193,21 @@ def test_index_join_probe_tiles(ctx, nS):
             assert np.array_equal(np.sort(outer[null, 1]), np.flatnonzero(~np.isin(S[:, 0], R[:, 0])))
         finally:
             ix.free()
+
+
+def test_index_memory_kept_for_the_next_build(ctx):
+    """A freed index's block serves the next one of its size, not a much smaller one, while other
+    indexes live: each keeps its own rows."""
+    rng = np.random.default_rng(77)
+    live = []
+    for i, n in enumerate([50_000, 49_000, 50_000, 3_000, 50_001, 26_000]):
+        R = np.stack([rng.integers(0, n, n), np.arange(n) + 10 ** 6 * i], 1).astype(np.int32)
+        S = np.stack([rng.integers(0, 2 * n, n // 2), np.arange(n // 2)], 1).astype(np.int32)
+        ix = ctx.hidx_build(R) if i % 2 else ctx.sidx_build(R)
+        live.append((ix, S, brute_join(R, S)))
+        if i in (1, 3):
+            live.pop(0)[0].free()
+        for other, S2, want in live:
+            assert same_multiset(other.join(S2), want)
+    for other, _, _ in live:
+        other.free()
