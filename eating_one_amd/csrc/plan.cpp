@@ -160,9 +160,11 @@ double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p) {
           p->passes = 1;
           p->lds_cap = lds;
           // half as long again as the mean share, so that ordinary partitions
-          // stay k tiles and one grown by skewed keys still splits
-          const uint64_t span = (uint64_t)(1.5 * s / k) + t.batch - 1;
-          p->s_span = (uint32_t)std::min<uint64_t>(span / t.batch * t.batch, 1u << 20);
+          // stay k tiles and one grown by skewed keys still splits; whole
+          // batches, at least one (a left outer join's S may hold fewer
+          // tuples than there are partitions)
+          const uint64_t batches = std::max<uint64_t>(1, ((uint64_t)(1.5 * s / k) + t.batch - 1) / t.batch);
+          p->s_span = (uint32_t)std::min<uint64_t>(batches * t.batch, 1u << 20);
         }
       }
     }

@@ -306,6 +306,37 @@ static void check_planner() {
   CHECK(eo::plan_hash_join(1 << 20, 1 << 20, &o, &hp) == EO_OK && hp.bits == 0 && hp.passes == 0);
 }
 
+// The time-model plans over every ratio of the sides (left outer joins keep a
+// large R beside a small S): tiles that cover both relations.
+static void check_time_model() {
+  std::mt19937_64 g(0x71);
+  auto sizes = [&] {
+    std::vector<uint64_t> v;
+    for (int l = 0; l < 31; ++l) {
+      v.push_back(1ull << l);
+      v.push_back((1ull << l) + g() % (1ull << l));
+    }
+    for (uint64_t n : {10ull, 50ull, 300ull, 500ull, 70000ull, 1000000ull, 5000000ull, (1ull << 31) - 1}) v.push_back(n);
+    return v;
+  };
+  for (int cus : {8, 256})
+    for (uint64_t nR : sizes())
+      for (uint64_t nS : sizes()) {
+        for (bool outer : {false, true}) {
+          const eo::DirectPlan d = eo::plan_direct(nR, nS, nullptr, cus, outer);
+          CHECK(d.table && d.chunk && d.chunk <= d.table && d.span);
+          CHECK((uint64_t)d.chunks * d.chunk >= nR && (uint64_t)(d.chunks - 1) * d.chunk < nR);
+          CHECK((uint64_t)d.spans * d.span >= nS && (uint64_t)(d.spans - 1) * d.span < nS);
+        }
+        eo::HashPlan p;
+        if (eo::plan_one_pass(nR, nS, cus, &p) == 0) continue;  // R needs more bits than one pass has
+        CHECK(p.passes == 1 && p.bits >= 1 && p.bits <= eo::kOneMaxBits && p.bits_pass1 == p.bits);
+        CHECK((nR >> p.bits) <= p.lds_cap);
+        const uint32_t batch = p.lds_cap == 16384 ? 8192 : 4096;
+        CHECK(p.s_span >= batch && p.s_span % batch == 0);
+      }
+}
+
 // One admission decision sequence of the request loop on a synthetic clock.
 static void check_serve_queue() {
   using eo::ServeQueue;
@@ -460,6 +491,7 @@ int main() {
   check_ref_files();
   check_tune_table();
   check_planner();
+  check_time_model();
   check_serve_queue();
   std::printf("host checks ok: %d checks\n", g_checks);
   return 0;

@@ -108,3 +108,14 @@ def test_few_digits(ctx, bits, order, flags):
         R[:, 0] &= -64
         S[:, 0] &= -64
     _check(ctx, R, S, 0, outer=False, radix_bits=bits, passes=1, flags=flags)
+
+
+@pytest.mark.parametrize("nR,nS", [(70_000, 1), (70_000, 10), (1_000_003, 50), (5_000_000, 300)])
+def test_planned_outer_join_of_few_probes(ctx, nR, nS):
+    """Fewer probes than partitions, no plan given: the spans are one batch at least."""
+    R, S = _relations(nR, nS, nR, nR + nS)
+    want = brute_join(R, S)
+    rows = ctx.hash_join(R, S, left_outer=True)
+    null = rows[:, 0] == _abi.EO_NULL_PAYLOAD
+    assert same_multiset(rows[~null], want)
+    assert np.array_equal(np.sort(rows[null, 1]), np.sort(S[~np.isin(S[:, 0], R[:, 0]), 1]))
