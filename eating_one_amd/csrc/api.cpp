@@ -624,16 +624,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const bool aligned = host || (aligned16(R) && aligned16(S));
   const bool fused_auto = !fx && !(eff.flags & (EO_F_DETERMINISTIC | EO_F_EXACT_PARTITIONS)) && !eff.radix_bits &&
                           !eff.passes && !eff.lds_tuples && !eff.s_tile && hp.passes <= 1;
-  if (fused_auto && aligned && nR) {
-    HashPlan one = hp;
-    const double us = plan_one_pass(nR, nS, c->props.cus, &one);
-    // (the model of the unpartitioned join is some 15 % low: 2^16 x 2^20 22.5
-    // us for 19.4, 100000 x 2^20 38.5 for 32, partitioned 31)
-    if (us < 1.2 * plan_direct(nR, nS, nullptr, c->props.cus, outer).us && one_pass_supported(nR, nS, one.bits))
-      hp = one;
-    else
-      hp.bits = hp.bits_pass1 = hp.passes = 0;
-  }
+  if (fused_auto && aligned && nR) plan_fused(nR, nS, c->props.cus, outer, &hp);
   // the fixed scratch holds the counts of this many stripes of a stable pass
   // (inputs that are not 16-byte aligned)
   if (fx) hp.stable_stripes = kNoAllocStripes;

@@ -267,6 +267,10 @@ hipError_t partition_msd2(uint64_t n, int bits_hi, int bits_lo, const eo_tuple *
 // kErrCapacity in *err (its tuples are then incomplete: redo the join with
 // partition_msd2).  Needs n >= kGapMinRows and 16-byte aligned in, tmp, out.
 constexpr uint64_t kGapMinRows = 1ull << 20;
+constexpr uint32_t kGapLineTuples = 16;  // 128-byte lines
+constexpr uint32_t kGapGroup = 16;       // lines per sampled line
+constexpr double kGapZ = 6.0;            // margin of a region in standard deviations
+constexpr uint32_t kGapPad = 16;         // plus a fixed margin, in tuples
 bool gap_supported(uint64_t n, int bits_hi, int bits_lo);
 // Tuples of a buffer that holds `parts` sampled regions of a relation of n
 // (for n >= kGapMinRows: enough for any sample whose variance is at most kappa

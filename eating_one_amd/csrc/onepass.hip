@@ -15,7 +15,6 @@
 // grouped keys only widen the margins.  A partition that proves too small all
 // the same raises kErrCapacity and the caller redoes the join exactly.
 #include <algorithm>
-#include <cmath>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -229,23 +228,7 @@ __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_s
   }
 }
 
-// Rows of a sampled relation's buffer that hold any layout of it: gap_bound of
-// partition.hip at the largest variance ratio a line of 16 allows.
-constexpr double kOneKappaMax = tile::kGapLineTuples;
-
 }  // namespace
-
-uint64_t one_pass_rows(uint64_t n, int bits) {
-  const uint64_t P = 1ull << bits;
-  if (n < kGapMinRows) return n + P * tile::kGapLineTuples;
-  return gap_rows(n, P, kOneKappaMax);
-}
-
-// 32-bit cursors start below the buffer size and grow by at most n.
-bool one_pass_supported(uint64_t nR, uint64_t nS, int bits) {
-  return bits >= 1 && bits <= kOneMaxBits && nR && nS && one_pass_rows(nR, bits) + nR < (1ull << 32) &&
-         one_pass_rows(nS, bits) + nS < (1ull << 32);
-}
 
 OneRel one_pass_rel(const eo_tuple *in, uint64_t n, int bits, eo_tuple *out, uint32_t *start, uint32_t *end,
                     uint32_t *cur) {

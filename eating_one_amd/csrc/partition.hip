@@ -1127,26 +1127,6 @@ __global__ void k_gap_ends(const uint32_t *__restrict__ cur2, const uint32_t *__
   if (b < FT) part_end[b] = min(cur2[gap_cur2<BL>(b)], re2[b]);
 }
 
-// Tuples a relation of n needs in a buffer of P sampled regions (the first
-// pass's 8 2^bh, the final 2^(bh+bl)) for any sample whose clumping ratios
-// are at most K.  A region of sampled count s and ratio kappa gets f kappa m w^3
-// with m = s / kappa + 1, and w <= 1 + z/(3 sqrt(m)) gives m w^3 <= m + z
-// sqrt(m) + z^2/3 + z^3/27, so its capacity is at most f (s + kappa + z
-// sqrt(kappa (s + kappa)) + kappa (z^2/3 + z^3/27)) + pad + line; over the P
-// regions, with kappa <= K and sum(sqrt(s_b + K)) <= sqrt(P (ns + K P))
-// (Cauchy-Schwarz), at most f (ns + K P (1 + z^2/3 + z^3/27) + z sqrt(K P (ns
-// + K P))) + P (pad + line + 1), and f ns = n; f = n / ns falls as the sample
-// grows, so the smallest sample (full tiles only) bounds it.  A layout whose
-// ratios pass K may not fit: it raises kErrCapacity before any tuple moves.
-uint64_t gap_bound(uint64_t n, uint64_t P, double K) {
-  const uint64_t full = n / kFastTile;
-  const double ns = (double)full * kGapLinesPerTile * kGapLineTuples;
-  if (ns <= 0.0) return ~0ull;
-  const double f = (double)n / ns, z = kGapZ, p = (double)P;
-  const double extra = f * (K * p * (1.0 + z * z / 3.0 + z * z * z / 27.0) + z * std::sqrt(K * p * (ns + K * p)));
-  return n + (uint64_t)std::ceil(extra) + P * (kGapPad + kGapLineTuples + 2);
-}
-
 struct GapLayout {
   size_t o_rows, o_hs, o_re2, o_cur2, o_rs1, o_re1, o_cur1, o_grp, total;
   uint32_t G, cols;
@@ -1195,7 +1175,7 @@ hipError_t launch_gap(uint64_t n, uint64_t group_len, uint32_t workers, const eo
     hipLaunchKernelGGL(k_gap_reduce, dim3((L.cols + 63) / 64), dim3(256), 0, stream, rows, L.G, L.cols, hs);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL((k_gap_layout<BH, BL>), dim3(1), dim3(kGapLayoutNT), 0, stream, hs, n, T, Tg,
-                       gap_bound(n, NSEG, kGapKappaMax), gap_bound(n, FT, kGapKappaMax), rs1, re1, cur1, part_start, re2,
+                       gap_rows(n, NSEG, kGapKappaMax), gap_rows(n, FT, kGapKappaMax), rs1, re1, cur1, part_start, re2,
                        cur2, err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -1396,18 +1376,16 @@ bool gap_supported(uint64_t n, int bits_hi, int bits_lo) {
   if (!msd2_supported(bits_hi, bits_lo) || bits_hi + bits_lo < 2 || n < kGapMinRows) return false;
   // the 32-bit region cursors start below the buffer size and grow by at
   // most n, so they never wrap
-  return gap_bound(n, 1ull << (bits_hi + bits_lo), kGapKappaMax) + n < (1ull << 32) &&
-         gap_bound(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax) + n < (1ull << 32);
+  return gap_rows(n, 1ull << (bits_hi + bits_lo), kGapKappaMax) + n < (1ull << 32) &&
+         gap_rows(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax) + n < (1ull << 32);
 }
 
-uint64_t gap_rows(uint64_t n, uint64_t parts, double kappa) { return gap_bound(n, parts, kappa); }
-
 uint64_t gap_tmp_rows(uint64_t n, int bits_hi, int /*bits_lo*/) {
-  return gap_bound(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax);
+  return gap_rows(n, (1ull << bits_hi) * kGapRanges, kGapKappaMax);
 }
 
 uint64_t gap_out_rows(uint64_t n, int bits_hi, int bits_lo) {
-  return gap_bound(n, 1ull << (bits_hi + bits_lo), kGapKappaMax);
+  return gap_rows(n, 1ull << (bits_hi + bits_lo), kGapKappaMax);
 }
 
 size_t gap_scratch_bytes(uint64_t n, int bits_hi, int bits_lo) { return gap_layout(n, bits_hi, bits_lo).total; }

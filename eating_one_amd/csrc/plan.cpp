@@ -1,6 +1,7 @@
 #include "plan.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 #include "kernels.hpp"
 
@@ -170,6 +171,51 @@ double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p) {
     }
   }
   return best;
+}
+
+// Tuples a relation of n needs in a buffer of P sampled regions (the first
+// pass's 8 2^bh, the final 2^(bh+bl)) for any sample whose clumping ratios
+// are at most K.  A region of sampled count s and ratio kappa gets f kappa m w^3
+// with m = s / kappa + 1, and w <= 1 + z/(3 sqrt(m)) gives m w^3 <= m + z
+// sqrt(m) + z^2/3 + z^3/27, so its capacity is at most f (s + kappa + z
+// sqrt(kappa (s + kappa)) + kappa (z^2/3 + z^3/27)) + pad + line; over the P
+// regions, with kappa <= K and sum(sqrt(s_b + K)) <= sqrt(P (ns + K P))
+// (Cauchy-Schwarz), at most f (ns + K P (1 + z^2/3 + z^3/27) + z sqrt(K P (ns
+// + K P))) + P (pad + line + 1), and f ns = n; f = n / ns falls as the sample
+// grows, so the smallest sample (full tiles only) bounds it.  A layout whose
+// ratios pass K may not fit: it raises kErrCapacity before any tuple moves.
+uint64_t gap_rows(uint64_t n, uint64_t P, double K) {
+  const uint64_t full = n / kPartTile;
+  const double ns = (double)full * (kPartTile / kGapGroup);
+  if (ns <= 0.0) return ~0ull;
+  const double f = (double)n / ns, z = kGapZ, p = (double)P;
+  const double extra = f * (K * p * (1.0 + z * z / 3.0 + z * z * z / 27.0) + z * std::sqrt(K * p * (ns + K * p)));
+  return n + (uint64_t)std::ceil(extra) + P * (kGapPad + kGapLineTuples + 2);
+}
+
+uint64_t one_pass_rows(uint64_t n, int bits) {
+  const uint64_t P = 1ull << bits;
+  if (n < kGapMinRows) return n + P * kGapLineTuples;
+  // the largest variance ratio that a line of 16 tuples allows
+  return gap_rows(n, P, kGapLineTuples);
+}
+
+// 32-bit cursors start below the buffer size and grow by at most n.
+bool one_pass_supported(uint64_t nR, uint64_t nS, int bits) {
+  return bits >= 1 && bits <= kOneMaxBits && nR && nS && one_pass_rows(nR, bits) + nR < (1ull << 32) &&
+         one_pass_rows(nS, bits) + nS < (1ull << 32);
+}
+
+void plan_fused(uint64_t nR, uint64_t nS, int cus, bool outer, HashPlan *p) {
+  HashPlan one = *p;
+  const double us = plan_one_pass(nR, nS, cus, &one);
+  if (us == 0) return;
+  // (the model of the unpartitioned join is some 15 % low: 2^16 x 2^20 22.5
+  // us for 19.4, 100000 x 2^20 38.5 for 32, partitioned 31)
+  if (us >= 1.2 * plan_direct(nR, nS, nullptr, cus, outer).us) p->bits = p->bits_pass1 = p->passes = 0;
+  else if (one_pass_supported(nR, nS, one.bits)) *p = one;
+  // (else relations of nearly 2^31 tuples: their counted pass, which takes any
+  // size; unpartitioned, 2^24 x (2^31 - 1) would read S 964 times)
 }
 
 uint32_t plan_span(uint64_t nR, uint64_t nS, uint32_t lds_cap, int bits, uint64_t s_pool, int cus) {

@@ -61,6 +61,12 @@ DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *opts, int c
 // model's estimate of the whole join in microseconds.
 double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p);
 
+// The plan of a fused join that no option, tuned entry or misaligned input
+// fixes, from plan_hash_join's *p of at most one pass: unpartitioned or both
+// relations together, as the time model has it, or *p as it is where the model's
+// one pass does not take the sizes.
+void plan_fused(uint64_t nR, uint64_t nS, int cus, bool outer, HashPlan *p);
+
 // Returns EO_OK and fills *out, or EO_EINVAL for inconsistent overrides.
 eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *opts, HashPlan *out, int cus = 256);
 

@@ -312,6 +312,7 @@ __device__ __forceinline__ uint64_t probe_tile(ProbeShared<C> &sh, const uint2 *
 constexpr int kFastNT = 1024;
 constexpr int kFastPairs = 8;                         // uint4 loads (2 tuples) per thread per tile
 constexpr int kFastTile = kFastNT * kFastPairs * 2;   // 16384 tuples: a 128 KB staging tile
+static_assert(kFastTile == kPartTile, "the planner's tile is the scatter's");
 // gfx9 buffer resource word 3 for untyped loads (32-bit data format, no swizzle)
 constexpr int kBufferRsrcWord3 = 0x00020000;
 constexpr int kFastWgPerCu = 1;                       // one workgroup per CU (LDS)
@@ -650,16 +651,16 @@ __device__ __forceinline__ void scatter_stripe(ScatterShared<BITS, ORDERED> &sh,
 // tuple tile's 1024 lines of 128 bytes one line in each group of 16 is read,
 // at an offset hashed from (tile, group), so 1/16 of the bytes, spread so that
 // no arrangement that repeats with the tile or the line skews it.
-constexpr uint32_t kGapLineTuples = 16;                                        // 128-byte lines
-constexpr uint32_t kGapGroup = 16;                                             // lines per sampled line
+using eo::kGapGroup;
+using eo::kGapLineTuples;
+using eo::kGapPad;
+using eo::kGapZ;
 constexpr uint32_t kGapLinesPerTile = kFastTile / kGapLineTuples / kGapGroup;  // 64
 constexpr int kGapSampleNT = kGapLinesPerTile * 8;  // 8 threads (16-byte pairs) per line
 constexpr int kGapSampleUnroll = 8;                 // tiles in flight per workgroup
 constexpr int kGapClumpEvery = 8;                   // the clumping sums count one sampled line in 8
 constexpr double kGapKappaMax = 2.0;                // clumping the single-join buffers are sized for
 constexpr double kGapKappaNoise = 0.25;             // taken off a measured clumping ratio (its noise)
-constexpr double kGapZ = 6.0;                       // margin in standard deviations
-constexpr uint32_t kGapPad = 16;                    // plus a fixed margin, in tuples
 
 // v from lane (lane ^ R) of the same 32-lane half (R < 8: the 8 lanes of one
 // sampled line), by ds_swizzle's bit-mask mode (and 0x1f, or 0, xor R)

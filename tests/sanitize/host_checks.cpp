@@ -334,6 +334,19 @@ static void check_time_model() {
         CHECK((nR >> p.bits) <= p.lds_cap);
         const uint32_t batch = p.lds_cap == 16384 ? 8192 : 4096;
         CHECK(p.s_span >= batch && p.s_span % batch == 0);
+        // the choice between them: never an unpartitioned join where the model
+        // has it slower than the partitioned one, whatever sizes that takes
+        for (bool outer : {false, true}) {
+          eo::HashPlan hp;
+          CHECK(eo::plan_hash_join(nR, nS, nullptr, &hp, cus) == EO_OK);
+          if (hp.passes > 1) continue;
+          const bool parted = hp.passes == 1;
+          const double one = eo::plan_one_pass(nR, nS, cus, &p);
+          const double direct = eo::plan_direct(nR, nS, nullptr, cus, outer).us;
+          eo::plan_fused(nR, nS, cus, outer, &hp);
+          CHECK(hp.passes == 1 || one >= 1.2 * direct || !parted);
+          CHECK(hp.passes == 0 || eo::one_pass_supported(nR, nS, hp.bits) || nS > 2000000000ull);
+        }
       }
 }
 
