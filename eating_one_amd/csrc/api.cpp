@@ -868,7 +868,8 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   uint64_t words[3] = {0, 0, 0};  // tiles, inner rows, null rows
   if (outer) EO_TRY_HIP(fill_u32(bits, 0u, matched_words(nS), s), "match bitmap reset");
   for (;;) {
-    EO_TRY_HIP(span_count(P, hp.s_span, cap, (uint32_t)n_tiles, Rp, r_start, Sp, s_start, tile_start, bits, tile_cnt, s),
+    EO_TRY_HIP(span_count(P, hp.s_span, cap, (uint32_t)n_tiles, n_tiles_dev, Rp, r_start, Sp, s_start, tile_start, bits,
+                          tile_cnt, s),
                "count");
     EO_TRY_HIP(scan_u64(tile_cnt, tile_cnt, n_tiles, cursor, cnt_scr, c->d_err, s), "count scan");
     if (outer) {

@@ -184,12 +184,17 @@ template <typename C>
 __global__ __launch_bounds__(kFNT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_span_count(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_start, const uint2 *__restrict__ S,
                   const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ tile_start, uint32_t P,
-                  uint32_t s_span, uint64_t *__restrict__ tile_count, uint32_t n, uint32_t *matched) {
+                  uint32_t s_span, uint64_t *__restrict__ tile_count, uint32_t n, uint32_t *matched,
+                  const uint64_t *__restrict__ n_tiles) {
   __shared__ tile::ProbeShared<C> sh;
+  // 2^31 tiles or more: tile_start may have wrapped, and the host, which reads
+  // *n_tiles, refuses the join
+  const bool too_many = *n_tiles >= (1ull << 31);
   for (uint32_t t = blockIdx.x; t < n; t += gridDim.x) {  // a grid below the tile count loops
     if (t != blockIdx.x) __syncthreads();
     SpanRef ref;
-    if (!resolve_span(t, tile_start, P, r_start, r_start + 1, s_start, s_start + 1, s_span, C::Cap, &ref)) {
+    if (too_many ||
+        !resolve_span(t, tile_start, P, r_start, r_start + 1, s_start, s_start + 1, s_span, C::Cap, &ref)) {
       if (threadIdx.x == 0) tile_count[t] = 0;  // past the last tile (uniform)
       continue;
     }
@@ -213,19 +218,28 @@ void k_span_write(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
   }
 }
 
-__global__ void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end, const uint32_t *s_start,
-                             const uint32_t *s_end, uint32_t P, uint32_t s_span, uint32_t cap, int outer,
-                             uint32_t *tiles) {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > P) return;
-  if (p == P) {
-    tiles[P] = 0;
-    return;
-  }
-  const uint32_t rn = r_end[p] - r_start[p];
-  const uint32_t sn = s_end[p] - s_start[p];
-  const uint32_t spans = (sn + s_span - 1) / s_span;
-  tiles[p] = outer ? spans : rn ? (rn + cap - 1) / cap * spans : 0u;
+// Probe tiles of a partition of rn x sn tuples (R chunks of `cap` x S spans;
+// outer: S spans, whatever R holds).
+__device__ __forceinline__ uint64_t span_tiles(uint32_t rn, uint32_t sn, uint32_t s_span, uint32_t cap, int outer) {
+  const uint64_t spans = ((uint64_t)sn + s_span - 1) / s_span;
+  return outer ? spans : rn ? ((uint64_t)rn + cap - 1) / cap * spans : 0ull;
+}
+
+// tiles[p] of every partition, and their 64-bit sum added to *n_tiles: a sum of
+// 2^31 or more is refused by the kernels that read it, since the 32-bit tile
+// numbers scanned from tiles[] may then have wrapped.
+constexpr int kPlanNT = 256;
+__global__ __launch_bounds__(kPlanNT) void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end,
+                                                        const uint32_t *s_start, const uint32_t *s_end, uint32_t P,
+                                                        uint32_t s_span, uint32_t cap, int outer, uint32_t *tiles,
+                                                        uint64_t *n_tiles) {
+  __shared__ uint64_t red[kPlanNT / kWave + 1];
+  const uint32_t p = blockIdx.x * kPlanNT + threadIdx.x;
+  uint64_t n = 0;
+  if (p < P) n = span_tiles(r_end[p] - r_start[p], s_end[p] - s_start[p], s_span, cap, outer);
+  if (p <= P) tiles[p] = (uint32_t)n;
+  const uint64_t sum = block_sum<kPlanNT, uint64_t>(n, red);
+  if (threadIdx.x == 0 && sum) atomic_add_agent(n_tiles, sum);
 }
 
 }  // namespace
@@ -251,11 +265,11 @@ hipError_t join_fused_plan(uint32_t parts, uint32_t s_span, uint32_t cap, const 
                            uint32_t *tile_start, uint64_t *n_tiles_dev, void *scan_scratch, uint32_t *err,
                            hipStream_t stream, bool outer) {
   const uint32_t n = parts + 1;
-  hipLaunchKernelGGL(k_plan_spans, dim3((n + 255) / 256), dim3(256), 0, stream, r_start, r_end, s_start, s_end,
-                     parts, s_span, cap, (int)outer, tile_start);
+  hipLaunchKernelGGL(k_plan_spans, dim3((n + kPlanNT - 1) / kPlanNT), dim3(kPlanNT), 0, stream, r_start, r_end,
+                     s_start, s_end, parts, s_span, cap, (int)outer, tile_start, n_tiles_dev);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return scan_u32(tile_start, tile_start, n, n_tiles_dev, scan_scratch, err, stream);
+  return scan_u32(tile_start, tile_start, n, nullptr, scan_scratch, err, stream);
 }
 
 // Largest grid of 1024-thread blocks one dispatch takes (2^32 work-items),
@@ -345,20 +359,20 @@ hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, cons
 #undef EO_DIRECT
 }
 
-hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const eo_tuple *R,
-                      const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start, const uint32_t *tile_start,
-                      uint32_t *matched, uint64_t *tile_count, hipStream_t stream) {
+hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const uint64_t *n_tiles_dev,
+                      const eo_tuple *R, const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start,
+                      const uint32_t *tile_start, uint32_t *matched, uint64_t *tile_count, hipStream_t stream) {
   if (n_tiles == 0) return hipSuccess;
   const uint32_t grid = exact_grid(n_tiles);
   const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
   if (cap == (uint32_t)tile::ProbeSmall::Cap)
     EO_TIMED("probe_count", stream,
              hipLaunchKernelGGL(k_span_count<tile::ProbeSmall>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, vS,
-                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched));
+                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched, n_tiles_dev));
   else if (cap == (uint32_t)tile::ProbeBig::Cap)
     EO_TIMED("probe_count", stream,
              hipLaunchKernelGGL(k_span_count<tile::ProbeBig>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, vS,
-                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched));
+                                s_start, tile_start, parts, s_span, tile_count, n_tiles, matched, n_tiles_dev));
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

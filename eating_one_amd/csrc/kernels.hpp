@@ -142,7 +142,7 @@ hipError_t one_pass_partition(const OneArgs &a, int bits, uint32_t s_span, uint3
 size_t join_plan_scratch_bytes(uint32_t parts);
 // Fused single-pass probe.  Tiles are (partition, R-chunk of join_fused_cap()
 // tuples, S span of s_span tuples); join_fused_plan counts and scans them
-// (tile_start: P+1 u32, *n_tiles_dev = total).  Partition p of R is
+// (tile_start: P+1 u32; their number is added to *n_tiles_dev, zero on entry).  Partition p of R is
 // [r_start[p], r_end[p]) (contiguous partitions: r_end = r_start + 1), of S
 // [s_start[p], s_end[p]).  *out_cursor must be zero on
 // entry and holds the match count afterwards; pairs beyond out_cap are
@@ -189,12 +189,13 @@ hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, cons
 hipError_t publish_results(uint64_t *words, int n, uint32_t *err, uint64_t *host, hipStream_t stream);
 // Deterministic order on the fused tiles (join_fused_plan's tile_start):
 // span_count writes the match counts of the first n_tiles tiles (0 past the
-// last one, so an estimate will do) and sets matched bits;
+// last one, so an estimate will do; all 0 when *n_tiles_dev, the plan's number,
+// is 2^31 or more) and sets matched bits;
 // span_write writes every tile's rows from tile_off[t] on, in an order fixed
 // by the inputs.
-hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const eo_tuple *R,
-                      const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start, const uint32_t *tile_start,
-                      uint32_t *matched, uint64_t *tile_count, hipStream_t stream);
+hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const uint64_t *n_tiles_dev,
+                      const eo_tuple *R, const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start,
+                      const uint32_t *tile_start, uint32_t *matched, uint64_t *tile_count, hipStream_t stream);
 hipError_t span_write(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const eo_tuple *R,
                       const uint32_t *r_start, const eo_tuple *S, const uint32_t *s_start, const uint32_t *tile_start,
                       const uint64_t *tile_off, eo_pair *out, uint64_t out_cap, bool wide, hipStream_t stream);

@@ -195,8 +195,7 @@ __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_s
   constexpr uint32_t F = 1u << BITS, BPT = F > (uint32_t)kOnePlanNT ? F / kOnePlanNT : 1;
   __shared__ uint64_t red[kOnePlanNT / kWave + 1];
   const uint32_t b0 = threadIdx.x * BPT;
-  uint32_t cnt[BPT];
-  uint64_t sum = 0;
+  uint64_t cnt[BPT], sum = 0;
 #pragma unroll
   for (uint32_t k = 0; k < BPT; ++k) {
     cnt[k] = 0;
@@ -210,8 +209,9 @@ __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_s
         r.end[p] = e;
         n[rel] = e - r.start[p];
       }
-      const uint32_t spans = (n[1] + s_span - 1) / s_span;
-      cnt[k] = outer ? spans : n[0] ? (n[0] + cap - 1) / cap * spans : 0u;
+      // (64 bits: a sum of 2^31 or more is refused by the probe)
+      const uint64_t spans = ((uint64_t)n[1] + s_span - 1) / s_span;
+      cnt[k] = outer ? spans : n[0] ? ((uint64_t)n[0] + cap - 1) / cap * spans : 0ull;
     }
     sum += cnt[k];
   }

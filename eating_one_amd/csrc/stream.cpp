@@ -173,7 +173,7 @@ struct Streamer {
   eo_status probe(int b, uint64_t nr, uint64_t n, bool write, uint64_t *count) {
     eo_pair *dst = write ? dOut[b] : nullptr;
     const uint64_t cap = write ? out_rows : 0;
-    EO_TRY_HIP(fill_u64(small + 1, 0, 1, cs), "cursor reset");
+    EO_TRY_HIP(fill_u64(small, 0, 2, cs), "tile count and cursor reset");
     const eo_tuple *probe_side = dS[b];
     hipError_t e = hipSuccess;
     if (hash) {

@@ -6,7 +6,8 @@ import ctypes
 import numpy as np
 import pytest
 
-from eating_one_amd import _abi
+import eating_one_amd as eo
+from eating_one_amd import DeviceArray, _abi
 from common import brute_join, same_multiset
 
 pytestmark = pytest.mark.gpu
@@ -71,3 +72,27 @@ def test_deterministic_join_with_more_tiles_than_estimated(ctx):
         assert np.array_equal(np.sort(inner[:, 1]), np.flatnonzero(hit))
         assert np.array_equal(R[inner[:, 0], 0], S[inner[:, 1], 0])
         assert len(a) - len(inner) == (np.count_nonzero(~hit) if outer else 0)
+
+
+@pytest.mark.parametrize("bits,deterministic", [(1, True), (-1, True), (1, False)])
+def test_too_many_tiles_are_refused(ctx, bits, deterministic):
+    """All keys in two partitions: 2^32 and more tiles of 8704 x 8192 tuples, whose 32-bit numbers
+    wrap.  The join is refused before a tile is probed, and the next one is answered."""
+    n, chunk = 800_000_000, 1 << 20
+    keys = np.zeros((chunk, 2), dtype=np.int32)
+    keys[1::2, 0] = 1
+    with eo.Context(0) as c:  # (its scratch is 26 GB)
+        rel = DeviceArray(c, 8 * n)
+        assert c.lib.eo_copy_h2d(c.handle, rel.ptr, keys.ctypes.data, 8 * chunk) == _abi.EO_OK
+        have = chunk
+        while have < n:
+            k = min(have, n - have)
+            assert c.lib.eo_copy_d2d(c.handle, rel.ptr + 8 * have, rel.ptr, 8 * k) == _abi.EO_OK
+            have += k
+        o = c.opts(where=_abi.EO_DEVICE, radix_bits=bits, lds_tuples=8192, s_tile=8192, deterministic=deterministic)
+        cnt = ctypes.c_uint64()
+        st = c.lib.eo_hash_join(c.handle, rel.ptr, n, rel.ptr, n, None, 0, ctypes.byref(cnt), ctypes.byref(o))
+        assert st == _abi.EO_EINTERNAL
+        R, S = _relations(3000, 9000, 2000)
+        assert same_multiset(c.hash_join(R, S, deterministic=deterministic), brute_join(R, S))
+        rel.close()
