@@ -82,8 +82,11 @@ eo_status read_u64(eo_ctx *ctx, const uint64_t *dev, uint64_t *host, int n, hipS
 }
 
 eo_status begin_results(eo_ctx *ctx, hipStream_t stream) {
-  if (ctx->words_dirty)
+  if (ctx->words_dirty) {
+    // the call before ended early: what it launched, on whichever stream, ends first
+    EO_TRY_HIP(hipDeviceSynchronize(), "sync");
     EO_TRY_HIP(fill_u64(ctx->d_words, 0, 8 + kCountWords / 2, stream), "result reset");
+  }
   ctx->words_dirty = true;
   return EO_OK;
 }
@@ -868,6 +871,10 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   uint64_t words[3] = {0, 0, 0};  // tiles, inner rows, null rows
   if (outer) EO_TRY_HIP(fill_u32(bits, 0u, matched_words(nS), s), "match bitmap reset");
   for (;;) {
+    if (side && (st = begin_results(c, s)) != EO_OK) {  // the words are in use again
+      free_side();
+      return st;
+    }
     EO_TRY_HIP(span_count(P, hp.s_span, cap, (uint32_t)n_tiles, n_tiles_dev, Rp, r_start, Sp, s_start, tile_start, bits,
                           tile_cnt, s),
                "count");
