@@ -101,6 +101,7 @@ struct ProbeTable {
   double tile(double r, double s) const { return fixed + build * r + probe * s; }
 };
 constexpr double kAtomicUs = 0.010;
+constexpr uint64_t kDirectTiles = (1ull << 22) - 1;  // of up to 1024 threads each
 constexpr ProbeTable kProbeTables[] = {{kFusedTableFull, 8192, 1, 2.0, 1.5e-4, 6e-4},
                                        {kFusedTableHalf, 4096, 2, 1.2, 2e-4, 1e-3},
                                        {kFusedTableQuarter, 2048, 4, 0.8, 2e-4, 7e-4}};
@@ -123,6 +124,10 @@ DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus,
     uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / side));
     uint64_t span = (batches + spans - 1) / spans * t.batch;
     if (span_opt) span = std::max<uint64_t>(t.batch, (uint64_t)span_opt);
+    // (a dispatch holds fewer than 2^32 work-items: a shorter span from the
+    // caller is lengthened until the tiles fit one launch)
+    const uint64_t most = std::max<uint64_t>(1, kDirectTiles / d.chunks);
+    span = std::max(span, (batches + most - 1) / most * t.batch);
     span = std::min<uint64_t>(span, 1u << 30);
     spans = std::max<uint64_t>(1, (nS + span - 1) / span);
     d.span = (uint32_t)span;

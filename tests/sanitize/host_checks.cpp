@@ -328,6 +328,16 @@ static void check_time_model() {
           CHECK((uint64_t)d.chunks * d.chunk >= nR && (uint64_t)(d.chunks - 1) * d.chunk < nR);
           CHECK((uint64_t)d.spans * d.span >= nS && (uint64_t)(d.spans - 1) * d.span < nS);
         }
+        // any span and table from the caller: a dispatch holds 2^32 work-items
+        for (int span : {1, 8192, 100000, 1 << 30})
+          for (int lds : {0, 4096, 8192, 16384}) {
+            eo_join_opts o{};
+            o.s_tile = span;
+            o.lds_tuples = lds;
+            const eo::DirectPlan d = eo::plan_direct(nR, nS, &o, cus);
+            CHECK((uint64_t)d.chunks * d.spans * 1024 < (1ull << 32));
+            CHECK((uint64_t)d.chunks * d.chunk >= nR && (uint64_t)d.spans * d.span >= nS);
+          }
         eo::HashPlan p;
         if (eo::plan_one_pass(nR, nS, cus, &p) == 0) continue;  // R needs more bits than one pass has
         CHECK(p.passes == 1 && p.bits >= 1 && p.bits <= eo::kOneMaxBits && p.bits_pass1 == p.bits);
