@@ -664,9 +664,8 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_sc = L.add(one ? P * sizeof(uint32_t) : 0);
   const size_t o_ts = L.add((P + 1) * sizeof(uint32_t));
   const DirectPlan dp = direct ? plan_direct(nR, nS, &eff, c->props.cus, outer) : DirectPlan{};
-  const uint64_t spans = direct ? dp.spans : (uint64_t)P + nS / hp.s_span + 1;
-  const size_t outer_bytes = outer ? outer_words(hp.passes ? sp_rows : nS, spans) * sizeof(uint32_t) : 0;
-  const size_t o_bits = L.add(outer && deterministic ? matched_words(nS) * sizeof(uint32_t) : outer_bytes);
+  const size_t bits_words = !outer ? 0 : one ? outer_words(sp_rows, P, hp.s_span) : matched_words(nS);
+  const size_t o_bits = L.add(bits_words * sizeof(uint32_t));
   const uint64_t ublocks = outer && deterministic ? unmatched_blocks(nS) : 0;  // null rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);
@@ -680,10 +679,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   const size_t o_tc = L.add(tiles_est * sizeof(uint64_t) + scan_scratch_bytes_u64(tiles_est));
   char *A = nullptr;
   if (fx) {  // the caller's fixed scratch: no allocation, no synchronisation
-    // (the spans' bitmaps take a little more than one bit a row: the buffer has
-    // room for that beyond its nominal size, so the sizes that fit stay the same)
-    const size_t over = std::min<size_t>(fx->slack, outer ? 8 * spans + 16 : 0);
-    if (L.total > fx->cap + over) {
+    if (L.total > fx->cap) {
       set_last_error("hash join needs " + std::to_string(L.total) + " bytes of scratch, the fixed buffer holds " +
                      std::to_string(fx->cap));
       return EO_EINVAL;
@@ -725,6 +721,8 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     a.rel[1] = one_pass_rel(dS, nS, hp.bits, sp, s_start, (uint32_t *)(A + o_se), (uint32_t *)(A + o_sc));
     a.hs = c->d_counts;
     a.ticket = c->d_counts + kCountWords - 2;
+    a.zero = (uint32_t *)(A + o_bits);
+    a.nzero = (uint32_t)bits_words;
     EO_TRY_HIP(one_pass_partition(a, hp.bits, hp.s_span, cap, outer, tile_start, n_tiles_dev, c->d_err, s),
                "one-pass partition");
     used_gap = true;
@@ -778,7 +776,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   // both orders use the fused probe's tiles: (partition, R chunk, S span)
   if (!direct && !one)
     EO_TRY_HIP(join_fused_plan(P, hp.s_span, cap, r_start, r_end, s_start, s_end, tile_start, n_tiles_dev, A + o_jscr,
-                               c->d_err, s, outer && !deterministic),
+                               c->d_err, s),
                "tile plan");
   if (stats) {
     stats->radix_bits = (uint32_t)hp.bits;
@@ -801,19 +799,25 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
       staged = true;
     }
     uint32_t *ow = outer ? (uint32_t *)(A + o_bits) : nullptr;
+    if (outer && !direct && !one) EO_TRY_HIP(fill_u32(ow, 0u, bits_words, s), "match bitmap reset");
     clk.mark();  // 2
     hipError_t e;
     if (direct)
       e = join_direct(dp, Rp, nR, Sp, nS, cap_dev ? dout : nullptr, cap_dev, cursor, wide, ow, swapped, "probe", s);
+    else if (outer && one)
+      e = join_outer(P, hp.s_span, cap, join_fused_grid(P, nR, nS, tiles_est, c->props.cus), n_tiles_dev, Rp, r_start,
+                     r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, cursor, wide, sp_rows, ow, c->d_err, s);
     else
       e = join_fused(P, hp.s_span, cap, join_fused_grid(P, nR, nS, tiles_est, c->props.cus), n_tiles_dev, Rp, r_start,
                      r_end, Sp, s_start, s_end, tile_start, dout, cap_dev, cursor, wide, ow, c->d_err, s, swapped);
+    if (e == hipSuccess && outer && !direct && !one)
+      e = emit_unmatched(Sp, nS, ow, cursor, dout, cap_dev, wide, s);
     clk.mark();  // 3
     uint64_t words[2] = {0, 0};  // tiles, matches
     uint32_t flags = 0;
     if (e == hipSuccess) {
       st = end_results(c, s, words, 2, &flags);
-      if (direct) words[0] = (uint64_t)(outer ? 1u : dp.chunks) * dp.spans;
+      if (direct) words[0] = (uint64_t)dp.chunks * dp.spans;
       total = words[1];
       if (st == EO_OK && used_gap && flags == kErrCapacity) {
         // a sampled region was too small: the rows are incomplete, so the
@@ -986,10 +990,11 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
   const size_t o_sin = L.add(host ? nS * sizeof(eo_tuple) : 0);
   const bool deterministic = o && (o->flags & EO_F_DETERMINISTIC);
   const size_t o_cnt = L.add(deterministic ? slots * sizeof(uint64_t) : 0);
-  const DirectPlan dp = plan_direct(nR, nS, nullptr, c->props.cus, outer);
-  const size_t o_bits = L.add(!outer ? 0
-                              : deterministic ? matched_words(nS) * sizeof(uint32_t)
-                                              : outer_words(nS, dp.spans) * sizeof(uint32_t));
+  // (the inner join's tiles also for a left outer one: with duplicates a tile's
+  // rows outweigh the two launches that several R chunks take; 2^14 x 2^13 tuples
+  // of two keys in one chunk, two workgroups, 39 ms, in four 3.3 ms)
+  const DirectPlan dp = plan_direct(nR, nS, nullptr, c->props.cus);
+  const size_t o_bits = L.add(outer ? matched_words(nS) * sizeof(uint32_t) : 0);
   const uint64_t ublocks = outer && deterministic ? unmatched_blocks(nS) : 0;  // null rows: block offsets
   const size_t o_ub = L.add(ublocks * sizeof(uint64_t));
   const size_t o_ubs = L.add(ublocks ? scan_scratch_bytes_u64(ublocks) : 0);

@@ -162,7 +162,6 @@ void fold_timer(const LaunchTimer &t, eo_join_stats *stats);
 struct FixedScratch {
   char *base;
   size_t cap;
-  size_t slack;  // bytes past cap, for left outer joins' bitmaps only
 };
 // Stripes of a stable partition pass in fixed scratch: 4 bytes per stripe and
 // digit (4096 stripes of 9 bits would take 8 MiB of it).

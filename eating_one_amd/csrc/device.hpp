@@ -270,6 +270,16 @@ __device__ __forceinline__ void mark_bits(uint32_t *bits, uint64_t base, uint64_
   if (v) atomic_or_agent(bits + (base >> 5) + lane, v);
 }
 
+__device__ __forceinline__ uint32_t ld_agent(const uint32_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until this wave's device-scope atomics are performed.  They are
+// performed at memory, so once every wave of a workgroup has waited and met a
+// barrier, a workgroup that finds the ticket taken after it may read what they
+// wrote, with device-scope atomic loads: of plain stores this says nothing.
+__device__ __forceinline__ void wait_atomics() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Workgroup -> work-item mapping that keeps consecutive work items on one XCD:
 // the hardware deals workgroup b to XCD b % 8, so item (b % 8) * (G/8) + b / 8
 // puts items [x*G/8, (x+1)*G/8) on XCD x.  Bijective on [0, G) for G % 8 == 0.

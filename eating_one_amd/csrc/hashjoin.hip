@@ -46,13 +46,14 @@ using namespace tile;
 __device__ __forceinline__ bool resolve_span(uint32_t t, const uint32_t *tile_start, uint32_t P,
                                              const uint32_t *r_start, const uint32_t *r_end,
                                              const uint32_t *s_start, const uint32_t *s_end, uint32_t s_span,
-                                             uint32_t cap, SpanRef *ref) {
+                                             uint32_t cap, SpanRef *ref, uint32_t *part = nullptr) {
   if (t >= tile_start[P]) return false;
   const uint32_t p = wave_find(tile_start, P, t);
+  if (part) *part = p;
   const uint32_t local = t - tile_start[p];
   const uint32_t rb = r_start[p], rn = r_end[p] - rb;
   const uint32_t sb = s_start[p], sn = s_end[p] - sb;
-  const uint32_t nc = (rn + cap - 1) / cap;
+  const uint32_t nc = max(1u, (rn + cap - 1) / cap);
   const uint32_t c = local % nc, j = local / nc;
   ref->r_beg = rb + c * cap;
   ref->r_n = min(cap, rn - c * cap);
@@ -76,7 +77,7 @@ void k_join_fused(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
                   const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ s_end,
                   const uint32_t *__restrict__ tile_start, uint32_t P,
                                                      uint32_t s_span, uint2 *__restrict__ out, uint64_t out_cap,
-                                                     uint64_t *out_cursor, int wide,
+                                                     uint64_t *out_cursor, int wide, uint32_t *matched,
                                                      const uint64_t *__restrict__ n_tiles, uint32_t *err,
                                                      int swapped) {
   __shared__ tile::ProbeShared<C> sh;
@@ -91,42 +92,53 @@ void k_join_fused(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
     if (t != blockIdx.x) __syncthreads();  // the previous tile's LDS reads are done
     SpanRef ref;
     if (!resolve_span(t, tile_start, P, r_start, r_end, s_start, s_end, s_span, C::Cap, &ref)) return;
-    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, out_cursor, wide != 0, nullptr, 0, swapped != 0);
+    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, out_cursor, wide != 0, matched, 0, swapped != 0);
   }
 }
 
-// Left outer join of one S span against R chunks [0, chunks) of one partition
-// (R[rb, rb + rn), equal chunks of at most C::Cap): the rows of every chunk,
-// and with the last one the null rows.  A span whose partition is one chunk
-// (the usual case) needs no bitmap; otherwise its words start at mw.
+// Null rows of the S tuples of a span whose bit (over S positions) is clear.
+// LDS is free for use; all threads of the workgroup.
 template <typename C>
-__device__ __forceinline__ void outer_span(tile::ProbeShared<C> &sh, const uint2 *__restrict__ R, uint32_t rb,
-                                           uint32_t rn, const uint2 *__restrict__ S, uint32_t s_beg, uint32_t s_n,
-                                           uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor, bool wide,
-                                           uint32_t *mw) {
-  const uint32_t nc = max(1u, (rn + C::Cap - 1) / C::Cap), chunk = (rn + nc - 1) / nc;
-  for (uint32_t c = 0; c < nc; ++c) {
-    SpanRef ref;
-    ref.r_beg = rb + c * chunk;
-    ref.r_n = min(chunk, rn - c * chunk);
-    ref.s_beg = s_beg;
-    ref.s_n = s_n;
-    tile::probe_tile<C, tile::kProbeFused, true>(sh, R, S, ref, out, out_cap, cursor, wide, nullptr, 0, false,
-                                                 nc > 1 ? mw : nullptr, c == 0, c + 1 == nc);
+__device__ __forceinline__ void null_rows(tile::ProbeShared<C> &sh, const uint2 *__restrict__ S, const SpanRef &ref,
+                                          const uint32_t *bits, uint2 *__restrict__ out, uint64_t out_cap,
+                                          uint64_t *cursor, bool wide) {
+  for (uint32_t b0 = 0; b0 < ref.s_n; b0 += C::Batch) {
+    uint32_t mask = 0;
+#pragma unroll
+    for (int u = 0; u < C::SPT; ++u) {
+      const uint32_t i = b0 + u * C::NT + threadIdx.x, pos = ref.s_beg + i;
+      if (i < ref.s_n && !((ld_agent(bits + pos / 32) >> (pos % 32)) & 1u)) mask |= 1u << u;
+    }
+    uint32_t tot;
+    const uint32_t ex = block_excl_scan<C::NT, uint32_t>((uint32_t)__popc(mask), sh.scan_tmp, &tot);
+    if (threadIdx.x == 0) sh.base_sh[0] = tot ? atomic_add_agent(cursor, (uint64_t)tot) : 0ull;
+    __syncthreads();
+    uint64_t pos = sh.base_sh[0] + ex;
+    for (; mask; mask &= mask - 1u, ++pos) {
+      const uint2 t = S[ref.s_beg + b0 + ((uint32_t)__ffs(mask) - 1u) * C::NT + threadIdx.x];
+      if (pos < out_cap) emit_null(out, pos, t.y, t.x, wide);
+    }
+    __syncthreads();
   }
 }
 
-// Left outer joins: tile t is S span t - tile_start[p] of its partition p.
-// words: the spans' bitmaps, span t's from s_beg / 32 + 2 t on.
+// Left outer join of one-pass partitions.  A partition whose R side is one
+// chunk (the usual case) writes its null rows with the others.  The chunks of a
+// larger one run beside each other, mark the matches of their span in bits
+// (over S positions, zero on entry), and the last of them (done: a ticket per
+// span, zero on entry) writes the null rows.  (One workgroup per span taking
+// the chunks in turn needed neither, and 5 ms instead of 0.1 where one
+// partition held all of 2^22 R tuples.)
 template <typename C>
 __global__ __launch_bounds__(kFNT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_join_outer(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_start,
                   const uint32_t *__restrict__ r_end, const uint2 *__restrict__ S,
                   const uint32_t *__restrict__ s_start, const uint32_t *__restrict__ s_end,
                   const uint32_t *__restrict__ tile_start, uint32_t P, uint32_t s_span, uint2 *__restrict__ out,
-                  uint64_t out_cap, uint64_t *cursor, int wide, uint32_t *words,
+                  uint64_t out_cap, uint64_t *cursor, int wide, uint32_t *bits, uint32_t *done,
                   const uint64_t *__restrict__ n_tiles, uint32_t *err) {
   __shared__ tile::ProbeShared<C> sh;
+  __shared__ uint32_t s_last;
   const uint64_t nt = *n_tiles;
   if (nt >= (1ull << 31)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) atomic_or_agent(err, kErrOverflow);
@@ -134,33 +146,50 @@ void k_join_outer(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
   }
   for (uint32_t t = blockIdx.x; t < (uint32_t)nt; t += gridDim.x) {
     if (t != blockIdx.x) __syncthreads();
-    const uint32_t p = wave_find(tile_start, P, t);
-    const uint32_t rb = r_start[p], rn = r_end[p] - rb;
-    const uint32_t j = t - tile_start[p], sb = s_start[p] + j * s_span;
-    outer_span<C>(sh, R, rb, rn, S, sb, min(s_span, s_end[p] - sb), out, out_cap, cursor, wide != 0,
-                  words + sb / 32 + 2ull * t);
+    SpanRef ref;
+    uint32_t p = 0;
+    if (!resolve_span(t, tile_start, P, r_start, r_end, s_start, s_end, s_span, C::Cap, &ref, &p)) return;
+    const uint32_t nc = (r_end[p] - r_start[p] + C::Cap - 1) / C::Cap;
+    tile::probe_tile<C, tile::kProbeFused, true>(sh, R, S, ref, out, out_cap, cursor, wide != 0,
+                                                 nc > 1 ? bits : nullptr);
+    if (nc <= 1) continue;
+    wait_atomics();
+    __syncthreads();
+    // (spans have a ticket each: a partition's lie one s_span apart)
+    if (threadIdx.x == 0) s_last = atomic_add_agent(done + p + ref.s_beg / s_span, 1u) == nc - 1;
+    __syncthreads();
+    if (s_last) null_rows<C>(sh, S, ref, bits, out, out_cap, cursor, wide != 0);
   }
 }
 
-template <typename C>
+// An unpartitioned left outer join whose R side is one chunk: one S span per
+// workgroup, the null rows with the others.  WRITE = false counts only.
+template <typename C, bool WRITE>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_join_direct_outer(const uint2 *__restrict__ R, uint32_t nR, const uint2 *__restrict__ S, uint32_t nS,
-                         uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor, int wide,
-                         uint32_t *words) {
+                         uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor, int wide) {
   __shared__ tile::ProbeShared<C> sh;
-  const uint32_t sb = blockIdx.x * span;
-  outer_span<C>(sh, R, 0, nR, S, sb, min(span, nS - sb), out, out_cap, cursor, wide != 0,
-                words + sb / 32 + 2ull * blockIdx.x);
+  SpanRef ref;
+  ref.r_beg = 0;
+  ref.r_n = nR;
+  ref.s_beg = blockIdx.x * span;
+  ref.s_n = min(span, nS - ref.s_beg);
+  if (WRITE) {
+    tile::probe_tile<C, tile::kProbeFused, true>(sh, R, S, ref, out, out_cap, cursor, wide != 0);
+  } else {
+    const uint64_t n = tile::probe_tile<C, tile::kProbeCount, true>(sh, R, S, ref, nullptr, 0, nullptr);
+    if (threadIdx.x == 0 && n) atomic_add_agent(cursor, n);
+  }
 }
 
 // An unpartitioned join: tile t is R chunk t % chunks against S span t /
 // chunks, so nothing is planned on the device and the join is this launch.
-// WRITE = false counts only.
+// WRITE = false counts only.  matched: as probe_tile's.
 template <typename C, bool WRITE>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::Cap <= 8704 ? 8 : 1)))
 void k_join_direct(const uint2 *__restrict__ R, uint64_t nR, const uint2 *__restrict__ S, uint64_t nS, uint32_t chunk,
                    uint32_t chunks, uint32_t span, uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor,
-                   int wide, int swapped) {
+                   int wide, uint32_t *matched, int swapped) {
   __shared__ tile::ProbeShared<C> sh;
   const uint32_t c = blockIdx.x % chunks, j = blockIdx.x / chunks;
   SpanRef ref;
@@ -169,9 +198,9 @@ void k_join_direct(const uint2 *__restrict__ R, uint64_t nR, const uint2 *__rest
   ref.s_beg = j * span;
   ref.s_n = (uint32_t)min((uint64_t)span, nS - ref.s_beg);
   if (WRITE) {
-    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, cursor, wide != 0, nullptr, 0, swapped != 0);
+    tile::probe_tile<C>(sh, R, S, ref, out, out_cap, cursor, wide != 0, matched, 0, swapped != 0);
   } else {
-    const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr);
+    const uint64_t n = tile::probe_tile<C, tile::kProbeCount>(sh, R, S, ref, nullptr, 0, nullptr, false, matched);
     if (threadIdx.x == 0 && n) atomic_add_agent(cursor, n);
   }
 }
@@ -218,25 +247,19 @@ void k_span_write(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
   }
 }
 
-// Probe tiles of a partition of rn x sn tuples (R chunks of `cap` x S spans;
-// outer: S spans, whatever R holds).
-__device__ __forceinline__ uint64_t span_tiles(uint32_t rn, uint32_t sn, uint32_t s_span, uint32_t cap, int outer) {
-  const uint64_t spans = ((uint64_t)sn + s_span - 1) / s_span;
-  return outer ? spans : rn ? ((uint64_t)rn + cap - 1) / cap * spans : 0ull;
-}
-
-// tiles[p] of every partition, and their 64-bit sum added to *n_tiles: a sum of
+// tiles[p] of every partition (R chunks x S spans), and their 64-bit sum added to *n_tiles: a sum of
 // 2^31 or more is refused by the kernels that read it, since the 32-bit tile
 // numbers scanned from tiles[] may then have wrapped.
 constexpr int kPlanNT = 256;
 __global__ __launch_bounds__(kPlanNT) void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end,
                                                         const uint32_t *s_start, const uint32_t *s_end, uint32_t P,
-                                                        uint32_t s_span, uint32_t cap, int outer, uint32_t *tiles,
+                                                        uint32_t s_span, uint32_t cap, uint32_t *tiles,
                                                         uint64_t *n_tiles) {
   __shared__ uint64_t red[kPlanNT / kWave + 1];
   const uint32_t p = blockIdx.x * kPlanNT + threadIdx.x;
   uint64_t n = 0;
-  if (p < P) n = span_tiles(r_end[p] - r_start[p], s_end[p] - s_start[p], s_span, cap, outer);
+  if (p < P)
+    n = ((uint64_t)(r_end[p] - r_start[p]) + cap - 1) / cap * (((uint64_t)(s_end[p] - s_start[p]) + s_span - 1) / s_span);
   if (p <= P) tiles[p] = (uint32_t)n;
   const uint64_t sum = block_sum<kPlanNT, uint64_t>(n, red);
   if (threadIdx.x == 0 && sum) atomic_add_agent(n_tiles, sum);
@@ -244,7 +267,9 @@ __global__ __launch_bounds__(kPlanNT) void k_plan_spans(const uint32_t *r_start,
 
 }  // namespace
 
-size_t outer_words(uint64_t s_rows, uint64_t spans) { return s_rows / 32 + 2 * spans + 4; }
+size_t outer_words(uint64_t s_rows, uint32_t parts, uint32_t s_span) {
+  return matched_words(s_rows) + parts + s_rows / s_span + 1;
+}
 
 size_t join_plan_scratch_bytes(uint32_t parts) { return scan_scratch_bytes_u32((uint64_t)parts + 1); }
 
@@ -263,10 +288,10 @@ uint32_t join_fused_cap(uint32_t lds_cap) {
 hipError_t join_fused_plan(uint32_t parts, uint32_t s_span, uint32_t cap, const uint32_t *r_start,
                            const uint32_t *r_end, const uint32_t *s_start, const uint32_t *s_end,
                            uint32_t *tile_start, uint64_t *n_tiles_dev, void *scan_scratch, uint32_t *err,
-                           hipStream_t stream, bool outer) {
+                           hipStream_t stream) {
   const uint32_t n = parts + 1;
   hipLaunchKernelGGL(k_plan_spans, dim3((n + kPlanNT - 1) / kPlanNT), dim3(kPlanNT), 0, stream, r_start, r_end,
-                     s_start, s_end, parts, s_span, cap, (int)outer, tile_start, n_tiles_dev);
+                     s_start, s_end, parts, s_span, cap, tile_start, n_tiles_dev);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return scan_u32(tile_start, tile_start, n, nullptr, scan_scratch, err, stream);
@@ -296,24 +321,16 @@ uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tile
 hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
                       const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
                       const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
-                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer, uint32_t *err,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched, uint32_t *err,
                       hipStream_t stream, bool swapped) {
   if (grid == 0) return hipSuccess;
   const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
   uint2 *vout = reinterpret_cast<uint2 *>(out);
-#define EO_FUSED(C)                                                                                                  \
-  do {                                                                                                               \
-    if (outer)                                                                                                       \
-      EO_TIMED("probe", stream,                                                                                      \
-               hipLaunchKernelGGL(k_join_outer<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,   \
-                                  s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,   \
-                                  outer, n_tiles_dev, err));                                                         \
-    else                                                                                                             \
-      EO_TIMED("probe", stream,                                                                                      \
-               hipLaunchKernelGGL(k_join_fused<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,   \
-                                  s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,   \
-                                  n_tiles_dev, err, (int)swapped));                                                  \
-  } while (0)
+#define EO_FUSED(C)                                                                                                \
+  EO_TIMED("probe", stream,                                                                                        \
+           hipLaunchKernelGGL(k_join_fused<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,     \
+                              s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,     \
+                              matched, n_tiles_dev, err, (int)swapped))
   if (cap == (uint32_t)tile::ProbeSmall::Cap) EO_FUSED(ProbeSmall);
   else if (cap == (uint32_t)tile::ProbeBig::Cap) EO_FUSED(ProbeBig);
   else return hipErrorInvalidValue;
@@ -321,24 +338,49 @@ hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t gr
   return hipGetLastError();
 }
 
+hipError_t join_outer(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
+                      const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
+                      const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint64_t s_rows, uint32_t *words, uint32_t *err,
+                      hipStream_t stream) {
+  if (grid == 0) return hipSuccess;
+  const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
+  uint2 *vout = reinterpret_cast<uint2 *>(out);
+  uint32_t *done = words + matched_words(s_rows);
+#define EO_OUTER(C)                                                                                                \
+  EO_TIMED("probe", stream,                                                                                        \
+           hipLaunchKernelGGL(k_join_outer<tile::C>, dim3(grid), dim3(kFNT), 0, stream, vR, r_start, r_end, vS,     \
+                              s_start, s_end, tile_start, parts, s_span, vout, out_cap, out_cursor, (int)wide,     \
+                              words, done, n_tiles_dev, err))
+  if (cap == (uint32_t)tile::ProbeSmall::Cap) EO_OUTER(ProbeSmall);
+  else if (cap == (uint32_t)tile::ProbeBig::Cap) EO_OUTER(ProbeBig);
+  else return hipErrorInvalidValue;
+#undef EO_OUTER
+  return hipGetLastError();
+}
+
 template <typename C>
 static hipError_t launch_direct(const DirectPlan &d, const uint2 *R, uint64_t nR, const uint2 *S, uint64_t nS,
-                                uint2 *out, uint64_t out_cap, uint64_t *cursor, bool wide, uint32_t *outer,
-                                bool swapped, const char *name, hipStream_t stream) {
-  const uint64_t grid = outer ? d.spans : (uint64_t)d.chunks * d.spans;
+                                uint2 *out, uint64_t out_cap, uint64_t *cursor, bool wide, uint32_t *matched,
+                                bool outer, bool swapped, const char *name, hipStream_t stream) {
+  const uint64_t grid = (uint64_t)d.chunks * d.spans;
   if (grid > 0xffffffffull / C::NT) return hipErrorInvalidValue;  // 2^32 work-items a dispatch
-  if (outer)
+  if (outer && !matched && out)
     EO_TIMED(name, stream,
-             hipLaunchKernelGGL(k_join_direct_outer<C>, dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, (uint32_t)nR,
-                                S, (uint32_t)nS, d.span, out, out_cap, cursor, (int)wide, outer));
+             hipLaunchKernelGGL((k_join_direct_outer<C, true>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R,
+                                (uint32_t)nR, S, (uint32_t)nS, d.span, out, out_cap, cursor, (int)wide));
+  else if (outer && !matched)
+    EO_TIMED(name, stream,
+             hipLaunchKernelGGL((k_join_direct_outer<C, false>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R,
+                                (uint32_t)nR, S, (uint32_t)nS, d.span, nullptr, 0ull, cursor, 0));
   else if (out)
     EO_TIMED(name, stream,
              hipLaunchKernelGGL((k_join_direct<C, true>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
-                                d.chunk, d.chunks, d.span, out, out_cap, cursor, (int)wide, (int)swapped));
+                                d.chunk, d.chunks, d.span, out, out_cap, cursor, (int)wide, matched, (int)swapped));
   else
     EO_TIMED(name, stream,
              hipLaunchKernelGGL((k_join_direct<C, false>), dim3((uint32_t)grid), dim3(C::NT), 0, stream, R, nR, S, nS,
-                                d.chunk, d.chunks, d.span, nullptr, 0ull, cursor, 0, 0));
+                                d.chunk, d.chunks, d.span, nullptr, 0ull, cursor, 0, matched, 0));
   return hipGetLastError();
 }
 
@@ -348,15 +390,22 @@ hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, cons
   if (nS == 0 || (nR == 0 && !outer)) return hipSuccess;
   const uint2 *vR = reinterpret_cast<const uint2 *>(R), *vS = reinterpret_cast<const uint2 *>(S);
   uint2 *vout = reinterpret_cast<uint2 *>(out);
+  // several R chunks: all tiles beside each other, the null rows from the
+  // matches they marked
+  uint32_t *matched = outer && d.chunks > 1 ? outer : nullptr;
+  hipError_t e = matched ? fill_u32(matched, 0u, matched_words(nS), stream) : hipSuccess;
+  if (e != hipSuccess) return e;
 #define EO_DIRECT(C) \
-  launch_direct<tile::C>(d, vR, nR, vS, nS, vout, out_cap, out_cursor, wide, outer, swapped, name, stream)
+  launch_direct<tile::C>(d, vR, nR, vS, nS, vout, out_cap, out_cursor, wide, matched, outer, swapped, name, stream)
   switch (d.table) {
-    case kFusedTableFull: return EO_DIRECT(ProbeBig);
-    case kFusedTableHalf: return EO_DIRECT(ProbeSmall);
-    case kFusedTableQuarter: return EO_DIRECT(ProbeQuarter);
+    case kFusedTableFull: e = EO_DIRECT(ProbeBig); break;
+    case kFusedTableHalf: e = EO_DIRECT(ProbeSmall); break;
+    case kFusedTableQuarter: e = EO_DIRECT(ProbeQuarter); break;
     default: return hipErrorInvalidValue;
   }
 #undef EO_DIRECT
+  if (e == hipSuccess && matched) e = emit_unmatched(S, nS, matched, out_cursor, out, out_cap, wide, stream);
+  return e;
 }
 
 hipError_t span_count(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t n_tiles, const uint64_t *n_tiles_dev,

@@ -125,6 +125,8 @@ struct OneArgs {
   OneRel rel[2];     // R, S
   uint32_t *hs;      // 2 kOneCopies one_hs_words(bits) words, zero on entry and again on completion
   uint32_t *ticket;  // 2 words, likewise
+  uint32_t *zero;    // nzero words to clear (join_outer's)
+  uint32_t nzero;
 };
 __host__ __device__ inline constexpr uint32_t one_hs_words(int bits) { return (1u << bits) + 2u; }
 uint64_t one_pass_rows(uint64_t n, int bits);
@@ -132,7 +134,7 @@ bool one_pass_supported(uint64_t nR, uint64_t nS, int bits);
 OneRel one_pass_rel(const eo_tuple *in, uint64_t n, int bits, eo_tuple *out, uint32_t *start, uint32_t *end,
                     uint32_t *cur);
 // tile_start: 2^bits + 1; *n_tiles: their number.  cap: R tuples per probe
-// tile; outer: the tiles of join_fused's left outer joins.  A partition that
+// tile; outer: join_outer's tiles.  A partition that
 // proves too small raises kErrCapacity in *err.
 hipError_t one_pass_partition(const OneArgs &a, int bits, uint32_t s_span, uint32_t cap, bool outer,
                               uint32_t *tile_start, uint64_t *n_tiles, uint32_t *err, hipStream_t stream);
@@ -153,7 +155,7 @@ uint32_t join_fused_cap(uint32_t lds_cap);
 hipError_t join_fused_plan(uint32_t parts, uint32_t s_span, uint32_t cap, const uint32_t *r_start,
                            const uint32_t *r_end, const uint32_t *s_start, const uint32_t *s_end,
                            uint32_t *tile_start, uint64_t *n_tiles_dev, void *scan_scratch, uint32_t *err,
-                           hipStream_t stream, bool outer = false);
+                           hipStream_t stream);
 // Grid of join_fused for `parts` partitions of nR x nS tuples, sized without
 // the tile count (tiles_est: the host's estimate of it).
 uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tiles_est, int cus);
@@ -161,24 +163,30 @@ uint32_t join_fused_grid(uint32_t parts, uint64_t nR, uint64_t nS, uint64_t tile
 // is correct; a tile count of 2^31 or more raises kErrOverflow in *err and
 // probes nothing).
 // wide: out holds 16-byte RESULT rows {R payload, key, S payload, key};
-// outer (optional): a left outer join — a null row per S tuple without a match
-// comes with the other rows, the plan is join_fused_plan's for outer joins, and
-// `outer` is scratch of outer_words(rows of the S buffer, spans) words (no
-// contents expected) for partitions whose R side takes several tables.
+// matched (optional): bitmap over S positions of the tuples that matched.
 // swapped: R is the caller's S and S its R (the smaller relation built into
 // the tables); the rows are written with the payloads exchanged.
 hipError_t join_fused(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
                       const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
                       const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
-                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer, uint32_t *err,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *matched, uint32_t *err,
                       hipStream_t stream, bool swapped = false);
-size_t outer_words(uint64_t s_rows, uint64_t spans);
+// The left outer join of one_pass_partition's tiles: a null row per S tuple
+// without a match comes with the other rows.  words: outer_words(rows of the S
+// buffer, parts, s_span) words, zero on entry.
+hipError_t join_outer(uint32_t parts, uint32_t s_span, uint32_t cap, uint32_t grid, const uint64_t *n_tiles_dev,
+                      const eo_tuple *R, const uint32_t *r_start, const uint32_t *r_end, const eo_tuple *S,
+                      const uint32_t *s_start, const uint32_t *s_end, const uint32_t *tile_start, eo_pair *out,
+                      uint64_t out_cap, uint64_t *out_cursor, bool wide, uint64_t s_rows, uint32_t *words, uint32_t *err,
+                      hipStream_t stream);
+size_t outer_words(uint64_t s_rows, uint32_t parts, uint32_t s_span);
 // One launch of the integer VALU probe `kind` (EO_VALU_COMPARE / EO_VALU_ADD)
 // over `blocks` 256-thread blocks; *ops = the operations it performs.
 hipError_t valu_kernel(int kind, uint32_t blocks, uint32_t reps, uint64_t *sink, hipStream_t s, double *ops);
-// The unpartitioned join on the host's tile plan, one launch.  *out_cursor must
-// be zero on entry; out == NULL counts only; outer: as join_fused's.  name: the
-// launch timer's.
+// The unpartitioned join on the host's tile plan, one launch (left outer joins
+// of several R chunks: three).  *out_cursor must be zero on entry; out == NULL
+// counts only; outer (optional): matched_words(nS) words of scratch, a null row
+// per S tuple without a match.  name: the launch timer's.
 struct DirectPlan;
 hipError_t join_direct(const DirectPlan &d, const eo_tuple *R, uint64_t nR, const eo_tuple *S, uint64_t nS,
                        eo_pair *out, uint64_t out_cap, uint64_t *out_cursor, bool wide, uint32_t *outer,

@@ -26,9 +26,7 @@ namespace {
 constexpr size_t kNoAllocScratchBytes = (size_t)EO_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 64;
 
-constexpr size_t kNoAllocSlack = 64 << 10;
-
-static __device__ __align__(256) char scratch[kNoAllocScratchBytes + kNoAllocSlack];
+static __device__ __align__(256) char scratch[kNoAllocScratchBytes];
 
 std::mutex g_mu;
 char *g_scratch[kMaxDevices] = {};  // device address of `scratch` on each device
@@ -71,6 +69,6 @@ extern "C" eo_status eo_hash_join_noalloc(eo_ctx *c, const eo_tuple *R, uint64_t
     set_last_error("eo_hash_join_noalloc: scratch not prepared on this device");
     return EO_EINTERNAL;
   }
-  FixedScratch fx{base, kNoAllocScratchBytes, kNoAllocSlack};
+  FixedScratch fx{base, kNoAllocScratchBytes};
   return hash_join_impl(c, R, nR, S, nS, out, out_cap, n_out, o, &fx);
 }

@@ -29,10 +29,6 @@ constexpr int kOneNT = tile::kGapSampleNT;           // 512
 constexpr uint32_t kOneTiles = tile::kGapSampleUnroll;  // tiles one workgroup samples
 constexpr int kOnePlanNT = 1024;
 
-__device__ __forceinline__ uint32_t ld_agent(const uint32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // A counter's kOneCopies copies, one_hs_words apart, are added to by different
 // XCDs' workgroups (atomics on one word queue up) and summed by the layout.
 __device__ __forceinline__ uint32_t sum_copies(const uint32_t *p, uint32_t stride) {
@@ -150,14 +146,11 @@ __global__ __launch_bounds__(kOneNT) void k_one_count(OneArgs a, uint32_t *err) 
   __syncthreads();
   for (uint32_t d = threadIdx.x; d < F; d += kOneNT)
     if (hist[d]) atomic_add_agent(hs + d, hist[d]);
-  // The relation's last workgroup lays it out.  Counts and ticket are device-
-  // scope atomics, performed at memory, and the layout reads the counts the
-  // same way, so all that is needed is that a thread's counts are performed
-  // before its workgroup's ticket: a wait for them.  (A release fence at device
-  // scope would also write the XCD's whole L2 back, once per workgroup: 15 M
-  // tuples 39 instead of 28 us; one counter copy instead of kOneCopies: 28
-  // instead of 13 us.)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // The relation's last workgroup lays it out, from counts that are device-scope
+  // atomics like the ticket.  (A release fence at device scope would also write
+  // the XCD's whole L2 back, once per workgroup: 15 M tuples 39 instead of 28
+  // us; one counter copy instead of kOneCopies: 28 instead of 13 us.)
+  wait_atomics();
   __syncthreads();
   if (threadIdx.x == 0) s_last = atomic_add_agent(a.ticket + rel, 1u) == r.units - 1;
   __syncthreads();
@@ -167,10 +160,11 @@ __global__ __launch_bounds__(kOneNT) void k_one_count(OneArgs a, uint32_t *err) 
 }
 
 // Blocks [0, round8(tiles of R)) scatter R, the rest S; consecutive tiles of a
-// relation on one XCD.
+// relation on one XCD.  Also clears the left outer probe's words.
 template <int BITS>
 __global__ __launch_bounds__(kFastNT) void k_one_scatter(OneArgs a, uint32_t *err) {
   __shared__ tile::ScatterShared<BITS> sh;
+  for (uint32_t i = blockIdx.x * kFastNT + threadIdx.x; i < a.nzero; i += gridDim.x * kFastNT) a.zero[i] = 0;
   const uint32_t g0 = (a.rel[0].tiles + kXcds - 1) / kXcds * kXcds;
   const uint32_t rel = blockIdx.x < g0 ? 0u : 1u;
   const OneRel &r = a.rel[rel];
@@ -188,7 +182,7 @@ __global__ __launch_bounds__(kFastNT) void k_one_scatter(OneArgs a, uint32_t *er
 }
 
 // One workgroup: every partition's filled end, its probe tiles (R chunks of
-// `cap` x S spans; outer: S spans, whatever R holds) and their scan.
+// `cap`, outer: at least one, x S spans) and their scan.
 template <int BITS>
 __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_span, uint32_t cap, int outer,
                                                           uint32_t *__restrict__ tile_start, uint64_t *n_tiles) {
@@ -211,7 +205,8 @@ __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_s
       }
       // (64 bits: a sum of 2^31 or more is refused by the probe)
       const uint64_t spans = ((uint64_t)n[1] + s_span - 1) / s_span;
-      cnt[k] = outer ? spans : n[0] ? ((uint64_t)n[0] + cap - 1) / cap * spans : 0ull;
+      const uint64_t chunks = ((uint64_t)n[0] + cap - 1) / cap;
+      cnt[k] = (outer ? max(chunks, (uint64_t)1) : chunks) * spans;
     }
     sum += cnt[k];
   }

@@ -120,8 +120,7 @@ DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus,
     d.chunks = (uint32_t)std::max<uint64_t>(1, (nR + d.chunk - 1) / d.chunk);
     const uint64_t slots = n_cu * t.per_cu, batches = std::max<uint64_t>(1, (nS + t.batch - 1) / t.batch);
     // as many S spans as fill the chip once, of whole batches
-    const uint64_t side = outer ? 1 : d.chunks;  // chunks of a span that run beside each other
-    uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / side));
+    uint64_t spans = std::min(batches, std::max<uint64_t>(1, slots / d.chunks));
     uint64_t span = (batches + spans - 1) / spans * t.batch;
     if (span_opt) span = std::max<uint64_t>(t.batch, (uint64_t)span_opt);
     // (a dispatch holds fewer than 2^32 work-items: a shorter span from the
@@ -132,8 +131,10 @@ DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *o, int cus,
     spans = std::max<uint64_t>(1, (nS + span - 1) / span);
     d.span = (uint32_t)span;
     d.spans = (uint32_t)spans;
-    const double waves = (double)((side * spans + slots - 1) / slots) * (double)(d.chunks / side);
+    const double waves = (double)((d.chunks * spans + slots - 1) / slots);
     d.us = waves * t.tile(d.chunk, (double)std::min(span, nS)) + kAtomicUs * (double)d.chunks * (double)batches;
+    // several chunks: the match bitmap is cleared before and read after the tiles
+    if (outer && d.chunks > 1) d.us += 10 + 2e-6 * (double)nS;
     if (!best.table || d.us < best.us) best = d;
   }
   return best;

@@ -53,7 +53,7 @@ struct DirectPlan {
   double us = 0;  // the time model's estimate of the launch
 };
 // opts: lds_tuples and s_tile overrides (0: chosen here).  outer: a left outer
-// join, whose spans take the chunks one after the other.
+// join, which adds two launches to tiles of several chunks.
 DirectPlan plan_direct(uint64_t nR, uint64_t nS, const eo_join_opts *opts, int cus, bool outer = false);
 
 // The plan of a fused join of one pass that partitions both relations together

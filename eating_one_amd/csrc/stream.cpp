@@ -177,6 +177,7 @@ struct Streamer {
     const eo_tuple *probe_side = dS[b];
     hipError_t e = hipSuccess;
     if (hash) {
+      if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(n), cs), "match bitmap reset");
       if (hp.passes) {
         eo_status s = partition_relation(c, dS[b], n, hp, tmp, sp, s_start, pscr, cs);
         if (s != EO_OK) return s;
@@ -187,15 +188,16 @@ struct Streamer {
       }
       const uint32_t cap_lds = join_fused_cap(hp.lds_cap);
       EO_TRY_HIP(join_fused_plan(P, hp.s_span, cap_lds, r_start, r_start + 1, s_start, s_start + 1, tile_start,
-                                 small, jscr, c->d_err, cs, outer),
+                                 small, jscr, c->d_err, cs),
                  "tile plan");
       // the probe's grid does not need the tile count: no readback before it
       const uint64_t tiles_est = (uint64_t)P + nr / cap_lds + n / hp.s_span + 1024;
       e = join_fused(P, hp.s_span, cap_lds, join_fused_grid(P, nr, n, tiles_est, c->props.cus), small, hp.passes ? rp : dR,
                      r_start, r_start + 1, probe_side, s_start, s_start + 1, tile_start, dst, cap, small + 1, wide,
                      outer ? matched : nullptr, c->d_err, cs);
+      if (e == hipSuccess && outer) e = emit_unmatched(probe_side, n, matched, small + 1, dst, cap, wide, cs);
     } else {
-      e = join_direct(plan_direct(nr, n, nullptr, c->props.cus, outer), dR, nr, dS[b], n, cap ? dst : nullptr, cap,
+      e = join_direct(plan_direct(nr, n, nullptr, c->props.cus), dR, nr, dS[b], n, cap ? dst : nullptr, cap,
                       small + 1, wide, outer ? matched : nullptr, false, dst ? "nlj_fused" : "nlj_count", cs);
     }
     if (e != hipSuccess) return hip_fail(e, hash ? "stream hash probe" : "stream nlj");
@@ -329,9 +331,7 @@ extern "C" eo_status eo_stream_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, c
   const size_t o_ss = L.add((x.P + 1) * sizeof(uint32_t));
   const size_t o_ts = L.add((x.P + 1) * sizeof(uint32_t));
   const size_t o_small = L.add(8 * sizeof(uint64_t));
-  // (spans: at most one short one per partition; an NLJ's are at least 2048 tuples)
-  const size_t o_bits =
-      L.add(outer ? outer_words(sc, x.hash ? x.P + sc / x.hp.s_span + 1 : sc / 2048 + 1) * sizeof(uint32_t) : 0);
+  const size_t o_bits = L.add(outer ? matched_words(sc) * sizeof(uint32_t) : 0);
   size_t pscr = 0;
   if (parted)
     for (uint64_t n : {std::min(rt, nR), r_last, sc, s_last}) pscr = std::max(pscr, partition_scratch(n, x.hp, cus));

@@ -66,11 +66,9 @@ constexpr int kProbeOrdered = 2;  // write rows from position base on, in an ord
 // nothing and returns the number of matches.  Positions >= out_cap are
 // counted only.  wide: 16-byte RESULT rows instead of pairs (see emit_pair).
 // matched (optional bitmap over S positions): sets the bit of every S tuple
-// that matched, for a left outer join.  OUTER (kProbeFused): also writes a null
-// row for every S tuple of the span that no R chunk matched: chunks of one
-// partition come one after the other (first, last), and with more than one of
-// them mw (2 words per 64 tuples of the span, the workgroup's own) carries the
-// matches so far.  swapped: the table side is the
+// that matched, for a left outer join.  OUTER (not kProbeOrdered) without
+// `matched`: the chunk is the whole R side, and every S tuple of the span that it
+// does not match gets (or counts as) a null row with the other rows.  swapped: the table side is the
 // caller's S and the streamed side its R (an inner join built on its smaller
 // relation), so every row is written with the two payloads exchanged.
 // All threads of the workgroup call it; it leaves LDS free for reuse.
@@ -79,9 +77,8 @@ __device__ __forceinline__ uint64_t probe_tile(ProbeShared<C> &sh, const uint2 *
                                                const uint2 *__restrict__ S, const SpanRef &ref,
                                                uint2 *__restrict__ out, uint64_t out_cap, uint64_t *cursor,
                                                bool wide = false, uint32_t *matched = nullptr, uint64_t base = 0,
-                                               bool swapped = false, uint32_t *mw = nullptr, bool first = true,
-                                               bool last = true) {
-  static_assert(!OUTER || MODE == kProbeFused, "null rows come with the fused rows");
+                                               bool swapped = false) {
+  static_assert(!OUTER || MODE != kProbeOrdered, "ordered rows: the null rows follow the others");
   constexpr int NW = C::NT / kWave;
   auto load_batch = [&](uint32_t b0, uint2 *dst) {
 #pragma unroll
@@ -207,6 +204,7 @@ __device__ __forceinline__ uint64_t probe_tile(ProbeShared<C> &sh, const uint2 *
     if (MODE == kProbeCount) {
 #pragma unroll
       for (int u = 0; u < C::SPT; ++u) {
+        if (OUTER && !matched && m[u] == 0 && b0 + u * C::NT + threadIdx.x < ref.s_n) m[u] = 1;
         mine += m[u];
         cur[u] = nxt[u];
       }
@@ -216,18 +214,7 @@ __device__ __forceinline__ uint64_t probe_tile(ProbeShared<C> &sh, const uint2 *
     if constexpr (OUTER) {
 #pragma unroll
       for (int u = 0; u < C::SPT; ++u) {
-        const uint32_t at = b0 + u * C::NT + w * kWave;  // the wave's 64 tuples of the span
-        bool hit = m[u] != 0;
-        if (mw && at < ref.s_n) {
-          uint64_t seen = __ballot(hit);
-          if (!first) seen |= (uint64_t)mw[at / 32 + 1] << 32 | mw[at / 32];
-          if (!last && lane == 0) {
-            mw[at / 32] = (uint32_t)seen;
-            mw[at / 32 + 1] = (uint32_t)(seen >> 32);
-          }
-          hit = (seen >> lane) & 1;
-        }
-        if (last && !hit && at + lane < ref.s_n) {  // (unmatched by this chunk too)
+        if (!matched && m[u] == 0 && b0 + u * C::NT + threadIdx.x < ref.s_n) {
           nul |= 1u << u;
           m[u] = 1;
           fp[u] = kNullPayload;
@@ -282,7 +269,7 @@ __device__ __forceinline__ uint64_t probe_tile(ProbeShared<C> &sh, const uint2 *
           else if (swapped) emit_pair<true>(out, pos, cur[u].y, fp[u], cur[u].x, wide);
           else emit_pair<true>(out, pos, fp[u], cur[u].y, cur[u].x, wide);
         }
-      } else {
+      } else if (pos < out_cap) {
         const uint32_t h = bucket_hash((int32_t)cur[u].x, C::Log2NB);
         const uint32_t e1 = sh.off[h + 1];
         for (uint32_t e = sh.off[h]; e < e1; ++e) {

@@ -328,6 +328,9 @@ static void check_time_model() {
           CHECK((uint64_t)d.chunks * d.chunk >= nR && (uint64_t)(d.chunks - 1) * d.chunk < nR);
           CHECK((uint64_t)d.spans * d.span >= nS && (uint64_t)(d.spans - 1) * d.span < nS);
         }
+        // a left outer join spreads its R chunks over the chip as an inner one does
+        CHECK(eo::plan_direct(nR, nS, nullptr, cus, true).us <=
+              eo::plan_direct(nR, nS, nullptr, cus, false).us + 10 + 2e-6 * (double)nS + 1e-6);
         // any span and table from the caller: a dispatch holds 2^32 work-items
         for (int span : {1, 8192, 100000, 1 << 30})
           for (int lds : {0, 4096, 8192, 16384}) {

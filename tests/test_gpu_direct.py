@@ -96,3 +96,36 @@ def test_too_many_tiles_are_refused(ctx, bits, deterministic):
         R, S = _relations(3000, 9000, 2000)
         assert same_multiset(c.hash_join(R, S, deterministic=deterministic), brute_join(R, S))
         rel.close()
+
+
+def _check_outer(join, R, S, **kw):
+    want = brute_join(R, S)
+    absent = S[~np.isin(S[:, 0], R[:, 0])]
+    rows = join(R, S, left_outer=True, **kw)
+    null = rows[:, 0] == _abi.EO_NULL_PAYLOAD
+    assert same_multiset(rows[~null], want)
+    assert np.array_equal(np.sort(rows[null, 1]), np.sort(absent[:, 1]))
+    assert join(R, S, left_outer=True, count_only=True, **kw) == len(want) + len(absent)
+
+
+@pytest.mark.parametrize("nR,nS", [(200_003, 1), (200_003, 63), (1 << 20, 1000), (70_001, 8193), (17409, 40_000)])
+def test_outer_joins_of_a_large_build_side(ctx, nR, nS):
+    """The R chunks of an unpartitioned left outer join run beside each other and mark what they
+    match; the null rows follow."""
+    R, S = _relations(nR, nS, 2 * nR)
+    _check_outer(ctx.nlj_join, R, S)
+    _check_outer(ctx.hash_join, R, S, radix_bits=-1)
+    _check_outer(ctx.hash_join, R, S, radix_bits=-1, lds_tuples=4096)
+
+
+@pytest.mark.parametrize("lds", [8192, 16384])
+@pytest.mark.parametrize("flags", [0, _abi.EO_F_EXACT_PARTITIONS])
+def test_outer_joins_of_one_large_partition(ctx, lds, flags):
+    """R in one of 32 partitions, several tables and S spans there: the last chunk of a span writes
+    its null rows; beside it partitions without R."""
+    rng = np.random.default_rng(lds + flags)
+    nR, nS = 60_000, 100_003
+    R = np.stack([rng.integers(0, nR, nR) << 5, np.arange(nR)], 1).astype(np.int32)
+    keys = rng.integers(0, 2 * nR, nS)
+    S = np.stack([np.where(rng.random(nS) < 0.7, keys << 5, keys), np.arange(nS)], 1).astype(np.int32)
+    _check_outer(ctx.hash_join, R, S, radix_bits=5, passes=1, lds_tuples=lds, s_tile=8192, flags=flags)
