@@ -110,7 +110,7 @@ hipError_t partition_bounds(const eo_tuple *sorted, uint64_t n, int bits, int sh
 // ---- onepass.hip -------------------------------------------------------------
 // One-pass partition of both relations of a fused join in three launches, the
 // last of them the probe's tile plan.  Up to 10 bits (at 11 the scatter's
-// staging tile and digit arrays fill the LDS, and two passes are faster).
+// staging tile and digit arrays fill the LDS).
 constexpr int kOneMaxBits = 10;
 constexpr uint32_t kOneCopies = 8;
 struct OneRel {

@@ -28,14 +28,8 @@ eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *o, HashPl
   // extra radix bit lands in the second pass (which moves the same bytes),
   // and two probe workgroups per CU hide each other's barrier and atomic
   // round trips (C2, 2^27 x 2^28: probe 1.32 -> 1.08 ms, join 5.09 -> 4.93 ms;
-  // deterministic order 7.35 -> 6.86 ms).  The fused order takes two passes
-  // from 11 bits on: a tile's runs of 2048 digits are 64 bytes (30 M x 60 M
-  // tuples: 1.14 ms in one pass of 11 bits, 0.99 in two of 6; 2^24 x 2^25: 0.57
-  // in one of 10, 0.64 in two).
-  const bool det = o && (o->flags & EO_F_DETERMINISTIC);
-  if (!cap_opt && !bits_opt && nR > 16384 &&
-      ceil_log2((nR + 16383) / 16384) > (det ? kMaxPassBits : kOneMaxBits))
-    p.lds_cap = 8192u;
+  // deterministic order 7.35 -> 6.86 ms).
+  if (!cap_opt && !bits_opt && nR > 16384 && ceil_log2((nR + 16383) / 16384) > kMaxPassBits) p.lds_cap = 8192u;
   if (bits_opt == -1) {
     p.bits = 0;
   } else if (bits_opt > 0) {
@@ -213,6 +207,17 @@ bool one_pass_supported(uint64_t nR, uint64_t nS, int bits) {
 }
 
 void plan_fused(uint64_t nR, uint64_t nS, int cus, bool outer, HashPlan *p) {
+  if (p->bits > kOneMaxBits) {
+    // 11 bits: where both relations' partitions are sampled two passes of the
+    // half table's 12 bits, since a tile's runs of 2048 digits are 64 bytes
+    // (one counted pass, two sampled: 17 M x 34 M tuples 0.68 and 0.68 ms, 30 M
+    // x 60 M 1.14 and 1.00; counted either way, 17 M x 34 M take 0.68 and
+    // 0.75, left outer 0.71 and 0.77)
+    eo_join_opts half{};
+    half.lds_tuples = 8192;
+    if (!outer) (void)plan_hash_join(nR, nS, &half, p, cus);
+    return;
+  }
   HashPlan one = *p;
   const double us = plan_one_pass(nR, nS, cus, &one);
   if (us == 0) return;

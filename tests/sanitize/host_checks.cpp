@@ -287,6 +287,24 @@ static void check_planner() {
         CHECK(chunks <= eo::kUnpartitionedChunks && chunks * nS <= eo::kUnpartitionedSReads);
       }
     }
+  // 11 radix bits: one pass wherever the partitions are counted (left outer,
+  // exact, misaligned, streamed and batched joins); two of the half table's 12
+  // for the fused inner join of sampled partitions
+  for (uint64_t nR : {(1ull << 24) + 1, 30000000ull, 1ull << 25}) {
+    for (int flags : {0, EO_F_LEFT_OUTER, EO_F_EXACT_PARTITIONS, EO_F_DETERMINISTIC}) {
+      eo_join_opts o{};
+      o.flags = flags;
+      eo::HashPlan hp;
+      CHECK(eo::plan_hash_join(nR, 2 * nR, &o, &hp) == EO_OK && hp.bits == 11 && hp.passes == 1 && hp.lds_cap == 16384);
+    }
+    for (bool outer : {false, true}) {
+      eo::HashPlan hp;
+      CHECK(eo::plan_hash_join(nR, 2 * nR, nullptr, &hp) == EO_OK);
+      eo::plan_fused(nR, 2 * nR, 256, outer, &hp);
+      CHECK(hp.bits == (outer ? 11 : 12) && hp.passes == (outer ? 1 : 2));
+      CHECK(hp.lds_cap == (outer ? 16384u : 8192u) && hp.s_span >= 8192);
+    }
+  }
   // overrides: accepted when consistent, refused otherwise
   eo_join_opts o{};
   eo::HashPlan hp;
