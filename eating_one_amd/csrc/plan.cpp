@@ -229,6 +229,53 @@ void plan_fused(uint64_t nR, uint64_t nS, int cus, bool outer, HashPlan *p) {
   // size; unpartitioned, 2^24 x (2^31 - 1) would read S 964 times)
 }
 
+std::vector<PlanChoice> tune_candidates(uint64_t nR, uint64_t nS, int cus) {
+  std::vector<PlanChoice> v;
+  // per LDS table (a full table, one 1024-thread workgroup per CU, or a half
+  // table with two): bits b0-1 .. b0+2 around the planner's for that table,
+  // passes 1 (bits <= 11) or 2, span auto / x2 / x0.5
+  for (int lds : {16384, 8192}) {
+    eo_join_opts lo{};
+    lo.lds_tuples = lds;
+    HashPlan base;
+    if (plan_hash_join(nR, nS, &lo, &base, cus) != EO_OK) continue;
+    for (int b = std::max(0, base.bits - 1); b <= std::min(kMaxJoinBits, base.bits + 2); ++b) {
+      for (int p = 1; p <= 2; ++p) {
+        if (b == 0 && p == 2) continue;
+        if (b > 0 && p == 1 && b > kMaxPassBits) continue;
+        if (p == 2 && (b < 2 || b > 2 * kMaxPassBits)) continue;
+        HashPlan hp;
+        eo_join_opts o{};
+        o.radix_bits = b ? b : -1;
+        o.passes = b ? p : 0;
+        o.lds_tuples = lds;
+        if (plan_hash_join(nR, nS, &o, &hp, cus) != EO_OK) continue;
+        for (int k = 0; k < 3; ++k) {
+          uint32_t span = hp.s_span;
+          if (k == 1) span = std::min<uint32_t>(span * 2, 1u << 18);
+          if (k == 2) span = std::max<uint32_t>(span / 2, 8192u);
+          if (k > 0 && span == hp.s_span) continue;
+          v.push_back({b, b ? p : 0, lds, k == 0 ? 0 : (int)span});
+        }
+        if (b == 0) break;
+      }
+    }
+  }
+  // the untuned join's own plan (built on the smaller side), whose bits, table
+  // and span may be none of those
+  const uint64_t r = std::min(nR, nS), s = std::max(nR, nS);
+  HashPlan own;
+  if (r && plan_hash_join(r, s, nullptr, &own, cus) == EO_OK && own.passes <= 1) {
+    plan_fused(r, s, cus, false, &own);
+    const DirectPlan d = plan_direct(r, s, nullptr, cus);
+    const PlanChoice c = own.passes
+                             ? PlanChoice{own.bits, own.passes, (int)own.lds_cap, (int)std::max(own.s_span, 8192u)}
+                             : PlanChoice{0, 0, (int)table_lds(d.table), 0};
+    v.push_back(c);
+  }
+  return v;
+}
+
 uint32_t plan_span(uint64_t nR, uint64_t nS, uint32_t lds_cap, int bits, uint64_t s_pool, int cus) {
   // Fused probe: S spans short enough to give every CU a few tiles of the
   // s_pool S tuples that share the GPU (this join's, or a whole batch's), and

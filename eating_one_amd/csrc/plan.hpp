@@ -10,6 +10,8 @@
 
 #include <stdint.h>
 
+#include <vector>
+
 #include "eojoin.h"
 
 namespace eo {
@@ -66,6 +68,18 @@ double plan_one_pass(uint64_t nR, uint64_t nS, int cus, HashPlan *p);
 // relations together, as the time model has it, or *p as it is where the model's
 // one pass does not take the sizes.
 void plan_fused(uint64_t nR, uint64_t nS, int cus, bool outer, HashPlan *p);
+
+// lds_tuples of an LDS table of `table` tuples (fused_table_tuples' inverse).
+inline uint32_t table_lds(uint32_t table) {
+  return table == kFusedTableQuarter ? 4096u : table == kFusedTableHalf ? 8192u : 16384u;
+}
+
+// Plans the autotuner times for a join of these sizes (radix_bits 0:
+// unpartitioned), the one that an untuned join takes among them.
+struct PlanChoice {
+  int radix_bits, passes, lds_tuples, s_tile;
+};
+std::vector<PlanChoice> tune_candidates(uint64_t nR, uint64_t nS, int cus);
 
 // Returns EO_OK and fills *out, or EO_EINVAL for inconsistent overrides.
 eo_status plan_hash_join(uint64_t nR, uint64_t nS, const eo_join_opts *opts, HashPlan *out, int cus = 256);

@@ -518,7 +518,8 @@ eo_status eo_batch_replay(eo_batch *batch);
 typedef struct eo_tune_result {
   int32_t radix_bits;   /* chosen plan (0 bits = no partitioning) */
   int32_t passes;
-  int32_t lds_tuples;   /* 16384 or 8192 (0 in a table saved before the LDS axis: the planner's) */
+  int32_t lds_tuples;   /* 16384 or 8192, unpartitioned also 4096 (0 in a table saved before the
+                           LDS axis: the planner's) */
   int32_t s_tile;       /* 0: the planner's S span */
   double ms;            /* best device time of the chosen plan */
   double default_ms;    /* device time of the untuned planner's plan */
@@ -528,7 +529,8 @@ typedef struct eo_tune_result {
 
 /* Times candidate plans (the LDS table size — a full table with one
  * workgroup per CU, or a half table with two — radix bits around the
- * planner's choice for it, one or two passes, three S spans) for the size
+ * planner's choice for it, one or two passes, three S spans, and the plan of an
+ * untuned join) for the size
  * class of (|R|, |S|) = (ceil log2 nR,
  * ceil log2 nS) on the given device inputs, best of `reps` runs each, and
  * stores the fastest in the ctx's table.  eo_hash_join and eo_batch_submit

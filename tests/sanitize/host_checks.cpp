@@ -381,6 +381,36 @@ static void check_time_model() {
       }
 }
 
+// The autotuner times the plan of an untuned join, so a tuned one is no slower.
+static void check_tune_candidates() {
+  for (int lr = 0; lr <= 30; ++lr)
+    for (int ls = 0; ls <= 30; ++ls) {
+      const uint64_t nR = (1ull << lr) + lr, nS = (1ull << ls) + 5, r = std::min(nR, nS), s = std::max(nR, nS);
+      eo::HashPlan own;
+      CHECK(eo::plan_hash_join(r, s, nullptr, &own) == EO_OK);
+      if (own.passes <= 1) eo::plan_fused(r, s, 256, false, &own);
+      const eo::DirectPlan d = eo::plan_direct(r, s, nullptr, 256);
+      bool found = false;
+      for (const eo::PlanChoice &c : eo::tune_candidates(nR, nS, 256)) {
+        eo_join_opts o{};
+        o.radix_bits = c.radix_bits ? c.radix_bits : -1;
+        o.passes = c.passes;
+        o.lds_tuples = c.lds_tuples;
+        o.s_tile = c.s_tile;
+        eo::HashPlan p;
+        CHECK(eo::plan_hash_join(r, s, &o, &p) == EO_OK);
+        if (p.bits != own.bits || p.passes != own.passes) continue;
+        if (p.passes) {
+          found |= p.lds_cap == own.lds_cap && (p.s_span == own.s_span || (own.s_span < 8192 && p.s_span == 8192));
+        } else {
+          const eo::DirectPlan e = eo::plan_direct(r, s, &o, 256);
+          found |= e.table == d.table && e.chunk == d.chunk && e.span == d.span;
+        }
+      }
+      CHECK(found || own.passes == 2);
+    }
+}
+
 // One admission decision sequence of the request loop on a synthetic clock.
 static void check_serve_queue() {
   using eo::ServeQueue;
@@ -536,6 +566,7 @@ int main() {
   check_tune_table();
   check_planner();
   check_time_model();
+  check_tune_candidates();
   check_serve_queue();
   std::printf("host checks ok: %d checks\n", g_checks);
   return 0;
