@@ -781,7 +781,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
   if (stats) {
     stats->radix_bits = (uint32_t)hp.bits;
     stats->passes = (uint32_t)hp.passes;
-    stats->lds_tuples = hp.lds_cap;
+    stats->lds_tuples = direct ? table_lds(dp.table) : hp.lds_cap;
     stats->sampled = sampled ? 1u : 0u;
   }
   eo_pair *dout = out;

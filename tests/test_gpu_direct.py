@@ -129,3 +129,15 @@ def test_outer_joins_of_one_large_partition(ctx, lds, flags):
     keys = rng.integers(0, 2 * nR, nS)
     S = np.stack([np.where(rng.random(nS) < 0.7, keys << 5, keys), np.arange(nS)], 1).astype(np.int32)
     _check_outer(ctx.hash_join, R, S, radix_bits=5, passes=1, lds_tuples=lds, s_tile=8192, flags=flags)
+
+
+@pytest.mark.parametrize("nR,nS,lds", [(1000, 4000, 4096), (4353, 70_000, 4096), (1 << 16, 1 << 20, 16384)])
+def test_stats_name_the_table_of_an_unpartitioned_join(ctx, nR, nS, lds):
+    """The table that the time model chose, whichever the partitioned plan had: one with fewer
+    tuples than the build side is several chunks of it."""
+    R, S = _relations(nR, nS, nR)
+    st = eo.JoinStats()
+    ctx.hash_join(R, S, stats=st)
+    assert st.radix_bits == 0 and st.lds_tuples == lds
+    table = {4096: 4352, 8192: 8704, 16384: 17408}[lds]
+    assert st.tiles % -(-nR // table) == 0
