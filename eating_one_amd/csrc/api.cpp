@@ -160,7 +160,7 @@ bool opts_ok(const eo_join_opts *o) {
 }
 
 eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const HashPlan &hp, eo_tuple *tmp,
-                             eo_tuple *out, uint32_t *part_start, void *scratch, hipStream_t s, bool stable,
+                             eo_tuple *out, uint32_t *part_start, void *scratch, uint32_t *err, hipStream_t s, bool stable,
                              bool fixed) {
   const int cus = ctx->props.cus;
   if (hp.passes == 1) {
@@ -168,14 +168,14 @@ eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const 
     const bool fast = aligned16(in) && !stable && (!fixed || hp.bits_pass1 <= 7);
     PartPassPlan pp = plan_partition_pass(n, hp.bits_pass1, 0, 0u, cus, fast, hp.stable_stripes);
     pp.ordered = fast && fixed;
-    EO_TRY_HIP(partition_pass(pp, in, out, part_start, scratch, ctx->d_err, s), "partition pass");
+    EO_TRY_HIP(partition_pass(pp, in, out, part_start, scratch, err, s), "partition pass");
     return EO_OK;
   }
   const int b_lo = hp.bits_pass1, b_hi = hp.bits_pass2;
   if (stable) {
     // fall through to the stable LSD passes below
   } else if (aligned16(in) && aligned16(tmp) && msd2_supported(b_hi, b_lo)) {
-    EO_TRY_HIP(partition_msd2(n, b_hi, b_lo, in, tmp, out, part_start, scratch, ctx->d_err, cus, s, fixed),
+    EO_TRY_HIP(partition_msd2(n, b_hi, b_lo, in, tmp, out, part_start, scratch, err, cus, s, fixed),
                "partition (two passes, one histogram)");
     return EO_OK;
   }
@@ -184,15 +184,15 @@ eo_status partition_relation(eo_ctx *ctx, const eo_tuple *in, uint64_t n, const 
     uint32_t *start1 = (uint32_t *)scratch;
     char *rest = (char *)scratch + ((F1 + 1) * sizeof(uint32_t) + 255) / 256 * 256;
     PartPassPlan p1 = plan_partition_pass(n, b_hi, b_lo, 0u, cus, true);
-    EO_TRY_HIP(partition_pass(p1, in, tmp, start1, rest, ctx->d_err, s), "partition pass 1");
+    EO_TRY_HIP(partition_pass(p1, in, tmp, start1, rest, err, s), "partition pass 1");
     SegPassPlan p2 = plan_seg_pass(n, F1, b_lo, 0, cus);
-    EO_TRY_HIP(partition_seg_pass(p2, tmp, out, start1, part_start, rest, ctx->d_err, s), "partition pass 2");
+    EO_TRY_HIP(partition_seg_pass(p2, tmp, out, start1, part_start, rest, err, s), "partition pass 2");
     return EO_OK;
   }
   PartPassPlan p1 = plan_partition_pass(n, b_lo, 0, 0u, cus, false, hp.stable_stripes);
   PartPassPlan p2 = plan_partition_pass(n, b_hi, b_lo, 0u, cus, false, hp.stable_stripes);
-  EO_TRY_HIP(partition_pass(p1, in, tmp, nullptr, scratch, ctx->d_err, s), "partition pass 1");
-  EO_TRY_HIP(partition_pass(p2, tmp, out, nullptr, scratch, ctx->d_err, s), "partition pass 2");
+  EO_TRY_HIP(partition_pass(p1, in, tmp, nullptr, scratch, err, s), "partition pass 1");
+  EO_TRY_HIP(partition_pass(p2, tmp, out, nullptr, scratch, err, s), "partition pass 2");
   EO_TRY_HIP(partition_bounds(out, n, hp.bits, 0, 0u, part_start, s), "partition bounds");
   return EO_OK;
 }
@@ -752,14 +752,14 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
       EO_TRY_HIP(gap(dR, nR, rp, r_start, r_end_g, o_gr, kGapScatter), "partition (sampled regions, R)");
       r_end = r_end_g;
     } else {
-      st = partition_relation(c, dR, nR, hp, tmp, rp, r_start, A + o_pscr, s, stable, fixed);
+      st = partition_relation(c, dR, nR, hp, tmp, rp, r_start, A + o_pscr, c->d_err, s, stable, fixed);
       if (st != EO_OK) return st;
     }
     if (gs) {
       EO_TRY_HIP(gap(dS, nS, sp, s_start, s_end_g, o_gs, kGapScatter), "partition (sampled regions, S)");
       s_end = s_end_g;
     } else {
-      st = partition_relation(c, dS, nS, hp, tmp, sp, s_start, A + o_pscr, s, stable, fixed);
+      st = partition_relation(c, dS, nS, hp, tmp, sp, s_start, A + o_pscr, c->d_err, s, stable, fixed);
       if (st != EO_OK) return st;
     }
     used_gap = sampled = gr || gs;

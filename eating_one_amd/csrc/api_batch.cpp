@@ -296,7 +296,8 @@ eo_status plan_batch(eo_batch *b, const eo_request *reqs, uint32_t n, const eo_j
   blob_bytes = (blob + 15) / 16 * 16;
   b->o_blob = L.add(blob_bytes);
   b->o_bits = L.add(b->bits_words * sizeof(uint32_t));
-  b->o_cursor = L.add(((size_t)nj + 2) * sizeof(uint64_t));  // per-join counts, the capacity flag, the queue head
+  // per-join counts, the capacity flag, the error flags, the queue head
+  b->o_cursor = L.add(((size_t)nj + 3) * sizeof(uint64_t));
   b->o_counts = L.add(max_counts * sizeof(uint64_t));
   b->o_cscr = L.add(max_counts ? scan_scratch_bytes_u64(max_counts) : 0);
   b->o_tmp = L.add(part_bytes(max_tmp));
@@ -416,21 +417,24 @@ eo_status enqueue_batch(eo_batch *b, hipStream_t s) {
   const uint32_t nj = (uint32_t)b->joins.size();
   uint64_t *cursor = reinterpret_cast<uint64_t *>(A + b->o_cursor);
   if (nj == 0) return EO_OK;
-  EO_TRY_HIP(fill_u64(cursor, 0, (uint64_t)nj + 2, s), "cursor reset");  // counts, capacity flag, queue head
+  EO_TRY_HIP(fill_u64(cursor, 0, (uint64_t)nj + 3, s), "cursor reset");  // counts, flags, queue head
   uint32_t *cap_flag = reinterpret_cast<uint32_t *>(cursor + nj);
-  uint32_t *head = reinterpret_cast<uint32_t *>(cursor + nj + 1);
+  // (the batch's own flags: a join of the context may run, and raise and clear
+  // the context's, while the batch is in flight)
+  uint32_t *err = reinterpret_cast<uint32_t *>(cursor + nj + 1);
+  uint32_t *head = reinterpret_cast<uint32_t *>(cursor + nj + 2);
   if (b->outer)
     EO_TRY_HIP(fill_u32(reinterpret_cast<uint32_t *>(A + b->o_bits), 0u, b->bits_words, s), "match bitmap reset");
   uint64_t *counts = reinterpret_cast<uint64_t *>(A + b->o_counts);
   for (auto &G : b->groups)
-    EO_TRY_HIP(batch_partition_group(G.g, counts, A + b->o_cscr, G.g.sampled ? cap_flag : c->d_err, s),
+    EO_TRY_HIP(batch_partition_group(G.g, counts, A + b->o_cscr, G.g.sampled ? cap_flag : err, s),
                "batch partition");
   for (auto &J : b->joins) {
     for (const SideInfo *sd : {&J.r, &J.s}) {
       if (sd->mode != 2) continue;
       eo_status st = partition_relation(c, sd->in, sd->n, J.hp, reinterpret_cast<eo_tuple *>(A + b->o_tmp),
                                         reinterpret_cast<eo_tuple *>(A + sd->o_part),
-                                        reinterpret_cast<uint32_t *>(A + sd->o_start), A + b->o_pscr, s);
+                                        reinterpret_cast<uint32_t *>(A + sd->o_start), A + b->o_pscr, err, s);
       if (st != EO_OK) return st;
     }
   }
@@ -438,7 +442,7 @@ eo_status enqueue_batch(eo_batch *b, hipStream_t s) {
   uint32_t *pair_join = reinterpret_cast<uint32_t *>(A + b->o_pair);
   uint32_t *tile_start = reinterpret_cast<uint32_t *>(A + b->o_tiles);
   BatchTile *tdesc = reinterpret_cast<BatchTile *>(A + b->o_tdesc);
-  EO_TRY_HIP(batch_plan(dj, nj, pair_join, b->npairs, tile_start, tdesc, b->tiles_cap, A + b->o_tscr, c->d_err, s),
+  EO_TRY_HIP(batch_plan(dj, nj, pair_join, b->npairs, tile_start, tdesc, b->tiles_cap, A + b->o_tscr, err, s),
              "batch plan");
   EO_TRY_HIP(batch_probe(dj, pair_join, tile_start, b->npairs, tdesc, b->tiles_cap, head, c->props.cus, s),
              "batch probe");
@@ -446,7 +450,7 @@ eo_status enqueue_batch(eo_batch *b, hipStream_t s) {
     EO_TRY_HIP(batch_emit_unmatched(dj, nj, reinterpret_cast<const uint32_t *>(A + b->o_blob + b->o_emit),
                                     b->emit_blocks, s),
                "outer rows");
-  EO_TRY_HIP(batch_publish(cursor, nj + 1, c->d_err, b->h_counts, s), "count readback");
+  EO_TRY_HIP(batch_publish(cursor, nj + 2, b->h_counts, s), "count readback");
   return EO_OK;
 }
 
@@ -520,7 +524,7 @@ eo_status eo_table_create(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_jo
       if (e != hipSuccess) return fail(hip_fail(e, "h2d R"));
       dR = reinterpret_cast<const eo_tuple *>(A + o_in);
     }
-    st = partition_relation(c, dR, nR, hp, reinterpret_cast<eo_tuple *>(A + o_tmp), t->part, t->start, A + o_scr, s);
+    st = partition_relation(c, dR, nR, hp, reinterpret_cast<eo_tuple *>(A + o_tmp), t->part, t->start, A + o_scr, c->d_err, s);
     if (st != EO_OK) return fail(st);
   }
   e = hipStreamSynchronize(s);
@@ -754,15 +758,10 @@ eo_status eo_batch_wait(eo_batch *b, eo_result *res, uint32_t n) {
     EO_TRY_HIP(hipEventSynchronize(b->done), "batch wait");
     // (the error flags came with the counts; a copy of their own cost 36 us)
     const size_t nj = b->joins.size();
-    eo_status st = EO_OK;
-    if (nj == 0 || b->h_counts[nj + 1]) {
-      st = check_device_errors(c, b->stream);  // and clears them
-      if (st == EO_OK && nj) {  // cleared by another call meanwhile: this batch still failed
-        set_last_error("device error flags 0x" + std::to_string(b->h_counts[nj + 1]));
-        st = EO_EINTERNAL;
-      }
+    if (nj && b->h_counts[nj + 1]) {
+      set_last_error("device error flags 0x" + std::to_string(b->h_counts[nj + 1]));
+      return EO_EINTERNAL;
     }
-    if (st != EO_OK) return st;
     if (!(b->any_sampled && nj && (b->h_counts[nj] & kErrCapacity))) break;
     // a sampled partition was too small: its join's rows are incomplete, so
     // the whole batch runs again with exact partitions (same requests and
@@ -771,7 +770,7 @@ eo_status eo_batch_wait(eo_batch *b, eo_result *res, uint32_t n) {
     eo_join_stats *stats = b->stats;
     eo_join_opts ro = so;
     ro.stats = stats;
-    st = submit_batch(b, b->reqs.data(), n, b->has_opts || stats ? &ro : nullptr, true);
+    const eo_status st = submit_batch(b, b->reqs.data(), n, b->has_opts || stats ? &ro : nullptr, true);
     if (st != EO_OK) return st;
     redone = true;
   }

@@ -323,10 +323,9 @@ __global__ void k_bplan(const BatchJoin *__restrict__ joins, uint32_t *__restric
 }
 
 // Pinned host memory: visible once the batch's event is.
-__global__ void k_bpublish(const uint64_t *__restrict__ words, uint32_t n, const uint32_t *__restrict__ err,
-                           uint64_t *__restrict__ host) {
+__global__ void k_bpublish(const uint64_t *__restrict__ words, uint32_t n, uint64_t *__restrict__ host) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= n) host[i] = i < n ? words[i] : (uint64_t)*err;
+  if (i < n) host[i] = words[i];
 }
 
 // Descriptor of probe tile t of pair q (tile_start[q] <= t < tile_start[q + 1]):
@@ -550,8 +549,8 @@ hipError_t batch_emit_unmatched(const BatchJoin *joins, uint32_t njoins, const u
   return hipGetLastError();
 }
 
-hipError_t batch_publish(const uint64_t *words, uint32_t n, const uint32_t *err, uint64_t *host, hipStream_t stream) {
-  hipLaunchKernelGGL(k_bpublish, dim3(n / 256 + 1), dim3(256), 0, stream, words, n, err, host);
+hipError_t batch_publish(const uint64_t *words, uint32_t n, uint64_t *host, hipStream_t stream) {
+  hipLaunchKernelGGL(k_bpublish, dim3(n / 256 + 1), dim3(256), 0, stream, words, n, host);
   return hipGetLastError();
 }
 

@@ -385,9 +385,8 @@ hipError_t batch_plan(const BatchJoin *joins, uint32_t njoins, uint32_t *pair_jo
 // join's unmatched_blocks(nS), emit_start[njoins] the grid.
 hipError_t batch_emit_unmatched(const BatchJoin *joins, uint32_t njoins, const uint32_t *emit_start,
                                 uint32_t blocks, hipStream_t stream);
-// The per-join counts, the capacity flag and the context's error flags to the
-// pinned host words [0, n) and n.
-hipError_t batch_publish(const uint64_t *words, uint32_t n, const uint32_t *err, uint64_t *host, hipStream_t stream);
+// The per-join counts, the capacity flag and the error flags to pinned host words.
+hipError_t batch_publish(const uint64_t *words, uint32_t n, uint64_t *host, hipStream_t stream);
 // *queue_head must be zero on entry; grid = one workgroup per CU.  Tiles
 // below tiles_cap read their descriptor; later ones resolve their pair by
 // search.

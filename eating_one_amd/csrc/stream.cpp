@@ -179,7 +179,7 @@ struct Streamer {
     if (hash) {
       if (outer) EO_TRY_HIP(fill_u32(matched, 0u, matched_words(n), cs), "match bitmap reset");
       if (hp.passes) {
-        eo_status s = partition_relation(c, dS[b], n, hp, tmp, sp, s_start, pscr, cs);
+        eo_status s = partition_relation(c, dS[b], n, hp, tmp, sp, s_start, pscr, c->d_err, cs);
         if (s != EO_OK) return s;
         probe_side = sp;
       } else {
@@ -378,7 +378,7 @@ extern "C" eo_status eo_stream_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, c
     EO_TRY_HIP(hipStreamWaitEvent(x.cs, x.ev.up[0], 0), "wait");
     if (x.hash) {
       if (parted) {
-        s = partition_relation(c, x.dR, nr, x.hp, x.tmp, x.rp, x.r_start, x.pscr, x.cs);
+        s = partition_relation(c, x.dR, nr, x.hp, x.tmp, x.rp, x.r_start, x.pscr, c->d_err, x.cs);
         if (s != EO_OK) return s;
       } else {
         EO_TRY_HIP(fill_u32(x.r_start, 0u, 1, x.cs), "fill");

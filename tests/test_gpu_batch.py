@@ -446,3 +446,36 @@ def test_relations_of_different_bits_partition_together(ctx):
         for k, (_, n, status) in enumerate(b.run(reqs)):
             assert status == 0 and n == len(want[k])
             assert same_multiset(keep[k][2].to_host(np.int32, (n, 2)), want[k])
+
+
+def test_batches_in_flight_beside_a_join_that_is_redone(ctx):
+    """A join whose sample proves too small raises the context's flags until it is redone; batches
+    in flight meanwhile keep flags of their own and finish with their results."""
+    from test_gpu_sampled import _sampled_lines
+
+    rng = np.random.default_rng(4)
+    n = 1 << 20
+    keys = np.full(n, 5)
+    for t in range(n // 16384):
+        for j in range(64):
+            b = t * 16384 + _sampled_lines(t, j) * 16
+            keys[b:b + 16] = rng.integers(0, 1 << 20, 16)
+    S = DeviceArray.from_host(ctx, np.stack([keys, np.arange(n)], 1).astype(np.int32))
+    R = DeviceArray.from_host(ctx, np.stack([rng.permutation(200_000), np.arange(200_000)], 1).astype(np.int32))
+    stats = eo.JoinStats()
+    alone, _ = ctx.hash_join_device(R, 200_000, S, n, None, 0, radix_bits=6, passes=1, stats=stats)
+    assert stats.sampled == 2
+    m = 1 << 23
+    bR, bS = DeviceArray(ctx, 8 << 16), DeviceArray(ctx, 8 * m)
+    ctx.gen_build(bR, 1 << 16, seed=1)
+    ctx.gen_probe(bS, m, 1 << 16, 0.5, seed=2)
+    sizes = [m * k // 64 for k in range(1, 65)]  # batches that end at any time of the join
+    want = [ctx.hash_join_device(bR, 1 << 16, bS, k, None, 0)[0] for k in sizes]
+    batches = [ctx.batch() for _ in range(3)]
+    for i in range(2, len(sizes)):
+        for k, b in enumerate(batches):
+            b.submit([eo.request(R=bR, nR=1 << 16, S=bS, nS=sizes[i - k])])
+        assert ctx.hash_join_device(R, 200_000, S, n, None, 0, radix_bits=6, passes=1)[0] == alone
+        assert [b.wait()[0][1] for b in batches] == want[i - 2:i + 1][::-1]
+    for b in batches:
+        b.free()
