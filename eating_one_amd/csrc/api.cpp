@@ -30,7 +30,7 @@ hipError_t Arena::reserve(size_t bytes) {
   release();
   size_t want = std::max<size_t>(bytes, (size_t)64 << 20);
   want = (want + (1u << 21) - 1) & ~(size_t)((1u << 21) - 1);
-  hipError_t e = hipMalloc((void **)&base, want);
+  hipError_t e = dev_malloc(spare, (void **)&base, want);
   if (e != hipSuccess) {
     base = nullptr;
     cap = 0;
@@ -232,6 +232,7 @@ eo_status eo_ctx_create(eo_ctx **out, int device, const eo_ctx_opts *opts) {
   if (device < 0 || device >= ndev) return EO_EINVAL;
   DeviceGuard g(device);
   eo_ctx *c = new eo_ctx();
+  c->arena.spare = &c->index_block;
   c->device = device;
   hipDeviceProp_t pr;
   if (hipGetDeviceProperties(&pr, device) != hipSuccess) {
@@ -326,7 +327,7 @@ eo_status eo_dev_alloc(eo_ctx *c, uint64_t bytes, void **dptr) {
   if (!c || !dptr) return EO_EINVAL;
   DeviceGuard g(c->device);
   *dptr = nullptr;
-  EO_TRY_HIP(hipMalloc(dptr, bytes ? bytes : 1), "eo_dev_alloc");
+  EO_TRY_HIP(dev_malloc(&c->index_block, dptr, bytes ? bytes : 1), "eo_dev_alloc");
   return EO_OK;
 }
 
@@ -795,7 +796,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     // count, the match count and the device error flags together.
     uint64_t cap_dev = out ? out_cap : 0;
     if (host && out && out_cap) {
-      EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
+      EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
     uint32_t *ow = outer ? (uint32_t *)(A + o_bits) : nullptr;
@@ -904,7 +905,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     Layout L2;
     const size_t o_cnt = L2.add(n_tiles * sizeof(uint64_t));
     const size_t o_cscr = L2.add(scan_scratch_bytes_u64(n_tiles));
-    EO_TRY_HIP(hipMallocAsync((void **)&side, L2.total, s), "tile count buffer");
+    EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&side, L2.total, s), "tile count buffer");
     tile_cnt = (uint64_t *)(side + o_cnt);
     cnt_scr = side + o_cscr;
   }
@@ -924,7 +925,7 @@ eo_status hash_join_impl(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tup
     return EO_ECAPACITY;
   }
   if (host && total) {
-    hipError_t e = hipMallocAsync((void **)&dout, total * row, s);
+    hipError_t e = dev_malloc_async(&c->index_block, (void **)&dout, total * row, s);
     if (e != hipSuccess) {
       free_side();
       return hip_fail(e, "output staging");
@@ -1021,7 +1022,7 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
     const uint64_t cap_dev = out ? out_cap : 0;
     bool staged = false;
     if (host && out && out_cap) {
-      EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
+      EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
     // every R block against every S block, the inner block looked up in an LDS
@@ -1072,7 +1073,7 @@ eo_status eo_nlj_join(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_tuple 
   if (total > out_cap) return EO_ECAPACITY;
   if (total) {
     eo_pair *dout = out;
-    if (host) EO_TRY_HIP(hipMallocAsync((void **)&dout, total * row, s), "output staging");
+    if (host) EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, total * row, s), "output staging");
     hipError_t e = inner ? nlj_write(np, dR, dS, cnt, dout, total, wide, s) : hipSuccess;
     if (e == hipSuccess && outer) e = emit_unmatched_at(dS, nS, bits, ub, inner, dout, total, wide, s);
     clk.mark();
@@ -1124,7 +1125,7 @@ eo_status eo_nlj_dist_join(eo_ctx *c, const eo_point3 *R, uint64_t nR, const eo_
   eo_pair *dout = out;
   bool staged = false;
   if (host && out && out_cap) {
-    EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * sizeof(eo_pair), s), "output staging");
+    EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, out_cap * sizeof(eo_pair), s), "output staging");
     staged = true;
   }
   if ((st = begin_results(c, s)) != EO_OK) {

@@ -491,7 +491,7 @@ eo_status eo_table_create(eo_ctx *c, const eo_tuple *R, uint64_t nR, const eo_jo
   const size_t o_part = T.add(part_bytes(nR));
   const size_t o_start = T.add((P + 1) * sizeof(uint32_t));
   t->bytes = T.total;
-  hipError_t e = hipMalloc(&t->mem, std::max<size_t>(T.total, 256));
+  hipError_t e = dev_malloc(&c->index_block, &t->mem, std::max<size_t>(T.total, 256));
   if (e != hipSuccess) {
     delete t;
     return hip_fail(e, "table allocation");
@@ -556,6 +556,7 @@ eo_status eo_batch_create(eo_ctx *c, eo_batch **out) {
   DeviceGuard g(c->device);
   eo_batch *b = new eo_batch();
   b->ctx = c;
+  b->arena.spare = &c->index_block;
   hipError_t e = hipStreamCreateWithFlags(&b->own_stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreate(&b->t0);

@@ -24,8 +24,7 @@ struct eo_index {
   eo_tuple *ent = nullptr;
   uint32_t *off = nullptr;  // hash: bucket offsets; sorted: the directory
   void *model = nullptr;
-  uint64_t bytes = 0;
-  size_t mem_bytes = 0;  // of mem: bytes, or more in a block kept from another index
+  uint64_t bytes = 0;  // of mem (in a block kept from another index: the block's)
   double build_ms = 0.0;
   int32_t max_err = 0;
   double mean_err = 0.0;
@@ -51,20 +50,18 @@ eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
     std::lock_guard<std::mutex> lk(k.mu);
     if (k.mem && k.bytes >= L.total && k.bytes / 2 <= L.total) {  // (a small index takes no large block)
       ix->mem = k.mem;
-      ix->mem_bytes = k.bytes;
+      ix->bytes = k.bytes;
       k.mem = nullptr;
     }
   }
   if (!ix->mem) {
-    hipError_t e = hipMalloc((void **)&ix->mem, L.total);
-    if (e == hipErrorOutOfMemory && k.release()) e = hipMalloc((void **)&ix->mem, L.total);
+    const hipError_t e = dev_malloc(&k, (void **)&ix->mem, L.total);
     if (e != hipSuccess) {
       ix->mem = nullptr;
       return hip_fail(e, "index allocation");
     }
-    ix->mem_bytes = L.total;
+    ix->bytes = L.total;
   }
-  ix->bytes = L.total;
   ix->ent = (eo_tuple *)(ix->mem + o_ent);
   ix->off = (uint32_t *)(ix->mem + o_off);
   if (model) ix->model = ix->mem + o_model;
@@ -74,14 +71,14 @@ eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
 void free_index(eo_index *ix) {
   if (!ix) return;
   char *mem = ix->mem;
-  if (mem && ix->mem_bytes <= kIndexKeepBytes) {
+  if (mem && ix->bytes <= kIndexKeepBytes) {
     // the last block stays with the context, once no stream uses it any more
     // (hipFree waits for that too)
     KeptBlock &k = ix->ctx->index_block;
     if (hipDeviceSynchronize() == hipSuccess) {
       std::lock_guard<std::mutex> lk(k.mu);
       std::swap(mem, k.mem);
-      k.bytes = ix->mem_bytes;
+      k.bytes = ix->bytes;
     }
   }
   if (mem) (void)hipFree(mem);
@@ -373,7 +370,7 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
     eo_pair *dout = out;
     bool staged = false;
     if (host && out && out_cap) {
-      EO_TRY_HIP(hipMallocAsync((void **)&dout, out_cap * row, s), "output staging");
+      EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, out_cap * row, s), "output staging");
       staged = true;
     }
     hipError_t e = hipSuccess;
@@ -421,7 +418,7 @@ eo_status eo_index_join(eo_ctx *c, const eo_index *ix, const eo_tuple *S, uint64
   if (total > out_cap) return EO_ECAPACITY;
   if (total) {
     eo_pair *dout = out;
-    if (host) EO_TRY_HIP(hipMallocAsync((void **)&dout, total * row, s), "output staging");
+    if (host) EO_TRY_HIP(dev_malloc_async(&c->index_block, (void **)&dout, total * row, s), "output staging");
     hipError_t e = index_probe(kind, true, ix->n, ix->log2nb, ix->ent, ix->off, ix->model, dS, nS, cnt,
                                nullptr, dout, total, nullptr, wide, outer, c->props.cus, s);
     clk.mark();

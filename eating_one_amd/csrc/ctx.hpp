@@ -17,10 +17,41 @@ namespace eo {
 
 void set_last_error(const std::string &msg);
 
+// One freed device block kept for the next allocation of its size.
+struct KeptBlock {
+  std::mutex mu;
+  char *mem = nullptr;
+  size_t bytes = 0;
+  bool release() {  // gives it back; whether there was one
+    std::lock_guard<std::mutex> lk(mu);
+    if (!mem) return false;
+    (void)hipFree(mem);
+    mem = nullptr;
+    return true;
+  }
+};
+
+// alloc(), and where memory has run out again once the kept block is given
+// back.  Every device allocation of a context goes through it.
+template <typename Fn>
+hipError_t alloc_device(KeptBlock *spare, Fn &&alloc) {
+  const hipError_t e = alloc();
+  if (e != hipErrorOutOfMemory || !spare || !spare->release()) return e;
+  (void)hipGetLastError();
+  return alloc();
+}
+inline hipError_t dev_malloc(KeptBlock *spare, void **p, size_t bytes) {
+  return alloc_device(spare, [&] { return hipMalloc(p, bytes); });
+}
+inline hipError_t dev_malloc_async(KeptBlock *spare, void **p, size_t bytes, hipStream_t s) {
+  return alloc_device(spare, [&] { return hipMallocAsync(p, bytes, s); });
+}
+
 // Bump allocator over one device buffer that only grows between calls.
 struct Arena {
   char *base = nullptr;
   size_t cap = 0;
+  KeptBlock *spare = nullptr;  // the context's, for when memory runs out
   hipError_t reserve(size_t bytes);  // may free and reallocate (caller has synchronised)
   void release();
 };
@@ -58,22 +89,6 @@ struct DeviceProps {
   size_t lds_per_wg = 0, hbm = 0, l2 = 0;
 };
 
-}  // namespace eo
-
-namespace eo {
-// One freed device block kept for the next allocation of its size.
-struct KeptBlock {
-  std::mutex mu;
-  char *mem = nullptr;
-  size_t bytes = 0;
-  bool release() {  // gives it back; whether there was one
-    std::lock_guard<std::mutex> lk(mu);
-    if (!mem) return false;
-    (void)hipFree(mem);
-    mem = nullptr;
-    return true;
-  }
-};
 }  // namespace eo
 
 struct eo_ctx {

@@ -126,7 +126,7 @@ struct Streamer {
         (void)hipFree(d);
         d = nullptr;
       }
-    for (eo_pair *&d : dOut) EO_TRY_HIP(hipMalloc((void **)&d, std::max<uint64_t>(rows, 1) * row), "output staging");
+    for (eo_pair *&d : dOut) EO_TRY_HIP(dev_malloc(&c->index_block, (void **)&d, std::max<uint64_t>(rows, 1) * row), "output staging");
     if (!out_pinned && out) {
       const size_t half = (std::max<uint64_t>(rows, 1) * row + 4095) & ~(size_t)4095;
       hout_buf.release();

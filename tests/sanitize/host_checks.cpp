@@ -54,6 +54,23 @@ uint64_t oracle_sidx_join_mt(const otuple *R, uint64_t nR, const otuple *S, uint
                              uint64_t cap);
 }
 
+// The device allocator, played: a card of g_free bytes.
+static size_t g_free = 0;
+static int g_frees = 0;
+extern "C" hipError_t hipMalloc(void **p, size_t bytes) {
+  if (bytes > g_free) return hipErrorOutOfMemory;
+  g_free -= bytes;
+  *p = &g_free;
+  return hipSuccess;
+}
+extern "C" hipError_t hipMallocAsync(void **p, size_t bytes, hipStream_t) { return hipMalloc(p, bytes); }
+extern "C" hipError_t hipFree(void *) {
+  g_free += 100;
+  ++g_frees;
+  return hipSuccess;
+}
+extern "C" hipError_t hipGetLastError() { return hipSuccess; }
+
 static int g_checks = 0;
 #define CHECK(cond)                                                            \
   do {                                                                         \
@@ -560,6 +577,27 @@ static void check_serve_queue() {
   }
 }
 
+// A kept block goes back when an allocation of its context would fail without it.
+static void check_kept_block() {
+  for (bool async : {false, true}) {
+    eo::KeptBlock k;
+    void *p = nullptr;
+    auto alloc = [&](size_t bytes) {
+      return async ? eo::dev_malloc_async(&k, &p, bytes, nullptr) : eo::dev_malloc(&k, &p, bytes);
+    };
+    g_free = 50;
+    g_frees = 0;
+    CHECK(alloc(60) == hipErrorOutOfMemory && g_frees == 0);  // none kept
+    k.mem = (char *)&k;
+    k.bytes = 100;
+    CHECK(alloc(10) == hipSuccess && k.mem && g_frees == 0);  // there is room beside it
+    CHECK(alloc(120) == hipSuccess && !k.mem && g_frees == 1);
+    CHECK(alloc(120) == hipErrorOutOfMemory && g_frees == 1);
+    k.mem = (char *)&k;
+    CHECK(alloc(1000) == hipErrorOutOfMemory && !k.mem && g_frees == 2);  // not enough all the same
+  }
+}
+
 int main() {
   check_oracle();
   check_ref_files();
@@ -568,6 +606,7 @@ int main() {
   check_time_model();
   check_tune_candidates();
   check_serve_queue();
+  check_kept_block();
   std::printf("host checks ok: %d checks\n", g_checks);
   return 0;
 }

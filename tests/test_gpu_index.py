@@ -211,3 +211,14 @@ def test_index_memory_kept_for_the_next_build(ctx):
             assert same_multiset(other.join(S2), want)
     for other, _, _ in live:
         other.free()
+
+
+def test_index_info_counts_the_block_it_holds(ctx):
+    """An index in a larger block kept from a freed one reports that block."""
+    big = np.stack([np.arange(60_000), np.arange(60_000)], 1).astype(np.int32)
+    ix = ctx.sidx_build(big)
+    held = ix.info()["bytes"]
+    ix.free()
+    ix = ctx.sidx_build(big[:40_000])
+    assert ix.info()["bytes"] == held
+    ix.free()

@@ -5,6 +5,7 @@ request loop's admission policy (deadlines, cancellation, budget), built with
 g++ from the sources and run as one program (tests/sanitize/host_checks.cpp).
 No GPU and no HIP runtime are involved."""
 import os
+import re
 import shutil
 import subprocess
 
@@ -46,3 +47,15 @@ def test_host_code_under_asan_ubsan(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
     assert "host checks ok" in r.stdout
     assert "runtime error" not in r.stderr and "AddressSanitizer" not in r.stderr
+
+
+def test_device_allocations_give_the_kept_block_back():
+    """Every device allocation of a context is dev_malloc's or dev_malloc_async's (ctx.hpp), which
+    release its kept index block when memory runs out; the context's own first one has none yet."""
+    raw = []
+    for name in sorted(os.listdir(CSRC)):
+        with open(os.path.join(CSRC, name)) as f:
+            raw += [(name, line.strip()) for line in f if re.search(r"\bhipMalloc(Async)?\(", line)]
+    assert [line for name, line in raw if name != "ctx.hpp"] == \
+        ["if (e == hipSuccess) e = hipMalloc((void **)&c->d_err, small_bytes);"]
+    assert len([name for name, _ in raw if name == "ctx.hpp"]) == 2
