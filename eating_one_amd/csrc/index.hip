@@ -36,11 +36,10 @@
 //         largest under- / over-prediction of the first position of any key
 //         routed to the leaf, measured with this same inference code.
 // A learned lookup is the lower bound within [pred - err_hi, pred + err_lo]
-// (clamped): every key present in R lies in its window, so results equal the
-// plain search exactly; absent keys find no equal key in any window.  The
-// position within the window is the directory's lower bound clamped to it, and
-// a learned index's join needs no window at all (its rows are those of the
-// plain search).
+// (clamped), found by searching that window alone: every key present in R lies
+// in its window, so results equal the plain search exactly; absent keys find no
+// equal key in any window.  A learned index's join searches the directory like
+// any sorted index's: the rows are the same, and it writes them at once.
 //
 // The deterministic order is count -> scan -> write: per tile of 2048 S tuples
 // a count, a u64 scan of those, then the write kernel re-probes and writes at
@@ -404,9 +403,53 @@ __device__ __forceinline__ void hash_count(const IndexView &ix, uint32_t key, ui
   }
 }
 
-// KIND 0: hash; 1: sorted; 2: sorted, positions of the learned model's windows
-// (lookups only).  U probes per thread and tile; workgroups walk the tiles, so
-// the top of the directory is read into LDS once per workgroup.
+// Lookups by the learned model: the lower bound of each key within its leaf's
+// window, searched there alone, so that a lookup shows what the model is worth.
+// First the window's nodes by level 1 of the directory, then the node, one line
+// of each for most probes.  Bound by the latency of those dependent loads and
+// by the lines of entries that miss L2: one probe per thread, a workgroup per
+// 256 probes (2^27 lookups of 2^26 lognormal keys 4.85 ms, the directory search
+// 5.09; the window's keys in an array of their own 4.74; two and four probes
+// per thread step by step 5.4 and 7.7, workgroups that walk the probes 5.1).
+constexpr int kLookNT = 256;
+__global__ __launch_bounds__(kLookNT) void k_learned_lookup(IndexView ix, const uint2 *__restrict__ S, uint64_t nS,
+                                                            uint64_t *__restrict__ pos) {
+  __shared__ int32_t kk[kKnots + 1];
+  __shared__ float kp[kKnots + 1];
+  for (int i = threadIdx.x; i <= kKnots; i += kLookNT) {
+    kk[i] = ix.knot_key[i];
+    kp[i] = ix.knot_pos[i];
+  }
+  __syncthreads();
+  const uint32_t *const dir = ix.off + ix.dir.off[0];
+  for (uint64_t i = (uint64_t)blockIdx.x * kLookNT + threadIdx.x; i < nS; i += (uint64_t)gridDim.x * kLookNT) {
+    const int32_t key = (int32_t)S[i].x;
+    const LeafModel m = ix.leaves[leaf_of(root_pred(kk, kp, key), ix.n)];
+    const int64_t pred = leaf_pred(m, key), n = (int64_t)ix.n;
+    const uint32_t lo = (uint32_t)min<int64_t>(max<int64_t>(0, pred - m.err_hi), n);
+    const uint32_t hi = (uint32_t)max<int64_t>(lo, min<int64_t>(n, pred + m.err_lo + 1));  // (none: an empty window)
+    // the first node of the window whose largest key is not below the probe's
+    uint32_t a = lo / kEntNode, b = hi > lo ? (hi - 1) / kEntNode + 1 : a;
+    while (a < b) {
+      const uint32_t mid = (a + b) / 2;
+      if ((int32_t)dir[mid] < key) a = mid + 1;
+      else b = mid;
+    }
+    // and its first such entry within the window
+    const uint64_t first = (uint64_t)a * kEntNode;
+    b = (uint32_t)min<uint64_t>(hi, first + kEntNode);
+    a = (uint32_t)min<uint64_t>(max<uint64_t>(lo, first), hi);
+    while (a < b) {
+      const uint32_t mid = (a + b) / 2;
+      if ((int32_t)ix.ent[mid].x < key) a = mid + 1;
+      else b = mid;
+    }
+    pos[i] = a;
+  }
+}
+
+// KIND 0: hash; 1: sorted.  U probes per thread and tile; workgroups walk the
+// tiles, so the top of the directory is read into LDS once per workgroup.
 template <int KIND, bool WRITE, int U, int NT>
 __global__ __launch_bounds__(NT) void k_index_probe(IndexView ix, const uint2 *__restrict__ S, uint64_t nS,
                                                         uint32_t tiles, uint64_t *__restrict__ tile_cnt,
@@ -414,20 +457,12 @@ __global__ __launch_bounds__(NT) void k_index_probe(IndexView ix, const uint2 *_
                                                         uint64_t *__restrict__ lb_out, int wide, int outer) {
   constexpr int NW = NT / kWave;
   __shared__ int32_t top[KIND != 0 ? kDirTop : 1];
-  __shared__ int32_t kk[KIND == 2 ? kKnots + 1 : 1];
-  __shared__ float kp[KIND == 2 ? kKnots + 1 : 1];
   __shared__ uint64_t red[NT / kWave + 1];
   __shared__ uint64_t wtot[U * NW];
   __shared__ uint64_t base_sh;
   if (KIND != 0) {
     const int l = ix.dir.levels - 1;
     for (uint32_t i = threadIdx.x; i < ix.dir.cnt[l]; i += NT) top[i] = (int32_t)ix.off[ix.dir.off[l] + i];
-  }
-  if (KIND == 2) {
-    for (int i = threadIdx.x; i <= kKnots; i += NT) {
-      kk[i] = ix.knot_key[i];
-      kp[i] = ix.knot_pos[i];
-    }
   }
   if (KIND != 0) __syncthreads();
   for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {
@@ -458,20 +493,7 @@ __global__ __launch_bounds__(NT) void k_index_probe(IndexView ix, const uint2 *_
       if constexpr (KIND == 0) hash_count(ix, s[u].x, b[u], e[u], m[u], fp[u]);
       else sorted_locate(ix, top, (int32_t)s[u].x, b[u], m[u], fp[u]);
       if (i >= nS) m[u] = 0;
-      if (lb_out && i < nS) {
-        uint64_t pos = b[u];
-        // (a present key is in its leaf's window, which was fitted over it: the
-        // model is read for absent keys only; 2^27 lookups of 2^26 keys 5.13 -> 4.71 ms)
-        if (KIND == 2 && m[u] == 0) {
-          const LeafModel mo = ix.leaves[leaf_of(root_pred(kk, kp, (int32_t)s[u].x), ix.n)];
-          const int64_t pred = leaf_pred(mo, (int32_t)s[u].x);
-          const int64_t lo = max<int64_t>(0, pred - mo.err_hi);
-          const int64_t hi = min<int64_t>((int64_t)ix.n, pred + mo.err_lo + 1);
-          pos = lo < hi ? (uint64_t)min<int64_t>(max<int64_t>((int64_t)pos, lo), hi)
-                        : (uint64_t)min<int64_t>(lo, (int64_t)ix.n);
-        }
-        lb_out[i] = pos;
-      }
+      if (lb_out && i < nS) lb_out[i] = b[u];
       if (outer && m[u] == 0 && i < nS) nul |= 1u << u;  // left outer join: one null-padded row
       total += (uint64_t)m[u] + ((nul >> u) & 1u);
     }
@@ -659,19 +681,25 @@ hipError_t index_probe(int kind, bool write, uint64_t n, int log2nb, const eo_tu
   ix.ent = reinterpret_cast<const uint2 *>(ent);
   ix.off = off;
   if (kind != 0) ix.dir = dir_geo(n);
-  if (kind == 2 && !lb_out) kind = 1;  // the rows are the plain search's
+  if (kind == 2 && (!lb_out || n == 0)) kind = 1;  // the rows are the plain search's
   if (kind == 2) {
+    if (write || tile_cnt || cursor) return hipErrorInvalidValue;  // lookups only
+    if (nS == 0) return hipSuccess;
     const char *mp = (const char *)model;
     ix.knot_key = (const int32_t *)mp;
     ix.knot_pos = (const float *)(mp + (kKnots + 1) * sizeof(int32_t));
     ix.leaves = (const LeafModel *)(mp + ((kKnots + 1) * (sizeof(int32_t) + sizeof(float)) + 63) / 64 * 64);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((nS + kLookNT - 1) / kLookNT, 1u << 20);
+    EO_TIMED("index_lookup", stream,
+             hipLaunchKernelGGL(k_learned_lookup, dim3(grid), dim3(kLookNT), 0, stream, ix,
+                                reinterpret_cast<const uint2 *>(S), nS, lb_out));
+    return hipGetLastError();
   }
 #define EO_PROBE(K, W) \
   launch_probe<K, W>(ix, S, nS, tile_cnt, cursor, out, out_cap, lb_out, wide, outer, cus, stream)
   switch (kind) {
     case 0: return write ? EO_PROBE(0, true) : EO_PROBE(0, false);
     case 1: return write ? EO_PROBE(1, true) : EO_PROBE(1, false);
-    case 2: return write ? hipErrorInvalidValue : EO_PROBE(2, false);
     default: return hipErrorInvalidValue;
   }
 #undef EO_PROBE

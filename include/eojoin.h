@@ -371,7 +371,8 @@ typedef enum eo_index_kind { EO_INDEX_HASH = 0, EO_INDEX_SORTED = 1 } eo_index_k
 /* Lookup methods of eo_index_lookup. */
 enum { EO_LOOKUP_DEFAULT = 0, EO_LOOKUP_BINARY = 1, EO_LOOKUP_LEARNED = 2 };
 
-/* eo_index_join on a learned sorted index: use plain binary search instead. */
+/* eo_index_join on a learned sorted index: use plain search.  Joins always do
+ * (the rows are the same); kept for callers that set it. */
 #define EO_F_BINARY_SEARCH 4
 
 typedef struct eo_index_info {
@@ -401,15 +402,16 @@ eo_status eo_sidx_build(eo_ctx *ctx, const eo_tuple *R, uint64_t nR, int learned
 /* Index join of S against a resident index: replaces join() of
  * joins/innerJoin_gpu/main_street/inner-idx-bnlj.cc:183-673 (hash) and
  * joins/innerJoin_gpu/sort_index/main_street/inner-idx-bnlj.cc:219-658
- * (sorted: binary search, or the learned model unless EO_F_BINARY_SEARCH).
+ * (sorted, learned or not: a search by the index's directory of largest keys).
  * Same sizing and error conventions as eo_hash_join. */
 eo_status eo_index_join(eo_ctx *ctx, const eo_index *index, const eo_tuple *S,
                         uint64_t nS, eo_pair *out, uint64_t out_cap,
                         uint64_t *n_out, const eo_join_opts *opts);
 
 /* Per probe, the index position its search starts from: the lower bound of
- * S[i].key (sorted index; method BINARY or LEARNED — equal for every key
- * present in R) or the bucket start (hash index).  pos: nS uint64, host or
+ * S[i].key (sorted index; method BINARY: in the whole index, LEARNED, the
+ * default of a learned index: in the window that the model predicts — equal for
+ * every key present in R) or the bucket start (hash index).  pos: nS uint64, host or
  * device per opts->where.  Used to check the learned model against binary
  * search probe by probe. */
 eo_status eo_index_lookup(eo_ctx *ctx, const eo_index *index, const eo_tuple *S,

@@ -4,6 +4,8 @@ Oracles: joins/CPU_JOIN/inner_cpu (hash index) and joins/CPU_JOIN/sortIndex_cpu
 (sorted index) restated in oracle/cpu_join.c; the learned model is checked probe
 by probe against the plain binary search of the same index.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -221,4 +223,31 @@ def test_index_info_counts_the_block_it_holds(ctx):
     ix.free()
     ix = ctx.sidx_build(big[:40_000])
     assert ix.info()["bytes"] == held
+    ix.free()
+
+
+def test_learned_lookups_come_from_the_model(ctx):
+    """A lookup that the model predicts wrongly is answered wrongly: with every leaf's intercept
+    moved, present keys are no longer found where the plain search finds them."""
+    n = 100_000
+    rng = np.random.default_rng(5)
+    keys = np.unique(rng.integers(0, 2 ** 31 - 1, n)).astype(np.int32)
+    R = np.stack([keys, np.arange(len(keys))], 1).astype(np.int32)
+    ix = ctx.sidx_build(R, learned=True)
+    binary = ix.lookup(R, _abi.EO_LOOKUP_BINARY)
+    assert np.array_equal(binary, np.arange(len(keys), dtype=np.uint64))
+    assert np.array_equal(ix.lookup(R, _abi.EO_LOOKUP_LEARNED), binary)
+    # eo_index (api_index.cpp): ctx, kind, learned, n, log2nb, mem, ent, off, model
+    word = lambda at: ctypes.c_uint64.from_address(ix.handle + at).value  # noqa: E731
+    assert word(8) == _abi.EO_INDEX_SORTED | 1 << 32 and word(16) == len(keys)
+    leaves = word(56) + (257 * 8 + 63) // 64 * 64  # behind 257 knots
+    leaf = np.empty((4096, 8), dtype=np.int32)  # a, b, k0, pad, err_lo, err_hi, first, last
+    assert ctx.lib.eo_copy_d2h(ctx.handle, leaf.ctypes.data, leaves, leaf.nbytes) == _abi.EO_OK
+    assert leaf[:, 7].max() == len(keys) and leaf[:, 4:6].max() == ix.info()["max_err"]
+    moved = leaf.copy()
+    moved[:, 0] = (np.ascontiguousarray(leaf[:, 0]).view(np.float32) + np.float32(3 * (leaf[:, 4:6].max() + 1))).view(np.int32)
+    assert ctx.lib.eo_copy_h2d(ctx.handle, leaves, moved.ctypes.data, moved.nbytes) == _abi.EO_OK
+    wrong = ix.lookup(R, _abi.EO_LOOKUP_LEARNED)
+    assert (wrong[:-4 * leaf[:, 4:6].max() - 8] > binary[:-4 * leaf[:, 4:6].max() - 8]).all()
+    assert np.array_equal(ix.lookup(R, _abi.EO_LOOKUP_BINARY), binary)
     ix.free()
