@@ -38,6 +38,7 @@ using namespace eo;
 // most: hipMalloc and hipFree take 11 us each, a sixth of building an index of
 // 2^18 tuples and joining it.
 constexpr size_t kIndexKeepBytes = 256u << 20;
+constexpr uint64_t kExportHostEntries = 1u << 15;
 
 // Allocates the index's memory: its entries, `words` u32 and `model` bytes.
 eo_status alloc_index(eo_index *ix, uint64_t words, size_t model) {
@@ -481,12 +482,23 @@ eo_status eo_index_export(eo_ctx *c, const eo_index *ix, uint32_t *keys, uint32_
   if (!c || !ix || (ix->n && (!keys || !pays))) return EO_EINVAL;
   DeviceGuard g(c->device);
   if (!ix->n) return EO_OK;
-  // the entries are pairs: split on the device, then two copies
+  // the entries are pairs: few are split here after one copy, more on the device
+  // before two (1000 entries 17 us, 41 by the device; 32000 123 and 145; 64000
+  // are 52 by the device)
+  if (ix->n <= kExportHostEntries) {
+    std::vector<eo_tuple> t(ix->n);
+    EO_TRY_HIP(hipMemcpy(t.data(), ix->ent, ix->n * sizeof(eo_tuple), hipMemcpyDeviceToHost), "export");
+    for (uint64_t i = 0; i < ix->n; ++i) {
+      keys[i] = (uint32_t)t[i].key;
+      pays[i] = (uint32_t)t[i].payload;
+    }
+    return EO_OK;
+  }
   hipStream_t s = c->stream;
   Layout L;
   const size_t o_k = L.add(ix->n * 4), o_p = L.add(ix->n * 4);
-  EO_TRY_HIP(hipStreamSynchronize(s), "sync");
-  EO_TRY_HIP(c->arena.reserve(L.total), "arena");
+  const eo_status st = ensure_arena(c, s, L.total);
+  if (st != EO_OK) return st;
   char *A = c->arena.base;
   EO_TRY_HIP(index_split(ix->ent, ix->n, (uint32_t *)(A + o_k), (uint32_t *)(A + o_p), s), "export split");
   EO_TRY_HIP(hipMemcpyAsync(keys, A + o_k, ix->n * 4, hipMemcpyDeviceToHost, s), "export keys");

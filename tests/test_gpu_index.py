@@ -251,3 +251,15 @@ def test_learned_lookups_come_from_the_model(ctx):
     assert (wrong[:-4 * leaf[:, 4:6].max() - 8] > binary[:-4 * leaf[:, 4:6].max() - 8]).all()
     assert np.array_equal(ix.lookup(R, _abi.EO_LOOKUP_BINARY), binary)
     ix.free()
+
+
+@pytest.mark.parametrize("n", [1, 17, 1 << 15, (1 << 15) + 1, 200_003])
+def test_export_returns_the_entries(ctx, n):
+    """Few entries are split on the host, more on the device."""
+    rng = np.random.default_rng(n)
+    R = np.stack([rng.integers(-n, n, n), np.arange(n)], 1).astype(np.int32)
+    ix = ctx.sidx_build(R)
+    keys, pays = ix.export()
+    order = np.argsort(R[:, 0], kind="stable")
+    assert np.array_equal(keys, R[order, 0]) and np.array_equal(pays, order)
+    ix.free()
