@@ -263,3 +263,20 @@ def test_export_returns_the_entries(ctx, n):
     order = np.argsort(R[:, 0], kind="stable")
     assert np.array_equal(keys, R[order, 0]) and np.array_equal(pays, order)
     ix.free()
+
+
+@pytest.mark.parametrize("dups", [15, 16, 17, 33, 500])
+def test_deterministic_hash_join_of_long_buckets(ctx, dups):
+    """Buckets of many duplicates, read two entries at a time from odd and even starts."""
+    rng = np.random.default_rng(dups)
+    keys = np.concatenate([np.repeat(np.arange(0, 40, 2), dups + rng.integers(0, 2, 20)), np.arange(1001, 1040)])
+    R = np.stack([rng.permutation(keys), np.arange(len(keys))], 1).astype(np.int32)
+    S = np.stack([rng.integers(0, 60, 300), np.arange(300)], 1).astype(np.int32)
+    ix = ctx.hidx_build(R)
+    rows = ix.join(S, deterministic=True)
+    assert same_multiset(rows, brute_join(R, S))
+    outer = ix.join(S, deterministic=True, left_outer=True)
+    null = outer[:, 0] == _abi.EO_NULL_PAYLOAD
+    assert same_multiset(outer[~null], rows)
+    assert np.array_equal(outer[null, 1], np.flatnonzero(~np.isin(S[:, 0], R[:, 0])))
+    ix.free()
