@@ -155,8 +155,9 @@ __global__ __launch_bounds__(kNljNT) void k_nlj(const uint2 *__restrict__ R, uin
 // passes a filter that never rejects a match:
 //   |r|^2 - 2 r.s + |s|^2 - d2 < 0,  lowered by a bound on the filter's error
 // and only pairs that pass it evaluate the predicate, on the coordinates as
-// given.  There are two filters, chosen by a workgroup for each of its R tiles
-// by the points in it.
+// given.  There are two filters: a workgroup takes the matrix filter up to its
+// first R tile with a point outside that filter's range (none, if its S tile has
+// one) and the FP64 filter from there on.
 //
 // Matrix filter (dist_matrix).  The sum is a contraction: coordinates about a
 // common origin o (a mean of the S tile's points, subtracted in FP64) as two
@@ -171,7 +172,8 @@ __global__ __launch_bounds__(kNljNT) void k_nlj(const uint2 *__restrict__ R, uin
 // and t and the FP64 steps stay below 2^-22 (N + d2).  Together under 14.2
 // 2^-18 (N + d2); kMatSlack is 16 2^-18.  (Measured over 2^24 pairs each in
 // boxes of 4 to 100, near each other or not: 6.9 2^-18 (N + d2) at most; 0.04
-// where the coordinates are bf16 numbers.)  It is used where every N stays within 2^15 d2, so that
+// where the coordinates are bf16 numbers, which is what the unit's additions are
+// off by.)  It is used where every N stays within 2^15 d2, so that
 // the slack is 2 d2 at the corners and few pairs pass that do not match, and
 // d2 is within 2^-60 .. 2^60 (no bf16 or 32-bit word overflows, and what is
 // flushed to zero is far below the slack).

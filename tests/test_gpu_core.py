@@ -484,3 +484,28 @@ def test_hash_join_builds_on_the_smaller_side(ctx, nR, nS, key_range):
     assert status == eo._abi.EO_ECAPACITY and n == len(want)
     rows = small.to_host(np.int32, (100, 2))
     assert np.array_equal(R[rows[:, 0], 0], S[rows[:, 1], 0])
+
+
+@pytest.mark.parametrize("flip", [(1, 1, 1), (1, -1, 1)])
+def test_nlj_dist_matrix_filter_at_its_worst_words(ctx, flip):
+    """Pairs a few roundings inside the distance whose coordinates leave the most behind their two
+    bf16 words, every product on the same side: what the words miss takes 0.47 of the filter's
+    slack, and a pair is lost if the matrix unit's sums are off by the rest."""
+    # above a bf16 number of exponent 5: just under half a step left to the second word, and
+    # just under half of that word's last step behind it
+    step = 2.0 ** -2
+    low = step / 2 - 2.0 ** -12 - 2.0 ** -17
+    a, b = 33.0 + low, 32.5 + low
+    flip = np.array(flip, dtype=np.float64)
+    S = np.zeros(2048, dtype=oracle.POINT3)
+    R = np.zeros(300, dtype=oracle.POINT3)
+    S["id"], R["id"] = np.arange(2048), np.arange(300)
+    side = np.where(np.arange(2048) // 32 % 2 == 0, 1.0, -1.0)  # the sampled points' mean is zero
+    S["v"] = side[:, None] * a * flip
+    R["v"] = np.where(np.arange(300) % 2 == 0, 1.0, -1.0)[:, None] * b * flip
+    dist = np.sqrt(0.75) * (1 + 2.0 ** -50)
+    assert 3 * a * a < 2.0 ** 14 * dist * dist  # within the matrix filter's range
+    want = oracle.nlj_dist_join(R, S, dist)
+    assert len(want) == 1024 * 300
+    assert same_multiset(ctx.nlj_dist_join(R, S, dist), want)
+    assert ctx.nlj_dist_join(R, S, np.sqrt(0.75) * (1 - 2.0 ** -50), count_only=True) == 0
