@@ -258,8 +258,8 @@ __global__ __launch_bounds__(kPlanNT) void k_plan_spans(const uint32_t *r_start,
   __shared__ uint64_t red[kPlanNT / kWave + 1];
   const uint32_t p = blockIdx.x * kPlanNT + threadIdx.x;
   uint64_t n = 0;
-  if (p < P)
-    n = ((uint64_t)(r_end[p] - r_start[p]) + cap - 1) / cap * (((uint64_t)(s_end[p] - s_start[p]) + s_span - 1) / s_span);
+  if (p < P)  // (below 2^31 tuples and spans below 2^31: the quotients fit 32 bits, their product need not)
+    n = (uint64_t)((r_end[p] - r_start[p] + cap - 1) / cap) * ((s_end[p] - s_start[p] + s_span - 1) / s_span);
   if (p <= P) tiles[p] = (uint32_t)n;
   const uint64_t sum = block_sum<kPlanNT, uint64_t>(n, red);
   if (threadIdx.x == 0 && sum) atomic_add_agent(n_tiles, sum);

@@ -203,10 +203,9 @@ __global__ __launch_bounds__(kOnePlanNT) void k_one_plan(OneArgs a, uint32_t s_s
         r.end[p] = e;
         n[rel] = e - r.start[p];
       }
-      // (64 bits: a sum of 2^31 or more is refused by the probe)
-      const uint64_t spans = ((uint64_t)n[1] + s_span - 1) / s_span;
-      const uint64_t chunks = ((uint64_t)n[0] + cap - 1) / cap;
-      cnt[k] = (outer ? max(chunks, (uint64_t)1) : chunks) * spans;
+      // (products in 64 bits: a sum of 2^31 or more is refused by the probe)
+      const uint32_t spans = (n[1] + s_span - 1) / s_span, chunks = (n[0] + cap - 1) / cap;
+      cnt[k] = (uint64_t)(outer ? max(chunks, 1u) : chunks) * spans;
     }
     sum += cnt[k];
   }
