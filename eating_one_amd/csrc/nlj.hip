@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kNljNT) void k_nlj(const uint2 *__restrict__ R, uin
 // of it pass.
 //
 // 2^17 x 2^17 points: 3.69 ms with the exact predicate on every pair, 2.27 ms
-// with the FP64 filter (issue bound, 0.89 of the VALU's cycles), 0.53 ms with
+// with the FP64 filter (issue bound, 0.89 of the VALU's cycles), 0.54 ms with
 // the matrix filter: a SIMD's MFMAs (0.44 of its cycles) and VALU (0.62) do not
 // run beside each other, so the signs cost as much as the products.  (Each MFMA
 // issued before the signs of the tile before it, four tiles to a test: 0.66

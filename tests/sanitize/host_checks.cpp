@@ -5,9 +5,10 @@
 //   - the library's host-only code: the reference table / index file readers
 //     and writers (well-formed, truncated and inconsistent files), the
 //     autotuner's table file (round trip, malformed rows), the hash join
-//     planner over a sweep of sizes and overrides, and the request loop's
-//     admission policy (FIFO batches, budget, deadlines, cancellation) on
-//     synthetic clocks.
+//     planner, the time-model plans and the autotuner's candidates over sweeps
+//     of sizes and overrides, the request loop's admission policy (FIFO
+//     batches, budget, deadlines, cancellation) on synthetic clocks, and the
+//     kept index block under a played allocator.
 // Exit status 0 and "host checks ok" on success; any sanitizer report aborts.
 #include <algorithm>
 #include <cmath>
