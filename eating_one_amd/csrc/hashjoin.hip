@@ -247,9 +247,9 @@ void k_span_write(const uint2 *__restrict__ R, const uint32_t *__restrict__ r_st
   }
 }
 
-// tiles[p] of every partition (R chunks x S spans), and their 64-bit sum added to *n_tiles: a sum of
-// 2^31 or more is refused by the kernels that read it, since the 32-bit tile
-// numbers scanned from tiles[] may then have wrapped.
+// tiles[p] of every partition (R chunks x S spans), and their 64-bit sum added
+// to *n_tiles: a sum of 2^31 or more is refused by the kernels that read it,
+// since the 32-bit tile numbers scanned from tiles[] may then have wrapped.
 constexpr int kPlanNT = 256;
 __global__ __launch_bounds__(kPlanNT) void k_plan_spans(const uint32_t *r_start, const uint32_t *r_end,
                                                         const uint32_t *s_start, const uint32_t *s_end, uint32_t P,

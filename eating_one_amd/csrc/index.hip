@@ -710,7 +710,7 @@ hipError_t index_probe(int kind, bool write, uint64_t n, int log2nb, const eo_tu
     ix.knot_pos = (const float *)(mp + (kKnots + 1) * sizeof(int32_t));
     ix.leaves = (const LeafModel *)(mp + ((kKnots + 1) * (sizeof(int32_t) + sizeof(float)) + 63) / 64 * 64);
     const uint32_t grid = (uint32_t)std::min<uint64_t>((nS + kLookNT - 1) / kLookNT, 1u << 20);
-    EO_TIMED("index_lookup", stream,
+    EO_TIMED("index_probe", stream,
              hipLaunchKernelGGL(k_learned_lookup, dim3(grid), dim3(kLookNT), 0, stream, ix,
                                 reinterpret_cast<const uint2 *>(S), nS, lb_out));
     return hipGetLastError();
